@@ -37,13 +37,12 @@ static __device__ __align__(256) char scratch[SVDAG_NOALLOC_SCRATCH_BYTES];
 namespace {
 
 const char* const kKernelNames[kNumKernelIds] = {
-    "sort_histogram", "sort_count",  "sort_scan",     "sort_scatter_keys", "sort_scatter_pairs", "fill",
-    "scan_counts",    "leaf_reduce", "leaf_compact",      "table_clear",        "leaf_insert",
-    "rank_of_slot",   "level_count", "level_build",   "level_check",       "extract_count",      "level_extract",
-    "final_count",    "final_positions", "final_write", "merge_insert",      "sketch",             "level_tail",
-    "slot_list",      "query_voxels",    "vox_setup",   "vox_count",         "vox_write",
-    "trace_paths",    "resident_insert", "sort_scatter_top", "seg_count",   "seg_scatter",
-    "pair_histogram", "pair_count"};
+    "sort_histogram", "sort_count",  "sort_scan",     "sort_scatter_keys",  "fill",
+    "scan_counts",    "leaf_reduce", "leaf_compact",  "table_clear",        "leaf_insert",
+    "leaf_order",     "level_count", "level_build",   "level_check",        "extract_count",      "level_extract",
+    "final_count",    "final_positions", "final_write", "merge_insert",     "sketch",             "level_tail",
+    "query_voxels",   "vox_setup",   "vox_count",     "vox_write",
+    "trace_paths",    "resident_insert", "sort_scatter_top", "seg_count",   "seg_scatter"};
 
 // Event pairs around the launches of the kernels selected by `mask`; resolved
 // into per-kernel totals once the stream has drained.
@@ -295,12 +294,12 @@ inline uint32_t table_lg(uint64_t count, uint32_t shift)
 struct BuildLayout {
     uint64_t total = 0;
     uint64_t zero_begin = 0, zero_end = 0;
-    uint64_t counters = 0, key_sort_zero = 0, leaf_sort_zero = 0, sketch = 0;
+    uint64_t counters = 0, key_sort_zero = 0, order_zero = 0, sketch = 0, order_split = 0;
     uint64_t sort_counts = 0, tile_counts = 0, tile_offsets = 0;
     uint64_t keys_a = 0, keys_b = 0;
     uint64_t lp_code = 0, lp_mask = 0, lp_slot = 0, leaf_table = 0, leaf_rank = 0;
     uint64_t reg_code = 0, reg_mask = 0;  // leaf-reduce regions, over the later stages' buffers
-    uint64_t list_keys[2] = {}, list_slots[2] = {}, sorted_slots = 0;
+    uint64_t list_keys[2] = {}, list_slots[2] = {};
     // Levels: build outputs (codes, slots, hashes) ping-pong between
     // consecutive level builds; every hashed level keeps its own records
     // (masks, children) and table until its extract, so that all level builds
@@ -312,7 +311,7 @@ struct BuildLayout {
     uint64_t tail_codes[2] = {}, tail_ranks[2] = {}, tail_masks = 0, tail_children = 0, tail_hash = 0;
     uint64_t n = 0, leaf_bound = 0, level_bound = 0, leaf_slots = 0, level_slots = 0;
     uint32_t group_bits = 0;
-    SortPlan key_plan{}, leaf_plan{};
+    SortPlan key_plan{};
     // Plain builds of 64-bit keys may sort top digit first
     // (launch_top_digit_sort): the 32-bit bucket-local keys over keys_b, the
     // bucket starts and the segmented sort's tables over the buffers from
@@ -340,17 +339,16 @@ BuildLayout plan_build(uint64_t n, int depth, int key_bytes, uint32_t load_shift
     const uint32_t code_bits = uint32_t(3 * depth - 6);
     L.group_bits = std::min(kLeafGroupBits, code_bits);
     L.key_plan = make_sort_plan(int(6 + std::min(L.group_bits, code_bits - 1)), 3 * depth, radix_bits, sort_ipt);
-    L.leaf_plan = make_sort_plan(0, 64);
     const uint64_t stage_tiles = std::max({tiles(n, kPackTileItems), tiles(L.leaf_bound, kBuildTileItems),
-                                           tiles(L.level_slots, kExtractTileItems),
-                                           tiles(L.leaf_slots, kListTileItems), uint64_t(1)});
+                                           tiles(L.level_slots, kExtractTileItems), uint64_t(1)});
     Carver c;
     L.zero_begin = c.off;
     L.counters = c.take(sizeof(BuildCounters));
     L.key_sort_zero = c.take(4 * sort_zero_words(L.key_plan));
-    L.leaf_sort_zero = c.take(4 * sort_zero_words(L.leaf_plan));
+    L.order_zero = c.take(4 * kOrderZeroWords);
     L.sketch = c.take(4 * kSketchRegs);
     L.zero_end = c.off;
+    L.order_split = c.take(8 * kOrderMaxBuckets);
     L.sort_counts = c.take(4 * sort_count_words(n));
     L.tile_counts = c.take(4 * stage_tiles);
     L.tile_offsets = c.take(8 * stage_tiles);
@@ -366,7 +364,6 @@ BuildLayout plan_build(uint64_t n, int depth, int key_bytes, uint32_t load_shift
         L.list_keys[i] = c.take(8 * L.leaf_bound);
         L.list_slots[i] = c.take(4 * L.leaf_bound);
     }
-    L.sorted_slots = c.take(4 * L.leaf_bound);
     for (int i = 0; i < 2; ++i) {
         L.codes[i] = c.take(8 * L.level_bound);
         L.slots[i] = c.take(4 * L.level_bound);
@@ -810,8 +807,8 @@ int build(svdag_context* ctx, const K* d_keys, uint64_t n, int depth, svdag_dag*
                                           batch->num_chunks, &c->n, n, sc, B.seg_lo, B.seg_chunk_bits, err,
                                           ctx->seg_first_bits);
         } else {
-            where = launch_sort<uint64_t>(st, L.key_plan, reinterpret_cast<const uint64_t*>(d_keys), nullptr, ka, kb,
-                                          nullptr, nullptr, nullptr, nullptr, &c->n, n,
+            where = launch_sort<uint64_t>(st, L.key_plan, reinterpret_cast<const uint64_t*>(d_keys), ka, kb,
+                                          nullptr, &c->n, n,
                                           reinterpret_cast<uint32_t*>(A + L.key_sort_zero), sort_counts, &c->key_or,
                                           prefix);
         }
@@ -840,8 +837,8 @@ int build(svdag_context* ctx, const K* d_keys, uint64_t n, int depth, svdag_dag*
             }
         }
         if (!L.top_first)
-            where = launch_sort<K>(st, L.key_plan, d_keys, nullptr, ka, kb, nullptr, nullptr, nullptr, nullptr, &c->n,
-                                   n, reinterpret_cast<uint32_t*>(A + L.key_sort_zero), sort_counts, &c->key_or);
+            where = launch_sort<K>(st, L.key_plan, d_keys, ka, kb, nullptr, &c->n, n,
+                                   reinterpret_cast<uint32_t*>(A + L.key_sort_zero), sort_counts, &c->key_or);
         sorted = where == 0 ? static_cast<const void*>(ka) : static_cast<const void*>(kb);
     }
     if (where < 0) return fail(set_error(SVDAG_ERR_INTERNAL, "sort plan failed"));
@@ -871,7 +868,6 @@ int build(svdag_context* ctx, const K* d_keys, uint64_t n, int depth, svdag_dag*
     uint64_t* lk1 = reinterpret_cast<uint64_t*>(A + L.list_keys[1]);
     uint32_t* ls0 = reinterpret_cast<uint32_t*>(A + L.list_slots[0]);
     uint32_t* ls1 = reinterpret_cast<uint32_t*>(A + L.list_slots[1]);
-    uint32_t* sorted_slots = reinterpret_cast<uint32_t*>(A + L.sorted_slots);
     // The leaf table is sized from a distinct-count estimate of the masks (or,
     // on a retry, from the leaf positions, an upper bound).
     const uint64_t* leaf_size = &c->leaf_positions;
@@ -883,8 +879,6 @@ int build(svdag_context* ctx, const K* d_keys, uint64_t n, int depth, svdag_dag*
     }
     launch_table_clear(st, leaf_table, leaf_size, leaf_lg, ctx->load_shift, 0, L.leaf_slots);
     launch_leaf_insert(st, lp_mask, &c->leaf_positions, leaf_table, leaf_lg, lp_slot, L.leaf_bound, err);
-    launch_slot_list(st, leaf_table, leaf_lg, L.leaf_slots, tile_counts, tile_offsets, &c->table_slots, lk0, ls0,
-                     &c->unique_leaves);
     // The unique leaves are ordered (sorted masks, slot -> rank) on the side
     // stream for large builds: the level above the leaves needs their ranks
     // only from its extract on, so its build overlaps this sort.  Small builds
@@ -904,11 +898,10 @@ int build(svdag_context* ctx, const K* d_keys, uint64_t n, int depth, svdag_dag*
     auto order_leaves = [&]() -> int {
         if (ordered) return 0;
         ordered = true;
-        if (launch_sort<uint64_t>(ls, L.leaf_plan, lk0, ls0, lk1, lk0, ls1, ls0, leaves_out, sorted_slots,
-                                  &c->unique_leaves, L.leaf_bound, reinterpret_cast<uint32_t*>(A + L.leaf_sort_zero),
-                                  sort_counts, nullptr) < 0)
-            return fail(set_error(SVDAG_ERR_INTERNAL, "leaf sort plan failed"));
-        launch_rank_of_slot(ls, sorted_slots, &c->unique_leaves, leaf_rank, L.leaf_bound);
+        launch_leaf_order(ls, LeafOrderArgs{leaf_table, leaf_lg, reinterpret_cast<uint64_t*>(A + L.order_split),
+                                            reinterpret_cast<uint32_t*>(A + L.order_zero), {lk0, lk1}, {ls0, ls1},
+                                            leaves_out, leaf_rank, &c->unique_leaves},
+                          L.leaf_slots, L.leaf_bound);
         if (forked && hipEventRecord(ctx->join_ev, ls) != hipSuccess)
             return fail(set_error(SVDAG_ERR_HIP, "event record failed"));
         return 0;
@@ -1109,16 +1102,14 @@ int merge_device(svdag_context* ctx, const svdag_dag* dags, uint64_t count, int 
     const uint32_t shift = ctx->load_shift;
     const uint64_t leaf_slots = 1ull << table_lg(total_leaves, shift);
     const uint64_t level_slots = (1ull << table_lg(std::max(max_total, nlive), shift)) + kTableOverflow;
-    const SortPlan leaf_plan = make_sort_plan(0, 64);
-
     const uint64_t stage_tiles =
         std::max({tiles(level_slots, kExtractTileItems), tiles(nlive, kBuildTileItems), uint64_t(1)});
     Carver cv;
     const uint64_t o_zero = cv.off;
     const uint64_t o_counters = cv.take(sizeof(BuildCounters));
-    const uint64_t o_leaf_sort_zero = cv.take(4 * sort_zero_words(leaf_plan));
+    const uint64_t o_order_zero = cv.take(4 * kOrderZeroWords);
     const uint64_t zero_end = cv.off;
-    const uint64_t o_sort_counts = cv.take(4 * sort_count_words(total_leaves));
+    const uint64_t o_order_split = cv.take(8 * kOrderMaxBuckets);
     const uint64_t o_tile_counts = cv.take(4 * stage_tiles);
     const uint64_t o_tile_offsets = cv.take(8 * stage_tiles);
     const uint64_t o_sources = cv.take(sizeof(MergeSource) * nlive * (lc_levels + 1));
@@ -1130,7 +1121,6 @@ int merge_device(svdag_context* ctx, const svdag_dag* dags, uint64_t count, int 
         o_lk[i] = cv.take(8 * total_leaves);
         o_ls[i] = cv.take(4 * total_leaves);
     }
-    const uint64_t o_sorted_slots = cv.take(4 * total_leaves);
     uint64_t o_slot_of[2];
     for (int i = 0; i < 2; ++i) o_slot_of[i] = cv.take(4 * std::max(max_total, nlive));
     const uint64_t o_masks = cv.take(max_total);
@@ -1198,8 +1188,7 @@ int merge_device(svdag_context* ctx, const svdag_dag* dags, uint64_t count, int 
         launch_fill_u64(st, &c->pre[k - 1], 1, groups);
     }
 
-    // Leaves: shared hashed table (first inserters append to the unique list),
-    // sort, rank.
+    // Leaves: shared hashed table, its order, ranks.
     uint64_t* leaf_table = reinterpret_cast<uint64_t*>(A + o_leaf_table);
     uint32_t* leaf_rank = reinterpret_cast<uint32_t*>(A + o_leaf_rank);
     uint32_t* leaf_slot_of = reinterpret_cast<uint32_t*>(A + o_leaf_slot_of);
@@ -1208,16 +1197,14 @@ int merge_device(svdag_context* ctx, const svdag_dag* dags, uint64_t count, int 
     uint64_t* lk1 = reinterpret_cast<uint64_t*>(A + o_lk[1]);
     uint32_t* ls0 = reinterpret_cast<uint32_t*>(A + o_ls[0]);
     uint32_t* ls1 = reinterpret_cast<uint32_t*>(A + o_ls[1]);
-    uint32_t* sorted_slots = reinterpret_cast<uint32_t*>(A + o_sorted_slots);
     launch_table_clear(st, leaf_table, &c->leaf_positions, leaf_lg, shift, 0, leaf_slots);
     launch_merge_insert(st, d_src, uint32_t(nlive), total_leaves, nullptr, nullptr, nullptr, nullptr, leaf_table,
-                        nullptr, leaf_lg, leaf_slot_of, c, 0, lk0, ls0);
+                        nullptr, leaf_lg, leaf_slot_of, c, 0);
     uint64_t* leaves_out = reinterpret_cast<uint64_t*>(O + S.leaves);
-    if (launch_sort<uint64_t>(st, leaf_plan, lk0, ls0, lk1, lk0, ls1, ls0, leaves_out, sorted_slots, &c->unique_leaves,
-                              total_leaves, reinterpret_cast<uint32_t*>(A + o_leaf_sort_zero),
-                              reinterpret_cast<uint32_t*>(A + o_sort_counts), nullptr) < 0)
-        return fail(set_error(SVDAG_ERR_INTERNAL, "leaf sort plan failed"));
-    launch_rank_of_slot(st, sorted_slots, &c->unique_leaves, leaf_rank, total_leaves);
+    launch_leaf_order(st, LeafOrderArgs{leaf_table, leaf_lg, reinterpret_cast<uint64_t*>(A + o_order_split),
+                                        reinterpret_cast<uint32_t*>(A + o_order_zero), {lk0, lk1}, {ls0, ls1},
+                                        leaves_out, leaf_rank, &c->unique_leaves},
+                      leaf_slots, total_leaves);
 
     const uint32_t* child_slot_of = leaf_slot_of;
     const uint32_t* child_rank = leaf_rank;
@@ -1251,7 +1238,7 @@ int merge_device(svdag_context* ctx, const svdag_dag* dags, uint64_t count, int 
         launch_table_clear(st, tk, &c->pre[l], &c->table_log2[l], shift, kTableOverflow, level_slots);
         launch_merge_insert(st, d_src + uint64_t(lc + 1) * nlive, uint32_t(nlive), totals[lc], child_slot_of,
                             child_rank, masks, children, tk, reinterpret_cast<uint32_t*>(A + o_trep[cur]),
-                            &c->table_log2[l], slot_of, c, 1, nullptr, nullptr);
+                            &c->table_log2[l], slot_of, c, 1);
         extract(l, cur);
         child_slot_of = slot_of;
         child_rank = reinterpret_cast<const uint32_t*>(A + o_trank[cur]);
@@ -1333,8 +1320,8 @@ int sort_keys_entry(svdag_context* ctx, const K* d_keys, uint64_t n, int32_t bit
     launch_fill_u64(st, reinterpret_cast<uint64_t*>(A + o_zero), (o_n - o_zero) / 8, 0);
     launch_fill_u64(st, reinterpret_cast<uint64_t*>(A + o_n), 1, n);
     launch_fill_u64(st, reinterpret_cast<uint64_t*>(A + o_or), 1, 0);
-    const int where = launch_sort<K>(st, plan, d_keys, nullptr, reinterpret_cast<K*>(A + o_a),
-                                     reinterpret_cast<K*>(A + o_b), nullptr, nullptr, d_out, nullptr,
+    const int where = launch_sort<K>(st, plan, d_keys, reinterpret_cast<K*>(A + o_a),
+                                     reinterpret_cast<K*>(A + o_b), d_out,
                                      reinterpret_cast<const uint64_t*>(A + o_n), n,
                                      reinterpret_cast<uint32_t*>(A + o_zero), reinterpret_cast<uint32_t*>(A + o_counts),
                                      reinterpret_cast<unsigned long long*>(A + o_or));
@@ -2502,24 +2489,22 @@ int svdag_resident_dag(svdag_resident* r, svdag_dag* out)
     hipStream_t st = ctx->stream;
     const uint64_t nslots = 1ull << (3 * r->top);
     const uint64_t L = r->occupied[r->rlevels];
-    const SortPlan leaf_plan = make_sort_plan(0, 64);
     uint64_t max_slots = r->leaf_slots;
     for (int i = 0; i < r->rlevels; ++i) max_slots = std::max(max_slots, r->slots[i]);
-    const uint64_t stage_tiles = std::max({tiles(max_slots, kExtractTileItems), tiles(r->leaf_slots, kListTileItems),
-                                           uint64_t(1)});
+    const uint64_t stage_tiles = std::max(tiles(max_slots, kExtractTileItems), uint64_t(1));
     Carver cv;
     const uint64_t o_zero = cv.off;
     const uint64_t o_counters = cv.take(sizeof(BuildCounters));
-    const uint64_t o_sort_zero = cv.take(4 * sort_zero_words(leaf_plan));
+    const uint64_t o_order_zero = cv.take(4 * kOrderZeroWords);
     const uint64_t zero_end = cv.off;
-    const uint64_t o_sort_counts = cv.take(4 * sort_count_words(L));
+    const uint64_t o_order_split = cv.take(8 * kOrderMaxBuckets);
     const uint64_t o_tile_counts = cv.take(4 * stage_tiles), o_tile_offsets = cv.take(8 * stage_tiles);
     uint64_t o_lk[2], o_ls[2];
     for (int i = 0; i < 2; ++i) {
         o_lk[i] = cv.take(8 * L);
         o_ls[i] = cv.take(4 * L);
     }
-    const uint64_t o_sorted = cv.take(4 * L), o_leaf_rank = cv.take(4 * r->leaf_slots);
+    const uint64_t o_leaf_rank = cv.take(4 * r->leaf_slots);
     const uint64_t o_rank[2] = {cv.take(4 * max_slots), cv.take(4 * max_slots)};
     const uint64_t o_codes = cv.take(8 * nslots), o_rslots = cv.take(4 * nslots), o_rcount = cv.take(8);
     uint64_t o_tcodes[2], o_tranks[2];
@@ -2551,16 +2536,13 @@ int svdag_resident_dag(svdag_resident* r, svdag_dag* out)
     uint64_t* lk1 = reinterpret_cast<uint64_t*>(A + o_lk[1]);
     uint32_t* ls0 = reinterpret_cast<uint32_t*>(A + o_ls[0]);
     uint32_t* ls1 = reinterpret_cast<uint32_t*>(A + o_ls[1]);
-    uint32_t* sorted = reinterpret_cast<uint32_t*>(A + o_sorted);
     uint32_t* leaf_rank = reinterpret_cast<uint32_t*>(A + o_leaf_rank);
     uint64_t* leaves_out = reinterpret_cast<uint64_t*>(O + S.leaves);
-    launch_slot_list(st, r->leaf_keys, r->d_lg + r->rlevels, r->leaf_slots, tile_counts, tile_offsets,
-                     &c->table_slots, lk0, ls0, &c->unique_leaves);
-    if (launch_sort<uint64_t>(st, leaf_plan, lk0, ls0, lk1, lk0, ls1, ls0, leaves_out, sorted, &c->unique_leaves, L,
-                              reinterpret_cast<uint32_t*>(A + o_sort_zero),
-                              reinterpret_cast<uint32_t*>(A + o_sort_counts), nullptr) < 0)
-        return fail(set_error(SVDAG_ERR_INTERNAL, "leaf sort plan failed"));
-    launch_rank_of_slot(st, sorted, &c->unique_leaves, leaf_rank, L);
+    launch_leaf_order(st, LeafOrderArgs{r->leaf_keys, r->d_lg + r->rlevels,
+                                        reinterpret_cast<uint64_t*>(A + o_order_split),
+                                        reinterpret_cast<uint32_t*>(A + o_order_zero), {lk0, lk1}, {ls0, ls1},
+                                        leaves_out, leaf_rank, &c->unique_leaves},
+                      r->leaf_slots, L);
     // Resident levels bottom-up, each in ascending hash order with its
     // children's slots turned into ranks of the level below.
     const uint32_t* below = leaf_rank;

@@ -5,9 +5,8 @@
 //       (one pass over the keys grouped by code >> 15: duplicates OR into the
 //       same 4^3 mask, so no separate unique step is needed)
 //   SortLevel(Leaves)               :1070-1071  -> k_table_clear / k_leaf_insert
-//       (hash table keyed by the mask; the first inserter of a mask appends it
-//       to the unique list) + a key/value radix sort of that list +
-//       k_rank_of_slot
+//       (hash table keyed by the mask) + a sample sort of its occupied slots
+//       (k_leaf_sample, k_order_*)
 //   ExtractLevel + ComputeHashes    :916-974, :827-833 -> k_level_count /
 //       k_level_build (parent masks, child ranks, Murmur hash, insert into the
 //       level's dedup table)
@@ -522,67 +521,6 @@ __global__ __launch_bounds__(kThreads) void k_leaf_insert(const uint64_t* __rest
     }
 }
 
-// Unique list of a hashed table: its occupied slots (key, slot index), by
-// count / scan / write over tiles of kListTile slots.
-constexpr int kListIpt = 16;
-constexpr uint32_t kListTile = kThreads * kListIpt;
-
-__global__ __launch_bounds__(kThreads) void k_slot_count(const uint64_t* __restrict__ tk,
-                                                         const uint32_t* __restrict__ log2_ptr,
-                                                         uint32_t* __restrict__ counts, uint64_t* __restrict__ slots_out)
-{
-    __shared__ uint64_t s_red[kThreads / kWave];
-    const uint64_t total = 1ull << *log2_ptr;
-    const uint64_t ntiles = (total + kListTile - 1) / kListTile;
-    if (blockIdx.x == 0 && threadIdx.x == 0) *slots_out = total;
-    for (uint64_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
-        uint32_t occ = 0;
-        // Unconditional loads (indices past the end read the last slot and are
-        // not counted), so that all are in flight at once.
-        uint64_t v[kListIpt];
-#pragma unroll
-        for (int j = 0; j < kListIpt; ++j) v[j] = tk[min(tile * kListTile + uint64_t(j) * kThreads + threadIdx.x, total - 1)];
-#pragma unroll
-        for (int j = 0; j < kListIpt; ++j) {
-            const uint64_t i = tile * kListTile + uint64_t(j) * kThreads + threadIdx.x;
-            occ += (i < total && v[j] != 0) ? 1u : 0u;
-        }
-        const uint64_t cnt = block_reduce_sum<kThreads>(occ, s_red);
-        if (threadIdx.x == 0) counts[tile] = uint32_t(cnt);
-    }
-}
-
-__global__ __launch_bounds__(kThreads) void k_slot_list(const uint64_t* __restrict__ tk,
-                                                        const uint32_t* __restrict__ log2_ptr,
-                                                        const uint64_t* __restrict__ offsets,
-                                                        uint64_t* __restrict__ list_keys,
-                                                        uint32_t* __restrict__ list_slots)
-{
-    __shared__ uint32_t s_scan[kThreads / kWave];
-    const uint64_t total = 1ull << *log2_ptr;
-    const uint64_t ntiles = (total + kListTile - 1) / kListTile;
-    for (uint64_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
-        uint64_t key[kListIpt];
-        uint32_t occ = 0;
-#pragma unroll
-        for (int j = 0; j < kListIpt; ++j) {
-            const uint64_t i = tile * kListTile + uint64_t(j) * kThreads + threadIdx.x;
-            key[j] = i < total ? tk[i] : 0ull;
-            occ |= (key[j] != 0 ? 1u : 0u) << j;
-        }
-        uint32_t unused;
-        uint64_t o = offsets[tile] + block_exclusive_scan<kThreads>(uint32_t(__popc(occ)), s_scan, unused);
-#pragma unroll
-        for (int j = 0; j < kListIpt; ++j) {
-            if ((occ >> j) & 1u) {
-                list_keys[o] = key[j];
-                list_slots[o] = uint32_t(tile * kListTile + uint64_t(j) * kThreads + threadIdx.x);
-                ++o;
-            }
-        }
-    }
-}
-
 // ---------------------------------------------------------------------------
 // Distinct-count estimate of the leaf masks (HyperLogLog: Flajolet, Fusy,
 // Gandouet, Meunier 2007), so the leaf table is sized by unique leaves rather
@@ -665,13 +603,314 @@ __global__ __launch_bounds__(kEstimateThreads) void k_sketch_estimate(const uint
     }
 }
 
-__global__ void k_rank_of_slot(const uint32_t* __restrict__ sorted_slots, const uint64_t* __restrict__ count_ptr,
-                               uint32_t* __restrict__ rank_of_slot)
+// ---------------------------------------------------------------------------
+// Leaf order: the occupied slots of a hashed table -> the masks in ascending
+// order, and each slot's rank.  A sample sort in four launches:
+//   k_leaf_sample   one workgroup: a sample of the masks, sorted, gives the
+//                   splitters of 2^b buckets of about 1024 masks.  The table is
+//                   hashed, so its first slots are a uniform sample; their
+//                   density also gives the mask count that b is chosen from.
+//   k_order_count   keys per bucket (each tile of slots classifies its masks by
+//                   binary search in the splitters, in LDS)
+//   k_order_scatter masks and slots into their buckets' ranges, in any order
+//   k_order_sort    one workgroup per bucket: LDS sort, masks and ranks out.
+//                   The masks are distinct, so the result does not depend on
+//                   the order of the scatter.
+// Bound by launches and by the dependent LDS steps of the two sorts, not by
+// bytes.  An LSD radix sort of the same pairs took eight passes of three
+// launches: 25 launches and 130 us (100k masks) to 330 us (360k masks) of
+// kernel time, 130 us of a 350 us build of 1000 keys.
+// A bucket too large for LDS (the sample missed, or over 4M masks) is sorted in
+// pieces that its workgroup merges in global memory.
+// ---------------------------------------------------------------------------
+constexpr int kSampleThreads = 1024;
+constexpr uint32_t kSampleMax = 4096;        // masks sampled at most
+constexpr uint32_t kSamplePerBucket = 8;     // aimed at; fewer past 2^9 buckets
+constexpr uint32_t kSampleScanMax = 1u << 18;  // slots looked at for a small sample
+constexpr uint32_t kOrderMean = 1024;        // masks per bucket aimed at
+constexpr uint32_t kOrderCap = 4096;         // masks one LDS sort takes
+constexpr int kOrderIpt = 16;
+constexpr uint32_t kOrderTile = kThreads * kOrderIpt;
+static_assert(kOrderTile <= 65536 && kOrderMaxBuckets <= 65536, "bucket and rank packed in 16 bits each");
+
+// Ascending bitonic sort of n2 (a power of two) keys in LDS, with their slots
+// when SLOTS (equal keys, padding only, then compare by slot).  Ends with a
+// barrier; every thread of the block must call it.
+template <int THREADS, bool SLOTS>
+__device__ __forceinline__ void lds_sort(uint64_t* key, uint32_t* slot, uint32_t n2)
 {
-    const uint64_t n = *count_ptr;
-    const uint64_t stride = uint64_t(gridDim.x) * blockDim.x;
-    for (uint64_t r = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x; r < n; r += stride)
-        rank_of_slot[sorted_slots[r]] = uint32_t(r);
+    for (uint32_t size = 2; size <= n2; size <<= 1) {
+        for (uint32_t stride = size >> 1; stride > 0; stride >>= 1) {
+            __syncthreads();
+            for (uint32_t t = threadIdx.x; t < n2 / 2; t += THREADS) {
+                const uint32_t lo = 2 * t - (t & (stride - 1));
+                const uint32_t hi = lo + stride;
+                const bool up = (lo & size) == 0;
+                const uint64_t a = key[lo], b = key[hi];
+                if constexpr (SLOTS) {
+                    const uint32_t sa = slot[lo], sb = slot[hi];
+                    const bool greater = a > b || (a == b && sa > sb);
+                    if (greater == up) {
+                        key[lo] = b;
+                        key[hi] = a;
+                        slot[lo] = sb;
+                        slot[hi] = sa;
+                    }
+                } else {
+                    if ((a > b) == up) {
+                        key[lo] = b;
+                        key[hi] = a;
+                    }
+                }
+            }
+        }
+    }
+    __syncthreads();
+}
+
+__device__ __forceinline__ uint32_t pow2_at_least(uint32_t v)
+{
+    uint32_t p = 1;
+    while (p < v) p <<= 1;
+    return p;
+}
+
+// split[1 .. 2^b): the splitters; split[0] = b.
+__global__ __launch_bounds__(kSampleThreads) void k_leaf_sample(const uint64_t* __restrict__ tk,
+                                                                const uint32_t* __restrict__ log2_ptr,
+                                                                uint64_t* __restrict__ split)
+{
+    constexpr int IPT = 4;
+    constexpr uint32_t kRound = kSampleThreads * IPT;
+    __shared__ uint64_t s_key[kSampleMax];
+    __shared__ uint32_t s_scan[kSampleThreads / kWave];
+    const uint64_t total = 1ull << *log2_ptr;
+    uint64_t scanned = 0, found = 0;
+    uint32_t m = 0, b = 0;
+    while (true) {
+        uint64_t v[IPT];
+#pragma unroll
+        for (int i = 0; i < IPT; ++i) v[i] = tk[min(scanned + uint64_t(i) * kSampleThreads + threadIdx.x, total - 1)];
+        uint32_t mine = 0;
+#pragma unroll
+        for (int i = 0; i < IPT; ++i) {
+            if (scanned + uint64_t(i) * kSampleThreads + threadIdx.x >= total) v[i] = 0;
+            mine += v[i] != 0 ? 1u : 0u;
+        }
+        uint32_t round;
+        uint32_t o = m + block_exclusive_scan<kSampleThreads>(mine, s_scan, round);
+#pragma unroll
+        for (int i = 0; i < IPT; ++i) {
+            if (v[i] != 0) {
+                if (o < kSampleMax) s_key[o] = v[i];
+                ++o;
+            }
+        }
+        found += round;
+        m = uint32_t(min(uint64_t(kSampleMax), m + uint64_t(round)));
+        scanned = min(scanned + kRound, total);
+        // Expected masks in the whole table, and the buckets for them.
+        const uint64_t expect = found * (total / scanned + (total % scanned ? 1 : 0));
+        b = 0;
+        while (b < kOrderMaxLog2 && (uint64_t(kOrderMean) << b) < expect) ++b;
+        const uint32_t want = min(max(kSamplePerBucket << b, 64u), kSampleMax);
+        if (scanned == total || m >= want || scanned >= kSampleScanMax) break;
+    }
+    while (b > 0 && (2u << b) > m) --b;  // at least two samples per bucket
+    const uint32_t n2 = pow2_at_least(m);
+    if (b > 0) {
+        for (uint32_t i = m + threadIdx.x; i < n2; i += kSampleThreads) s_key[i] = ~0ull;
+        lds_sort<kSampleThreads, false>(s_key, nullptr, n2);
+        const uint32_t buckets = 1u << b;
+        for (uint32_t j = 1 + threadIdx.x; j < buckets; j += kSampleThreads)
+            split[j] = s_key[uint32_t(uint64_t(j) * m >> b)];
+    }
+    if (threadIdx.x == 0) split[0] = b;
+}
+
+// Bucket of key: the number of splitters at or below it.
+__device__ __forceinline__ uint32_t bucket_by_split(const uint64_t* s_split, uint32_t b, uint64_t key)
+{
+    uint32_t idx = 0;
+    for (uint32_t step = (1u << b) >> 1; step > 0; step >>= 1)
+        if (s_split[idx + step] <= key) idx += step;
+    return idx;
+}
+
+__global__ __launch_bounds__(kThreads) void k_order_count(const uint64_t* __restrict__ tk,
+                                                          const uint32_t* __restrict__ log2_ptr,
+                                                          const uint64_t* __restrict__ split,
+                                                          uint32_t* __restrict__ totals)
+{
+    __shared__ uint64_t s_split[kOrderMaxBuckets];
+    __shared__ uint32_t s_cnt[kOrderMaxBuckets];
+    const uint64_t total = 1ull << *log2_ptr;
+    const uint64_t ntiles = (total + kOrderTile - 1) / kOrderTile;
+    if (blockIdx.x >= ntiles) return;
+    const uint32_t b = uint32_t(split[0]), buckets = 1u << b;
+    for (uint32_t i = threadIdx.x; i < buckets; i += kThreads) {
+        s_split[i] = split[i];
+        s_cnt[i] = 0;
+    }
+    __syncthreads();
+    for (uint64_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
+        uint64_t v[kOrderIpt];
+#pragma unroll
+        for (int j = 0; j < kOrderIpt; ++j)
+            v[j] = tk[min(tile * kOrderTile + uint64_t(j) * kThreads + threadIdx.x, total - 1)];
+#pragma unroll
+        for (int j = 0; j < kOrderIpt; ++j) {
+            const bool here = tile * kOrderTile + uint64_t(j) * kThreads + threadIdx.x < total && v[j] != 0;
+            if (b == 0) {
+                // One bucket: one add per wave instead of one word for all.
+                const uint32_t c = uint32_t(__popcll(__ballot(here)));
+                if (lane_id() == 0 && c) atomicAdd(&s_cnt[0], c);
+            } else if (here) {
+                atomicAdd(&s_cnt[bucket_by_split(s_split, b, v[j])], 1u);
+            }
+        }
+    }
+    __syncthreads();
+    for (uint32_t i = threadIdx.x; i < buckets; i += kThreads)
+        if (s_cnt[i]) atomicAdd(&totals[i], s_cnt[i]);
+}
+
+__global__ __launch_bounds__(kThreads) void k_order_scatter(const uint64_t* __restrict__ tk,
+                                                            const uint32_t* __restrict__ log2_ptr,
+                                                            const uint64_t* __restrict__ split,
+                                                            const uint32_t* __restrict__ totals,
+                                                            uint32_t* __restrict__ cursors,
+                                                            uint64_t* __restrict__ list_keys,
+                                                            uint32_t* __restrict__ list_slots)
+{
+    constexpr int BPT = int(kOrderMaxBuckets) / kThreads;  // buckets per thread in the scan
+    __shared__ uint64_t s_split[kOrderMaxBuckets];
+    __shared__ uint32_t s_start[kOrderMaxBuckets];
+    __shared__ uint32_t s_cnt[kOrderMaxBuckets];
+    __shared__ uint32_t s_scan[kThreads / kWave];
+    const uint64_t total = 1ull << *log2_ptr;
+    const uint64_t ntiles = (total + kOrderTile - 1) / kOrderTile;
+    if (blockIdx.x >= ntiles) return;
+    const uint32_t b = uint32_t(split[0]), buckets = 1u << b;
+    for (uint32_t i = threadIdx.x; i < buckets; i += kThreads) s_split[i] = split[i];
+    // Bucket starts: exclusive scan of the totals, BPT consecutive per thread.
+    uint32_t t[BPT], sum = 0;
+#pragma unroll
+    for (int k = 0; k < BPT; ++k) {
+        const uint32_t i = threadIdx.x * BPT + k;
+        t[k] = i < buckets ? totals[i] : 0u;
+        sum += t[k];
+    }
+    uint32_t unused;
+    uint32_t run = block_exclusive_scan<kThreads>(sum, s_scan, unused);
+#pragma unroll
+    for (int k = 0; k < BPT; ++k) {
+        const uint32_t i = threadIdx.x * BPT + k;
+        if (i < buckets) s_start[i] = run;
+        run += t[k];
+    }
+    for (uint64_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
+        __syncthreads();  // the previous tile's counts have been read
+        for (uint32_t i = threadIdx.x; i < buckets; i += kThreads) s_cnt[i] = 0;
+        uint64_t v[kOrderIpt];
+        uint32_t br[kOrderIpt];  // bucket << 16 | rank within the tile's bucket
+#pragma unroll
+        for (int j = 0; j < kOrderIpt; ++j)
+            v[j] = tk[min(tile * kOrderTile + uint64_t(j) * kThreads + threadIdx.x, total - 1)];
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < kOrderIpt; ++j) {
+            if (tile * kOrderTile + uint64_t(j) * kThreads + threadIdx.x >= total) v[j] = 0;
+            if (v[j] != 0) {
+                const uint32_t k = bucket_by_split(s_split, b, v[j]);
+                br[j] = k << 16 | atomicAdd(&s_cnt[k], 1u);
+            }
+        }
+        __syncthreads();
+        // The tile's place in each bucket's range.
+        for (uint32_t i = threadIdx.x; i < buckets; i += kThreads) {
+            const uint32_t c = s_cnt[i];
+            if (c) s_cnt[i] = s_start[i] + atomicAdd(&cursors[i], c);
+        }
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < kOrderIpt; ++j) {
+            if (v[j] != 0) {
+                const uint32_t o = s_cnt[br[j] >> 16] + (br[j] & 0xFFFFu);
+                list_keys[o] = v[j];
+                list_slots[o] = uint32_t(tile * kOrderTile + uint64_t(j) * kThreads + threadIdx.x);
+            }
+        }
+    }
+}
+
+__global__ __launch_bounds__(kThreads) void k_order_sort(const uint64_t* __restrict__ split,
+                                                         const uint32_t* __restrict__ totals, uint64_t* keys_a,
+                                                         uint32_t* slots_a, uint64_t* keys_b, uint32_t* slots_b,
+                                                         uint64_t* __restrict__ out, uint32_t* __restrict__ rank_of_slot,
+                                                         uint64_t* __restrict__ count)
+{
+    __shared__ uint64_t s_key[kOrderCap];
+    __shared__ uint32_t s_slot[kOrderCap];
+    __shared__ uint64_t s_red[kThreads / kWave];
+    const uint32_t buckets = 1u << uint32_t(split[0]);
+    for (uint32_t bucket = blockIdx.x; bucket < buckets; bucket += gridDim.x) {
+        uint64_t below = 0;
+        for (uint32_t i = threadIdx.x; i < bucket; i += kThreads) below += totals[i];
+        const uint64_t start = block_reduce_sum<kThreads>(below, s_red);
+        const uint32_t cnt = totals[bucket];
+        if (bucket + 1 == buckets && threadIdx.x == 0) *count = start + cnt;
+        for (uint32_t c0 = 0; c0 < cnt; c0 += kOrderCap) {
+            const uint32_t n = min(kOrderCap, cnt - c0), n2 = pow2_at_least(n);
+            for (uint32_t i = threadIdx.x; i < n2; i += kThreads) {
+                s_key[i] = i < n ? keys_a[start + c0 + i] : ~0ull;
+                s_slot[i] = i < n ? slots_a[start + c0 + i] : ~0u;
+            }
+            lds_sort<kThreads, true>(s_key, s_slot, n2);
+            for (uint32_t i = threadIdx.x; i < n; i += kThreads) {
+                if (cnt <= kOrderCap) {
+                    out[start + i] = s_key[i];
+                    rank_of_slot[s_slot[i]] = uint32_t(start + i);
+                } else {
+                    keys_a[start + c0 + i] = s_key[i];
+                    slots_a[start + c0 + i] = s_slot[i];
+                }
+            }
+            __syncthreads();
+        }
+        if (cnt <= kOrderCap) continue;
+        // Pairs of sorted pieces, merged by each key's place in the other one.
+        uint64_t *ka = keys_a + start, *kb = keys_b + start;
+        uint32_t *sa = slots_a + start, *sb = slots_b + start;
+        for (uint64_t piece = kOrderCap; piece < cnt; piece *= 2) {
+            for (uint64_t i = threadIdx.x; i < cnt; i += kThreads) {
+                const uint64_t first = i / (2 * piece) * (2 * piece);
+                const uint64_t mid = min(first + piece, uint64_t(cnt)), last = min(first + 2 * piece, uint64_t(cnt));
+                const uint64_t key = ka[i];
+                uint64_t lo = i < mid ? mid : first, hi = i < mid ? last : mid;
+                const uint64_t own = i < mid ? i : i - mid + first, base = lo;
+                while (lo < hi) {
+                    const uint64_t at = (lo + hi) / 2;
+                    if (ka[at] < key) lo = at + 1;
+                    else hi = at;
+                }
+                kb[own + (lo - base)] = key;
+                sb[own + (lo - base)] = sa[i];
+            }
+            __syncthreads();
+            uint64_t* const kt = ka;
+            ka = kb;
+            kb = kt;
+            uint32_t* const st = sa;
+            sa = sb;
+            sb = st;
+        }
+        for (uint64_t i = threadIdx.x; i < cnt; i += kThreads) {
+            out[start + i] = ka[i];
+            rank_of_slot[sa[i]] = uint32_t(start + i);
+        }
+        __syncthreads();
+    }
 }
 
 // Ordered-table probe: home = top lg bits of the hash, linear probing forward
@@ -1251,7 +1490,7 @@ __global__ __launch_bounds__(kThreads) void k_level_extract(LevelExtractArgs g)
 constexpr int kFinalIpt = 16;
 constexpr int kFinalTile = kThreads * kFinalIpt;
 static_assert(kBuildTile == kBuildTileItems && kExtractTile == kExtractTileItems &&
-                  kFinalTile == kFinalTileItems && kListTile == kListTileItems,
+                  kFinalTile == kFinalTileItems,
               "tile sizes shared with the scratch planner");
 
 // Per-level starts and arrays of the layout, staged in LDS once per block:
@@ -1399,18 +1638,14 @@ __global__ void k_merge_insert(const MergeSource* __restrict__ src, uint32_t nsr
                                const uint32_t* __restrict__ child_rank_of_slot, uint8_t* __restrict__ masks_out,
                                uint32_t* __restrict__ children_out, uint64_t* __restrict__ tk,
                                uint32_t* __restrict__ trep, const uint32_t* __restrict__ log2_ptr,
-                               uint32_t* __restrict__ slot_of, BuildCounters* __restrict__ c, int ordered,
-                               uint64_t* __restrict__ list_keys, uint32_t* __restrict__ list_slots)
+                               uint32_t* __restrict__ slot_of, BuildCounters* __restrict__ c, int ordered)
 {
     const uint32_t lg = *log2_ptr;
     const uint64_t limit = (1ull << lg) + kTableOverflow;
     const uint64_t stride = uint64_t(gridDim.x) * blockDim.x;
-    // Wave-uniform trip count: the leaf mode's list reservation is a wave ballot.
-    for (uint64_t base = uint64_t(blockIdx.x) * blockDim.x; base < total; base += stride) {
-        const uint64_t gi = base + threadIdx.x;
-        const bool active = gi < total;
+    for (uint64_t gi = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x; gi < total; gi += stride) {
         uint32_t lo = 0, hi = nsrc;  // src[lo].first <= gi < src[hi].first
-        while (active && hi - lo > 1) {
+        while (hi - lo > 1) {
             const uint32_t mid = (lo + hi) / 2;
             if (src[mid].first <= gi) lo = mid;
             else hi = mid;
@@ -1418,31 +1653,10 @@ __global__ void k_merge_insert(const MergeSource* __restrict__ src, uint32_t nsr
         const MergeSource& s = src[lo];
         const uint64_t i = gi - s.first;
         if (!ordered) {
-            bool won = false;
-            uint32_t slot = 0;
-            uint64_t key = 0;
-            if (active) {
-                key = s.hashes[i];
-                slot = hashed_insert(tk, lg, key, won, (unsigned long long*)&c->error);
-                slot_of[gi] = slot;
-            }
-            // One list reservation per wave for the keys this wave placed.
-            const uint64_t wins = __ballot(won);
-            if (wins) {
-                const uint32_t leader = uint32_t(__ffsll((long long)wins) - 1);
-                uint64_t start = 0;
-                if (lane_id() == leader)
-                    start = atomicAdd((unsigned long long*)&c->unique_leaves, (unsigned long long)__popcll(wins));
-                start = __shfl(start, leader, kWave);
-                if (won) {
-                    const uint64_t idx = start + uint32_t(__popcll(wins & lanemask_lt()));
-                    list_keys[idx] = key;
-                    list_slots[idx] = slot;
-                }
-            }
+            bool won;
+            slot_of[gi] = hashed_insert(tk, lg, s.hashes[i], won, (unsigned long long*)&c->error);
             continue;
         }
-        if (!active) continue;
         const uint64_t key = s.hashes[i];
         const uint4* cs = reinterpret_cast<const uint4*>(s.children + 8 * i);
         const uint4 a = cs[0], b = cs[1];
@@ -1713,22 +1927,19 @@ void launch_leaf_insert(hipStream_t s, const uint64_t* lp_mask, const uint64_t* 
                        dim3(kThreads), 0, s, lp_mask, count_ptr, table_keys, log2_ptr, lp_slot, err);
 }
 
-void launch_slot_list(hipStream_t s, const uint64_t* table_keys, const uint32_t* log2_ptr, uint64_t slot_bound,
-                      uint32_t* tile_counts, uint64_t* tile_offsets, uint64_t* slots_scratch, uint64_t* list_keys,
-                      uint32_t* list_slots, uint64_t* list_count)
+void launch_leaf_order(hipStream_t s, const LeafOrderArgs& a, uint64_t slot_bound, uint64_t leaf_bound)
 {
-    const int grid = grid_for((slot_bound + kListTile - 1) / kListTile, 8);
-    {
-        TimedLaunch t(kKSlotList, s);
-        hipLaunchKernelGGL(k_slot_count, dim3(grid), dim3(kThreads), 0, s, table_keys, log2_ptr, tile_counts,
-                           slots_scratch);
-    }
-    launch_scan_counts(s, tile_counts, tile_offsets, slots_scratch, kListTile, list_count);
-    {
-        TimedLaunch t(kKSlotList, s);
-        hipLaunchKernelGGL(k_slot_list, dim3(grid), dim3(kThreads), 0, s, table_keys, log2_ptr, tile_offsets,
-                           list_keys, list_slots);
-    }
+    TimedLaunch t(kKLeafOrder, s);
+    const int grid = grid_for((slot_bound + kOrderTile - 1) / kOrderTile, 4);
+    hipLaunchKernelGGL(k_leaf_sample, dim3(1), dim3(kSampleThreads), 0, s, a.table_keys, a.table_log2, a.split);
+    hipLaunchKernelGGL(k_order_count, dim3(grid), dim3(kThreads), 0, s, a.table_keys, a.table_log2, a.split, a.totals);
+    hipLaunchKernelGGL(k_order_scatter, dim3(grid), dim3(kThreads), 0, s, a.table_keys, a.table_log2, a.split, a.totals,
+                       a.totals + kOrderMaxBuckets, a.list_keys[0], a.list_slots[0]);
+    // At most one bucket per kOrderMean / 2 leaves (the sample's error aside;
+    // the workgroups stride over the buckets there are).
+    const uint64_t buckets = std::min<uint64_t>(kOrderMaxBuckets, std::max<uint64_t>(1, leaf_bound / (kOrderMean / 2)));
+    hipLaunchKernelGGL(k_order_sort, dim3(uint32_t(buckets)), dim3(kThreads), 0, s, a.split, a.totals, a.list_keys[0],
+                       a.list_slots[0], a.list_keys[1], a.list_slots[1], a.out, a.rank_of_slot, a.count);
 }
 
 void launch_sketch(hipStream_t s, const uint64_t* values, const uint64_t* count_ptr, uint32_t* regs, uint64_t n_bound)
@@ -1743,14 +1954,6 @@ void launch_sketch_estimate(hipStream_t s, const uint32_t* regs, const uint64_t*
 {
     TimedLaunch t(kKSketch, s);
     hipLaunchKernelGGL(k_sketch_estimate, dim3(1), dim3(kEstimateThreads), 0, s, regs, bound_ptr, estimate);
-}
-
-void launch_rank_of_slot(hipStream_t s, const uint32_t* sorted_slots, const uint64_t* count_ptr,
-                         uint32_t* rank_of_slot, uint64_t n_bound)
-{
-    TimedLaunch t(kKRankOfSlot, s);
-    hipLaunchKernelGGL(k_rank_of_slot, dim3(grid_for((n_bound + kThreads - 1) / kThreads, 8)), dim3(kThreads), 0, s,
-                       sorted_slots, count_ptr, rank_of_slot);
 }
 
 void launch_level_build(hipStream_t s, const LevelBuildArgs& a, uint64_t child_bound, const TableClearArgs* clear)
@@ -1930,14 +2133,13 @@ void launch_resident_root_list(hipStream_t s, const uint32_t* root_slot, uint32_
 void launch_merge_insert(hipStream_t s, const MergeSource* d_sources, uint32_t num_sources, uint64_t total,
                          const uint32_t* child_slot_of, const uint32_t* child_rank_of_slot, uint8_t* masks_out,
                          uint32_t* children_out, uint64_t* table_keys, uint32_t* table_rep, const uint32_t* table_log2,
-                         uint32_t* slot_of, BuildCounters* counters, int ordered, uint64_t* list_keys,
-                         uint32_t* list_slots)
+                         uint32_t* slot_of, BuildCounters* counters, int ordered)
 {
     if (total == 0) return;
     TimedLaunch t(kKMergeInsert, s);
     hipLaunchKernelGGL(k_merge_insert, dim3(grid_for((total + kThreads - 1) / kThreads, 8)), dim3(kThreads), 0, s,
                        d_sources, num_sources, total, child_slot_of, child_rank_of_slot, masks_out, children_out,
-                       table_keys, table_rep, table_log2, slot_of, counters, ordered, list_keys, list_slots);
+                       table_keys, table_rep, table_log2, slot_of, counters, ordered);
 }
 
 }  // namespace svdag

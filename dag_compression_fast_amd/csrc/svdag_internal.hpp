@@ -23,14 +23,13 @@ enum KernelId : int {
     kKSortCount,
     kKSortScan,
     kKSortScatterKeys,
-    kKSortScatterPairs,
     kKFill,
     kKScanCounts,
     kKLeafReduce,
     kKLeafCompact,
     kKTableClear,
     kKLeafInsert,
-    kKRankOfSlot,
+    kKLeafOrder,  // ascending order of the unique leaves
     kKLevelCount,
     kKLevelBuild,
     kKLevelCheck,
@@ -42,7 +41,6 @@ enum KernelId : int {
     kKMergeInsert,
     kKSketch,
     kKLevelTail,
-    kKSlotList,
     kKQueryVoxels,
     kKVoxSetup,
     kKVoxCount,
@@ -52,8 +50,6 @@ enum KernelId : int {
     kKSortScatterTop,  // top-digit pass of a top-digit-first key sort (64-bit in, 32-bit out)
     kKSegCount,        // segmented sort: per-tile counts
     kKSegScatter,      // segmented sort: scatter passes
-    kKPairHistogram,   // key/value sorts (the unique-leaf order): first read
-    kKPairCount,       // key/value sorts: per-tile counts of the later passes
     kNumKernelIds
 };
 
@@ -85,10 +81,8 @@ struct TimedLaunch {
 constexpr int kMaxRadixBits = 9;
 constexpr int kRadix = 1 << kMaxRadixBits;
 constexpr int kMaxPasses = 8;
-// A tile is 256 threads x ipt keys: 16 (4096 keys; key/value sorts) or 32
-// (8192 keys; keys-only sorts).
+// A tile is 256 threads x ipt keys: 16 (4096 keys) or 32 (8192 keys).
 constexpr int kSortThreads = 256;
-constexpr int kSortIptPairs = 8;   // u64 key/value sorts
 constexpr int kSortIptSmall = 16;
 constexpr int kSortIptLarge = 32;
 
@@ -115,15 +109,14 @@ inline uint64_t sort_tiles(uint64_t n, int ipt)
 // u32, zero before launch_sort) and the per-tile digit counts
 // (sort_count_words u32 for any tile size, any contents).
 inline uint64_t sort_zero_words(const SortPlan& p) { return uint64_t(p.passes) * kRadix; }
-inline uint64_t sort_count_words(uint64_t n_bound) { return uint64_t(kRadix) * sort_tiles(n_bound, kSortIptPairs); }
+inline uint64_t sort_count_words(uint64_t n_bound) { return uint64_t(kRadix) * sort_tiles(n_bound, kSortIptSmall); }
 
-// LSD radix sort of keys (and optionally u32 values) on the plan's bits.  With
-// values, or with plan.stable, keys equal on those bits keep their input order;
-// otherwise their order is unspecified (the first pass ranks unstably).
+// LSD radix sort of keys on the plan's bits.  With plan.stable, keys equal on
+// those bits keep their input order; otherwise their order is unspecified (the first pass ranks unstably).
 // n is read from device memory (*n_ptr, < 2^30); n_bound is a host upper bound
 // sizing the grid and the count buffer.  Passes ping-pong between (keys_a,
 // keys_b); the first pass reads keys_in.  Returns which buffer holds the result
-// (0 = a, 1 = b, 2 = final); if final_keys / final_vals are non-null the last
+// (0 = a, 1 = b, 2 = final); if final_keys is non-null the last
 // pass writes there instead.  key_or (optional) receives the OR of all keys.
 // Chunk-local input of a batched build: key i, with offsets[c] <= i <
 // offsets[c + 1], becomes (c << chunk_bits) | key when the sort first reads it
@@ -191,8 +184,7 @@ int launch_top_digit_sort(hipStream_t stream, const uint64_t* keys_in, uint32_t*
                           unsigned long long* err);
 
 template <typename K>
-int launch_sort(hipStream_t stream, const SortPlan& plan, const K* keys_in, const uint32_t* vals_in,
-                K* keys_a, K* keys_b, uint32_t* vals_a, uint32_t* vals_b, K* final_keys, uint32_t* final_vals,
+int launch_sort(hipStream_t stream, const SortPlan& plan, const K* keys_in, K* keys_a, K* keys_b, K* final_keys,
                 const uint64_t* n_ptr, uint64_t n_bound, uint32_t* zero, uint32_t* counts,
                 unsigned long long* key_or, const ChunkPrefix& prefix = ChunkPrefix{});
 
@@ -229,7 +221,6 @@ constexpr uint64_t kLeafRegionItems = kPackTileItems + (1u << kLeafGroupBits);  
 constexpr uint64_t kBuildTileItems = 1024;    // child codes per level-build tile
 constexpr uint64_t kExtractTileItems = 256;   // table slots per extract tile
 constexpr uint64_t kFinalTileItems = 4096;    // nodes per final-layout tile
-constexpr uint64_t kListTileItems = 4096;     // table slots per slot-list tile
 inline uint64_t tiles(uint64_t n, uint64_t per) { return (n + per - 1) / per; }
 
 int device_cu_count();
@@ -290,13 +281,24 @@ void launch_table_clear(hipStream_t s, uint64_t* keys, const uint64_t* count_ptr
 void launch_leaf_insert(hipStream_t s, const uint64_t* lp_mask, const uint64_t* count_ptr, uint64_t* table_keys,
                         const uint32_t* log2_ptr, uint32_t* lp_slot, uint64_t n_bound, unsigned long long* err);
 
-// The occupied slots of a hashed table (2^*log2_ptr slots, at most slot_bound)
-// as a list (key, slot index); their number goes to *list_count.  tile_counts
-// and tile_offsets need tiles(slot_bound, 4096) entries; *slots_scratch
-// receives the slot count.
-void launch_slot_list(hipStream_t s, const uint64_t* table_keys, const uint32_t* log2_ptr, uint64_t slot_bound,
-                      uint32_t* tile_counts, uint64_t* tile_offsets, uint64_t* slots_scratch, uint64_t* list_keys,
-                      uint32_t* list_slots, uint64_t* list_count);
+// The occupied slots of a hashed table (2^*table_log2 slots, at most
+// slot_bound; at most leaf_bound occupied): their keys in ascending order to
+// out, each slot's rank to rank_of_slot, their number to *count.
+constexpr uint32_t kOrderMaxLog2 = 11;
+constexpr uint32_t kOrderMaxBuckets = 1u << kOrderMaxLog2;
+constexpr uint64_t kOrderZeroWords = 2 * kOrderMaxBuckets;  // u32 words that must be zero at launch
+struct LeafOrderArgs {
+    const uint64_t* table_keys;
+    const uint32_t* table_log2;
+    uint64_t* split;          // kOrderMaxBuckets entries
+    uint32_t* totals;         // kOrderZeroWords, zero: bucket totals, then cursors
+    uint64_t* list_keys[2];   // leaf_bound entries each
+    uint32_t* list_slots[2];
+    uint64_t* out;
+    uint32_t* rank_of_slot;
+    uint64_t* count;
+};
+void launch_leaf_order(hipStream_t s, const LeafOrderArgs& a, uint64_t slot_bound, uint64_t leaf_bound);
 
 // Distinct-count sketch (HyperLogLog, kSketchRegs registers, zero before the
 // first launch) of values[0, *count_ptr), and the count a hashed table is sized
@@ -305,9 +307,6 @@ constexpr int kSketchBits = 12;
 constexpr int kSketchRegs = 1 << kSketchBits;
 void launch_sketch(hipStream_t s, const uint64_t* values, const uint64_t* count_ptr, uint32_t* regs, uint64_t n_bound);
 void launch_sketch_estimate(hipStream_t s, const uint32_t* regs, const uint64_t* bound_ptr, uint64_t* estimate);
-
-void launch_rank_of_slot(hipStream_t s, const uint32_t* sorted_slots, const uint64_t* count_ptr,
-                         uint32_t* rank_of_slot, uint64_t n_bound);
 
 // Children come in one of two forms.  With child_hash_seq, child i's hash is
 // child_hash_seq[i] and its table slot is recorded as the pointer (the level's
@@ -501,8 +500,7 @@ struct MergeSource {
 void launch_merge_insert(hipStream_t s, const MergeSource* d_sources, uint32_t num_sources, uint64_t total,
                          const uint32_t* child_slot_of, const uint32_t* child_rank_of_slot, uint8_t* masks_out,
                          uint32_t* children_out, uint64_t* table_keys, uint32_t* table_rep, const uint32_t* table_log2,
-                         uint32_t* slot_of, BuildCounters* counters, int ordered, uint64_t* list_keys,
-                         uint32_t* list_slots);
+                         uint32_t* slot_of, BuildCounters* counters, int ordered);
 
 // ---- gathered chunks ------------------------------------------------------
 // Source i's keys go to dst[start, start of source i + 1) (the last source up

@@ -1,7 +1,7 @@
 // svdag_sort.hip -- LSD radix sort for gfx950 (wave64), reduce-then-scan.
 //
 // Replaces the CUB DeviceRadixSort calls of the reference (SortKeys,
-// src/DAGCompression.cu:336-357; SortPairs, :359-394).  Digits are up to 9
+// src/DAGCompression.cu:336-357).  Digits are up to 9
 // bits wide.  No workgroup ever waits on another one: every pass is
 //   k_sort_count    tile t (a fixed range of 4096 keys) -> per-digit counts
 //   k_sort_scan     one workgroup per digit scans that digit's row of tile
@@ -339,10 +339,8 @@ enum RankMode { kRankUnstable = 0, kRankStable = 1, kRankAdaptive = 2 };
 
 // KO narrower than K (the top-digit pass of a 64-bit key sort): each key is
 // written without its digit and the bits above it, as a key local to its digit.
-template <typename K, bool PAIRS, int MODE, int IPT, int THREADS, typename KO = K>
+template <typename K, int MODE, int IPT, int THREADS, typename KO = K>
 __global__ __launch_bounds__(THREADS) void k_sort_scatter(const K* __restrict__ keys_in, KO* __restrict__ keys_out,
-                                                               const uint32_t* __restrict__ vals_in,
-                                                               uint32_t* __restrict__ vals_out,
                                                                const uint64_t* __restrict__ n_ptr, uint32_t shift,
                                                                uint32_t digit_mask,
                                                                const uint32_t* __restrict__ offsets, uint64_t stride,
@@ -360,7 +358,6 @@ __global__ __launch_bounds__(THREADS) void k_sort_scatter(const K* __restrict__ 
     // size, so 16 bits hold them.
     static_assert(kTile <= 65535, "16-bit tile-local counters");
     __shared__ K s_keys[kTile];
-    __shared__ uint32_t s_vals[PAIRS ? kTile : 1];
     // Stable ranking: per-wave digit counts and the per-wave match table (zeroed
     // once; each key's ranking clears the word it set, so it is zero again at
     // the end of every tile).  Unstable ranking: the tile's digit counts.
@@ -385,28 +382,22 @@ __global__ __launch_bounds__(THREADS) void k_sort_scatter(const K* __restrict__ 
     const uint32_t wave_base = w * kWave * IPT;
     TileWalk walk = xcd_tiles(ntiles);
     K key[IPT];
-    uint32_t val[PAIRS ? IPT : 1];
     // Keys of tile t (loaded one tile ahead).  Full tiles, the common case, load
     // without per-key guards.
     auto load_tile = [&](uint64_t t) {
         const uint64_t base = t * kTile;
         const uint32_t cnt = t < walk.end ? uint32_t(min(uint64_t(kTile), n - base)) : 0u;
         const K* src = keys_in + base + wave_base + lane;
-        const uint32_t* vs = PAIRS ? vals_in + base + wave_base + lane : nullptr;
         if (cnt == kTile) {
             // Each key is read once: non-temporal loads (measured 4% faster
             // per pass than cached ones; non-temporal stores were 2x slower).
 #pragma unroll
-            for (int i = 0; i < IPT; ++i) {
-                key[i] = __builtin_nontemporal_load(src + i * kWave);
-                if constexpr (PAIRS) val[i] = vs[i * kWave];
-            }
+            for (int i = 0; i < IPT; ++i) key[i] = __builtin_nontemporal_load(src + i * kWave);
         } else {
 #pragma unroll
             for (int i = 0; i < IPT; ++i) {
                 const bool valid = wave_base + i * kWave + lane < cnt;
                 key[i] = valid ? src[i * kWave] : K(0);
-                if constexpr (PAIRS) val[i] = valid ? vs[i * kWave] : 0u;
             }
         }
         if (prefix.offsets && cnt) {
@@ -549,7 +540,6 @@ __global__ __launch_bounds__(THREADS) void k_sort_scatter(const K* __restrict__ 
                 const uint32_t d = dr[i] & 0xFFFFu;
                 const uint32_t pos = s_lstart[d] + (MATCH && stable ? uint32_t(s_wcnt[w][d]) : 0u) + (dr[i] >> 16);
                 s_keys[pos] = key[i];
-                if constexpr (PAIRS) s_vals[pos] = val[i];
             }
         }
         };
@@ -566,7 +556,6 @@ __global__ __launch_bounds__(THREADS) void k_sort_scatter(const K* __restrict__ 
                 keys_out[o] = KO(k & ((K(1) << shift) - 1));
             else
                 keys_out[o] = k;
-            if constexpr (PAIRS) vals_out[o] = s_vals[j];
         };
         if (tile_n == kTile) {
 #pragma unroll
@@ -609,8 +598,7 @@ int device_cu_count()
 constexpr unsigned kUnstableExtraLds = 20 * 1024;
 
 template <typename K, int IPT>
-static void launch_pass(hipStream_t stream, const K* src, K* dst, const uint32_t* vsrc, uint32_t* vdst,
-                        const uint64_t* n_ptr, uint32_t shift, uint32_t dmask, uint32_t* counts, uint32_t* hist,
+static void launch_pass(hipStream_t stream, const K* src, K* dst, const uint64_t* n_ptr, uint32_t shift, uint32_t dmask, uint32_t* counts, uint32_t* hist,
                         uint64_t stride, uint32_t grid, bool first, const ChunkPrefix& prefix, uint32_t sorted_lo,
                         bool stable, const unsigned long long* key_or, uint32_t end_bit)
 {
@@ -621,16 +609,11 @@ static void launch_pass(hipStream_t stream, const K* src, K* dst, const uint32_t
     const uint32_t sorted_mask = span_fits ? (1u << (shift - sorted_lo)) - 1u : 0u;
     // Key sorts (tens of millions of keys) launch about one workgroup per tile
     // (up to 64 per CU): the dispatcher then balances the tiles, which measured
-    // 4% faster than 8 per CU walking several tiles each.  Key/value sorts are
-    // small and sized from a loose bound, where the empty workgroups would cost
-    // more than they balance.
-    const uint32_t scatter_grid =
-        vsrc ? grid
-             : uint32_t(std::max<uint64_t>(
-                   kXcds, std::min<uint64_t>((stride + kXcds - 1) / kXcds * kXcds, uint64_t(device_cu_count()) * 64) /
-                              kXcds * kXcds));
+    // 4% faster than 8 per CU walking several tiles each.
+    const uint32_t scatter_grid = uint32_t(std::max<uint64_t>(
+        kXcds, std::min<uint64_t>((stride + kXcds - 1) / kXcds * kXcds, uint64_t(device_cu_count()) * 64) / kXcds * kXcds));
     if (!counted) {
-        TimedLaunch t(vsrc ? kKPairCount : kKSortCount, stream);
+        TimedLaunch t(kKSortCount, stream);
         hipLaunchKernelGGL((k_sort_count<K, IPT>), dim3(grid), dim3(kSortThreads), 0, stream, src, n_ptr, shift, dmask,
                            counts, stride, hist);
     }
@@ -646,47 +629,38 @@ static void launch_pass(hipStream_t stream, const K* src, K* dst, const uint32_t
     // A stable key-only sort ranks adaptively when it can (see k_sort_scatter);
     // its first pass has no earlier bits, so every tile is uniform there.
     const unsigned long long* wide_or = stable ? key_or : nullptr;
-    if (vsrc) {
-        TimedLaunch t(kKSortScatterPairs, stream);
-        hipLaunchKernelGGL((k_sort_scatter<K, true, kRankStable, IPT, kSortThreads>), dim3(scatter_grid),
-                           dim3(kSortThreads), 0, stream, src, dst, vsrc, vdst, n_ptr, shift, dmask, counts, stride,
-                           prefix, sorted_lo, sorted_mask, nullptr, 64u);
-    } else if (first && !stable) {
+    if (first && !stable) {
         // Key-only first pass: the order within a digit is free.  Its kernel
         // needs fewer registers and would fit three workgroups per CU; the extra
         // LDS holds it to two, as the stable pass, which measured faster (more
         // tiles in flight spread the scattered writes over more open lines).
         TimedLaunch t(kKSortScatterKeys, stream);
-        hipLaunchKernelGGL((k_sort_scatter<K, false, kRankUnstable, IPT, kSortThreads>), dim3(scatter_grid),
-                           dim3(kSortThreads), kUnstableExtraLds, stream, src, dst, nullptr, nullptr, n_ptr, shift,
+        hipLaunchKernelGGL((k_sort_scatter<K, kRankUnstable, IPT, kSortThreads>), dim3(scatter_grid),
+                           dim3(kSortThreads), kUnstableExtraLds, stream, src, dst, n_ptr, shift,
                            dmask, counts, stride, prefix, sorted_lo, sorted_mask, nullptr, 64u);
     } else if (span_fits || (first && wide_or)) {
         // Later key-only passes: tiles uniform in the earlier passes' bits (the
         // common case: the input is sorted on them, in runs longer than a tile)
         // rank unstably, the others stably.
         TimedLaunch t(kKSortScatterKeys, stream);
-        hipLaunchKernelGGL((k_sort_scatter<K, false, kRankAdaptive, IPT, kSortThreads>), dim3(scatter_grid),
-                           dim3(kSortThreads), 0, stream, src, dst, nullptr, nullptr, n_ptr, shift, dmask, counts,
+        hipLaunchKernelGGL((k_sort_scatter<K, kRankAdaptive, IPT, kSortThreads>), dim3(scatter_grid),
+                           dim3(kSortThreads), 0, stream, src, dst, n_ptr, shift, dmask, counts,
                            stride, prefix, sorted_lo, sorted_mask, wide_or, end_bit);
     } else {
         TimedLaunch t(kKSortScatterKeys, stream);
-        hipLaunchKernelGGL((k_sort_scatter<K, false, kRankStable, IPT, kSortThreads>), dim3(scatter_grid),
-                           dim3(kSortThreads), 0, stream, src, dst, nullptr, nullptr, n_ptr, shift, dmask, counts,
+        hipLaunchKernelGGL((k_sort_scatter<K, kRankStable, IPT, kSortThreads>), dim3(scatter_grid),
+                           dim3(kSortThreads), 0, stream, src, dst, n_ptr, shift, dmask, counts,
                            stride, prefix, sorted_lo, sorted_mask, nullptr, 64u);
     }
 }
 
 template <typename K>
-int launch_sort(hipStream_t stream, const SortPlan& plan, const K* keys_in, const uint32_t* vals_in, K* keys_a,
-                K* keys_b, uint32_t* vals_a, uint32_t* vals_b, K* final_keys, uint32_t* final_vals,
+int launch_sort(hipStream_t stream, const SortPlan& plan, const K* keys_in, K* keys_a, K* keys_b, K* final_keys,
                 const uint64_t* n_ptr, uint64_t n_bound, uint32_t* zero, uint32_t* counts, unsigned long long* key_or,
                 const ChunkPrefix& prefix)
 {
     if (plan.passes == 0 || n_bound == 0) return -1;
-    const bool pairs = vals_in != nullptr;
-    // Key/value sorts (the unique-leaf order: a few hundred thousand keys) use
-    // 2048-key tiles for u64 keys, so that more workgroups share each pass.
-    const int ipt = pairs ? (sizeof(K) == 8 ? kSortIptPairs : kSortIptSmall) : plan.ipt;
+    const int ipt = plan.ipt;
     uint32_t* hist = zero;
     const uint64_t stride = sort_tiles(n_bound, ipt);
     HistPlan hp{};
@@ -703,44 +677,38 @@ int launch_sort(hipStream_t stream, const SortPlan& plan, const K* keys_in, cons
         constexpr int I = decltype(ipt_tag)::value;
         {
             // Also writes the first pass's tile counts.
-            TimedLaunch t(vals_in ? kKPairHistogram : kKHistogram, stream);
+            TimedLaunch t(kKHistogram, stream);
             hipLaunchKernelGGL((k_histogram<K, I>), dim3(histogram_grid<K, I>(stride)), dim3(kSortThreads), 0, stream,
                                keys_in, n_ptr, hp, hist, key_or, counts, stride, prefix);
         }
         const K* src = keys_in;
-        const uint32_t* vsrc = vals_in;
         int where = -1;
         for (int p = 0; p < plan.passes; ++p) {
             const bool last = p + 1 == plan.passes;
             K* dst = (p % 2 == 0) ? keys_a : keys_b;
-            uint32_t* vdst = (p % 2 == 0) ? vals_a : vals_b;
             where = p % 2;
             if (last && final_keys) {
                 dst = final_keys;
                 where = 2;
             }
-            if (last && final_vals) vdst = final_vals;
             const uint32_t dmask = (1u << plan.bits[p]) - 1u;
-            launch_pass<K, I>(stream, src, dst, vsrc, vdst, n_ptr, plan.shift[p], dmask, counts, hist + p * kRadix,
+            launch_pass<K, I>(stream, src, dst, n_ptr, plan.shift[p], dmask, counts, hist + p * kRadix,
                               stride, grid, p == 0, p == 0 ? prefix : ChunkPrefix{}, plan.shift[0], plan.stable,
                               key_or, plan.shift[plan.passes - 1] + plan.bits[plan.passes - 1]);
             src = dst;
-            vsrc = vdst;
         }
         return where;
     };
     if (ipt == kSortIptLarge) return run(std::integral_constant<int, kSortIptLarge>{});
-    if constexpr (sizeof(K) == 8)
-        if (ipt == kSortIptPairs) return run(std::integral_constant<int, kSortIptPairs>{});
     return run(std::integral_constant<int, kSortIptSmall>{});
 }
 
-template int launch_sort<uint64_t>(hipStream_t, const SortPlan&, const uint64_t*, const uint32_t*, uint64_t*,
-                                   uint64_t*, uint32_t*, uint32_t*, uint64_t*, uint32_t*, const uint64_t*, uint64_t,
-                                   uint32_t*, uint32_t*, unsigned long long*, const ChunkPrefix&);
-template int launch_sort<uint32_t>(hipStream_t, const SortPlan&, const uint32_t*, const uint32_t*, uint32_t*,
-                                   uint32_t*, uint32_t*, uint32_t*, uint32_t*, uint32_t*, const uint64_t*, uint64_t,
-                                   uint32_t*, uint32_t*, unsigned long long*, const ChunkPrefix&);
+template int launch_sort<uint64_t>(hipStream_t, const SortPlan&, const uint64_t*, uint64_t*, uint64_t*, uint64_t*,
+                                   const uint64_t*, uint64_t, uint32_t*, uint32_t*, unsigned long long*,
+                                   const ChunkPrefix&);
+template int launch_sort<uint32_t>(hipStream_t, const SortPlan&, const uint32_t*, uint32_t*, uint32_t*, uint32_t*,
+                                   const uint64_t*, uint64_t, uint32_t*, uint32_t*, unsigned long long*,
+                                   const ChunkPrefix&);
 
 // ---------------------------------------------------------------------------
 // Segmented key sort of a batched build.  The chunks arrive one after the
@@ -1253,9 +1221,8 @@ int launch_top_digit_sort(hipStream_t stream, const uint64_t* keys_in, uint32_t*
         // CU: this pass writes half the bytes and measured faster at four
         // (207 against 243 us on 70M keys).
         TimedLaunch t(kKSortScatterTop, stream);
-        hipLaunchKernelGGL((k_sort_scatter<uint64_t, false, kRankUnstable, I, kSortThreads, uint32_t>),
-                           dim3(scatter_grid), dim3(kSortThreads), 0, stream, keys_in, local, nullptr,
-                           nullptr, n_ptr, top_shift, dmask, counts, stride, ChunkPrefix{}, 0u, 0u, nullptr, 64u);
+        hipLaunchKernelGGL((k_sort_scatter<uint64_t, kRankUnstable, I, kSortThreads, uint32_t>),
+                           dim3(scatter_grid), dim3(kSortThreads), 0, stream, keys_in, local, n_ptr, top_shift, dmask, counts, stride, ChunkPrefix{}, 0u, 0u, nullptr, 64u);
     };
     if (ipt == kSortIptLarge) run(std::integral_constant<int, kSortIptLarge>{});
     else run(std::integral_constant<int, kSortIptSmall>{});

@@ -629,50 +629,70 @@ constexpr uint32_t kSamplePerBucket = 8;     // aimed at; fewer past 2^9 buckets
 constexpr uint32_t kSampleScanMax = 1u << 18;  // slots looked at for a small sample
 constexpr uint32_t kOrderMean = 1024;        // masks per bucket aimed at
 constexpr uint32_t kOrderCap = 4096;         // masks one LDS sort takes
+constexpr int kOrderSortThreads = 512;
 constexpr int kOrderIpt = 16;
 constexpr uint32_t kOrderTile = kThreads * kOrderIpt;
 static_assert(kOrderTile <= 65536 && kOrderMaxBuckets <= 65536, "bucket and rank packed in 16 bits each");
 
-// Ascending bitonic sort of n2 (a power of two) keys in LDS, with their slots
-// when SLOTS (equal keys, padding only, then compare by slot).  Ends with a
-// barrier; every thread of the block must call it.
-template <int THREADS, bool SLOTS>
-__device__ __forceinline__ void lds_sort(uint64_t* key, uint32_t* slot, uint32_t n2)
+// Ascending sort of the n <= THREADS * E keys of s_key (LDS; the rest of its
+// THREADS * E entries is overwritten with ~0), E consecutive ones per thread: a
+// sort in registers, then log2(n / E) rounds in which each thread finds its
+// place in a pair of runs (merge path) and merges its E keys.  Bound by the
+// chain of dependent LDS reads, about 16 per round; a bitonic network's n log^2 n
+// exchanges kept the CU's LDS busy for 40 us at 4096 keys.  Ends with a barrier;
+// every thread of the block must call it.
+template <int THREADS, int E>
+__device__ __forceinline__ void block_merge_sort(uint64_t* s_key, uint32_t n)
 {
-    for (uint32_t size = 2; size <= n2; size <<= 1) {
-        for (uint32_t stride = size >> 1; stride > 0; stride >>= 1) {
-            __syncthreads();
-            for (uint32_t t = threadIdx.x; t < n2 / 2; t += THREADS) {
-                const uint32_t lo = 2 * t - (t & (stride - 1));
-                const uint32_t hi = lo + stride;
-                const bool up = (lo & size) == 0;
-                const uint64_t a = key[lo], b = key[hi];
-                if constexpr (SLOTS) {
-                    const uint32_t sa = slot[lo], sb = slot[hi];
-                    const bool greater = a > b || (a == b && sa > sb);
-                    if (greater == up) {
-                        key[lo] = b;
-                        key[hi] = a;
-                        slot[lo] = sb;
-                        slot[hi] = sa;
-                    }
-                } else {
-                    if ((a > b) == up) {
-                        key[lo] = b;
-                        key[hi] = a;
-                    }
-                }
-            }
+    const uint32_t first = threadIdx.x * E;
+    uint64_t v[E];
+    __syncthreads();
+#pragma unroll
+    for (int e = 0; e < E; ++e) v[e] = first + e < n ? s_key[first + e] : ~0ull;
+#pragma unroll
+    for (int r = 0; r < E; ++r) {
+#pragma unroll
+        for (int e = r & 1; e + 1 < E; e += 2) {
+            const uint64_t a = v[e], b = v[e + 1];
+            v[e] = a < b ? a : b;
+            v[e + 1] = a < b ? b : a;
         }
     }
+#pragma unroll
+    for (int e = 0; e < E; ++e) s_key[first + e] = v[e];
     __syncthreads();
-}
-
-__device__ __forceinline__ uint32_t pow2_at_least(uint32_t v)
-{
-    uint32_t p = 1;
-    while (p < v) p <<= 1;
-    return p;
+    for (uint32_t run = E; run < n; run *= 2) {
+        const uint32_t base = first & ~(2 * run - 1), diag = first - base;
+        const bool live = base < n;  // threads past the keys hold padding only
+        if (live) {
+            const uint64_t *A = s_key + base, *B = A + run;
+            uint32_t lo = diag > run ? diag - run : 0u, hi = min(diag, run);
+            while (lo < hi) {
+                const uint32_t mid = (lo + hi) / 2;
+                if (A[mid] <= B[diag - 1 - mid]) lo = mid + 1;
+                else hi = mid;
+            }
+            uint32_t ia = lo, ib = diag - lo;
+            // Reads past a run's end stay inside s_key and are not taken.
+            uint64_t ka = A[min(ia, run - 1)], kb = B[min(ib, run - 1)];
+#pragma unroll
+            for (int e = 0; e < E; ++e) {
+                const bool take = ib >= run || (ia < run && ka <= kb);
+                v[e] = take ? ka : kb;
+                ia += take ? 1u : 0u;
+                ib += take ? 0u : 1u;
+                const uint64_t next = take ? A[min(ia, run - 1)] : B[min(ib, run - 1)];
+                ka = take ? next : ka;
+                kb = take ? kb : next;
+            }
+        }
+        __syncthreads();
+        if (live) {
+#pragma unroll
+            for (int e = 0; e < E; ++e) s_key[first + e] = v[e];
+        }
+        __syncthreads();
+    }
 }
 
 // split[1 .. 2^b): the splitters; split[0] = b.
@@ -710,17 +730,15 @@ __global__ __launch_bounds__(kSampleThreads) void k_leaf_sample(const uint64_t* 
         m = uint32_t(min(uint64_t(kSampleMax), m + uint64_t(round)));
         scanned = min(scanned + kRound, total);
         // Expected masks in the whole table, and the buckets for them.
-        const uint64_t expect = found * (total / scanned + (total % scanned ? 1 : 0));
+        const float expect = float(found) * (float(total) / float(scanned));
         b = 0;
-        while (b < kOrderMaxLog2 && (uint64_t(kOrderMean) << b) < expect) ++b;
+        while (b < kOrderMaxLog2 && float(kOrderMean << b) < expect) ++b;
         const uint32_t want = min(max(kSamplePerBucket << b, 64u), kSampleMax);
         if (scanned == total || m >= want || scanned >= kSampleScanMax) break;
     }
     while (b > 0 && (2u << b) > m) --b;  // at least two samples per bucket
-    const uint32_t n2 = pow2_at_least(m);
     if (b > 0) {
-        for (uint32_t i = m + threadIdx.x; i < n2; i += kSampleThreads) s_key[i] = ~0ull;
-        lds_sort<kSampleThreads, false>(s_key, nullptr, n2);
+        block_merge_sort<kSampleThreads, int(kSampleMax) / kSampleThreads>(s_key, m);
         const uint32_t buckets = 1u << b;
         for (uint32_t j = 1 + threadIdx.x; j < buckets; j += kSampleThreads)
             split[j] = s_key[uint32_t(uint64_t(j) * m >> b)];
@@ -728,13 +746,18 @@ __global__ __launch_bounds__(kSampleThreads) void k_leaf_sample(const uint64_t* 
     if (threadIdx.x == 0) split[0] = b;
 }
 
-// Bucket of key: the number of splitters at or below it.
-__device__ __forceinline__ uint32_t bucket_by_split(const uint64_t* s_split, uint32_t b, uint64_t key)
+// Buckets of N keys: the number of splitters at or below each.  The N searches
+// run in step, so that their LDS reads are in flight together.
+template <int N>
+__device__ __forceinline__ void buckets_by_split(const uint64_t* s_split, uint32_t b, const uint64_t (&key)[N],
+                                                 uint32_t (&idx)[N])
 {
-    uint32_t idx = 0;
-    for (uint32_t step = (1u << b) >> 1; step > 0; step >>= 1)
-        if (s_split[idx + step] <= key) idx += step;
-    return idx;
+#pragma unroll
+    for (int j = 0; j < N; ++j) idx[j] = 0;
+    for (uint32_t step = (1u << b) >> 1; step > 0; step >>= 1) {
+#pragma unroll
+        for (int j = 0; j < N; ++j) idx[j] += s_split[idx[j] + step] <= key[j] ? step : 0u;
+    }
 }
 
 __global__ __launch_bounds__(kThreads) void k_order_count(const uint64_t* __restrict__ tk,
@@ -758,6 +781,8 @@ __global__ __launch_bounds__(kThreads) void k_order_count(const uint64_t* __rest
 #pragma unroll
         for (int j = 0; j < kOrderIpt; ++j)
             v[j] = tk[min(tile * kOrderTile + uint64_t(j) * kThreads + threadIdx.x, total - 1)];
+        uint32_t k[kOrderIpt];
+        buckets_by_split(s_split, b, v, k);
 #pragma unroll
         for (int j = 0; j < kOrderIpt; ++j) {
             const bool here = tile * kOrderTile + uint64_t(j) * kThreads + threadIdx.x < total && v[j] != 0;
@@ -766,7 +791,7 @@ __global__ __launch_bounds__(kThreads) void k_order_count(const uint64_t* __rest
                 const uint32_t c = uint32_t(__popcll(__ballot(here)));
                 if (lane_id() == 0 && c) atomicAdd(&s_cnt[0], c);
             } else if (here) {
-                atomicAdd(&s_cnt[bucket_by_split(s_split, b, v[j])], 1u);
+                atomicAdd(&s_cnt[k[j]], 1u);
             }
         }
     }
@@ -818,13 +843,11 @@ __global__ __launch_bounds__(kThreads) void k_order_scatter(const uint64_t* __re
         for (int j = 0; j < kOrderIpt; ++j)
             v[j] = tk[min(tile * kOrderTile + uint64_t(j) * kThreads + threadIdx.x, total - 1)];
         __syncthreads();
+        buckets_by_split(s_split, b, v, br);
 #pragma unroll
         for (int j = 0; j < kOrderIpt; ++j) {
             if (tile * kOrderTile + uint64_t(j) * kThreads + threadIdx.x >= total) v[j] = 0;
-            if (v[j] != 0) {
-                const uint32_t k = bucket_by_split(s_split, b, v[j]);
-                br[j] = k << 16 | atomicAdd(&s_cnt[k], 1u);
-            }
+            if (v[j] != 0) br[j] = br[j] << 16 | atomicAdd(&s_cnt[br[j]], 1u);
         }
         __syncthreads();
         // The tile's place in each bucket's range.
@@ -844,46 +867,73 @@ __global__ __launch_bounds__(kThreads) void k_order_scatter(const uint64_t* __re
     }
 }
 
-__global__ __launch_bounds__(kThreads) void k_order_sort(const uint64_t* __restrict__ split,
-                                                         const uint32_t* __restrict__ totals, uint64_t* keys_a,
-                                                         uint32_t* slots_a, uint64_t* keys_b, uint32_t* slots_b,
-                                                         uint64_t* __restrict__ out, uint32_t* __restrict__ rank_of_slot,
-                                                         uint64_t* __restrict__ count)
+// The place of `key` among the n ascending keys of s_key that hold it.
+__device__ __forceinline__ uint32_t place_in(const uint64_t* s_key, uint32_t n, uint64_t key)
 {
+    uint32_t lo = 0;
+    for (uint32_t len = n; len > 1;) {
+        const uint32_t half = len / 2;
+        lo += s_key[lo + half] <= key ? half : 0u;
+        len -= half;
+    }
+    return lo;
+}
+
+// Only the masks are sorted; a slot's rank is its mask's place among them.
+__global__ __launch_bounds__(kOrderSortThreads) void k_order_sort(const uint64_t* __restrict__ split,
+                                                                  const uint32_t* __restrict__ totals,
+                                                                  uint64_t* keys_a, uint32_t* slots_a,
+                                                                  uint64_t* keys_b, uint32_t* slots_b,
+                                                                  uint64_t* __restrict__ out,
+                                                                  uint32_t* __restrict__ rank_of_slot,
+                                                                  uint64_t* __restrict__ count)
+{
+    constexpr uint32_t T = kOrderSortThreads;
+    constexpr int E = int(kOrderCap / T);
     __shared__ uint64_t s_key[kOrderCap];
-    __shared__ uint32_t s_slot[kOrderCap];
-    __shared__ uint64_t s_red[kThreads / kWave];
+    __shared__ uint64_t s_red[T / kWave];
     const uint32_t buckets = 1u << uint32_t(split[0]);
     for (uint32_t bucket = blockIdx.x; bucket < buckets; bucket += gridDim.x) {
         uint64_t below = 0;
-        for (uint32_t i = threadIdx.x; i < bucket; i += kThreads) below += totals[i];
-        const uint64_t start = block_reduce_sum<kThreads>(below, s_red);
+        for (uint32_t i = threadIdx.x; i < bucket; i += T) below += totals[i];
+        const uint64_t start = block_reduce_sum<T>(below, s_red);
         const uint32_t cnt = totals[bucket];
         if (bucket + 1 == buckets && threadIdx.x == 0) *count = start + cnt;
+        const bool whole = cnt <= kOrderCap;
         for (uint32_t c0 = 0; c0 < cnt; c0 += kOrderCap) {
-            const uint32_t n = min(kOrderCap, cnt - c0), n2 = pow2_at_least(n);
-            for (uint32_t i = threadIdx.x; i < n2; i += kThreads) {
-                s_key[i] = i < n ? keys_a[start + c0 + i] : ~0ull;
-                s_slot[i] = i < n ? slots_a[start + c0 + i] : ~0u;
+            const uint32_t n = min(kOrderCap, cnt - c0);
+            const uint64_t at = start + c0;
+            // The thread's masks and slots, kept for their ranks.
+            uint64_t key[E];
+            uint32_t slot[E];
+#pragma unroll
+            for (int e = 0; e < E; ++e) {
+                const uint32_t i = min(threadIdx.x + uint32_t(e) * T, n - 1);
+                key[e] = keys_a[at + i];
+                slot[e] = slots_a[at + i];
             }
-            lds_sort<kThreads, true>(s_key, s_slot, n2);
-            for (uint32_t i = threadIdx.x; i < n; i += kThreads) {
-                if (cnt <= kOrderCap) {
-                    out[start + i] = s_key[i];
-                    rank_of_slot[s_slot[i]] = uint32_t(start + i);
-                } else {
-                    keys_a[start + c0 + i] = s_key[i];
-                    slots_a[start + c0 + i] = s_slot[i];
+#pragma unroll
+            for (int e = 0; e < E; ++e)
+                if (threadIdx.x + uint32_t(e) * T < n) s_key[threadIdx.x + uint32_t(e) * T] = key[e];
+            block_merge_sort<int(T), E>(s_key, n);
+            uint64_t* const dst = whole ? out + start : keys_b + at;
+            for (uint32_t i = threadIdx.x; i < n; i += T) dst[i] = s_key[i];
+#pragma unroll
+            for (int e = 0; e < E; ++e) {
+                if (threadIdx.x + uint32_t(e) * T < n) {
+                    const uint32_t p = place_in(s_key, n, key[e]);
+                    if (whole) rank_of_slot[slot[e]] = uint32_t(start) + p;
+                    else slots_b[at + p] = slot[e];
                 }
             }
             __syncthreads();
         }
-        if (cnt <= kOrderCap) continue;
+        if (whole) continue;
         // Pairs of sorted pieces, merged by each key's place in the other one.
-        uint64_t *ka = keys_a + start, *kb = keys_b + start;
-        uint32_t *sa = slots_a + start, *sb = slots_b + start;
+        uint64_t *ka = keys_b + start, *kb = keys_a + start;
+        uint32_t *sa = slots_b + start, *sb = slots_a + start;
         for (uint64_t piece = kOrderCap; piece < cnt; piece *= 2) {
-            for (uint64_t i = threadIdx.x; i < cnt; i += kThreads) {
+            for (uint64_t i = threadIdx.x; i < cnt; i += T) {
                 const uint64_t first = i / (2 * piece) * (2 * piece);
                 const uint64_t mid = min(first + piece, uint64_t(cnt)), last = min(first + 2 * piece, uint64_t(cnt));
                 const uint64_t key = ka[i];
@@ -905,7 +955,7 @@ __global__ __launch_bounds__(kThreads) void k_order_sort(const uint64_t* __restr
             sa = sb;
             sb = st;
         }
-        for (uint64_t i = threadIdx.x; i < cnt; i += kThreads) {
+        for (uint64_t i = threadIdx.x; i < cnt; i += T) {
             out[start + i] = ka[i];
             rank_of_slot[sa[i]] = uint32_t(start + i);
         }
@@ -1938,7 +1988,7 @@ void launch_leaf_order(hipStream_t s, const LeafOrderArgs& a, uint64_t slot_boun
     // At most one bucket per kOrderMean / 2 leaves (the sample's error aside;
     // the workgroups stride over the buckets there are).
     const uint64_t buckets = std::min<uint64_t>(kOrderMaxBuckets, std::max<uint64_t>(1, leaf_bound / (kOrderMean / 2)));
-    hipLaunchKernelGGL(k_order_sort, dim3(uint32_t(buckets)), dim3(kThreads), 0, s, a.split, a.totals, a.list_keys[0],
+    hipLaunchKernelGGL(k_order_sort, dim3(uint32_t(buckets)), dim3(kOrderSortThreads), 0, s, a.split, a.totals, a.list_keys[0],
                        a.list_slots[0], a.list_keys[1], a.list_slots[1], a.out, a.rank_of_slot, a.count);
 }
 

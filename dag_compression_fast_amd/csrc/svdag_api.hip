@@ -150,7 +150,6 @@ struct svdag_context {
     uint32_t seg_first_bits = 0;
     int top_first = kTopFirstAuto;
     bool table_estimate = true;
-    uint64_t vox_stage_max = kVoxStageMaxBytes;
     int host_threads = 1;
     // Stage markers of the work in flight (bounded completion wait).
     static constexpr int kMaxMarks = 64;
@@ -1400,8 +1399,7 @@ int svdag_set_option(svdag_context* ctx, int32_t option, int64_t value)
         return 0;
     case SVDAG_OPT_VOXEL_STAGE_BYTES:
         if (value < 0) return set_error(SVDAG_ERR_ARGUMENT, "stage bytes must be >= 0");
-        ctx->vox_stage_max = uint64_t(value);
-        return 0;
+        return 0;  // no staging area is used
     case SVDAG_OPT_SORT_TILE:
         if (value != 4096 && value != 8192) return set_error(SVDAG_ERR_ARGUMENT, "sort tile must be 4096 or 8192 keys");
         ctx->sort_ipt = value == 8192 ? kSortIptLarge : kSortIptSmall;
@@ -1891,7 +1889,7 @@ int svdag_voxelize_triangles(svdag_context* ctx, const double* d_tris, uint64_t 
     if (n_tris == 0) return 0;
     hipStream_t st = ctx->stream;
     // Triangle stage in the arena: constants, row counts and offsets, and the
-    // counters [triangles, rows, columns, keys, rectangle columns, error].
+    // counters [triangles, rows, units, keys, rectangle columns, error].
     Carver cv;
     const uint64_t o_setup = cv.take(sizeof(TriSetup) * n_tris);
     const uint64_t o_rows = cv.take(4 * n_tris);
@@ -1913,51 +1911,51 @@ int svdag_voxelize_triangles(svdag_context* ctx, const double* d_tris, uint64_t 
     if (h[5] & kErrKeyRange) return set_error(SVDAG_ERR_ARGUMENT, "a triangle has a non-finite coordinate");
     const uint64_t n_rows = h[1], rect_columns = h[4];
     if (n_rows == 0 || rect_columns == 0) return 0;
-    // Row table and tile arrays (sized for the rectangles' columns, which bound
-    // the kept ones), then the keys (the caller's, svdag_free_keys).
-    const uint64_t ntiles = tiles(rect_columns, kVoxTileItems);
+    // Row table, then the unit stage's arrays, then the keys (the caller's,
+    // svdag_free_keys).
     Carver rows_cv;
     const uint64_t o_tri = rows_cv.take(4 * n_rows), o_u = rows_cv.take(4 * n_rows), o_w0 = rows_cv.take(4 * n_rows);
-    const uint64_t o_cols = rows_cv.take(4 * n_rows), o_coff = rows_cv.take(8 * n_rows);
-    const uint64_t o_tcnt = rows_cv.take(4 * ntiles), o_toff = rows_cv.take(8 * ntiles), o_trow = rows_cv.take(8 * (ntiles + 1));
+    const uint64_t o_cols = rows_cv.take(4 * n_rows), o_uoff = rows_cv.take(8 * n_rows);
     const uint64_t nrt = tiles(n_rows, kVoxTileItems);
-    const uint64_t o_rtc = rows_cv.take(4 * nrt), o_rto = rows_cv.take(8 * nrt);
+    const uint64_t o_rtu = rows_cv.take(4 * nrt), o_rto = rows_cv.take(8 * nrt);
     void* mem = nullptr;
     TRY(device_alloc(ctx, &mem, rows_cv.off));
     char* M = static_cast<char*>(mem);
     const VoxRows R{reinterpret_cast<uint32_t*>(M + o_tri), reinterpret_cast<uint32_t*>(M + o_u),
                     reinterpret_cast<uint32_t*>(M + o_w0), reinterpret_cast<uint32_t*>(M + o_cols),
-                    reinterpret_cast<uint64_t*>(M + o_coff)};
-    uint32_t* tcounts = reinterpret_cast<uint32_t*>(M + o_tcnt);
-    uint64_t* toffs = reinterpret_cast<uint64_t*>(M + o_toff);
-    uint64_t* trow = reinterpret_cast<uint64_t*>(M + o_trow);
-    launch_row_setup(st, setup, roff, cnt, cnt + 1, n_rows, R, reinterpret_cast<uint32_t*>(M + o_rtc),
+                    reinterpret_cast<uint64_t*>(M + o_uoff)};
+    launch_row_setup(st, setup, roff, cnt, cnt + 1, n_rows, R, reinterpret_cast<uint32_t*>(M + o_rtu),
                      reinterpret_cast<uint64_t*>(M + o_rto), cnt + 2, reinterpret_cast<unsigned long long*>(cnt + 5));
     uint64_t h2[6] = {};
     if (hipMemcpyAsync(h2, cnt, sizeof(h2), hipMemcpyDeviceToHost, st) != hipSuccess) {
         device_release(ctx, mem);
-        return set_error(SVDAG_ERR_HIP, "column read-back failed");
+        return set_error(SVDAG_ERR_HIP, "unit read-back failed");
     }
     int rc = finish(ctx, "voxelize (rows)");
     if (rc == 0 && h2[5]) rc = set_error(SVDAG_ERR_CAPACITY, "a block of %llu rows spans 2^32 or more voxel columns",
                                          (unsigned long long)kVoxTileItems);
     if (rc == 0 && h2[2] > rect_columns) rc = set_error(SVDAG_ERR_INTERNAL, "row ranges exceed the rectangles");
-    const uint64_t columns = h2[2];
-    if (rc != 0 || columns == 0) {
+    const uint64_t units = h2[2];
+    if (rc != 0 || units == 0) {
         device_release(ctx, mem);
         return rc;
     }
-    // One evaluation of the columns with a staging area of 16 bytes per
-    // column; past the context's limit (or if it cannot be allocated), two
-    // (count, then write in place).
-    const uint64_t stage_bytes = tiles(columns, kVoxTileItems) * 2 * kVoxTileItems * sizeof(uint64_t);
-    void* stage = nullptr;
-    if (stage_bytes <= ctx->vox_stage_max && device_alloc(ctx, &stage, stage_bytes) != 0) stage = nullptr;
-    if (stage)
-        launch_vox_emit(st, setup, R, cnt + 1, cnt + 2, columns, depth, trow, tcounts, static_cast<uint64_t*>(stage));
-    else
-        launch_vox_count(st, setup, R, cnt + 1, cnt + 2, columns, depth, trow, tcounts);
-    launch_scan_counts(st, tcounts, toffs, cnt + 2, kVoxTileItems, cnt + 3);
+    const uint64_t ntiles = tiles(units, kVoxUnitTile);
+    Carver unit_cv;
+    const uint64_t o_bits = unit_cv.take(2 * units);
+    const uint64_t o_tcnt = unit_cv.take(4 * ntiles), o_toff = unit_cv.take(8 * ntiles), o_trow = unit_cv.take(8 * (ntiles + 1));
+    void* unit_mem = nullptr;
+    if ((rc = device_alloc(ctx, &unit_mem, unit_cv.off)) != 0) {
+        device_release(ctx, mem);
+        return rc;
+    }
+    char* W = static_cast<char*>(unit_mem);
+    uint16_t* bits = reinterpret_cast<uint16_t*>(W + o_bits);
+    uint32_t* tcounts = reinterpret_cast<uint32_t*>(W + o_tcnt);
+    uint64_t* toffs = reinterpret_cast<uint64_t*>(W + o_toff);
+    uint64_t* trow = reinterpret_cast<uint64_t*>(W + o_trow);
+    launch_vox_count(st, setup, R, cnt + 1, cnt + 2, units, depth, trow, bits, tcounts);
+    launch_scan_counts(st, tcounts, toffs, cnt + 2, kVoxUnitTile, cnt + 3);
     if (hipMemcpyAsync(h, cnt, sizeof(h), hipMemcpyDeviceToHost, st) != hipSuccess)
         rc = set_error(SVDAG_ERR_HIP, "count read-back failed");
     if (rc == 0) rc = finish(ctx, "voxelize (count)");
@@ -1965,15 +1963,11 @@ int svdag_voxelize_triangles(svdag_context* ctx, const double* d_tris, uint64_t 
     void* out = nullptr;
     if (rc == 0 && keys) rc = device_alloc(ctx, &out, 8 * keys);
     if (rc == 0 && keys) {
-        if (stage)
-            launch_vox_compact(st, static_cast<const uint64_t*>(stage), tcounts, toffs, cnt + 2, columns,
-                               static_cast<uint64_t*>(out));
-        else
-            launch_vox_write(st, setup, R, trow, cnt + 1, cnt + 2, columns, depth, toffs, static_cast<uint64_t*>(out));
+        launch_vox_write(st, setup, R, trow, cnt + 2, units, depth, bits, toffs, static_cast<uint64_t*>(out));
         rc = hipGetLastError() == hipSuccess ? finish(ctx, "voxelize (write)")
                                              : set_error(SVDAG_ERR_HIP, "voxelizer launch failed");
     }
-    device_release(ctx, stage);
+    device_release(ctx, unit_mem);
     device_release(ctx, mem);
     if (rc != 0) {
         device_release(ctx, out);

@@ -434,16 +434,16 @@ struct TriSetup {
     uint32_t nw;
     int32_t a, u, w, planes;
 };
-constexpr uint64_t kVoxTileItems = 2048;  // columns per voxeliser tile
-constexpr uint64_t kVoxStageMaxBytes = 4ull << 30;  // default largest one-pass staging area
+constexpr uint64_t kVoxTileItems = 2048;  // rows per tile of the row stages
+constexpr uint64_t kVoxUnitTile = 256;    // units (at most 8 columns of one row) per voxeliser tile
 
 // Per-row table of the triangles' column rectangles (a row runs along w).
 struct VoxRows {
-    uint32_t* tri;      // triangle of the row
-    uint32_t* u;        // its u coordinate
-    uint32_t* w0;       // first column kept
-    uint32_t* cols;     // columns kept (a conservative superset of those the rule can emit)
-    uint64_t* col_off;  // exclusive scan of cols
+    uint32_t* tri;       // triangle of the row
+    uint32_t* u;         // its u coordinate
+    uint32_t* w0;        // first column kept
+    uint32_t* cols;      // columns kept (a conservative superset of those the rule can emit)
+    uint64_t* unit_off;  // exclusive scan of the rows' units
 };
 
 // rows[t] = rows of triangle t's rectangle (tris: 9 doubles per triangle);
@@ -451,32 +451,25 @@ struct VoxRows {
 // non-finite coordinate sets kErrKeyRange in *err.
 void launch_tri_setup(hipStream_t s, const double* tris, uint64_t n_tris, int depth, TriSetup* setup, uint32_t* rows,
                       uint64_t* rect_columns, unsigned long long* err);
-// rows.tri / u / w0 / cols / col_off for the *n_rows_dev rows (n_rows on the
-// host), the column total into *total_cols_dev; row_off = exclusive scan of
-// the per-triangle row counts; tile_cols / tile_off: one entry per
+// rows.tri / u / w0 / cols / unit_off for the *n_rows_dev rows (n_rows on the
+// host), the unit total into *total_units_dev; row_off = exclusive scan of
+// the per-triangle row counts; tile_units / tile_off: one entry per
 // kVoxTileItems rows; a tile of rows with 2^32 or more columns sets
 // kErrInternal in *err.
 void launch_row_setup(hipStream_t s, const TriSetup* setup, const uint64_t* row_off, const uint64_t* n_tris_dev,
-                      const uint64_t* n_rows_dev, uint64_t n_rows, const VoxRows& rows, uint32_t* tile_cols,
-                      uint64_t* tile_off, uint64_t* total_cols_dev, unsigned long long* err);
-// Voxels per tile of kVoxTileItems global columns (*total_cols_dev in all, at
-// most total_cols_bound).  tile_row (tiles + 1 entries) receives each tile's
-// first row; the write pass reads it.
+                      const uint64_t* n_rows_dev, uint64_t n_rows, const VoxRows& rows, uint32_t* tile_units,
+                      uint64_t* tile_off, uint64_t* total_units_dev, unsigned long long* err);
+// Voxels per tile of kVoxUnitTile units (total_units in all, also in
+// *total_units_dev) into tile_counts, and per unit the voxels that are in
+// (bits).  tile_row (tiles + 1 entries) receives each tile's first row; the
+// write pass reads both.
 void launch_vox_count(hipStream_t s, const TriSetup* setup, const VoxRows& rows, const uint64_t* n_rows_dev,
-                      const uint64_t* total_cols_dev, uint64_t total_cols_bound, int depth, uint64_t* tile_row,
-                      uint32_t* tile_counts);
+                      const uint64_t* total_units_dev, uint64_t total_units, int depth, uint64_t* tile_row,
+                      uint16_t* bits, uint32_t* tile_counts);
+// The keys, each tile's at tile_offsets[tile] (exclusive scan of the counts).
 void launch_vox_write(hipStream_t s, const TriSetup* setup, const VoxRows& rows, const uint64_t* tile_row,
-                      const uint64_t* n_rows_dev, const uint64_t* total_cols_dev, uint64_t total_cols_bound, int depth,
+                      const uint64_t* total_units_dev, uint64_t total_units, int depth, const uint16_t* bits,
                       const uint64_t* tile_offsets, uint64_t* keys);
-// One evaluation of the columns: tile t's keys go to stage[t * 2 * kVoxTileItems
-// ...] (2 * kVoxTileItems keys per tile of staging), their count to
-// tile_counts[t]; total_cols = the columns (known on the host).  Then each
-// tile's keys move to tile_offsets[t] (exclusive scan of the counts).
-void launch_vox_emit(hipStream_t s, const TriSetup* setup, const VoxRows& rows, const uint64_t* n_rows_dev,
-                     const uint64_t* total_cols_dev, uint64_t total_cols, int depth, uint64_t* tile_row,
-                     uint32_t* tile_counts, uint64_t* stage);
-void launch_vox_compact(hipStream_t s, const uint64_t* stage, const uint32_t* tile_counts, const uint64_t* tile_offsets,
-                        const uint64_t* total_cols_dev, uint64_t total_cols, uint64_t* keys);
 
 // Per pixel: the first voxel hit and its colour (the reference's trace_paths).
 void launch_trace_paths(hipStream_t s, const uint32_t* words, uint64_t n_words, int depth,

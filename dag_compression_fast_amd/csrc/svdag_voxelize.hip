@@ -17,15 +17,21 @@
 //   k_row_setup     per row: the columns whose centres can pass the dominant
 //                   projection's edge tests (a conservative superset, so the
 //                   exact per-column test below decides; about a fifth of the
-//                   rectangle for the triangle workload)
-//   (scan)          column offsets per row
-//   k_vox_emit      tile of 2048 global columns: its keys (at most two per
-//                   column) into the tile's 4096-key staging region, and
-//                   their count
+//                   rectangle for the triangle workload), cut into units of at
+//                   most 8 columns
+//   (scan)          unit offsets per row
+//   k_vox_count     one thread per unit: its columns' tests, two result bits
+//                   per column, keys per tile of 256 units
 //   (scan)          key offsets per tile
-//   k_vox_compact   each tile's staged keys to its offset
-// When the staging area would be too large, k_vox_count counts the keys per
-// tile and k_vox_write evaluates the columns again to write them in place.
+//   k_vox_write     the columns with a bit set again, now only for their keys,
+//                   staged in LDS and written in runs
+// A unit never leaves its row, so a thread keeps its triangle's edge functions
+// in registers and the wave has no row changes to diverge on.  Threads that
+// walked 8 columns across rows reloaded them at nearly every column (some lane
+// of the wave always changed rows) and held their keys in scratch memory: 1307
+// us for 47.9M voxels of 20k triangles in a 2048^3 grid, and 172 us more to move
+// the keys out of per-tile staging areas; now 350 + 246 us.  Bound by the float64
+// divisions and edge tests and by the row lookups.
 #pragma clang fp contract(off)
 
 #include "svdag_device.hpp"
@@ -36,9 +42,11 @@ namespace svdag {
 namespace {
 
 constexpr int kVoxThreads = 256;
-constexpr int kVoxIpt = 8;
+constexpr int kVoxIpt = 8;  // rows per thread and tile in the row kernels
 constexpr uint64_t kVoxTile = uint64_t(kVoxThreads) * kVoxIpt;
 static_assert(kVoxTile == kVoxTileItems, "tile size shared with the planner");
+constexpr int kUnitCols = 8;  // columns per unit of work
+static_assert(kVoxThreads == kVoxUnitTile && 2 * kUnitCols <= 16, "one unit per thread, two result bits per column");
 
 __device__ __forceinline__ double pick3(const double (&v)[3], int i) { return i == 0 ? v[0] : (i == 1 ? v[1] : v[2]); }
 
@@ -149,9 +157,9 @@ __device__ __forceinline__ uint64_t owner_of(const uint64_t* __restrict__ off, u
 // one side at c* = -(nx * cu + d) / ny.  The bound is widened by the rounding
 // error of the test and of c* (far below 2^-46 of their magnitudes) plus one
 // column, so it never drops a column the test keeps.
-// Rows are handled in tiles of kVoxTile; each tile's column total goes to
-// tile_cols for the scan that k_row_offsets finishes (a total of 2^32 or more
-// sets kErrInternal in *err).
+// Rows are handled in tiles of kVoxTile; each tile's unit total goes to
+// tile_units for the scan that k_row_offsets finishes (a column total of 2^32 or
+// more sets kErrInternal in *err).
 __global__ __launch_bounds__(kVoxThreads) void k_row_setup(const TriSetup* __restrict__ setup,
                                                            const uint64_t* __restrict__ row_off,
                                                            const uint64_t* __restrict__ n_tris_ptr,
@@ -159,14 +167,14 @@ __global__ __launch_bounds__(kVoxThreads) void k_row_setup(const TriSetup* __res
                                                            uint32_t* __restrict__ row_tri, uint32_t* __restrict__ row_u,
                                                            uint32_t* __restrict__ row_w0,
                                                            uint32_t* __restrict__ row_cols,
-                                                           uint32_t* __restrict__ tile_cols,
+                                                           uint32_t* __restrict__ tile_units,
                                                            unsigned long long* __restrict__ err)
 {
     __shared__ uint64_t s_red[kVoxThreads / kWave];
     const uint64_t n_tris = *n_tris_ptr, n_rows = *n_rows_ptr;
     const uint64_t ntiles = (n_rows + kVoxTile - 1) / kVoxTile;
     for (uint64_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
-        uint64_t tile_sum = 0;
+        uint64_t tile_sum = 0, unit_sum = 0;
         const uint64_t end = min(n_rows, (tile + 1) * kVoxTile);
         for (uint64_t r = tile * kVoxTile + threadIdx.x; r < end; r += kVoxThreads) {
             const uint64_t t = owner_of(row_off, 0, n_tris, r);
@@ -198,20 +206,22 @@ __global__ __launch_bounds__(kVoxThreads) void k_row_setup(const TriSetup* __res
             row_w0[r] = uint32_t(lo);
             row_cols[r] = cols;
             tile_sum += cols;
+            unit_sum += (cols + kUnitCols - 1) / kUnitCols;
         }
         const uint64_t sum = block_reduce_sum<kVoxThreads>(tile_sum, s_red);
+        const uint64_t units = block_reduce_sum<kVoxThreads>(unit_sum, s_red);
         if (threadIdx.x == 0) {
-            tile_cols[tile] = uint32_t(sum);
+            tile_units[tile] = uint32_t(units);
             if (sum > 0xFFFFFFFFull) atomicOr(err, (unsigned long long)kErrInternal);
         }
     }
 }
 
-// col_off[r] = tile_off[tile] + the columns of the tile's rows before r.
+// unit_off[r] = tile_off[tile] + the units of the tile's rows before r.
 __global__ __launch_bounds__(kVoxThreads) void k_row_offsets(const uint32_t* __restrict__ row_cols,
                                                              const uint64_t* __restrict__ tile_off,
                                                              const uint64_t* __restrict__ n_rows_ptr,
-                                                             uint64_t* __restrict__ col_off)
+                                                             uint64_t* __restrict__ unit_off)
 {
     __shared__ uint32_t s_scan[kVoxThreads / kWave];
     const uint64_t n_rows = *n_rows_ptr;
@@ -222,218 +232,183 @@ __global__ __launch_bounds__(kVoxThreads) void k_row_offsets(const uint32_t* __r
         uint32_t mine = 0;
 #pragma unroll
         for (int i = 0; i < kVoxIpt; ++i) {
-            c[i] = r0 + i < n_rows ? row_cols[r0 + i] : 0u;
+            c[i] = r0 + i < n_rows ? (row_cols[r0 + i] + kUnitCols - 1) / kUnitCols : 0u;
             mine += c[i];
         }
         uint32_t unused;
         uint64_t o = tile_off[tile] + block_exclusive_scan<kVoxThreads>(mine, s_scan, unused);
 #pragma unroll
         for (int i = 0; i < kVoxIpt; ++i) {
-            if (r0 + i < n_rows) col_off[r0 + i] = o;
+            if (r0 + i < n_rows) unit_off[r0 + i] = o;
             o += c[i];
         }
     }
 }
 
-// Voxels of column (iu, iw) of triangle S (at most two), appended to k[] at
-// `found`; returns the new count.
-template <int N>
-__device__ __forceinline__ int column_voxels(const TriSetup& S, int64_t iu, int64_t iw, int64_t side, uint64_t (&k)[N],
-                                             int found)
+// The voxels [lo, hi] along the dominant axis whose centres are within one of
+// column crossing `ac` (at most two; lo > hi: none).
+__device__ __forceinline__ void column_range(double ac, int64_t side, int32_t& lo, int32_t& hi)
 {
-    const double cu = double(iu) + 0.5, cw = double(iw) + 0.5;
-    // The dominant projection (the plane of u and w) sees only the column:
-    // its edge tests are the same for every voxel of it.
-    for (int e = 0; e < 3; ++e)
-        if (S.ex[S.u][e] * cu + S.ey[S.u][e] * cw + S.ed[S.u][e] < 0) return found;
-    const double na = pick3(S.n, S.a), nu = pick3(S.n, S.u), nw = pick3(S.n, S.w);
-    const double ac = (S.nd - nu * cu - nw * cw) / na;
-    const int64_t k0 = int64_t(floor(ac - 1.0)), k1 = int64_t(floor(ac));
-    for (int64_t kk = max(k0, int64_t(0)); kk <= min(k1, side - 1); ++kk) {
-        const double ck = double(kk) + 0.5;
-        if (fabs(ck - ac) > 0.5) continue;
-        // Voxel centre: k + 1/2 along a, cu along u, cw along w.
-        const double cc[3] = {S.a == 0 ? ck : (S.u == 0 ? cu : cw), S.a == 1 ? ck : (S.u == 1 ? cu : cw),
-                              S.a == 2 ? ck : (S.u == 2 ? cu : cw)};
-        bool inside = true;
-        for (int p = 0; p < 3 && inside; ++p) {
-            if (!((S.planes >> p) & 1) || p == S.u) continue;  // edge-on here, or tested above
-            const double c0 = pick3(cc, p), c1 = pick3(cc, (p + 1) % 3);
-            for (int e = 0; e < 3; ++e)
-                if (S.ex[p][e] * c0 + S.ey[p][e] * c1 + S.ed[p][e] < 0) {
-                    inside = false;
-                    break;
-                }
-        }
-        if (!inside) continue;
-        const int64_t x = S.a == 0 ? kk : (S.u == 0 ? iu : iw);
-        const int64_t y = S.a == 1 ? kk : (S.u == 1 ? iu : iw);
-        const int64_t z = S.a == 2 ? kk : (S.u == 2 ? iu : iw);
-        k[found++] = morton3(uint32_t(x), uint32_t(y), uint32_t(z));
+    if (fabs(ac) < 0x1p30) {
+        lo = max(int32_t(floor(ac - 1.0)), 0);
+        hi = min(int32_t(floor(ac)), int32_t(side - 1));
+    } else {  // far outside the grid, or not a number
+        const int64_t k0 = max(int64_t(floor(ac - 1.0)), int64_t(0)), k1 = min(int64_t(floor(ac)), side - 1);
+        lo = k0 <= k1 ? int32_t(k0) : 1;
+        hi = k0 <= k1 ? int32_t(k1) : 0;
     }
-    return found;
 }
 
-// The rows of tile t's columns lie in [tile_row[t], tile_row[t + 1] + 1)
-// (tile_row[t] = row of the tile's first column, one entry past the last
-// tile), found by one thread per tile.
-__global__ __launch_bounds__(kVoxThreads) void k_tile_rows(const uint64_t* __restrict__ col_off,
+// The unit rows: unit_off is the exclusive scan of the rows' unit counts.
+struct RowTable {
+    const uint32_t* tri;
+    const uint32_t* u;
+    const uint32_t* w0;
+    const uint32_t* cols;
+    const uint64_t* unit_off;
+};
+
+// Rows of unit tile t lie in [tile_row[t], tile_row[t + 1] + 1) (tile_row[t] =
+// row of the tile's first unit, one entry past the last tile), found by one
+// thread per tile.
+__global__ __launch_bounds__(kVoxThreads) void k_tile_rows(const uint64_t* __restrict__ unit_off,
                                                            const uint64_t* __restrict__ n_rows_ptr,
                                                            const uint64_t* __restrict__ total_ptr,
                                                            uint64_t* __restrict__ tile_row)
 {
     const uint64_t n_rows = *n_rows_ptr, total = *total_ptr;
-    const uint64_t ntiles = (total + kVoxTile - 1) / kVoxTile;
+    const uint64_t ntiles = (total + kVoxThreads - 1) / kVoxThreads;
     for (uint64_t t = uint64_t(blockIdx.x) * kVoxThreads + threadIdx.x; t <= ntiles;
          t += uint64_t(gridDim.x) * kVoxThreads)
-        tile_row[t] = t < ntiles ? owner_of(col_off, 0, n_rows, t * kVoxTile) : n_rows - 1;
+        tile_row[t] = t < ntiles ? owner_of(unit_off, 0, n_rows, t * kVoxThreads) : n_rows - 1;
 }
 
-struct RowTable {
-    const uint32_t* tri;
-    const uint32_t* u;
-    const uint32_t* w0;
-    const uint64_t* col_off;  // exclusive scan of the rows' column counts
+// The thread's unit of tile `tile`: its triangle, row, first column and columns.
+struct Unit {
+    uint32_t tri, u, w0;
+    int cols;  // 0: past the last unit
 };
-
-// Keys of the thread's kVoxIpt consecutive columns of tile `tile` (at most two
-// per column) into k[]; returns how many.  One row search per thread; the
-// columns then step along w, to the next non-empty row at a row's end.
-constexpr int kVoxKeys = 2 * kVoxIpt;
-
-__device__ __forceinline__ int thread_columns(const TriSetup* __restrict__ setup, const RowTable& R,
-                                              const uint64_t* __restrict__ tile_row, uint64_t n_rows, uint64_t total,
-                                              uint64_t tile, int64_t side, uint64_t (&k)[kVoxKeys])
+__device__ __forceinline__ Unit unit_of(const RowTable& R, const uint64_t* __restrict__ tile_row, uint64_t total,
+                                        uint64_t tile)
 {
-    const uint64_t g0 = tile * kVoxTile + uint64_t(threadIdx.x) * kVoxIpt;
-    if (g0 >= total) return 0;
-    const uint64_t g1 = min(g0 + uint64_t(kVoxIpt), total);
-    const uint64_t hi = tile_row[tile + 1] + 1;
-    uint64_t r = owner_of(R.col_off, tile_row[tile], hi, g0);
-    uint64_t r_end = r + 1 < n_rows ? R.col_off[r + 1] : total;
-    uint32_t t = R.tri[r];
-    int64_t iu = R.u[r], iw = int64_t(R.w0[r]) + int64_t(g0 - R.col_off[r]);
-    int found = 0;
-#pragma unroll 1
-    for (uint64_t g = g0; g < g1; ++g) {
-        if (g >= r_end) {  // the next row with columns starts at g
-            r = owner_of(R.col_off, r + 1, hi, g);
-            r_end = r + 1 < n_rows ? R.col_off[r + 1] : total;
-            t = R.tri[r];
-            iu = R.u[r];
-            iw = R.w0[r];
-        }
-        found = column_voxels(setup[t], iu, iw, side, k, found);
-        ++iw;
-    }
-    return found;
+    const uint64_t g = tile * kVoxThreads + threadIdx.x;
+    if (g >= total) return Unit{0, 0, 0, 0};
+    const uint64_t r = owner_of(R.unit_off, tile_row[tile], tile_row[tile + 1] + 1, g);
+    const uint32_t first = uint32_t(g - R.unit_off[r]) * kUnitCols;
+    return Unit{R.tri[r], R.u[r], R.w0[r] + first, int(min(uint32_t(kUnitCols), R.cols[r] - first))};
 }
 
+// bits[unit]: bit 2i + j says that voxel lo + j of the unit's column i is in
+// (lo: column_range); counts[tile] = the tile's bits set.
 __global__ __launch_bounds__(kVoxThreads) void k_vox_count(const TriSetup* __restrict__ setup, RowTable R,
                                                            const uint64_t* __restrict__ tile_row,
-                                                           const uint64_t* __restrict__ n_rows_ptr,
                                                            const uint64_t* __restrict__ total_ptr, int64_t side,
-                                                           uint32_t* __restrict__ counts)
+                                                           uint16_t* __restrict__ bits, uint32_t* __restrict__ counts)
 {
     __shared__ uint64_t s_red[kVoxThreads / kWave];
-    const uint64_t n_rows = *n_rows_ptr, total = *total_ptr;
-    const uint64_t ntiles = (total + kVoxTile - 1) / kVoxTile;
+    const uint64_t total = *total_ptr;
+    const uint64_t ntiles = (total + kVoxThreads - 1) / kVoxThreads;
     for (uint64_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
-        uint64_t k[kVoxKeys];
-        const int mine = thread_columns(setup, R, tile_row, n_rows, total, tile, side, k);
-        const uint64_t sum = block_reduce_sum<kVoxThreads>(uint64_t(mine), s_red);
+        const Unit U = unit_of(R, tile_row, total, tile);
+        uint32_t found = 0;
+        if (U.cols) {
+            const TriSetup& S = setup[U.tri];
+            const int a = S.a, u = S.u, w = S.w, planes = S.planes;
+            const double cu = double(int64_t(U.u)) + 0.5;
+            // Edge functions of the planes (u, w), (a, u) and (w, a), with the
+            // terms that the row fixes multiplied out.
+            double uu[3], uw[3], ud[3], aa[3], au[3], ad[3], ww[3], wa[3], wd[3];
+#pragma unroll
+            for (int e = 0; e < 3; ++e) {
+                uu[e] = S.ex[u][e] * cu;
+                uw[e] = S.ey[u][e];
+                ud[e] = S.ed[u][e];
+                aa[e] = S.ex[a][e];
+                au[e] = S.ey[a][e] * cu;
+                ad[e] = S.ed[a][e];
+                ww[e] = S.ex[w][e];
+                wa[e] = S.ey[w][e];
+                wd[e] = S.ed[w][e];
+            }
+            const double q = S.nd - pick3(S.n, u) * cu, nw = pick3(S.n, w), na = pick3(S.n, a);
+            const bool plane_a = (planes >> a) & 1, plane_w = (planes >> w) & 1;  // else edge-on there
+#pragma unroll 1
+            for (int i = 0; i < U.cols; ++i) {
+                const double cw = double(int64_t(U.w0) + i) + 0.5;
+                // The dominant projection sees only the column.
+                bool in = true;
+#pragma unroll
+                for (int e = 0; e < 3; ++e) in &= !(uu[e] + uw[e] * cw + ud[e] < 0);
+                if (!in) continue;
+                const double ac = (q - nw * cw) / na;
+                int32_t lo, hi;
+                column_range(ac, side, lo, hi);
+                double wx[3];
+#pragma unroll
+                for (int e = 0; e < 3; ++e) wx[e] = ww[e] * cw;
+                for (int32_t kk = lo; kk <= hi; ++kk) {
+                    const double ck = double(kk) + 0.5;
+                    bool ok = !(fabs(ck - ac) > 0.5);
+#pragma unroll
+                    for (int e = 0; e < 3; ++e) {
+                        ok &= !(plane_a && aa[e] * ck + au[e] + ad[e] < 0);
+                        ok &= !(plane_w && wx[e] + wa[e] * ck + wd[e] < 0);
+                    }
+                    found |= uint32_t(ok) << (2 * i + (kk - lo));
+                }
+            }
+            bits[tile * kVoxThreads + threadIdx.x] = uint16_t(found);
+        }
+        const uint64_t sum = block_reduce_sum<kVoxThreads>(uint64_t(__popc(found)), s_red);
         if (threadIdx.x == 0) counts[tile] = uint32_t(sum);
     }
 }
 
+// The keys of the voxels whose bit is set, in unit, column and voxel order.
 __global__ __launch_bounds__(kVoxThreads) void k_vox_write(const TriSetup* __restrict__ setup, RowTable R,
                                                            const uint64_t* __restrict__ tile_row,
-                                                           const uint64_t* __restrict__ n_rows_ptr,
                                                            const uint64_t* __restrict__ total_ptr, int64_t side,
+                                                           const uint16_t* __restrict__ bits,
                                                            const uint64_t* __restrict__ tile_offsets,
                                                            uint64_t* __restrict__ keys)
 {
+    constexpr uint64_t kThirds = 0x1249249249249249ull;
     __shared__ uint32_t s_scan[kVoxThreads / kWave];
-    const uint64_t n_rows = *n_rows_ptr, total = *total_ptr;
-    const uint64_t ntiles = (total + kVoxTile - 1) / kVoxTile;
+    __shared__ uint64_t s_keys[kVoxThreads * 2 * kUnitCols];
+    const uint64_t total = *total_ptr;
+    const uint64_t ntiles = (total + kVoxThreads - 1) / kVoxThreads;
     for (uint64_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
-        uint64_t k[kVoxKeys];
-        const int mine = thread_columns(setup, R, tile_row, n_rows, total, tile, side, k);
-        uint32_t unused;
-        const uint64_t o = tile_offsets[tile] + block_exclusive_scan<kVoxThreads>(uint32_t(mine), s_scan, unused);
-#pragma unroll
-        for (int j = 0; j < kVoxKeys; ++j)
-            if (j < mine) keys[o + j] = k[j];
-    }
-}
-
-// As k_vox_write, but the keys go to the tile's staging region
-// stage[tile * 2 * kVoxTile ...] and the tile's count to counts[tile].
-__global__ __launch_bounds__(kVoxThreads) void k_vox_emit(const TriSetup* __restrict__ setup, RowTable R,
-                                                          const uint64_t* __restrict__ tile_row,
-                                                          const uint64_t* __restrict__ n_rows_ptr,
-                                                          const uint64_t* __restrict__ total_ptr, int64_t side,
-                                                          uint32_t* __restrict__ counts, uint64_t* __restrict__ stage)
-{
-    __shared__ uint32_t s_scan[kVoxThreads / kWave];
-    const uint64_t n_rows = *n_rows_ptr, total = *total_ptr;
-    const uint64_t ntiles = (total + kVoxTile - 1) / kVoxTile;
-    for (uint64_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
-        uint64_t k[kVoxKeys];
-        const int mine = thread_columns(setup, R, tile_row, n_rows, total, tile, side, k);
+        const uint64_t g = tile * kVoxThreads + threadIdx.x;
+        uint32_t left = g < total ? bits[g] : 0u;
         uint32_t tile_keys;
-        const uint64_t o = tile * 2 * kVoxTile + block_exclusive_scan<kVoxThreads>(uint32_t(mine), s_scan, tile_keys);
-#pragma unroll
-        for (int j = 0; j < kVoxKeys; ++j)
-            if (j < mine) stage[o + j] = k[j];
-        if (threadIdx.x == 0) counts[tile] = tile_keys;
-    }
-}
-
-// keys[offsets[tile] + j] = stage[tile * 2 * kVoxTile + j] for j < counts[tile].
-__global__ __launch_bounds__(kVoxThreads) void k_vox_compact(const uint64_t* __restrict__ stage,
-                                                             const uint32_t* __restrict__ counts,
-                                                             const uint64_t* __restrict__ offsets,
-                                                             const uint64_t* __restrict__ total_ptr,
-                                                             uint64_t* __restrict__ keys)
-{
-    const uint64_t ntiles = (*total_ptr + kVoxTile - 1) / kVoxTile;
-    for (uint64_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
-        const uint32_t c = counts[tile];
-        const uint64_t* src = stage + tile * 2 * kVoxTile;
-        uint64_t* dst = keys + offsets[tile];
-        for (uint32_t j = threadIdx.x; j < c; j += kVoxThreads) dst[j] = src[j];
+        uint32_t o = block_exclusive_scan<kVoxThreads>(uint32_t(__popc(left)), s_scan, tile_keys);
+        if (left) {
+            const Unit U = unit_of(R, tile_row, total, tile);
+            const TriSetup& S = setup[U.tri];
+            const int a = S.a, u = S.u, w = S.w;
+            const double cu = double(int64_t(U.u)) + 0.5;
+            const double q = S.nd - pick3(S.n, u) * cu, nw = pick3(S.n, w), na = pick3(S.n, a);
+            const uint64_t row = split_by_3(U.u) << (2 - u);
+            uint64_t col = split_by_3(U.w0);
+#pragma unroll 1
+            for (uint32_t i = 0; left; ++i, left >>= 2, col = ((col | ~kThirds) + 1) & kThirds) {
+                if (!(left & 3u)) continue;
+                const double cw = double(int64_t(U.w0) + i) + 0.5;
+                int32_t lo, hi;
+                column_range((q - nw * cw) / na, side, lo, hi);
+                const uint64_t rc = row | col << (2 - w);
+                if (left & 1u) s_keys[o++] = rc | split_by_3(uint32_t(lo)) << (2 - a);
+                if (left & 2u) s_keys[o++] = rc | split_by_3(uint32_t(lo) + 1) << (2 - a);
+            }
+        }
+        __syncthreads();
+        uint64_t* const dst = keys + tile_offsets[tile];
+        for (uint32_t j = threadIdx.x; j < tile_keys; j += kVoxThreads) dst[j] = s_keys[j];
+        __syncthreads();  // s_keys is rewritten by the next tile
     }
 }
 
 }  // namespace
-
-static int vox_grid(uint64_t columns_bound)
-{
-    const uint64_t tiles = (columns_bound + kVoxTile - 1) / kVoxTile;
-    return int(std::max<uint64_t>(1, std::min<uint64_t>(tiles, uint64_t(device_cu_count()) * 8)));
-}
-
-void launch_vox_emit(hipStream_t s, const TriSetup* setup, const VoxRows& rows, const uint64_t* n_rows_dev,
-                     const uint64_t* total_cols_dev, uint64_t total_cols, int depth, uint64_t* tile_row,
-                     uint32_t* tile_counts, uint64_t* stage)
-{
-    TimedLaunch t(kKVoxCount, s);
-    const uint64_t tiles = (total_cols + kVoxTile - 1) / kVoxTile;
-    hipLaunchKernelGGL(k_tile_rows, dim3(uint32_t((tiles + kVoxThreads) / kVoxThreads)), dim3(kVoxThreads), 0, s,
-                       rows.col_off, n_rows_dev, total_cols_dev, tile_row);
-    const RowTable R{rows.tri, rows.u, rows.w0, rows.col_off};
-    hipLaunchKernelGGL(k_vox_emit, dim3(vox_grid(total_cols)), dim3(kVoxThreads), 0, s, setup, R, tile_row,
-                       n_rows_dev, total_cols_dev, int64_t(1) << depth, tile_counts, stage);
-}
-
-void launch_vox_compact(hipStream_t s, const uint64_t* stage, const uint32_t* tile_counts, const uint64_t* tile_offsets,
-                        const uint64_t* total_cols_dev, uint64_t total_cols, uint64_t* keys)
-{
-    TimedLaunch t(kKVoxWrite, s);
-    hipLaunchKernelGGL(k_vox_compact, dim3(vox_grid(total_cols)), dim3(kVoxThreads), 0, s, stage, tile_counts,
-                       tile_offsets, total_cols_dev, keys);
-}
 
 void launch_tri_setup(hipStream_t s, const double* tris, uint64_t n_tris, int depth, TriSetup* setup, uint32_t* rows,
                       uint64_t* rect_columns, unsigned long long* err)
@@ -446,43 +421,44 @@ void launch_tri_setup(hipStream_t s, const double* tris, uint64_t n_tris, int de
 }
 
 void launch_row_setup(hipStream_t s, const TriSetup* setup, const uint64_t* row_off, const uint64_t* n_tris_dev,
-                      const uint64_t* n_rows_dev, uint64_t n_rows, const VoxRows& rows, uint32_t* tile_cols,
-                      uint64_t* tile_off, uint64_t* total_cols_dev, unsigned long long* err)
+                      const uint64_t* n_rows_dev, uint64_t n_rows, const VoxRows& rows, uint32_t* tile_units,
+                      uint64_t* tile_off, uint64_t* total_units_dev, unsigned long long* err)
 {
     if (n_rows == 0) return;
     const uint32_t grid = uint32_t(std::min<uint64_t>((n_rows + kVoxTile - 1) / kVoxTile, device_cu_count() * 8ull));
     {
         TimedLaunch t(kKVoxSetup, s);
         hipLaunchKernelGGL(k_row_setup, dim3(grid), dim3(kVoxThreads), 0, s, setup, row_off, n_tris_dev, n_rows_dev,
-                           rows.tri, rows.u, rows.w0, rows.cols, tile_cols, err);
+                           rows.tri, rows.u, rows.w0, rows.cols, tile_units, err);
     }
-    launch_scan_counts(s, tile_cols, tile_off, n_rows_dev, kVoxTile, total_cols_dev);
+    launch_scan_counts(s, tile_units, tile_off, n_rows_dev, kVoxTile, total_units_dev);
     TimedLaunch t(kKVoxSetup, s);
     hipLaunchKernelGGL(k_row_offsets, dim3(grid), dim3(kVoxThreads), 0, s, rows.cols, tile_off, n_rows_dev,
-                       rows.col_off);
+                       rows.unit_off);
 }
 
 void launch_vox_count(hipStream_t s, const TriSetup* setup, const VoxRows& rows, const uint64_t* n_rows_dev,
-                      const uint64_t* total_cols_dev, uint64_t total_cols_bound, int depth, uint64_t* tile_row,
-                      uint32_t* tile_counts)
+                      const uint64_t* total_units_dev, uint64_t total_units, int depth, uint64_t* tile_row,
+                      uint16_t* bits, uint32_t* tile_counts)
 {
     TimedLaunch t(kKVoxCount, s);
-    const uint64_t tiles = (total_cols_bound + kVoxTile - 1) / kVoxTile;
+    const uint64_t tiles = (total_units + kVoxThreads - 1) / kVoxThreads;
     hipLaunchKernelGGL(k_tile_rows, dim3(uint32_t((tiles + kVoxThreads) / kVoxThreads)), dim3(kVoxThreads), 0, s,
-                       rows.col_off, n_rows_dev, total_cols_dev, tile_row);
-    const RowTable R{rows.tri, rows.u, rows.w0, rows.col_off};
-    hipLaunchKernelGGL(k_vox_count, dim3(vox_grid(total_cols_bound)), dim3(kVoxThreads), 0, s, setup, R, tile_row,
-                       n_rows_dev, total_cols_dev, int64_t(1) << depth, tile_counts);
+                       rows.unit_off, n_rows_dev, total_units_dev, tile_row);
+    const RowTable R{rows.tri, rows.u, rows.w0, rows.cols, rows.unit_off};
+    hipLaunchKernelGGL(k_vox_count, dim3(resident_grid(k_vox_count, kVoxThreads, tiles)), dim3(kVoxThreads), 0, s, setup,
+                       R, tile_row, total_units_dev, int64_t(1) << depth, bits, tile_counts);
 }
 
 void launch_vox_write(hipStream_t s, const TriSetup* setup, const VoxRows& rows, const uint64_t* tile_row,
-                      const uint64_t* n_rows_dev, const uint64_t* total_cols_dev, uint64_t total_cols_bound, int depth,
+                      const uint64_t* total_units_dev, uint64_t total_units, int depth, const uint16_t* bits,
                       const uint64_t* tile_offsets, uint64_t* keys)
 {
     TimedLaunch t(kKVoxWrite, s);
-    const RowTable R{rows.tri, rows.u, rows.w0, rows.col_off};
-    hipLaunchKernelGGL(k_vox_write, dim3(vox_grid(total_cols_bound)), dim3(kVoxThreads), 0, s, setup, R, tile_row,
-                       n_rows_dev, total_cols_dev, int64_t(1) << depth, tile_offsets, keys);
+    const uint64_t tiles = (total_units + kVoxThreads - 1) / kVoxThreads;
+    const RowTable R{rows.tri, rows.u, rows.w0, rows.cols, rows.unit_off};
+    hipLaunchKernelGGL(k_vox_write, dim3(resident_grid(k_vox_write, kVoxThreads, tiles)), dim3(kVoxThreads), 0, s, setup,
+                       R, tile_row, total_units_dev, int64_t(1) << depth, bits, tile_offsets, keys);
 }
 
 }  // namespace svdag

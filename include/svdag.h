@@ -88,10 +88,8 @@ typedef enum svdag_option {
                                          estimate of the leaf masks (default); 0: from the leaf
                                          positions.  An estimate that proves too small makes the
                                          call rebuild with the bound-sized table. */
-    SVDAG_OPT_VOXEL_STAGE_BYTES = 9,  /* largest staging area of svdag_voxelize_triangles
-                                         (16 bytes per voxel column, default 4 GiB): within it
-                                         the columns are evaluated once, past it twice (count,
-                                         then write); 0 always takes two passes */
+    SVDAG_OPT_VOXEL_STAGE_BYTES = 9,  /* accepted (>= 0) and without effect: the voxelizer no
+                                         longer stages its keys */
     SVDAG_OPT_SEG_FIRST_BITS = 10,    /* batched builds that sort inside each chunk (chunk
                                          depth <= 9): digit width of that sort's first pass,
                                          0 = half the chunk-local bits (default); clamped so

@@ -317,6 +317,11 @@ struct BuildLayout {
     // lp_code on (nothing there is live before the leaf reduce).
     bool top_first = false;
     uint32_t top_shift = 0, top_bits = 0;
+    // Plain builds whose keys end grouped by 64^3 cell (launch_cell_reduce):
+    // after one pass (depths 7 to 9), or after a top digit and one segmented
+    // pass below it.  The cells' starts lie behind the keys in keys_b.
+    uint64_t cells = 0, cell_starts = 0;
+    uint32_t sort_lo = 0;  // lowest bit a top-digit-first sort orders
     uint64_t bucket_start = 0, seg_tiles = 0, seg_ct = 0, seg_counts = 0, seg_totals = 0, seg_starts = 0,
              seg_ntiles = 0;
 };
@@ -398,13 +403,28 @@ BuildLayout plan_build(uint64_t n, int depth, int key_bytes, uint32_t load_shift
     L.total = std::max(L.total, L.reg_mask + region_bytes);
     // Top digit first: a digit of radix_bits at the top of the code, whose
     // bucket-local keys fit 32 bits, with at most kSegMaxBits sorted below it.
-    const uint32_t lo = L.key_plan.shift[0];
-    const uint32_t top_shift = uint32_t(3 * depth - radix_bits);
+    // Grouping by 64^3 cell is enough where one pass below the top digit does
+    // it, and orders 3 bits less.
+    const uint32_t bits = uint32_t(3 * depth);
+    const uint32_t top_shift = bits - uint32_t(radix_bits);
+    const uint64_t cells = depth > 6 ? pow8_capped(depth - 6, 1ull << 30) : 0;
+    const bool cell_sort = top_first != kTopFirstNever && !batched && cells > 1 && cells_pay(cells, n) &&
+                           4 * cells <= uint64_t(kb) * n;
+    if (cell_sort && top_first == kTopFirstAuto && bits - kCellShift <= uint32_t(radix_bits)) {
+        L.cells = cells;
+        L.cell_starts = L.keys_b;
+        return L;
+    }
+    uint32_t lo = L.key_plan.shift[0];
+    const bool cells_below = cell_sort && top_shift > kCellShift && top_shift - kCellShift <= kMaxSegDigitBits &&
+                             4 * (cells + n) <= uint64_t(kb) * n;
+    if (cells_below) lo = kCellShift;
     L.top_first = top_first != kTopFirstNever && !batched && key_bytes == 8 && L.key_plan.passes >= 2 &&
                   (top_first == kTopFirstAlways || n >= kTopFirstMinKeys) && top_shift <= 32 && top_shift > lo &&
                   top_shift - lo <= kSegMaxBits;
     if (L.top_first) {
         L.top_shift = top_shift;
+        L.sort_lo = lo;
         L.top_bits = uint32_t(radix_bits);
         Carver t;
         t.off = L.lp_code;
@@ -416,6 +436,11 @@ BuildLayout plan_build(uint64_t n, int depth, int key_bytes, uint32_t load_shift
         L.seg_totals = t.take(4 * (uint64_t(kRadix) << kMaxSegDigitBits));
         L.seg_starts = t.take(4 * (uint64_t(kRadix) << kMaxSegDigitBits));
         L.seg_ntiles = t.take(8);
+        if (cells_below) {
+            L.cells = cells;
+            L.cell_starts = L.keys_b + 4 * n;  // the bucket-local keys fill half of keys_b
+            L.seg_starts = L.cell_starts;
+        }
         L.total = std::max(L.total, t.off);
     }
     return L;
@@ -673,9 +698,10 @@ struct BatchLayout {
     uint64_t offsets = 0, seg_tiles = 0, seg_ct = 0, seg_counts = 0, seg_totals = 0, seg_starts = 0, seg_ntiles = 0;
     bool segmented = false;
     uint32_t seg_lo = 0, seg_chunk_bits = 0;
+    uint64_t cells = 0;  // the sort's one pass groups the keys by 64^3 cell
 };
 
-BatchLayout plan_batch(const BuildLayout& L, uint64_t n, const BatchInfo* batch)
+BatchLayout plan_batch(const BuildLayout& L, uint64_t n, const BatchInfo* batch, uint32_t first_bits)
 {
     BatchLayout B;
     if (!batch) return B;
@@ -688,6 +714,17 @@ BatchLayout plan_batch(const BuildLayout& L, uint64_t n, const BatchInfo* batch)
     B.seg_lo = uint32_t(L.key_plan.shift[0]);
     B.seg_chunk_bits = uint32_t(3 * batch->chunk_depth);
     B.segmented = L.key_plan.passes > 0 && B.seg_chunk_bits > B.seg_lo && B.seg_chunk_bits - B.seg_lo <= kSegMaxBits;
+    // Grouping by 64^3 cell takes one pass where at most 9 bits lie above a
+    // cell's (chunk depths 7 to 9); asked for a first digit, the sort keeps to
+    // its two passes.
+    if (B.segmented && first_bits == 0 && batch->chunk_depth > 6 &&
+        B.seg_chunk_bits - kCellShift <= kMaxSegDigitBits) {
+        const uint64_t cells = batch->num_chunks << (B.seg_chunk_bits - kCellShift);
+        if (cells_pay(cells, n)) {
+            B.cells = cells;
+            B.seg_lo = kCellShift;
+        }
+    }
     if (B.segmented) {
         const uint64_t tb = seg_tile_bound(n, batch->num_chunks);
         B.seg_tiles = c.take(sizeof(SegTile) * tb);
@@ -723,7 +760,7 @@ int build(svdag_context* ctx, const K* d_keys, uint64_t n, int depth, svdag_dag*
 
     const BuildLayout L = plan_build(n, depth, int(sizeof(K)), ctx->load_shift, batch != nullptr, ctx->radix_bits,
                                      ctx->sort_ipt, ctx->top_first);
-    const BatchLayout B = plan_batch(L, n, batch);
+    const BatchLayout B = plan_batch(L, n, batch, ctx->seg_first_bits);
     const uint64_t scratch_need = L.total + B.total;
     if (fixed && scratch_need > fixed->arena_bytes)
         return set_error(SVDAG_ERR_MEMORY, "build needs %llu scratch bytes, the fixed scratch holds %llu",
@@ -827,7 +864,7 @@ int build(svdag_context* ctx, const K* d_keys, uint64_t n, int depth, svdag_dag*
                 sc.ntiles = reinterpret_cast<uint64_t*>(A + L.seg_ntiles);
                 where = launch_top_digit_sort(st, d_keys, reinterpret_cast<uint32_t*>(kb),
                                               reinterpret_cast<uint32_t*>(ka), reinterpret_cast<uint32_t*>(kb),
-                                              L.key_plan.ipt, L.top_shift, L.top_bits, L.key_plan.shift[0], &c->n, n,
+                                              L.key_plan.ipt, L.top_shift, L.top_bits, L.sort_lo, &c->n, n,
                                               reinterpret_cast<uint32_t*>(A + L.key_sort_zero), sort_counts,
                                               &c->key_or, reinterpret_cast<uint64_t*>(A + L.bucket_start), sc, err);
                 buckets.offsets = reinterpret_cast<const uint64_t*>(A + L.bucket_start);
@@ -835,7 +872,12 @@ int build(svdag_context* ctx, const K* d_keys, uint64_t n, int depth, svdag_dag*
                 buckets.chunk_bits = L.top_shift;
             }
         }
-        if (!L.top_first)
+        if (L.cells && !L.top_first)
+            where = launch_cell_sort<K>(st, d_keys, reinterpret_cast<uint32_t*>(ka), L.key_plan.ipt, kCellShift,
+                                        uint32_t(3 * depth) - kCellShift, &c->n, n,
+                                        reinterpret_cast<uint32_t*>(A + L.key_sort_zero), sort_counts, &c->key_or,
+                                        reinterpret_cast<uint32_t*>(A + L.cell_starts));
+        else if (!L.top_first)
             where = launch_sort<K>(st, L.key_plan, d_keys, ka, kb, nullptr, &c->n, n,
                                    reinterpret_cast<uint32_t*>(A + L.key_sort_zero), sort_counts, &c->key_or);
         sorted = where == 0 ? static_cast<const void*>(ka) : static_cast<const void*>(kb);
@@ -850,7 +892,20 @@ int build(svdag_context* ctx, const K* d_keys, uint64_t n, int depth, svdag_dag*
     // Leaf ReduceByKey (DAGCompression.cu:1044-1068).
     uint64_t* reg_code = reinterpret_cast<uint64_t*>(A + L.reg_code);
     uint64_t* reg_mask = reinterpret_cast<uint64_t*>(A + L.reg_mask);
-    if (buckets.offsets || (!batch && sizeof(K) == 4))
+    if (L.cells || B.cells) {
+        CellArgs ca{};
+        ca.keys = static_cast<const uint32_t*>(sorted);
+        ca.starts = reinterpret_cast<const uint32_t*>(A + (batch ? B.seg_starts : L.cell_starts));
+        ca.cells = batch ? B.cells : L.cells;
+        ca.run_cells = cell_run_length(ca.cells, sort_count_words(n));
+        ca.reg_mask = reg_code;
+        ca.reg_code = reinterpret_cast<uint32_t*>(reg_mask);
+        ca.run_counts = sort_counts;  // free once the sort is done
+        ca.lp_code = lp_code;
+        ca.lp_mask = lp_mask;
+        ca.lp_capacity = L.leaf_bound;
+        launch_cell_reduce(st, ca, c, depth - 3);
+    } else if (buckets.offsets || (!batch && sizeof(K) == 4))
         launch_leaf_reduce<uint32_t>(st, static_cast<const uint32_t*>(sorted), c, L.group_bits, reg_code, reg_mask,
                                      lp_code, lp_mask, L.leaf_bound, tile_counts, tile_offsets, n, depth - 3,
                                      code_mask, buckets);
@@ -2165,7 +2220,7 @@ int svdag_batched_graph_create(svdag_context* ctx, const uint64_t* d_keys, const
     const BatchInfo batch{nullptr, num_chunks, chunk_depth, d_offsets};
     const BuildLayout L = plan_build(max_keys, depth, 8, g->ctx->load_shift, true, g->ctx->radix_bits,
                                      g->ctx->sort_ipt);
-    const uint64_t arena_bytes = L.total + plan_batch(L, max_keys, &batch).total;
+    const uint64_t arena_bytes = L.total + plan_batch(L, max_keys, &batch, g->ctx->seg_first_bits).total;
     const uint64_t storage_bytes = result_bytes(max_keys, depth);
     if (ctx->budget && arena_bytes + storage_bytes > ctx->budget)
         return fail(set_error(SVDAG_ERR_MEMORY, "graph needs %llu bytes, the budget is %llu",

@@ -412,6 +412,213 @@ __global__ __launch_bounds__(kThreads) void k_leaf_compact(const uint64_t* __res
     }
 }
 
+// ---------------------------------------------------------------------------
+// Leaf reduce of keys grouped by 64^3 cell (code >> kCellShift) with known cell
+// starts: one workgroup ORs a cell's keys into a table of its 4096 leaves in
+// LDS (32 KB: four workgroups of 8 waves per CU) and writes the leaves present
+// in order.  Against the 32^3 groups of k_leaf_reduce the sort orders 3 bits
+// less (one pass instead of two up to depth 9 in a chunk), no wave looks for
+// group starts, and the table words are 32 bits wide (64-bit LDS atomics take
+// twice the bank cycles).  Bound by the keys' read and the LDS atomics where
+// cells are full (512^3 noise, 67M keys: 304 -> 62 us, with 268 us of sort
+// saved), by the two barriers and the table pass a cell where they are not
+// (512 chunks, 645 keys a cell: 364 -> 415 us, with 640 us of sort saved; 690
+// before the next cell's keys were loaded ahead).
+// A cell of k keys emits at most min(k, 4096) leaves, so a run of cells writes
+// into its own keys' positions of the regions; codes there are 32-bit, local to
+// the run.
+// ---------------------------------------------------------------------------
+constexpr int kCellThreads = 512;
+constexpr int kCellWaves = kCellThreads / kWave;
+constexpr int kCellKeys = 8;  // keys per thread in flight
+constexpr int kCellRows = int(kCellLeaves) / kCellThreads;
+static_assert(kCellRows * kCellThreads == int(kCellLeaves) && kMaxRunCells < kWave, "rows and starts per lane");
+
+__global__ __launch_bounds__(kCellThreads) void k_cell_reduce(CellArgs a, const uint64_t* __restrict__ n_ptr,
+                                                              uint64_t* __restrict__ next_count)
+{
+    __shared__ uint64_t s_tab[kCellLeaves];
+    __shared__ uint32_t s_cnt[kCellWaves];
+    uint32_t* const tab = reinterpret_cast<uint32_t*>(s_tab);
+    const uint32_t lane = lane_id();
+    const uint32_t w = uint32_t(__builtin_amdgcn_readfirstlane(int(threadIdx.x / kWave)));
+    for (uint32_t i = threadIdx.x; i < kCellLeaves; i += kCellThreads) s_tab[i] = 0ull;
+    __syncthreads();
+    const uint32_t n = uint32_t(*n_ptr);
+    const uint64_t runs = cell_runs(a.cells, a.run_cells);
+    uint32_t parent_lanes = 0;  // per lane: parents counted by the flushes
+    // Bounds of a run's cells: lane l holds cell l's start (l == cells: the last
+    // one's end).  No keys (or offsets a check rejected): every cell is empty.
+    auto bounds_of = [&](uint64_t run) -> uint32_t {
+        const uint64_t c = run * a.run_cells + min(lane, a.run_cells);
+        return n != 0 && run < runs && c < a.cells ? a.starts[c] : n;
+    };
+    // Walk over the workgroup's cells that hold keys; the next run's bounds are
+    // in flight while a run is walked.
+    uint64_t run = blockIdx.x;
+    uint32_t bound = bounds_of(run), ahead = bounds_of(run + gridDim.x);
+    uint64_t todo = 0;  // cells of the run left to do
+    bool fresh = true;  // no cell of the run has been taken yet
+    uint32_t cell = 0, s = 0, e = 0;
+    auto cells_with_keys = [&]() -> uint64_t {
+        const uint32_t end = uint32_t(__shfl_down(int(bound), 1, kWave));
+        return __ballot(lane < a.run_cells && bound < end);
+    };
+    auto next_cell = [&]() -> bool {
+        while (todo == 0) {
+            if (run >= runs) return false;
+            if (fresh && threadIdx.x == 0) a.run_counts[run] = 0;  // no keys at all
+            run += gridDim.x;
+            bound = ahead;
+            ahead = bounds_of(run + gridDim.x);
+            todo = run < runs ? cells_with_keys() : 0ull;
+            fresh = true;
+        }
+        fresh = false;
+        cell = uint32_t(__builtin_amdgcn_readfirstlane(int(__ffsll((long long)todo) - 1)));
+        todo &= todo - 1ull;
+        s = uint32_t(__builtin_amdgcn_readlane(int(bound), int(cell)));
+        e = uint32_t(__builtin_amdgcn_readlane(int(bound), int(cell + 1)));
+        return true;
+    };
+    // The keys of one round, from p on; rows past the cell's end stay unread.
+    uint32_t k[kCellKeys];
+    auto load = [&](uint32_t p, uint32_t left) {
+#pragma unroll
+        for (int i = 0; i < kCellKeys; ++i)
+            if (uint32_t(i) * kCellThreads < left)
+                k[i] = __builtin_nontemporal_load(a.keys + p + min(uint32_t(i) * kCellThreads + threadIdx.x, left - 1));
+    };
+    todo = run < runs ? cells_with_keys() : 0ull;
+    bool have = next_cell();
+    if (have) load(s, e - s);
+    uint32_t written = 0;
+    while (have) {
+        const uint64_t cur_run = run;
+        const uint32_t cur_cell = cell;
+        const uint32_t base = uint32_t(__builtin_amdgcn_readlane(int(bound), 0));
+        for (uint32_t p = s;;) {
+            const uint32_t left = e - p;
+#pragma unroll
+            for (int i = 0; i < kCellKeys; ++i)
+                if (uint32_t(i) * kCellThreads + threadIdx.x < left)
+                    atomicOr(&tab[(k[i] >> 5) & (2 * kCellLeaves - 1)], 1u << (k[i] & 31u));
+            if (left <= uint32_t(kCellThreads * kCellKeys)) break;
+            p += kCellThreads * kCellKeys;
+            load(p, e - p);
+        }
+        // The next cell's first keys are in flight while this one is written.
+        have = next_cell();
+        if (have) load(s, e - s);
+        __syncthreads();
+        // Wave w holds the leaves [w * 512, ...) in rows of 64; lane l of a
+        // row counts the parent of leaves l .. l + 7 when l % 8 == 0.
+        uint64_t m[kCellRows];
+        uint32_t cnt = 0;
+#pragma unroll
+        for (int r = 0; r < kCellRows; ++r) {
+            const uint32_t leaf = (w * kCellRows + uint32_t(r)) * kWave + lane;
+            m[r] = s_tab[leaf];
+            s_tab[leaf] = 0ull;
+        }
+#pragma unroll
+        for (int r = 0; r < kCellRows; ++r) {
+            const uint64_t B = __ballot(m[r] != 0ull);
+            parent_lanes += ((lane & 7u) == 0u && ((B >> (lane & 56u)) & 0xFFull) != 0ull) ? 1u : 0u;
+            cnt += uint32_t(__popcll(B));
+        }
+        if (lane == 0) s_cnt[w] = cnt;
+        __syncthreads();
+        uint32_t pos = base + written;
+#pragma unroll
+        for (int i = 0; i < kCellWaves; ++i) {
+            const uint32_t x = s_cnt[i];
+            pos += uint32_t(i) < w ? x : 0u;
+            written += x;
+        }
+#pragma unroll
+        for (int r = 0; r < kCellRows; ++r) {
+            const uint64_t B = __ballot(m[r] != 0ull);
+            if (m[r]) {
+                const uint32_t q = pos + uint32_t(__popcll(B & lanemask_lt()));
+                a.reg_code[q] = cur_cell * kCellLeaves + (w * kCellRows + uint32_t(r)) * kWave + lane;
+                a.reg_mask[q] = m[r];
+            }
+            pos += uint32_t(__popcll(B));
+        }
+        if (!have || run != cur_run) {
+            if (threadIdx.x == 0) a.run_counts[cur_run] = written;
+            written = 0;
+        }
+    }
+    const uint32_t parents = wave_reduce_sum32(parent_lanes);
+    __syncthreads();
+    if (lane == 0) s_cnt[w] = parents;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        uint64_t t = 0;
+        for (int i = 0; i < kCellWaves; ++i) t += s_cnt[i];
+        if (t) atomicAdd((unsigned long long*)next_count, (unsigned long long)t);
+    }
+}
+
+// The runs' leaves, concatenated.  A workgroup takes consecutive runs, a wave a
+// run at a time, and finds its place by summing the counts before them (at most
+// a few tens of KB from L2; a scan kernel and its launch cost more).
+constexpr int kCompactAhead = 8;
+
+__global__ __launch_bounds__(kThreads) void k_cell_compact(CellArgs a, const uint64_t* __restrict__ n_ptr,
+                                                           uint64_t* __restrict__ total_out,
+                                                           unsigned long long* __restrict__ err)
+{
+    __shared__ uint64_t s_red[kThreads / kWave];
+    const uint64_t runs = cell_runs(a.cells, a.run_cells);
+    const uint64_t first = runs * blockIdx.x / gridDim.x, last = runs * (blockIdx.x + 1) / gridDim.x;
+    const uint32_t lane = lane_id(), w = threadIdx.x / kWave;
+    uint64_t sum = 0;
+    for (uint64_t i = threadIdx.x; i < first; i += kThreads) sum += a.run_counts[i];
+    uint64_t before = block_reduce_sum<kThreads>(sum, s_red);
+    const bool any = *n_ptr != 0;
+    for (uint64_t batch = first; batch < last; batch += kWave) {
+        // Lane l holds run batch + l's count, place and first key.
+        const bool mine = any && batch + lane < last;
+        const uint32_t count = mine ? a.run_counts[batch + lane] : 0u;
+        const uint32_t start = mine ? a.starts[(batch + lane) * a.run_cells] : 0u;
+        const uint32_t upto = wave_inclusive_scan(count);
+        const uint32_t here = uint32_t(min(uint64_t(kWave), last - batch));
+        for (uint32_t r = w; r < here; r += kThreads / kWave) {
+            const uint32_t cnt = uint32_t(__shfl(int(count), int(r), kWave));
+            const uint64_t src = uint32_t(__shfl(int(start), int(r), kWave));
+            const uint64_t dst = before + uint32_t(__shfl(int(upto), int(r), kWave)) - cnt;
+            const uint64_t high = (batch + r) * a.run_cells * kCellLeaves;
+            if (dst + cnt > a.lp_capacity) {
+                if (lane == 0) atomicOr(err, (unsigned long long)kErrInternal);
+                continue;
+            }
+            for (uint32_t j0 = 0; j0 < cnt; j0 += kWave * kCompactAhead) {
+                uint32_t code[kCompactAhead];
+                uint64_t mask[kCompactAhead];
+#pragma unroll
+                for (int q = 0; q < kCompactAhead; ++q) {
+                    const uint32_t j = min(j0 + uint32_t(q) * kWave + lane, cnt - 1);
+                    code[q] = a.reg_code[src + j];
+                    mask[q] = a.reg_mask[src + j];
+                }
+#pragma unroll
+                for (int q = 0; q < kCompactAhead; ++q) {
+                    const uint32_t j = j0 + uint32_t(q) * kWave + lane;
+                    if (j < cnt) {
+                        a.lp_code[dst + j] = high + code[q];
+                        a.lp_mask[dst + j] = mask[q];
+                    }
+                }
+            }
+        }
+        before += uint32_t(__shfl(int(upto), kWave - 1, kWave));
+    }
+    if (blockIdx.x + 1 == gridDim.x && threadIdx.x == 0) *total_out = before;
+}
+
 // Clears slots [0, 2^lg + overflow) with lg = max(8, ceil(log2(count << load_shift))).
 __global__ void k_table_clear(uint64_t* __restrict__ keys, const uint64_t* __restrict__ count_ptr,
                               uint32_t* __restrict__ log2_out, uint32_t load_shift, uint32_t overflow)
@@ -1910,6 +2117,19 @@ void launch_scan_counts(hipStream_t s, const uint32_t* counts, uint64_t* offsets
     TimedLaunch t(kKScanCounts, s);
     hipLaunchKernelGGL(k_scan_counts, dim3(1), dim3(kScanThreads), 0, s, counts, offsets, items_dev, per_tile, total_out,
                        items_host);
+}
+
+void launch_cell_reduce(hipStream_t s, const CellArgs& a, BuildCounters* c, int leaf_level)
+{
+    const uint64_t runs = cell_runs(a.cells, a.run_cells);
+    {
+        TimedLaunch t(kKLeafReduce, s);
+        hipLaunchKernelGGL(k_cell_reduce, dim3(resident_grid(k_cell_reduce, kCellThreads, runs)), dim3(kCellThreads), 0,
+                           s, a, &c->n, &c->pre[leaf_level]);
+    }
+    TimedLaunch t(kKLeafCompact, s);
+    hipLaunchKernelGGL(k_cell_compact, dim3(resident_grid(k_cell_compact, kThreads, runs)), dim3(kThreads), 0, s, a,
+                       &c->n, &c->leaf_positions, reinterpret_cast<unsigned long long*>(&c->error));
 }
 
 template <typename K>

@@ -183,6 +183,15 @@ int launch_top_digit_sort(hipStream_t stream, const uint64_t* keys_in, uint32_t*
                           unsigned long long* key_or, uint64_t* bucket_start, const SegScratch& sc,
                           unsigned long long* err);
 
+// One pass grouping the keys by their top digit [shift, shift + bits) (shift +
+// bits <= 32), written as 32-bit keys (the bits below shift at least); starts[d]
+// = first key of digit d, 2^bits entries.  zero, counts, key_or as above.
+// Returns 0, or -1 when the digit does not fit.
+template <typename K>
+int launch_cell_sort(hipStream_t stream, const K* keys_in, uint32_t* keys_out, int ipt, uint32_t shift, uint32_t bits,
+                     const uint64_t* n_ptr, uint64_t n_bound, uint32_t* zero, uint32_t* counts,
+                     unsigned long long* key_or, uint32_t* starts);
+
 template <typename K>
 int launch_sort(hipStream_t stream, const SortPlan& plan, const K* keys_in, K* keys_a, K* keys_b, K* final_keys,
                 const uint64_t* n_ptr, uint64_t n_bound, uint32_t* zero, uint32_t* counts,
@@ -271,6 +280,39 @@ void launch_leaf_reduce(hipStream_t s, const K* sorted, BuildCounters* c, uint32
                         uint64_t* reg_mask, uint64_t* lp_code, uint64_t* lp_mask, uint64_t lp_capacity,
                         uint32_t* tile_counts, uint64_t* tile_offsets, uint64_t n_bound, int leaf_level,
                         uint64_t code_mask, const ChunkPrefix& buckets = ChunkPrefix{});
+
+// Leaf ReduceByKey over keys grouped by cell (code >> kCellShift: 64^3 voxels,
+// 4096 leaves), cell c at keys[starts[c], starts[c + 1]) (the last up to
+// c->n): one workgroup per cell.  Runs of run_cells cells write their leaves
+// into reg_code / reg_mask from their first key's position on (n_bound
+// entries), counted in run_counts (cell_runs entries), then compacted as
+// above.  Which builds take it: cells_pay.
+constexpr uint32_t kCellShift = 18;
+constexpr uint32_t kCellLeaves = 1u << (kCellShift - 6);
+constexpr uint32_t kMaxRunCells = 32;
+inline uint32_t cell_run_length(uint64_t cells, uint64_t max_runs)
+{
+    const uint64_t runs = std::min<uint64_t>(16384, max_runs);
+    return uint32_t(std::max<uint64_t>(1, std::min<uint64_t>(kMaxRunCells, (cells + runs - 1) / runs)));
+}
+__host__ __device__ inline uint64_t cell_runs(uint64_t cells, uint32_t run_cells) { return (cells + run_cells - 1) / run_cells; }
+// A cell costs its workgroup a pass over 4096 table words however few keys it
+// holds: below 16 keys a cell the wave-sized groups of launch_leaf_reduce read
+// less, unless there are so few cells that launches cost more than the tables.
+inline bool cells_pay(uint64_t cells, uint64_t n) { return cells <= 8192 || cells <= n / 16; }
+struct CellArgs {
+    const uint32_t* keys;
+    const uint32_t* starts;
+    uint64_t cells;
+    uint32_t run_cells;
+    uint32_t* reg_code;
+    uint64_t* reg_mask;
+    uint32_t* run_counts;
+    uint64_t* lp_code;
+    uint64_t* lp_mask;
+    uint64_t lp_capacity;
+};
+void launch_cell_reduce(hipStream_t s, const CellArgs& a, BuildCounters* c, int leaf_level);
 
 // Clears an ordered (load_shift, overflow) or hashed table sized from *count_ptr
 // and records its log2 size.

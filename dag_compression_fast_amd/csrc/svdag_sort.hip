@@ -284,7 +284,8 @@ __global__ __launch_bounds__(kSortThreads) void k_sort_count(const K* __restrict
 }
 
 // Block d: exclusive scan of row d of the tile counts, offset by the digit's
-// global start (sum of the pass histogram below d).  In place.  Rows of at
+// global start (sum of the pass histogram below d; also to starts[d] when
+// given).  In place.  Rows of at
 // most kScanItems waves' worth of tiles take a one-wave block.
 constexpr int kScanThreads = 1024;
 constexpr int kScanItems = 4;
@@ -294,7 +295,7 @@ template <int kScanThreads>
 __global__ __launch_bounds__(kScanThreads) void k_sort_scan(uint32_t* __restrict__ counts,
                                                             const uint32_t* __restrict__ hist,
                                                             const uint64_t* __restrict__ n_ptr, uint64_t stride,
-                                                            uint64_t tile_keys)
+                                                            uint64_t tile_keys, uint32_t* __restrict__ starts)
 {
     __shared__ uint64_t s_red[kScanThreads / kWave];
     __shared__ uint32_t s_scan[kScanThreads / kWave];
@@ -305,6 +306,7 @@ __global__ __launch_bounds__(kScanThreads) void k_sort_scan(uint32_t* __restrict
     uint64_t below = 0;
     for (uint32_t i = threadIdx.x; i < d; i += kScanThreads) below += hist[i];
     uint64_t running = block_reduce_sum<kScanThreads>(below, s_red);
+    if (starts && threadIdx.x == 0) starts[d] = uint32_t(running);
     uint32_t* row = counts + uint64_t(d) * stride;
     // kScanItems consecutive counts per thread per block scan.
     for (uint64_t chunk = 0; chunk < ntiles; chunk += uint64_t(kScanThreads) * kScanItems) {
@@ -621,10 +623,10 @@ static void launch_pass(hipStream_t stream, const K* src, K* dst, const uint64_t
         TimedLaunch t(kKSortScan, stream);
         if (stride <= kSmallScanTiles)
             hipLaunchKernelGGL(k_sort_scan<kWave>, dim3(dmask + 1), dim3(kWave), 0, stream, counts, hist, n_ptr,
-                               stride, uint64_t(kSortThreads) * IPT);
+                               stride, uint64_t(kSortThreads) * IPT, nullptr);
         else
             hipLaunchKernelGGL(k_sort_scan<kScanThreads>, dim3(dmask + 1), dim3(kScanThreads), 0, stream, counts,
-                               hist, n_ptr, stride, uint64_t(kSortThreads) * IPT);
+                               hist, n_ptr, stride, uint64_t(kSortThreads) * IPT, nullptr);
     }
     // A stable key-only sort ranks adaptively when it can (see k_sort_scatter);
     // its first pass has no earlier bits, so every tile is uniform there.
@@ -1211,10 +1213,10 @@ int launch_top_digit_sort(hipStream_t stream, const uint64_t* keys_in, uint32_t*
             TimedLaunch t(kKSortScan, stream);
             if (stride <= kSmallScanTiles)
                 hipLaunchKernelGGL(k_sort_scan<kWave>, dim3(R), dim3(kWave), 0, stream, counts, zero, n_ptr, stride,
-                                   uint64_t(kSortThreads) * I);
+                                   uint64_t(kSortThreads) * I, nullptr);
             else
                 hipLaunchKernelGGL(k_sort_scan<kScanThreads>, dim3(R), dim3(kScanThreads), 0, stream, counts, zero,
-                                   n_ptr, stride, uint64_t(kSortThreads) * I);
+                                   n_ptr, stride, uint64_t(kSortThreads) * I, nullptr);
             hipLaunchKernelGGL(k_digit_starts, dim3(1), dim3(kRadix), 0, stream, zero, R, n_ptr, bucket_start);
         }
         // Without the LDS that holds the 64-bit LSD pass to two workgroups per
@@ -1229,5 +1231,53 @@ int launch_top_digit_sort(hipStream_t stream, const uint64_t* keys_in, uint32_t*
     return launch_segmented_sort<uint32_t>(stream, local, keys_a, keys_b, bucket_start, R, n_ptr, n_bound, sc, lo,
                                            top_shift, err, 0);
 }
+
+template <typename K>
+int launch_cell_sort(hipStream_t stream, const K* keys_in, uint32_t* keys_out, int ipt, uint32_t shift, uint32_t bits,
+                     const uint64_t* n_ptr, uint64_t n_bound, uint32_t* zero, uint32_t* counts,
+                     unsigned long long* key_or, uint32_t* starts)
+{
+    if (bits < 1 || bits > uint32_t(kMaxRadixBits) || shift + bits > 32 || n_bound == 0) return -1;
+    const uint32_t dmask = (1u << bits) - 1u, R = dmask + 1;
+    HistPlan hp{};
+    hp.passes = 1;
+    hp.shift[0] = shift;
+    hp.mask[0] = dmask;
+    auto run = [&](auto ipt_tag) {
+        constexpr int I = decltype(ipt_tag)::value;
+        const uint64_t stride = sort_tiles(n_bound, I);
+        const uint32_t scatter_grid =
+            uint32_t(std::max<uint64_t>(kXcds, std::min<uint64_t>((stride + kXcds - 1) / kXcds * kXcds,
+                                                                  uint64_t(device_cu_count()) * 64) / kXcds * kXcds));
+        {
+            TimedLaunch t(kKHistogram, stream);
+            hipLaunchKernelGGL((k_histogram<K, I>), dim3(histogram_grid<K, I>(stride)), dim3(kSortThreads), 0, stream,
+                               keys_in, n_ptr, hp, zero, key_or, counts, stride, ChunkPrefix{});
+        }
+        {
+            TimedLaunch t(kKSortScan, stream);
+            if (stride <= kSmallScanTiles)
+                hipLaunchKernelGGL(k_sort_scan<kWave>, dim3(R), dim3(kWave), 0, stream, counts, zero, n_ptr, stride,
+                                   uint64_t(kSortThreads) * I, starts);
+            else
+                hipLaunchKernelGGL(k_sort_scan<kScanThreads>, dim3(R), dim3(kScanThreads), 0, stream, counts, zero,
+                                   n_ptr, stride, uint64_t(kSortThreads) * I, starts);
+        }
+        TimedLaunch t(kKSortScatterKeys, stream);
+        hipLaunchKernelGGL((k_sort_scatter<K, kRankUnstable, I, kSortThreads, uint32_t>), dim3(scatter_grid),
+                           dim3(kSortThreads), 0, stream, keys_in, keys_out, n_ptr, shift, dmask, counts, stride,
+                           ChunkPrefix{}, 0u, 0u, nullptr, 64u);
+    };
+    if (ipt == kSortIptLarge) run(std::integral_constant<int, kSortIptLarge>{});
+    else run(std::integral_constant<int, kSortIptSmall>{});
+    return 0;
+}
+
+template int launch_cell_sort<uint64_t>(hipStream_t, const uint64_t*, uint32_t*, int, uint32_t, uint32_t,
+                                        const uint64_t*, uint64_t, uint32_t*, uint32_t*, unsigned long long*,
+                                        uint32_t*);
+template int launch_cell_sort<uint32_t>(hipStream_t, const uint32_t*, uint32_t*, int, uint32_t, uint32_t,
+                                        const uint64_t*, uint64_t, uint32_t*, uint32_t*, unsigned long long*,
+                                        uint32_t*);
 
 }  // namespace svdag

@@ -838,6 +838,8 @@ int build(svdag_context* ctx, const K* d_keys, uint64_t n, int depth, svdag_dag*
             sc.totals = reinterpret_cast<uint32_t*>(A + B.seg_totals);
             sc.starts = reinterpret_cast<uint32_t*>(A + B.seg_starts);
             sc.ntiles = reinterpret_cast<uint64_t*>(A + B.seg_ntiles);
+            sc.slices = sort_counts;  // not used by this sort otherwise
+            sc.slice_words = sort_count_words(n);
             where = launch_segmented_sort(st, reinterpret_cast<const uint64_t*>(d_keys),
                                           reinterpret_cast<uint32_t*>(ka), reinterpret_cast<uint32_t*>(kb), d_off,
                                           batch->num_chunks, &c->n, n, sc, B.seg_lo, B.seg_chunk_bits, err,
@@ -862,6 +864,8 @@ int build(svdag_context* ctx, const K* d_keys, uint64_t n, int depth, svdag_dag*
                 sc.totals = reinterpret_cast<uint32_t*>(A + L.seg_totals);
                 sc.starts = reinterpret_cast<uint32_t*>(A + L.seg_starts);
                 sc.ntiles = reinterpret_cast<uint64_t*>(A + L.seg_ntiles);
+                sc.slices = sort_counts;  // free after the top digit's scatter
+                sc.slice_words = sort_count_words(n);
                 where = launch_top_digit_sort(st, d_keys, reinterpret_cast<uint32_t*>(kb),
                                               reinterpret_cast<uint32_t*>(ka), reinterpret_cast<uint32_t*>(kb),
                                               L.key_plan.ipt, L.top_shift, L.top_bits, L.sort_lo, &c->n, n,

@@ -162,6 +162,8 @@ struct SegScratch {
     uint32_t* totals;
     uint32_t* starts;
     uint64_t* ntiles;
+    uint32_t* slices;      // sums over several tiles, slice_words words (any number)
+    uint64_t slice_words;
 };
 template <typename KI>
 int launch_segmented_sort(hipStream_t stream, const KI* keys_in, uint32_t* keys_a, uint32_t* keys_b,

@@ -728,31 +728,50 @@ template int launch_sort<uint32_t>(hipStream_t, const SortPlan&, const uint32_t*
 // ---------------------------------------------------------------------------
 namespace {
 
+// A tile is THREADS x kSegIpt keys: 256 threads (4096 keys), or 1024 (16384)
+// where a chunk holds kSegWideKeys keys or more on average.  A chunk that long
+// spreads a 4096-key tile over 512 digits in runs of 8 keys, 32 bytes: 67M keys
+// a chunk took 2170 us of scatter with 256 threads, 1515 with 1024 (1630 with
+// 512); buckets of 140k keys and 64 digits 105 and 162 us, chunks of 330k keys
+// and 512 digits 436 and 460.
 constexpr int kSegThreads = 256;
+constexpr int kSegWideThreads = 1024;
+constexpr uint64_t kSegWideKeys = 1ull << 22;
+constexpr uint64_t kSegUnits = 4096;   // workgroups that the count of a long key list keeps
+constexpr uint32_t kSegMaxSlice = 32;  // tiles per slice at most
 constexpr int kSegIpt = 16;
 constexpr uint32_t kSegTile = uint32_t(kSegThreads) * kSegIpt;
 constexpr uint32_t kSegMaxBins = 1u << kSegMaxBits;  // combined bins of the second pass
-constexpr int kSegBinsPerThread = kSegMaxBins / kSegThreads;
 constexpr uint32_t kSegMaxDigits = 1u << kMaxSegDigitBits;
 constexpr uint32_t kSegSubCounters = 4;  // LDS words per digit in the count kernel
 constexpr int kSegDigitsPerThread = int(kSegMaxDigits / kSegThreads);
 static_assert(kSegDigitsPerThread * kSegThreads == int(kSegMaxDigits), "digits spread evenly over the threads");
 static_assert(kSegTile == kSegTileItems, "tile size shared with the planner");
-static_assert(kSegTile <= 65536 && kSegMaxBins <= 65536, "bin and rank packed in 16 bits each");
-static_assert(kSegMaxBins == kSegThreads * kSegBinsPerThread && kSegBinsPerThread * kWave * (kSegThreads / kWave) ==
-                  kSegMaxBins, "bins covered by the row-wise scan");
+static_assert(kSegWideThreads * kSegIpt <= 65536 && kSegMaxBins <= 65536, "bin and rank packed in 16 bits each");
 
-// Counts of tile t, tile-major: counts[t * R + d] (one contiguous run per
-// tile, written and read whole).
-__device__ __forceinline__ uint64_t seg_count_index(uint64_t t, uint32_t R, uint32_t d)
+// Where the counts of the tiles are.  A workgroup of the count kernel takes
+// `per` consecutive tiles and keeps counting over them, so that only slices
+// (its tiles of one chunk) are left to scan: slice (t / per + chunk) of tile t
+// (both terms only grow, so no two slices share a row) holds the keys of each
+// digit before the slice, tile t's row those before the tile in the slice.
+// per == 1: the tile rows alone, as slice rows.  (8 chunks of 67M keys have so
+// many tiles and so few workgroups in the scan that scanning tile rows took 415
+// us a pass; slices take 11.)  All rows are R words, written
+// and read whole.
+struct SegRows {
+    uint32_t* tile;   // per > 1: ntiles rows
+    uint32_t* slice;  // per == 1: ntiles rows; else ntiles / per + num_chunks rows
+    uint32_t per;
+};
+__device__ __forceinline__ uint64_t seg_slice(const SegRows& rows, uint64_t t, uint64_t chunk)
 {
-    return t * R + d;
+    return rows.per == 1 ? t : uint32_t(t) / rows.per + chunk;
 }
 
 // Tile table of the segmented sort, planned on the device from the chunk
 // offsets (no host planning, so a captured build replays for any offsets
 // within its bounds): chunk c's tiles start at chunk_tiles[c] (exclusive scan
-// of ceil(keys / kSegTile)), *ntiles = their total.  *n_ptr == 0 (no keys, or
+// of ceil(keys / tile_keys)), *ntiles = their total.  *n_ptr == 0 (no keys, or
 // offsets a check rejected) plans no tiles.
 constexpr int kPlanThreads = 1024;
 
@@ -760,7 +779,7 @@ __global__ __launch_bounds__(kPlanThreads) void k_seg_plan_chunks(const uint64_t
                                                                   uint64_t num_chunks,
                                                                   const uint64_t* __restrict__ n_ptr,
                                                                   uint32_t* __restrict__ chunk_tiles,
-                                                                  uint64_t* __restrict__ ntiles)
+                                                                  uint64_t* __restrict__ ntiles, uint32_t tile_keys)
 {
     __shared__ uint32_t s_scan[kPlanThreads / kWave];
     const bool any = *n_ptr != 0;
@@ -768,7 +787,7 @@ __global__ __launch_bounds__(kPlanThreads) void k_seg_plan_chunks(const uint64_t
     for (uint64_t base = 0; base < num_chunks; base += kPlanThreads) {
         const uint64_t c = base + threadIdx.x;
         uint32_t t = 0;
-        if (any && c < num_chunks) t = uint32_t((offsets[c + 1] - offsets[c] + kSegTile - 1) / kSegTile);
+        if (any && c < num_chunks) t = uint32_t((offsets[c + 1] - offsets[c] + tile_keys - 1) / tile_keys);
         uint32_t total;
         const uint32_t ex = block_exclusive_scan<kPlanThreads>(t, s_scan, total);
         if (c < num_chunks) chunk_tiles[c] = carry + ex;
@@ -783,7 +802,7 @@ __global__ __launch_bounds__(kPlanThreads) void k_seg_plan_chunks(const uint64_t
 // Tile t: the chunk whose tile range holds it (last c with chunk_tiles[c] <= t).
 __global__ void k_seg_plan_tiles(const uint64_t* __restrict__ offsets, const uint32_t* __restrict__ chunk_tiles,
                                  uint64_t num_chunks, const uint64_t* __restrict__ ntiles_ptr,
-                                 SegTile* __restrict__ tiles)
+                                 SegTile* __restrict__ tiles, uint32_t tile_keys)
 {
     const uint64_t ntiles = *ntiles_ptr;
     const uint64_t stride = uint64_t(gridDim.x) * blockDim.x;
@@ -794,8 +813,8 @@ __global__ void k_seg_plan_tiles(const uint64_t* __restrict__ offsets, const uin
             if (chunk_tiles[mid] <= t) lo = mid;
             else hi = mid;
         }
-        const uint64_t start = offsets[lo] + (t - chunk_tiles[lo]) * kSegTile;
-        tiles[t] = SegTile{start, uint32_t(min(uint64_t(kSegTile), offsets[lo + 1] - start)), uint32_t(lo)};
+        const uint64_t start = offsets[lo] + (t - chunk_tiles[lo]) * tile_keys;
+        tiles[t] = SegTile{start, uint32_t(min(uint64_t(tile_keys), offsets[lo + 1] - start)), uint32_t(lo)};
     }
 }
 
@@ -804,67 +823,82 @@ __global__ void k_seg_plan_tiles(const uint64_t* __restrict__ offsets, const uin
 // is split over kSegSubCounters LDS words by lane: the second pass's tiles hold
 // few distinct digits, and lanes of one wave adding to one word serialise
 // (measured 187 -> 140 us for that count on 169M keys).
-template <bool FIRST, typename KI>
-__global__ __launch_bounds__(kSegThreads) void k_seg_count(const KI* __restrict__ keys,
-                                                           const SegTile* __restrict__ tiles,
-                                                           const uint64_t* __restrict__ ntiles_ptr, uint32_t shift,
-                                                           uint32_t dmask, uint32_t chunk_bits,
-                                                           uint32_t* __restrict__ counts,
-                                                           unsigned long long* __restrict__ err)
+template <bool FIRST, typename KI, int THREADS>
+__global__ __launch_bounds__(THREADS) void k_seg_count(const KI* __restrict__ keys,
+                                                       const SegTile* __restrict__ tiles,
+                                                       const uint64_t* __restrict__ ntiles_ptr, uint32_t shift,
+                                                       uint32_t dmask, uint32_t chunk_bits, SegRows rows,
+                                                       unsigned long long* __restrict__ err)
 {
     __shared__ uint32_t s_cnt[kSegMaxDigits * kSegSubCounters];
     const uint64_t ntiles = *ntiles_ptr;
     const uint32_t R = dmask + 1;
     bool bad = false;
-    // Tiles XCD by XCD: a chunk's neighbouring tiles have adjacent counts in
-    // every digit row, which then combine in one L2.
-    const TileWalk walk = xcd_tiles(ntiles);
-    for (uint64_t t = walk.tile; t < walk.end; t += walk.step) {
-        const SegTile tile = tiles[t];
-        // The whole tile's keys are in flight before the counters are cleared:
-        // positions past the tile's end read its last key (a tile holds at
-        // least one), so no load sits behind a branch, and are not counted.
-        KI key[kSegIpt];
-#pragma unroll
-        for (int i = 0; i < kSegIpt; ++i) {
-            const uint32_t j = min(uint32_t(i) * kSegThreads + threadIdx.x, tile.count - 1);
-            key[i] = __builtin_nontemporal_load(keys + tile.start + j);
-        }
-        for (uint32_t i = threadIdx.x; i < kSegSubCounters * R; i += kSegThreads) s_cnt[i] = 0;
-        __syncthreads();
-        const uint32_t sub = threadIdx.x & (kSegSubCounters - 1);
-#pragma unroll
-        for (int i = 0; i < kSegIpt; ++i) {
-            if (uint32_t(i) * kSegThreads + threadIdx.x < tile.count) {
-                if constexpr (FIRST) bad |= chunk_bits < 8 * sizeof(KI) && (uint64_t(key[i]) >> chunk_bits) != 0;
-                atomicAdd(&s_cnt[(uint32_t(uint64_t(key[i]) >> shift) & dmask) * kSegSubCounters + sub], 1u);
-            }
-        }
-        __syncthreads();
-        for (uint32_t d = threadIdx.x; d < R; d += kSegThreads) {
+    auto write_row = [&](uint32_t* row) {
+        for (uint32_t d = threadIdx.x; d < R; d += THREADS) {
             uint32_t c = 0;
 #pragma unroll
             for (uint32_t q = 0; q < kSegSubCounters; ++q) c += s_cnt[d * kSegSubCounters + q];
-            counts[seg_count_index(t, R, d)] = c;
+            row[d] = c;
         }
+    };
+    // Units XCD by XCD: neighbouring tiles' rows then combine in one L2.
+    const TileWalk walk = xcd_tiles((ntiles + rows.per - 1) / rows.per);
+    for (uint64_t u = walk.tile; u < walk.end; u += walk.step) {
+        const uint64_t t0 = u * rows.per, t1 = min(t0 + rows.per, ntiles);
+        uint32_t chunk = 0;
+        for (uint64_t t = t0; t < t1; ++t) {
+            const SegTile tile = tiles[t];
+            // The whole tile's keys are in flight before the counters are used:
+            // positions past the tile's end read its last key (a tile holds at
+            // least one), so no load sits behind a branch, and are not counted.
+            KI key[kSegIpt];
+#pragma unroll
+            for (int i = 0; i < kSegIpt; ++i) {
+                const uint32_t j = min(uint32_t(i) * THREADS + threadIdx.x, tile.count - 1);
+                key[i] = __builtin_nontemporal_load(keys + tile.start + j);
+            }
+            if (t == t0 || tile.chunk != chunk) {
+                if (t != t0) {
+                    write_row(rows.slice + seg_slice(rows, t - 1, chunk) * R);
+                    __syncthreads();
+                }
+                for (uint32_t i = threadIdx.x; i < kSegSubCounters * R; i += THREADS) s_cnt[i] = 0;
+                chunk = tile.chunk;
+                __syncthreads();
+            }
+            if (rows.per != 1) {
+                write_row(rows.tile + t * R);
+                __syncthreads();
+            }
+            const uint32_t sub = threadIdx.x & (kSegSubCounters - 1);
+#pragma unroll
+            for (int i = 0; i < kSegIpt; ++i) {
+                if (uint32_t(i) * THREADS + threadIdx.x < tile.count) {
+                    if constexpr (FIRST) bad |= chunk_bits < 8 * sizeof(KI) && (uint64_t(key[i]) >> chunk_bits) != 0;
+                    atomicAdd(&s_cnt[(uint32_t(uint64_t(key[i]) >> shift) & dmask) * kSegSubCounters + sub], 1u);
+                }
+            }
+            __syncthreads();
+        }
+        write_row(rows.slice + seg_slice(rows, t1 - 1, chunk) * R);
         __syncthreads();
     }
     if (FIRST && bad) atomicOr(err, (unsigned long long)kErrKeyRange);
 }
 
 // One block per (chunk, 64 digits): lane l of every wave owns digit d = group
-// * 64 + l; the chunk's tiles are split into kColWaves consecutive slices, one
-// per wave.  Each wave sums its slice (reading 64 adjacent counts of one tile
-// per step, kScanAhead tiles in flight), the slice sums are combined in LDS,
-// and each wave rewrites its slice with exclusive prefixes; the digit's total
-// goes to totals[c * R + d].
+// * 64 + l; the chunk's slice rows are split into kColWaves consecutive parts,
+// one per wave.  Each wave sums its part (reading 64 adjacent counts of one row
+// per step, kScanAhead rows in flight), the sums are combined in LDS, and each
+// wave rewrites its part with exclusive prefixes; the digit's total goes to
+// totals[c * R + d].
 constexpr uint32_t kScanAhead = 8;
-constexpr int kColWaves = 8;
+constexpr int kColWaves = 16;
 constexpr int kColThreads = kColWaves * kWave;
 
 __global__ __launch_bounds__(kColThreads) void k_seg_scan_cols(const uint32_t* __restrict__ chunk_tiles,
-                                                               uint64_t num_chunks, uint32_t R,
-                                                               uint32_t* __restrict__ counts,
+                                                               uint64_t num_chunks, uint32_t R, SegRows rows,
                                                                uint32_t* __restrict__ totals)
 {
     __shared__ uint32_t s_part[kColWaves][kWave];
@@ -873,10 +907,12 @@ __global__ __launch_bounds__(kColThreads) void k_seg_scan_cols(const uint32_t* _
     for (uint64_t job = blockIdx.x; job < num_chunks * groups; job += gridDim.x) {
         const uint64_t c = job / groups;
         const uint32_t d = uint32_t(job % groups) * kWave + lane;
-        const uint32_t t0 = chunk_tiles[c], nt = chunk_tiles[c + 1] - t0;
+        const uint32_t tile0 = chunk_tiles[c], tile1 = chunk_tiles[c + 1];
+        const uint64_t t0 = seg_slice(rows, tile0, c);
+        const uint32_t nt = tile1 > tile0 ? uint32_t(seg_slice(rows, tile1 - 1, c) - t0) + 1u : 0u;
         const uint32_t per = (nt + kColWaves - 1) / kColWaves;
         const uint32_t b = min(nt, w * per), e = min(nt, b + per);
-        uint32_t* col = counts + uint64_t(t0) * R + d;
+        uint32_t* col = rows.slice + t0 * R + d;
         const bool mine = d < R;
         uint32_t sum = 0;
         for (uint32_t i0 = b; i0 < e; i0 += kScanAhead) {
@@ -945,25 +981,26 @@ __global__ __launch_bounds__(kSegThreads) void k_seg_scan_digits(const uint64_t*
 // FIRST: bins = the pass digit.  Else: bins = digit * span + (previous digit -
 // the tile's smallest previous digit), span = the tile's range of previous
 // digits (the input is sorted on them, so a tile usually holds one or two).
-// Output offset of tile t's digit d: starts[c * R + d] plus the row prefix in
-// counts.  The first pass needs only R <= kSegMaxDigits bins, which keeps its
+// Output offset of tile t's digit d: starts[c * R + d] plus the prefixes in its
+// slice's and its own row.  The first pass needs only R <= kSegMaxDigits bins, which keeps its
 // LDS (and so its workgroups per CU) within reach of the later passes' double.
 // Tiles are walked XCD by XCD (the grid is a multiple of kXcds), so
 // neighbouring tiles, whose runs of one digit are adjacent in the output, are
 // written through one L2.
-template <bool FIRST, typename KI>
-__global__ __launch_bounds__(kSegThreads) void k_seg_scatter(const KI* __restrict__ keys_in,
-                                                             uint32_t* __restrict__ keys_out,
-                                                             const SegTile* __restrict__ tiles,
-                                                             const uint64_t* __restrict__ ntiles_ptr, uint32_t shift,
-                                                             uint32_t dmask, uint32_t prev_shift, uint32_t prev_bits,
-                                                             const uint32_t* __restrict__ counts,
-                                                             const uint32_t* __restrict__ starts)
+template <bool FIRST, typename KI, int THREADS>
+__global__ __launch_bounds__(THREADS) void k_seg_scatter(const KI* __restrict__ keys_in,
+                                                         uint32_t* __restrict__ keys_out,
+                                                         const SegTile* __restrict__ tiles,
+                                                         const uint64_t* __restrict__ ntiles_ptr, uint32_t shift,
+                                                         uint32_t dmask, uint32_t prev_shift, uint32_t prev_bits,
+                                                         SegRows rows, const uint32_t* __restrict__ starts)
 {
-    using KS = KI;  // staged key
+    // Keys are staged as they are written; the digit lies in the low 32 bits.
+    using KS = uint32_t;
+    constexpr uint32_t kSegTile = uint32_t(THREADS) * kSegIpt;
+    constexpr int kSegThreads = THREADS;
     constexpr uint32_t kBins = FIRST ? kSegMaxDigits : kSegMaxBins;
-    constexpr int kBinsPerThread = int(kBins / kSegThreads);
-    static_assert(kBinsPerThread * kSegThreads == int(kBins), "bins covered by the row-wise scan");
+    constexpr int kBinsPerThread = int((kBins + kSegThreads - 1) / kSegThreads);
     __shared__ KS s_keys[kSegTile];
     __shared__ uint32_t s_bin[kBins];
     __shared__ uint32_t s_base[kSegMaxDigits];
@@ -1062,8 +1099,8 @@ __global__ __launch_bounds__(kSegThreads) void k_seg_scatter(const KI* __restric
         __syncthreads();
         // Digit d's keys start at its first bin inside the tile.
         for (uint32_t d = threadIdx.x; d < R; d += kSegThreads)
-            s_base[d] = starts[uint64_t(tile.chunk) * R + d] + counts[seg_count_index(t, R, d)] -
-                        s_bin[d * span];
+            s_base[d] = starts[uint64_t(tile.chunk) * R + d] + rows.slice[seg_slice(rows, t, tile.chunk) * R + d] +
+                        (rows.per != 1 ? rows.tile[t * R + d] : 0u) - s_bin[d * span];
 #pragma unroll
         for (int i = 0; i < kSegIpt; ++i) {
             const uint32_t j = uint32_t(i) * kSegThreads + threadIdx.x;
@@ -1097,56 +1134,59 @@ int launch_segmented_sort(hipStream_t stream, const KI* keys_in, uint32_t* keys_
     const uint32_t b2 = B - b1;                                  // second (0: one pass)
     const uint64_t tile_bound = seg_tile_bound(n_bound, num_chunks);
     const int cus = device_cu_count();
+    const bool wide = n_bound / num_chunks >= kSegWideKeys;
+    const uint32_t tile_keys = uint32_t(wide ? kSegWideThreads : kSegThreads) * kSegIpt;
+    const uint64_t tile_count = n_bound / tile_keys + num_chunks;
     // A multiple of kXcds, as the scatter's tile walk assumes.
     const int grid = int(std::max<uint64_t>(
-        kXcds, std::min<uint64_t>((tile_bound + kXcds - 1) / kXcds * kXcds, uint64_t(cus) * 64) / kXcds * kXcds));
+        kXcds, std::min<uint64_t>((tile_count + kXcds - 1) / kXcds * kXcds, uint64_t(cus) * 64) / kXcds * kXcds));
     const int chunk_grid = int(std::max<uint64_t>(1, std::min<uint64_t>(num_chunks, uint64_t(cus) * 8)));
     {
         TimedLaunch t(kKSortScan, stream);
         hipLaunchKernelGGL(k_seg_plan_chunks, dim3(1), dim3(kPlanThreads), 0, stream, chunk_start, num_chunks, n_ptr,
-                           sc.chunk_tiles, sc.ntiles);
+                           sc.chunk_tiles, sc.ntiles, tile_keys);
         hipLaunchKernelGGL(k_seg_plan_tiles, dim3(int(std::max<uint64_t>(1, std::min<uint64_t>((tile_bound + 255) / 256,
                                                                                            uint64_t(cus) * 8)))),
-                           dim3(256), 0, stream, chunk_start, sc.chunk_tiles, num_chunks, sc.ntiles, sc.tiles);
+                           dim3(256), 0, stream, chunk_start, sc.chunk_tiles, num_chunks, sc.ntiles, sc.tiles,
+                           tile_keys);
     }
     // The first pass reads the caller's keys (KI), the second the first's output.
-    auto pass = [&](bool first, const void* src, uint32_t* dst, uint32_t shift, uint32_t bits) {
+    auto pass = [&](auto first_tag, auto threads_tag, const auto* src, uint32_t* dst, uint32_t shift, uint32_t bits) {
+        constexpr bool FIRST = decltype(first_tag)::value;
+        constexpr int THREADS = decltype(threads_tag)::value;
+        using KS = std::remove_const_t<std::remove_pointer_t<decltype(src)>>;
         const uint32_t mask = (1u << bits) - 1u, R = mask + 1;
         const uint64_t col_jobs = num_chunks * ((R + kWave - 1) / kWave);
         const int col_grid = int(std::max<uint64_t>(1, std::min<uint64_t>(col_jobs, uint64_t(cus) * 16)));
+        // Slices of several tiles where that leaves kSegUnits workgroups to
+        // count them and the rows have room beside the tiles'.
+        SegRows rows{sc.counts, sc.counts, 1};
+        const uint32_t per = uint32_t(std::min<uint64_t>(kSegMaxSlice, tile_count / kSegUnits));
+        if (per > 1 && (tile_count / per + num_chunks + 1) * R <= sc.slice_words)
+            rows = SegRows{sc.counts, sc.slices, per};
         {
             TimedLaunch t(kKSegCount, stream);
-            if (first)
-                hipLaunchKernelGGL((k_seg_count<true, KI>), dim3(grid), dim3(kSegThreads), 0, stream,
-                                   static_cast<const KI*>(src), sc.tiles, sc.ntiles, shift, mask,
-                                   chunk_bits, sc.counts, err);
-            else
-                hipLaunchKernelGGL((k_seg_count<false, uint32_t>), dim3(grid), dim3(kSegThreads), 0, stream,
-                                   static_cast<const uint32_t*>(src), sc.tiles, sc.ntiles, shift,
-                                   mask, chunk_bits, sc.counts, err);
+            hipLaunchKernelGGL((k_seg_count<FIRST, KS, THREADS>), dim3(grid), dim3(THREADS), 0, stream, src, sc.tiles,
+                               sc.ntiles, shift, mask, chunk_bits, rows, err);
         }
         {
             TimedLaunch t(kKSortScan, stream);
             hipLaunchKernelGGL(k_seg_scan_cols, dim3(col_grid), dim3(kColThreads), 0, stream, sc.chunk_tiles,
-                               num_chunks, R,
-                               sc.counts, sc.totals);
+                               num_chunks, R, rows, sc.totals);
             hipLaunchKernelGGL(k_seg_scan_digits, dim3(chunk_grid), dim3(kSegThreads), 0, stream, chunk_start,
                                num_chunks, R, sc.totals, sc.starts);
         }
         TimedLaunch t(kKSegScatter, stream);
-        if (first)
-            hipLaunchKernelGGL((k_seg_scatter<true, KI>), dim3(grid), dim3(kSegThreads), 0, stream,
-                               static_cast<const KI*>(src), dst, sc.tiles, sc.ntiles, shift, mask, 0u, 0u, sc.counts,
-                               sc.starts);
-        else
-            hipLaunchKernelGGL((k_seg_scatter<false, uint32_t>), dim3(grid), dim3(kSegThreads), 0, stream,
-                               static_cast<const uint32_t*>(src), dst, sc.tiles, sc.ntiles, shift, mask, lo, b1,
-                               sc.counts, sc.starts);
+        hipLaunchKernelGGL((k_seg_scatter<FIRST, KS, THREADS>), dim3(grid), dim3(THREADS), 0, stream, src, dst,
+                           sc.tiles, sc.ntiles, shift, mask, FIRST ? 0u : lo, FIRST ? 0u : b1, rows, sc.starts);
     };
-    pass(true, keys_in, keys_a, lo, b1);
-    if (b2 == 0) return 0;
-    pass(false, keys_a, keys_b, lo + b1, b2);
-    return 1;
+    auto run = [&](auto threads_tag) -> int {
+        pass(std::true_type{}, threads_tag, keys_in, keys_a, lo, b1);
+        if (b2 == 0) return 0;
+        pass(std::false_type{}, threads_tag, static_cast<const uint32_t*>(keys_a), keys_b, lo + b1, b2);
+        return 1;
+    };
+    return wide ? run(std::integral_constant<int, kSegWideThreads>{}) : run(std::integral_constant<int, kSegThreads>{});
 }
 
 template int launch_segmented_sort<uint64_t>(hipStream_t, const uint64_t*, uint32_t*, uint32_t*, const uint64_t*,

@@ -307,6 +307,8 @@ struct BuildLayout {
     uint64_t masks[SVDAG_MAX_LEVELS] = {}, children[SVDAG_MAX_LEVELS] = {};
     uint64_t tkeys[SVDAG_MAX_LEVELS] = {}, trep[SVDAG_MAX_LEVELS] = {}, trank[2] = {};
     uint64_t level_nodes[SVDAG_MAX_LEVELS] = {}, level_slots_of[SVDAG_MAX_LEVELS] = {};
+    // Per hashed level: counts per part of its children and of its table's slots.
+    uint64_t build_parts[SVDAG_MAX_LEVELS] = {}, extract_parts[SVDAG_MAX_LEVELS] = {};
     uint64_t tail_codes[2] = {}, tail_ranks[2] = {}, tail_masks = 0, tail_children = 0, tail_hash = 0;
     uint64_t n = 0, leaf_bound = 0, level_bound = 0, leaf_slots = 0, level_slots = 0;
     uint32_t group_bits = 0;
@@ -343,15 +345,27 @@ BuildLayout plan_build(uint64_t n, int depth, int key_bytes, uint32_t load_shift
     const uint32_t code_bits = uint32_t(3 * depth - 6);
     L.group_bits = std::min(kLeafGroupBits, code_bits);
     L.key_plan = make_sort_plan(int(6 + std::min(L.group_bits, code_bits - 1)), 3 * depth, radix_bits, sort_ipt);
-    const uint64_t stage_tiles = std::max({tiles(n, kPackTileItems), tiles(L.leaf_bound, kBuildTileItems),
-                                           tiles(L.level_slots, kExtractTileItems), uint64_t(1)});
+    const uint64_t stage_tiles = std::max<uint64_t>(tiles(n, kPackTileItems), 1);  // leaf reduce chunks
+    // Hashed levels tail_top + 1 .. depth - 3: at most min(level bound, 8^l)
+    // nodes each.
+    const int tail_top = std::min(depth - 3, kTailTopLevel);
+    for (int l = tail_top + 1; l <= depth - 3; ++l) {
+        L.level_nodes[l] = std::min<uint64_t>(L.level_bound, pow8_capped(l, L.level_bound));
+        L.level_slots_of[l] = (1ull << table_lg(L.level_nodes[l], load_shift)) + kTableOverflow;
+    }
     Carver c;
     L.zero_begin = c.off;
     L.counters = c.take(sizeof(BuildCounters));
     L.key_sort_zero = c.take(4 * sort_zero_words(L.key_plan));
     L.order_zero = c.take(4 * kOrderZeroWords);
     L.sketch = c.take(4 * kSketchRegs);
+    for (int l = tail_top + 1; l <= depth - 3; ++l) {
+        const uint64_t children = l == depth - 3 ? L.leaf_bound : L.level_nodes[l + 1];
+        L.build_parts[l] = c.take(4 * std::min<uint64_t>(kMaxParts, tiles(children, kBuildTileItems)));
+    }
     L.zero_end = c.off;
+    for (int l = tail_top + 1; l <= depth - 3; ++l)
+        L.extract_parts[l] = c.take(4 * std::min<uint64_t>(kMaxParts, tiles(L.level_slots_of[l], kExtractTileItems)));
     L.order_split = c.take(8 * kOrderMaxBuckets);
     L.sort_counts = c.take(4 * sort_count_words(n));
     L.tile_counts = c.take(4 * stage_tiles);
@@ -373,13 +387,8 @@ BuildLayout plan_build(uint64_t n, int depth, int key_bytes, uint32_t load_shift
         L.slots[i] = c.take(4 * L.level_bound);
         L.hashes[i] = c.take(8 * L.level_bound);
     }
-    // Hashed levels tail_top + 1 .. depth - 3: at most min(level bound, 8^l)
-    // nodes each.
-    const int tail_top = std::min(depth - 3, kTailTopLevel);
     uint64_t widest_slots = 1;
     for (int l = tail_top + 1; l <= depth - 3; ++l) {
-        L.level_nodes[l] = std::min<uint64_t>(L.level_bound, pow8_capped(l, L.level_bound));
-        L.level_slots_of[l] = (1ull << table_lg(L.level_nodes[l], load_shift)) + kTableOverflow;
         widest_slots = std::max(widest_slots, L.level_slots_of[l]);
         L.masks[l] = c.take(L.level_nodes[l]);
         L.children[l] = c.take(32 * L.level_nodes[l]);
@@ -908,14 +917,14 @@ int build(svdag_context* ctx, const K* d_keys, uint64_t n, int depth, svdag_dag*
         ca.lp_code = lp_code;
         ca.lp_mask = lp_mask;
         ca.lp_capacity = L.leaf_bound;
-        launch_cell_reduce(st, ca, c, depth - 3);
+        launch_cell_reduce(st, ca, c);
     } else if (buckets.offsets || (!batch && sizeof(K) == 4))
         launch_leaf_reduce<uint32_t>(st, static_cast<const uint32_t*>(sorted), c, L.group_bits, reg_code, reg_mask,
-                                     lp_code, lp_mask, L.leaf_bound, tile_counts, tile_offsets, n, depth - 3,
+                                     lp_code, lp_mask, L.leaf_bound, tile_counts, tile_offsets, n,
                                      code_mask, buckets);
     else
         launch_leaf_reduce<uint64_t>(st, static_cast<const uint64_t*>(sorted), c, L.group_bits, reg_code, reg_mask,
-                                     lp_code, lp_mask, L.leaf_bound, tile_counts, tile_offsets, n, depth - 3,
+                                     lp_code, lp_mask, L.leaf_bound, tile_counts, tile_offsets, n,
                                      code_mask);
 
     // SortLevel(Leaves) (DAGCompression.cu:1070-1071): dedup table, then order.
@@ -935,7 +944,20 @@ int build(svdag_context* ctx, const K* d_keys, uint64_t n, int depth, svdag_dag*
         launch_sketch_estimate(st, regs, &c->leaf_positions, &c->leaf_estimate);
         leaf_size = &c->leaf_estimate;
     }
-    launch_table_clear(st, leaf_table, leaf_size, leaf_lg, ctx->load_shift, 0, L.leaf_slots);
+    // Node counts of every hashed level, from the leaf codes; with them all
+    // tables are cleared at once.
+    const int tail_top = std::min(depth - 3, kTailTopLevel);
+    auto build_parts = [&](int l) { return reinterpret_cast<uint32_t*>(A + L.build_parts[l]); };
+    TableClears clears{};
+    clears.load_shift = ctx->load_shift;
+    clears.add(leaf_table, leaf_size, leaf_lg, 0, L.leaf_slots);
+    if (depth - 3 > tail_top)
+        launch_level_count(st, lp_code, &c->leaf_positions, L.leaf_bound, build_parts(depth - 3), c->pre, depth - 3,
+                           tail_top + 1);
+    for (int l = depth - 3; l > tail_top; --l)
+        clears.add(reinterpret_cast<uint64_t*>(A + L.tkeys[l]), &c->pre[l], &c->table_log2[l], kTableOverflow,
+                   L.level_slots_of[l]);
+    launch_table_clear(st, clears);
     launch_leaf_insert(st, lp_mask, &c->leaf_positions, leaf_table, leaf_lg, lp_slot, L.leaf_bound, err);
     // The unique leaves are ordered (sorted masks, slot -> rank) on the side
     // stream for large builds: the level above the leaves needs their ranks
@@ -983,7 +1005,6 @@ int build(svdag_context* ctx, const K* d_keys, uint64_t n, int depth, svdag_dag*
     // order) and table slots, not their ranks, so every level build is issued
     // first; the extracts follow in order (each turns its children's slots
     // into ranks of the level below), the first one after the leaf order.
-    const int tail_top = std::min(depth - 3, kTailTopLevel);
     for (int l = depth - 3; l > tail_top; --l) {
         const int cur = (depth - 3 - l) & 1;
         LevelBuildArgs a{};
@@ -1006,16 +1027,14 @@ int build(svdag_context* ctx, const K* d_keys, uint64_t n, int depth, svdag_dag*
         a.table_keys = reinterpret_cast<uint64_t*>(A + L.tkeys[l]);
         a.table_rep = reinterpret_cast<uint32_t*>(A + L.trep[l]);
         a.table_log2 = &c->table_log2[l];
-        a.tile_counts = tile_counts;
-        a.offsets = tile_offsets;
-        a.next_count = l > 0 ? &c->pre[l - 1] : nullptr;
+        a.parts = build_parts(l);
+        if (l - 1 > tail_top) {
+            a.next_parts = build_parts(l - 1);
+            a.next_num = level_build_parts(L.level_nodes[l]);
+            a.parent_count = &c->pre[l];
+        }
         a.counters = c;
-        // The table is sized from the level's node count (the build of the
-        // level below, or the leaf reduce, counted it) and cleared by the
-        // level's count kernel.
-        const TableClearArgs clear{a.table_keys, &c->pre[l], &c->table_log2[l], ctx->load_shift, kTableOverflow,
-                                   L.level_slots_of[l]};
-        launch_level_build(st, a, l == depth - 3 ? L.leaf_bound : L.level_nodes[l + 1], &clear);
+        launch_level_build(st, a, l == depth - 3 ? L.leaf_bound : L.level_nodes[l + 1]);
         if (ctx->check_collisions)
             launch_level_check(st, a.parent_slots, a.table_rep, a.parent_masks, a.parent_children, &c->pre[l],
                                &c->collisions, L.level_nodes[l]);
@@ -1029,6 +1048,11 @@ int build(svdag_context* ctx, const K* d_keys, uint64_t n, int depth, svdag_dag*
     // go between stage groups only: each event record leaves the GPU idle for
     // a few microseconds.
     if (!capture) mark(ctx, "level builds");
+    ExtractCounts occupied{};
+    for (int l = depth - 3; l > tail_top; --l)
+        occupied.add(reinterpret_cast<const uint64_t*>(A + L.tkeys[l]), &c->table_log2[l],
+                     reinterpret_cast<uint32_t*>(A + L.extract_parts[l]), level_extract_parts(L.level_slots_of[l]));
+    launch_extract_count(st, occupied);
     TRY(join());
     const uint32_t* below = leaf_rank;  // slot -> rank map of the level below
     for (int l = depth - 3; l > tail_top; --l) {
@@ -1044,9 +1068,7 @@ int build(svdag_context* ctx, const K* d_keys, uint64_t n, int depth, svdag_dag*
         e.out_hashes = reinterpret_cast<uint64_t*>(O + S.hashes[l]);
         e.out_masks = reinterpret_cast<uint8_t*>(O + S.masks[l]);
         e.out_children = reinterpret_cast<uint32_t*>(O + S.children[l]);
-        e.tile_counts = tile_counts;
-        e.offsets = tile_offsets;
-        e.slots_scratch = &c->table_slots;
+        e.parts = reinterpret_cast<const uint32_t*>(A + L.extract_parts[l]);
         e.q_count = &c->uniq[l];
         e.w_count = &c->words[l];
         launch_level_extract(st, e, L.level_slots_of[l]);
@@ -1160,17 +1182,17 @@ int merge_device(svdag_context* ctx, const svdag_dag* dags, uint64_t count, int 
     const uint32_t shift = ctx->load_shift;
     const uint64_t leaf_slots = 1ull << table_lg(total_leaves, shift);
     const uint64_t level_slots = (1ull << table_lg(std::max(max_total, nlive), shift)) + kTableOverflow;
-    const uint64_t stage_tiles =
-        std::max({tiles(level_slots, kExtractTileItems), tiles(nlive, kBuildTileItems), uint64_t(1)});
+    // The uploaded part: the counters as they start, the source tables and the
+    // chunk codes.
     Carver cv;
-    const uint64_t o_zero = cv.off;
     const uint64_t o_counters = cv.take(sizeof(BuildCounters));
-    const uint64_t o_order_zero = cv.take(4 * kOrderZeroWords);
-    const uint64_t zero_end = cv.off;
-    const uint64_t o_order_split = cv.take(8 * kOrderMaxBuckets);
-    const uint64_t o_tile_counts = cv.take(4 * stage_tiles);
-    const uint64_t o_tile_offsets = cv.take(8 * stage_tiles);
     const uint64_t o_sources = cv.take(sizeof(MergeSource) * nlive * (lc_levels + 1));
+    uint64_t o_codes[2];
+    o_codes[0] = cv.take(8 * nlive);
+    const uint64_t upload_bytes = cv.off;
+    const uint64_t o_order_zero = cv.take(4 * kOrderZeroWords);
+    const uint64_t o_order_split = cv.take(8 * kOrderMaxBuckets);
+    const uint64_t o_parts = cv.take(4 * kMaxParts);
     const uint64_t o_leaf_slot_of = cv.take(4 * total_leaves);
     const uint64_t o_leaf_table = cv.take(8 * leaf_slots);
     const uint64_t o_leaf_rank = cv.take(4 * leaf_slots);
@@ -1189,13 +1211,21 @@ int merge_device(svdag_context* ctx, const svdag_dag* dags, uint64_t count, int 
         o_trep[i] = cv.take(4 * level_slots);
         o_trank[i] = cv.take(4 * level_slots);
     }
-    uint64_t o_codes[2];
-    for (int i = 0; i < 2; ++i) o_codes[i] = cv.take(8 * nlive);
+    o_codes[1] = cv.take(8 * nlive);
+    // Few enough chunk levels take the one-workgroup tail (at most
+    // kTailMaxChildren roots below it).
+    const bool tail = k >= 1 && k - 1 <= kTailTopLevel;
+    uint64_t o_tcodes[2], o_tranks[2];
+    for (int i = 0; i < 2; ++i) {
+        o_tcodes[i] = cv.take(8 * kTailMaxParents);
+        o_tranks[i] = cv.take(4 * kTailMaxParents);
+    }
+    const uint64_t o_tmasks = cv.take(kTailMaxParents), o_tchildren = cv.take(32 * kTailMaxParents);
+    const uint64_t o_thash = cv.take(64 * kTailMaxParents);
     TRY(ensure_arena(ctx, cv.off));
     char* A = ctx->arena;
     BuildCounters* c = reinterpret_cast<BuildCounters*>(A + o_counters);
-    uint32_t* tile_counts = reinterpret_cast<uint32_t*>(A + o_tile_counts);
-    uint64_t* tile_offsets = reinterpret_cast<uint64_t*>(A + o_tile_offsets);
+    uint32_t* parts = reinterpret_cast<uint32_t*>(A + o_parts);
 
     uint64_t caps[SVDAG_MAX_LEVELS];
     for (int l = 0; l < levels; ++l) caps[l] = l < k ? pow8_capped(l, nlive) : totals[l - k];
@@ -1209,7 +1239,8 @@ int merge_device(svdag_context* ctx, const svdag_dag* dags, uint64_t count, int 
     };
 
     // Source tables: block 0 = leaves, block 1 + l = level l of every live input.
-    std::vector<MergeSource> src(nlive * (lc_levels + 1));
+    std::vector<char> up(upload_bytes, 0);
+    MergeSource* const src = reinterpret_cast<MergeSource*>(up.data() + o_sources);
     for (int blk = 0; blk <= lc_levels; ++blk) {
         uint64_t first = 0, child_first = 0;
         for (uint64_t j = 0; j < nlive; ++j) {
@@ -1227,24 +1258,22 @@ int merge_device(svdag_context* ctx, const svdag_dag* dags, uint64_t count, int 
         }
     }
     MergeSource* d_src = reinterpret_cast<MergeSource*>(A + o_sources);
-    if (hipMemcpyAsync(d_src, src.data(), sizeof(MergeSource) * src.size(), hipMemcpyHostToDevice, st) != hipSuccess)
-        return fail(set_error(SVDAG_ERR_HIP, "merge source upload failed"));
-    std::vector<uint64_t> codes(nlive);
+    uint64_t* const codes = reinterpret_cast<uint64_t*>(up.data() + o_codes[0]);
     for (uint64_t j = 0; j < nlive; ++j) codes[j] = live[j];
-    if (hipMemcpyAsync(A + o_codes[0], codes.data(), 8 * nlive, hipMemcpyHostToDevice, st) != hipSuccess)
-        return fail(set_error(SVDAG_ERR_HIP, "chunk code upload failed"));
-    // The upload buffers must outlive the copies: finish them before returning.
+    // Node counts known beforehand: the inputs' levels, and the level over the
+    // chunk roots.
+    BuildCounters* const start = reinterpret_cast<BuildCounters*>(up.data() + o_counters);
+    start->leaf_positions = total_leaves;
+    for (int l = k; l < levels; ++l) start->pre[l] = totals[l - k];
+    for (int l = 0; l < k; ++l)
+        for (uint64_t j = 0; j < nlive; ++j)
+            start->pre[l] += j == 0 || (live[j] >> (3 * (k - l))) != (live[j - 1] >> (3 * (k - l))) ? 1 : 0;
+    if (hipMemcpyAsync(A, up.data(), upload_bytes, hipMemcpyHostToDevice, st) != hipSuccess)
+        return fail(set_error(SVDAG_ERR_HIP, "merge source upload failed"));
+    // The upload buffer must outlive the copy: finish it before returning.
     if (hipStreamSynchronize(st) != hipSuccess) return fail(set_error(SVDAG_ERR_HIP, "merge upload failed"));
 
-    launch_fill_u64(st, reinterpret_cast<uint64_t*>(A + o_zero), (zero_end - o_zero) / 8, 0);
-    launch_fill_u64(st, &c->leaf_positions, 1, total_leaves);
-    for (int l = k; l < levels; ++l) launch_fill_u64(st, &c->pre[l], 1, totals[l - k]);
-    if (k > 0) {
-        uint64_t groups = 0;
-        for (uint64_t j = 0; j < nlive; ++j)
-            if (j == 0 || (live[j] >> 3) != (live[j - 1] >> 3)) ++groups;
-        launch_fill_u64(st, &c->pre[k - 1], 1, groups);
-    }
+    launch_fill_u64(st, reinterpret_cast<uint64_t*>(A + o_order_zero), kOrderZeroWords / 2, 0);
 
     // Leaves: shared hashed table, its order, ranks.
     uint64_t* leaf_table = reinterpret_cast<uint64_t*>(A + o_leaf_table);
@@ -1255,7 +1284,16 @@ int merge_device(svdag_context* ctx, const svdag_dag* dags, uint64_t count, int 
     uint64_t* lk1 = reinterpret_cast<uint64_t*>(A + o_lk[1]);
     uint32_t* ls0 = reinterpret_cast<uint32_t*>(A + o_ls[0]);
     uint32_t* ls1 = reinterpret_cast<uint32_t*>(A + o_ls[1]);
-    launch_table_clear(st, leaf_table, &c->leaf_positions, leaf_lg, shift, 0, leaf_slots);
+    // Tables alternate; each is cleared beside the count of the one before.
+    auto add_clear = [&](TableClears& t, int l, int cur) {
+        t.load_shift = shift;
+        t.add(reinterpret_cast<uint64_t*>(A + o_tk[cur]), &c->pre[l], &c->table_log2[l], kTableOverflow, level_slots);
+    };
+    TableClears first_clears{};
+    first_clears.load_shift = shift;
+    first_clears.add(leaf_table, &c->leaf_positions, leaf_lg, 0, leaf_slots);
+    add_clear(first_clears, levels - 1, 0);
+    launch_table_clear(st, first_clears);
     launch_merge_insert(st, d_src, uint32_t(nlive), total_leaves, nullptr, nullptr, nullptr, nullptr, leaf_table,
                         nullptr, leaf_lg, leaf_slot_of, c, 0);
     uint64_t* leaves_out = reinterpret_cast<uint64_t*>(O + S.leaves);
@@ -1279,11 +1317,14 @@ int merge_device(svdag_context* ctx, const svdag_dag* dags, uint64_t count, int 
         e.out_hashes = reinterpret_cast<uint64_t*>(O + S.hashes[l]);
         e.out_masks = reinterpret_cast<uint8_t*>(O + S.masks[l]);
         e.out_children = reinterpret_cast<uint32_t*>(O + S.children[l]);
-        e.tile_counts = tile_counts;
-        e.offsets = tile_offsets;
-        e.slots_scratch = &c->table_slots;
+        e.parts = parts;
         e.q_count = &c->uniq[l];
         e.w_count = &c->words[l];
+        ExtractCounts occupied{};
+        occupied.add(e.table_keys, e.table_log2, parts, level_extract_parts(level_slots));
+        TableClears next{};
+        if (l > 0 && !(tail && l == k)) add_clear(next, l - 1, cur ^ 1);
+        launch_extract_count(st, occupied, &next);
         launch_level_extract(st, e, level_slots);
     };
     // Levels below the sub-DAG roots.
@@ -1293,7 +1334,6 @@ int merge_device(svdag_context* ctx, const svdag_dag* dags, uint64_t count, int 
         const int cur = step & 1;
         uint64_t* tk = reinterpret_cast<uint64_t*>(A + o_tk[cur]);
         uint32_t* slot_of = reinterpret_cast<uint32_t*>(A + o_slot_of[cur]);
-        launch_table_clear(st, tk, &c->pre[l], &c->table_log2[l], shift, kTableOverflow, level_slots);
         launch_merge_insert(st, d_src + uint64_t(lc + 1) * nlive, uint32_t(nlive), totals[lc], child_slot_of,
                             child_rank, masks, children, tk, reinterpret_cast<uint32_t*>(A + o_trep[cur]),
                             &c->table_log2[l], slot_of, c, 1);
@@ -1302,7 +1342,30 @@ int merge_device(svdag_context* ctx, const svdag_dag* dags, uint64_t count, int 
         child_rank = reinterpret_cast<const uint32_t*>(A + o_trank[cur]);
     }
     // New top levels over the chunk roots (DAGCompression.cu:1505-1533).
-    for (int l = k - 1; l >= 0; --l, ++step) {
+    if (tail) {
+        TailArgs t{};
+        t.top = k - 1;
+        t.child_codes = reinterpret_cast<const uint64_t*>(A + o_codes[0]);
+        t.child_slots = child_slot_of;
+        t.child_hashes = reinterpret_cast<const uint64_t*>(O + S.hashes[k]);
+        t.child_count = &c->pre[k];
+        t.child_rank_of_slot = child_rank;
+        for (int i = 0; i < 2; ++i) {
+            t.codes[i] = reinterpret_cast<uint64_t*>(A + o_tcodes[i]);
+            t.ranks[i] = reinterpret_cast<uint32_t*>(A + o_tranks[i]);
+        }
+        t.masks = reinterpret_cast<uint8_t*>(A + o_tmasks);
+        t.children = reinterpret_cast<uint32_t*>(A + o_tchildren);
+        t.child_hash = reinterpret_cast<uint64_t*>(A + o_thash);
+        for (int l = 0; l < k; ++l) {
+            t.out_hashes[l] = reinterpret_cast<uint64_t*>(O + S.hashes[l]);
+            t.out_masks[l] = reinterpret_cast<uint8_t*>(O + S.masks[l]);
+            t.out_children[l] = reinterpret_cast<uint32_t*>(O + S.children[l]);
+        }
+        t.counters = c;
+        launch_level_tail(st, t);
+    }
+    for (int l = tail ? -1 : k - 1; l >= 0; --l, ++step) {
         const int cur = step & 1;
         LevelBuildArgs a{};
         a.child_codes = reinterpret_cast<const uint64_t*>(A + o_codes[(k - 1 - l) & 1]);
@@ -1317,11 +1380,9 @@ int merge_device(svdag_context* ctx, const svdag_dag* dags, uint64_t count, int 
         a.table_keys = reinterpret_cast<uint64_t*>(A + o_tk[cur]);
         a.table_rep = reinterpret_cast<uint32_t*>(A + o_trep[cur]);
         a.table_log2 = &c->table_log2[l];
-        a.tile_counts = tile_counts;
-        a.offsets = tile_offsets;
-        a.next_count = l > 0 ? &c->pre[l - 1] : nullptr;
+        a.parts = parts;
         a.counters = c;
-        launch_table_clear(st, a.table_keys, &c->pre[l], &c->table_log2[l], shift, kTableOverflow, level_slots);
+        launch_level_count(st, a.child_codes, a.child_count, nlive, parts, nullptr, 0, 0);
         launch_level_build(st, a, nlive);
         extract(l, cur);
         child_slot_of = a.parent_slots;
@@ -1706,15 +1767,13 @@ int svdag_create_final_dag(svdag_context* ctx, const svdag_dag* dag, uint32_t** 
     const uint64_t ntiles = std::max<uint64_t>(1, tiles(nodes, kFinalTileItems));
     Carver cv;
     const uint64_t o_counts = cv.take(4 * ntiles);
-    const uint64_t o_offsets = cv.take(8 * ntiles);
     const uint64_t o_pos = cv.take(4 * std::max<uint64_t>(nodes, 1));
     TRY(ensure_arena(ctx, cv.off));
     void* words = nullptr;
     TRY(device_alloc(ctx, &words, 4 * std::max<uint64_t>(total_words, 1)));
     a.words = static_cast<uint32_t*>(words);
     a.positions = reinterpret_cast<uint32_t*>(ctx->arena + o_pos);
-    a.counts = reinterpret_cast<uint32_t*>(ctx->arena + o_counts);
-    a.offsets = reinterpret_cast<uint64_t*>(ctx->arena + o_offsets);
+    a.parts = reinterpret_cast<uint32_t*>(ctx->arena + o_counts);
     launch_final(ctx->stream, a);
     const hipError_t e = hipGetLastError();
     mark(ctx, "final layout");
@@ -2544,14 +2603,13 @@ int svdag_resident_dag(svdag_resident* r, svdag_dag* out)
     const uint64_t L = r->occupied[r->rlevels];
     uint64_t max_slots = r->leaf_slots;
     for (int i = 0; i < r->rlevels; ++i) max_slots = std::max(max_slots, r->slots[i]);
-    const uint64_t stage_tiles = std::max(tiles(max_slots, kExtractTileItems), uint64_t(1));
     Carver cv;
     const uint64_t o_zero = cv.off;
     const uint64_t o_counters = cv.take(sizeof(BuildCounters));
     const uint64_t o_order_zero = cv.take(4 * kOrderZeroWords);
     const uint64_t zero_end = cv.off;
     const uint64_t o_order_split = cv.take(8 * kOrderMaxBuckets);
-    const uint64_t o_tile_counts = cv.take(4 * stage_tiles), o_tile_offsets = cv.take(8 * stage_tiles);
+    const uint64_t o_parts = cv.take(4 * kMaxParts * r->rlevels);
     uint64_t o_lk[2], o_ls[2];
     for (int i = 0; i < 2; ++i) {
         o_lk[i] = cv.take(8 * L);
@@ -2570,8 +2628,6 @@ int svdag_resident_dag(svdag_resident* r, svdag_dag* out)
     TRY(ensure_arena(ctx, cv.off));
     char* A = ctx->arena;
     BuildCounters* c = reinterpret_cast<BuildCounters*>(A + o_counters);
-    uint32_t* tile_counts = reinterpret_cast<uint32_t*>(A + o_tile_counts);
-    uint64_t* tile_offsets = reinterpret_cast<uint64_t*>(A + o_tile_offsets);
 
     uint64_t caps[SVDAG_MAX_LEVELS];
     for (int l = 0; l < levels; ++l) caps[l] = l < r->top ? (1ull << (3 * l)) : r->occupied[l - r->top];
@@ -2598,6 +2654,11 @@ int svdag_resident_dag(svdag_resident* r, svdag_dag* out)
                       r->leaf_slots, L);
     // Resident levels bottom-up, each in ascending hash order with its
     // children's slots turned into ranks of the level below.
+    uint32_t* const level_parts = reinterpret_cast<uint32_t*>(A + o_parts);
+    ExtractCounts occupied{};
+    for (int i = 0; i < r->rlevels; ++i)
+        occupied.add(r->tkeys[i], r->d_lg + i, level_parts + uint64_t(kMaxParts) * i, level_extract_parts(r->slots[i]));
+    launch_extract_count(st, occupied);
     const uint32_t* below = leaf_rank;
     int cur = 0;
     for (int i = r->rlevels - 1; i >= 0; --i, cur ^= 1) {
@@ -2613,9 +2674,7 @@ int svdag_resident_dag(svdag_resident* r, svdag_dag* out)
         e.out_hashes = reinterpret_cast<uint64_t*>(O + S.hashes[l]);
         e.out_masks = reinterpret_cast<uint8_t*>(O + S.masks[l]);
         e.out_children = reinterpret_cast<uint32_t*>(O + S.children[l]);
-        e.tile_counts = tile_counts;
-        e.offsets = tile_offsets;
-        e.slots_scratch = &c->table_slots;
+        e.parts = level_parts + uint64_t(kMaxParts) * i;
         e.q_count = &c->uniq[l];
         e.w_count = &c->words[l];
         launch_level_extract(st, e, r->slots[i]);

@@ -17,9 +17,10 @@
 //   CreateFinalDAG / WriteTo        :834-861, :1550-1610 -> k_final_count /
 //       k_final_positions / k_final_write
 // Every compaction is reduce-then-scan: a count kernel writes one count per
-// tile, k_scan_counts (one workgroup) turns them into offsets, and the main
-// kernel handles tile blockIdx.x + k * gridDim.x.  No workgroup waits on
-// another; element counts come from device memory, so the build runs without
+// part (the consecutive tiles of one workgroup of the main kernel), and each
+// workgroup of the main kernel sums the counts before its own; k_leaf_compact
+// takes its offsets from a one-workgroup scan (k_scan_counts).  No workgroup
+// waits on another; element counts come from device memory, so the build runs without
 // host round trips.
 #include "svdag_device.hpp"
 #include "svdag_internal.hpp"
@@ -79,6 +80,28 @@ __global__ __launch_bounds__(kScanThreads) void k_scan_counts(const uint32_t* __
         running += total;
     }
     if (total_out && threadIdx.x == 0) *total_out = running;
+}
+
+// Parts of a stage: workgroup b of P takes the consecutive tiles [t0, t1) of
+// ntiles.  A tile t lies in part part_of_tile.
+__device__ __forceinline__ void part_tiles(uint64_t ntiles, uint32_t b, uint32_t P, uint64_t& t0, uint64_t& t1)
+{
+    t0 = ntiles * b / P;
+    t1 = ntiles * (uint64_t(b) + 1) / P;
+}
+__device__ __forceinline__ uint32_t part_of_tile(uint64_t ntiles, uint64_t t, uint32_t P)
+{
+    return uint32_t(((t + 1) * P - 1) / ntiles);
+}
+
+// Sum of the parts before this workgroup's (two barriers; every thread must
+// call it).  At most kMaxParts words from L2: a scan kernel between the count
+// and the main kernel took 4.6 us at the smallest, 27 us over 65536 tiles.
+__device__ __forceinline__ uint64_t parts_before(const uint32_t* __restrict__ parts, uint64_t* scratch)
+{
+    uint64_t sum = 0;
+    for (uint32_t i = threadIdx.x; i < blockIdx.x; i += kThreads) sum += parts[i];
+    return block_reduce_sum<kThreads>(sum, scratch);
 }
 
 // ---------------------------------------------------------------------------
@@ -166,11 +189,9 @@ __global__ __launch_bounds__(kThreads) void k_leaf_reduce(const K* __restrict__ 
                                                           uint32_t r, uint64_t* __restrict__ reg_code,
                                                           uint64_t* __restrict__ reg_mask,
                                                           uint32_t* __restrict__ counts,
-                                                          uint64_t* __restrict__ next_count,
                                                           unsigned long long* __restrict__ err, ChunkPrefix bk)
 {
     __shared__ uint64_t s_tab[kReduceWaves][kReduceTable];
-    __shared__ uint64_t s_parents[kReduceWaves];
     constexpr int G = kReduceGroups<K>;
     constexpr bool BUCKETED = BM != kBucketsNone;
     // Keys and group indices in registers: 32-bit for 32-bit keys (a group
@@ -199,7 +220,6 @@ __global__ __launch_bounds__(kThreads) void k_leaf_reduce(const K* __restrict__ 
     const uint64_t nchunks = (n + kReduceChunk - 1) / kReduceChunk;
     const uint32_t sh = 6 + r;
     const uint32_t low_mask = (1u << r) - 1u;
-    uint32_t parent_lanes = 0;  // per lane: parents counted by the flushes
     bool overflow = false;
 
     for (uint64_t chunk = uint64_t(blockIdx.x) * kReduceWaves + w; chunk < nchunks;
@@ -252,8 +272,7 @@ __global__ __launch_bounds__(kThreads) void k_leaf_reduce(const K* __restrict__ 
 
         // Writes the open group's leaves in order and clears the table.  Row e
         // of the table is read by lanes 0..63 (leaves 64e + lane), so a leaf's
-        // output position is the count of nonzero rows' ballots before it;
-        // the 8 leaves of one parent are 8 consecutive lanes of one row.
+        // output position is the count of nonzero rows' ballots before it.
         auto flush = [&]() {
             __builtin_amdgcn_wave_barrier();
             // A full table fits the region for valid bounds: the groups before
@@ -264,15 +283,13 @@ __global__ __launch_bounds__(kThreads) void k_leaf_reduce(const K* __restrict__ 
             // Row by row, with the per-row bookkeeping in vector registers:
             // this runs once per group and its scalar work had been about half
             // of the kernel's scalar instructions (the scalar unit is its
-            // limit).  Lane l of row e counts parent 8e + l/8 when l % 8 == 0
-            // and one of its 8 leaves is present.
+            // limit).
             uint32_t pos = written;
 #pragma unroll
             for (int e = 0; e < 8; ++e) {
                 const uint64_t m = tab[e * kWave + lane];
                 tab[e * kWave + lane] = 0ull;
                 const uint64_t B = __ballot(m != 0ull);
-                parent_lanes += ((lane & 7u) == 0u && ((B >> (lane & 56u)) & 0xFFull) != 0ull) ? 1u : 0u;
                 if (m && room) {
                     const uint32_t p = pos + uint32_t(__popcll(B & lanemask_lt()));
                     oc[p] = (uint64_t(cur_b) << r) | uint64_t(e * kWave + lane);
@@ -369,17 +386,7 @@ __global__ __launch_bounds__(kThreads) void k_leaf_reduce(const K* __restrict__ 
         }
         if (lane == 0) counts[chunk] = written;
     }
-    uint64_t parents = parent_lanes;
-#pragma unroll
-    for (int d = kWave / 2; d >= 1; d >>= 1) parents += uint64_t(uint32_t(__shfl_xor(int(uint32_t(parents)), d, kWave)));
-    if (lane == 0) s_parents[w] = parents;
     if (overflow && lane == 0) atomicOr(err, (unsigned long long)kErrInternal);
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        uint64_t t = 0;
-        for (int i = 0; i < kReduceWaves; ++i) t += s_parents[i];
-        if (t) atomicAdd((unsigned long long*)next_count, (unsigned long long)t);
-    }
 }
 
 // Region of chunk c (counts[c] leaves) -> lp_code / lp_mask at offsets[c].
@@ -434,8 +441,7 @@ constexpr int kCellKeys = 8;  // keys per thread in flight
 constexpr int kCellRows = int(kCellLeaves) / kCellThreads;
 static_assert(kCellRows * kCellThreads == int(kCellLeaves) && kMaxRunCells < kWave, "rows and starts per lane");
 
-__global__ __launch_bounds__(kCellThreads) void k_cell_reduce(CellArgs a, const uint64_t* __restrict__ n_ptr,
-                                                              uint64_t* __restrict__ next_count)
+__global__ __launch_bounds__(kCellThreads) void k_cell_reduce(CellArgs a, const uint64_t* __restrict__ n_ptr)
 {
     __shared__ uint64_t s_tab[kCellLeaves];
     __shared__ uint32_t s_cnt[kCellWaves];
@@ -446,7 +452,6 @@ __global__ __launch_bounds__(kCellThreads) void k_cell_reduce(CellArgs a, const 
     __syncthreads();
     const uint32_t n = uint32_t(*n_ptr);
     const uint64_t runs = cell_runs(a.cells, a.run_cells);
-    uint32_t parent_lanes = 0;  // per lane: parents counted by the flushes
     // Bounds of a run's cells: lane l holds cell l's start (l == cells: the last
     // one's end).  No keys (or offsets a check rejected): every cell is empty.
     auto bounds_of = [&](uint64_t run) -> uint32_t {
@@ -511,8 +516,7 @@ __global__ __launch_bounds__(kCellThreads) void k_cell_reduce(CellArgs a, const 
         have = next_cell();
         if (have) load(s, e - s);
         __syncthreads();
-        // Wave w holds the leaves [w * 512, ...) in rows of 64; lane l of a
-        // row counts the parent of leaves l .. l + 7 when l % 8 == 0.
+        // Wave w holds the leaves [w * 512, ...) in rows of 64.
         uint64_t m[kCellRows];
         uint32_t cnt = 0;
 #pragma unroll
@@ -522,11 +526,7 @@ __global__ __launch_bounds__(kCellThreads) void k_cell_reduce(CellArgs a, const 
             s_tab[leaf] = 0ull;
         }
 #pragma unroll
-        for (int r = 0; r < kCellRows; ++r) {
-            const uint64_t B = __ballot(m[r] != 0ull);
-            parent_lanes += ((lane & 7u) == 0u && ((B >> (lane & 56u)) & 0xFFull) != 0ull) ? 1u : 0u;
-            cnt += uint32_t(__popcll(B));
-        }
+        for (int r = 0; r < kCellRows; ++r) cnt += uint32_t(__popcll(__ballot(m[r] != 0ull)));
         if (lane == 0) s_cnt[w] = cnt;
         __syncthreads();
         uint32_t pos = base + written;
@@ -550,15 +550,6 @@ __global__ __launch_bounds__(kCellThreads) void k_cell_reduce(CellArgs a, const 
             if (threadIdx.x == 0) a.run_counts[cur_run] = written;
             written = 0;
         }
-    }
-    const uint32_t parents = wave_reduce_sum32(parent_lanes);
-    __syncthreads();
-    if (lane == 0) s_cnt[w] = parents;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        uint64_t t = 0;
-        for (int i = 0; i < kCellWaves; ++i) t += s_cnt[i];
-        if (t) atomicAdd((unsigned long long*)next_count, (unsigned long long)t);
     }
 }
 
@@ -619,18 +610,23 @@ __global__ __launch_bounds__(kThreads) void k_cell_compact(CellArgs a, const uin
     if (blockIdx.x + 1 == gridDim.x && threadIdx.x == 0) *total_out = before;
 }
 
-// Clears slots [0, 2^lg + overflow) with lg = max(8, ceil(log2(count << load_shift))).
-__global__ void k_table_clear(uint64_t* __restrict__ keys, const uint64_t* __restrict__ count_ptr,
-                              uint32_t* __restrict__ log2_out, uint32_t load_shift, uint32_t overflow)
+// Clears slots [0, 2^lg + overflow) of each table, lg = max(8,
+// ceil(log2(count << load_shift))), and records lg.
+__device__ __forceinline__ void clear_tables(const TableClears& a)
 {
-    const uint64_t cnt = *count_ptr;
-    const uint32_t need = ceil_log2_u64((cnt ? cnt : 1ull) << load_shift);
-    const uint32_t lg = need > 8u ? need : 8u;
-    const uint64_t total = (1ull << lg) + overflow;
-    if (blockIdx.x == 0 && threadIdx.x == 0) *log2_out = lg;
     const uint64_t stride = uint64_t(gridDim.x) * blockDim.x;
-    for (uint64_t i = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x; i < total; i += stride) keys[i] = 0;
+    for (int t = 0; t < a.num; ++t) {
+        const uint64_t cnt = *a.table[t].count;
+        const uint32_t need = ceil_log2_u64((cnt ? cnt : 1ull) << a.load_shift);
+        const uint32_t lg = need > 8u ? need : 8u;
+        const uint64_t total = (1ull << lg) + a.table[t].overflow;
+        uint64_t* __restrict__ keys = a.table[t].keys;
+        if (blockIdx.x == 0 && threadIdx.x == 0) *a.table[t].log2_out = lg;
+        for (uint64_t i = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x; i < total; i += stride) keys[i] = 0;
+    }
 }
+
+__global__ void k_table_clear(TableClears a) { clear_tables(a); }
 
 // Inserts key h (never 0) into a wrap-around table of 2^lg slots; `won` tells
 // whether this call placed the key.  A probe never exceeds the table size; a
@@ -1213,50 +1209,51 @@ constexpr int kBuildIpt = 4;
 constexpr int kBuildTile = kThreads * kBuildIpt;
 
 __device__ __forceinline__ void parent_runs(const uint64_t* __restrict__ codes, uint64_t n, uint64_t first,
-                                            uint64_t (&code)[kBuildIpt], uint32_t& starts, uint32_t& gcount)
+                                            uint64_t (&code)[kBuildIpt], uint32_t& starts, uint32_t& gstarts)
 {
     // Unconditional loads (positions past the end read the last code and are
     // never starts), so that all of them are in flight at once.  n >= 1 here.
 #pragma unroll
     for (int j = 0; j < kBuildIpt; ++j) code[j] = codes[min(first + j, n - 1)];
     const uint64_t before = first > 0 ? codes[min(first - 1, n - 1)] : ~0ull;
-    starts = 0;
-    gcount = 0;
+    starts = 0;   // bit j: child j starts a parent
+    gstarts = 0;  // bit j: it starts a grandparent too
 #pragma unroll
     for (int j = 0; j < kBuildIpt; ++j) {
         const uint64_t prev = j ? code[j - 1] : before;
         const bool head = first + j == 0;
         if (first + j < n && (head || (code[j] >> 3) != (prev >> 3))) {
             starts |= 1u << j;
-            gcount += (head || (code[j] >> 6) != (prev >> 6)) ? 1u : 0u;
+            gstarts |= (head || (code[j] >> 6) != (prev >> 6)) ? 1u << j : 0u;
         }
     }
 }
 
-// With clear.keys set, the kernel also clears the level's table (as
-// k_table_clear: the table's node count is not the one this kernel adds to).
+// The parents that each part of the children starts (the workgroups of
+// k_level_build take the same parts).  With pre set, also the node counts of
+// all levels from `level` down to `lowest`, from the children's codes alone:
+// child i starts a node of level `level - j` when its code differs from its
+// predecessor's above bit 3 (j + 1).
 __global__ __launch_bounds__(kThreads) void k_level_count(const uint64_t* __restrict__ codes,
                                                           const uint64_t* __restrict__ n_ptr,
-                                                          uint32_t* __restrict__ counts,
-                                                          uint64_t* __restrict__ next_count, TableClearArgs clear)
+                                                          uint32_t* __restrict__ parts, uint64_t* __restrict__ pre,
+                                                          int level, int lowest)
 {
-    if (clear.keys) {
-        const uint64_t cnt = *clear.count;
-        const uint32_t need = ceil_log2_u64((cnt ? cnt : 1ull) << clear.load_shift);
-        const uint32_t lg = need > 8u ? need : 8u;
-        const uint64_t total = (1ull << lg) + clear.overflow;
-        if (blockIdx.x == 0 && threadIdx.x == 0) *clear.log2_out = lg;
-        const uint64_t stride = uint64_t(gridDim.x) * blockDim.x;
-        for (uint64_t i = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x; i < total; i += stride) clear.keys[i] = 0;
-    }
+    constexpr int kTriples = 22;  // of a 64-bit code
+    __shared__ uint32_t s_diff[kTriples];
     __shared__ uint64_t s_red[kThreads / kWave];
     const uint64_t n = *n_ptr;
     const uint64_t ntiles = (n + kBuildTile - 1) / kBuildTile;
-    uint64_t gtot = 0;
-    for (uint64_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
-        // The same run starts as parent_runs, counted with coalesced reads:
-        // lane i of a round reads code i and its predecessor (all loads
-        // issued first, indices clamped into [0, n)).
+    if (threadIdx.x < uint32_t(kTriples)) s_diff[threadIdx.x] = 0;
+    __syncthreads();
+    uint64_t t0, t1;
+    part_tiles(ntiles, blockIdx.x, gridDim.x, t0, t1);
+    // Starts of parents, grandparents; the levels above them from a histogram
+    // of the highest triple that differs (one child in 64 or fewer).
+    uint32_t starts = 0, gstarts = 0;
+    for (uint64_t tile = t0; tile < t1; ++tile) {
+        // Coalesced: lane i of a round reads code i and its predecessor (all
+        // loads issued first, indices clamped into [0, n)).
         const uint64_t base = tile * kBuildTile + threadIdx.x;
         uint64_t cv[kBuildIpt], pv[kBuildIpt];
 #pragma unroll
@@ -1265,22 +1262,23 @@ __global__ __launch_bounds__(kThreads) void k_level_count(const uint64_t* __rest
             cv[j] = codes[min(i, n - 1)];
             pv[j] = codes[i > 0 ? min(i - 1, n - 1) : 0];
         }
-        uint32_t starts = 0, gcount = 0;
 #pragma unroll
         for (int j = 0; j < kBuildIpt; ++j) {
             const uint64_t i = base + uint64_t(j) * kThreads;
-            if (i < n && (i == 0 || (cv[j] >> 3) != (pv[j] >> 3))) {
-                ++starts;
-                gcount += (i == 0 || (cv[j] >> 6) != (pv[j] >> 6)) ? 1u : 0u;
-            }
+            const uint64_t x = i == 0 ? ~0ull : i < n ? cv[j] ^ pv[j] : 0ull;
+            starts += (x >> 3) != 0 ? 1u : 0u;
+            gstarts += (x >> 6) != 0 ? 1u : 0u;
+            if (pre && (x >> 9) != 0) atomicAdd(&s_diff[(63 - __clzll((long long)x)) / 3], 1u);
         }
-        const uint64_t cnt = block_reduce_sum<kThreads>(starts, s_red);
-        gtot += gcount;
-        if (threadIdx.x == 0) counts[tile] = uint32_t(cnt);
     }
-    if (next_count) {
-        gtot = block_reduce_sum<kThreads>(gtot, s_red);
-        if (threadIdx.x == 0 && gtot) atomicAdd((unsigned long long*)next_count, (unsigned long long)gtot);
+    const uint64_t heads = block_reduce_sum<kThreads>(starts, s_red);
+    const uint64_t ghead = block_reduce_sum<kThreads>(gstarts, s_red);
+    if (threadIdx.x == 0) parts[blockIdx.x] = uint32_t(heads);
+    if (!pre) return;
+    for (int j = int(threadIdx.x); level - j >= lowest; j += kThreads) {
+        uint64_t sum = j == 0 ? heads : j == 1 ? ghead : 0;
+        for (int t = j + 1; j >= 2 && t < kTriples; ++t) sum += s_diff[t];
+        if (sum) atomicAdd((unsigned long long*)&pre[level - j], (unsigned long long)sum);
     }
 }
 
@@ -1331,24 +1329,44 @@ __device__ __forceinline__ uint64_t acc_emit(const ParentAcc& a, uint64_t p, con
 __global__ __launch_bounds__(kThreads) void k_level_build(LevelBuildArgs g)
 {
     __shared__ uint32_t s_scan[kThreads / kWave];
+    __shared__ uint64_t s_red[kThreads / kWave];
+    __shared__ uint32_t s_heads[kThreads / kWave];
     __shared__ uint64_t s_hash[kBuildTile];
     __shared__ uint32_t s_elect[kThreads / kWave][kElectBuckets];
     const uint64_t n = *g.child_count;
     const uint64_t ntiles = (n + kBuildTile - 1) / kBuildTile;
+    const uint64_t next_tiles = g.next_parts ? (*g.parent_count + kBuildTile - 1) / kBuildTile : 0;
+    uint64_t t0, t1;
+    part_tiles(ntiles, blockIdx.x, gridDim.x, t0, t1);
+    if (t0 >= t1) return;  // the whole workgroup
+    uint64_t p0 = parts_before(g.parts, s_red);
     const uint32_t lg = *g.table_log2;
     const uint64_t limit = (1ull << lg) + kTableOverflow;
     const uint32_t* __restrict__ slots = g.child_slots;
     const uint32_t* __restrict__ rank_of_slot = g.child_rank_of_slot;
     const uint64_t* __restrict__ hashes = g.child_hashes;
     const uint64_t* __restrict__ seq = g.child_hash_seq;
-    for (uint64_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
+    for (uint64_t tile = t0; tile < t1; ++tile) {
         const uint64_t first = tile * kBuildTile + uint64_t(threadIdx.x) * kBuildIpt;
         uint64_t code[kBuildIpt];
-        uint32_t starts, gcount;
-        parent_runs(g.child_codes, n, first, code, starts, gcount);
+        uint32_t starts, gstarts;
+        parent_runs(g.child_codes, n, first, code, starts, gstarts);
         uint32_t tile_parents;
         const uint32_t local = block_exclusive_scan<kThreads>(__popc(starts), s_scan, tile_parents);
-        const uint64_t p0 = g.offsets[tile];
+        if (g.next_parts) {
+            // Parents of this level's nodes, for the parts of the next build:
+            // the tile's nodes [p0, p0 + tile_parents) lie in at most two of
+            // its tiles (low half: the first, high half: the second).
+            const uint32_t cut = uint32_t(kBuildTile - p0 % kBuildTile);
+            uint32_t heads = 0;
+#pragma unroll
+            for (int j = 0; j < kBuildIpt; ++j) {
+                const uint32_t q = local + uint32_t(__popc(starts & ((1u << j) - 1u)));
+                heads += ((gstarts >> j) & 1u) ? (q < cut ? 1u : 1u << 16) : 0u;
+            }
+            heads = wave_reduce_sum32(heads);
+            if (lane_id() == 0) s_heads[threadIdx.x / kWave] = heads;
+        }
 
         // Indices are clamped into [0, n): loads past the end read a valid child
         // that is then ignored.
@@ -1399,6 +1417,13 @@ __global__ __launch_bounds__(kThreads) void k_level_build(LevelBuildArgs g)
             s_hash[q] = acc_emit(acc, p0 + q, g);
         }
         __syncthreads();
+        if (g.next_parts && threadIdx.x < 2) {
+            uint32_t sum = 0;
+#pragma unroll
+            for (int i = 0; i < kThreads / kWave; ++i) sum += (s_heads[i] >> (16 * threadIdx.x)) & 0xFFFFu;
+            const uint64_t t = p0 / kBuildTile + threadIdx.x;
+            if (sum) atomicAdd(&g.next_parts[part_of_tile(next_tiles, t, g.next_num)], sum);
+        }
         // Equal parents (identical subtrees) often sit side by side: one lane
         // per distinct hash in a wave probes the table, the others take its slot.
         for (uint32_t k0 = 0; k0 < tile_parents; k0 += kThreads) {
@@ -1413,6 +1438,7 @@ __global__ __launch_bounds__(kThreads) void k_level_build(LevelBuildArgs g)
             slot = uint32_t(__shfl(int(slot), int(leader), kWave));
             if (valid) g.parent_slots[p0 + k] = slot;
         }
+        p0 += tile_parents;
         __syncthreads();  // s_hash is rewritten by the next tile
     }
 }
@@ -1610,29 +1636,35 @@ constexpr int kExtractIpt = 1;
 constexpr int kExtractTile = kThreads * kExtractIpt;
 constexpr int kHalo = 128;
 
-__global__ __launch_bounds__(kThreads) void k_extract_count(const uint64_t* __restrict__ table_keys,
-                                                            const uint32_t* __restrict__ table_log2,
-                                                            uint32_t* __restrict__ counts,
-                                                            uint64_t* __restrict__ slots_out)
+// Occupied slots of every part of the tables given (one workgroup per part;
+// the workgroups of k_level_extract take the same parts).  With clear.num, the
+// workgroups also clear those tables.
+__global__ __launch_bounds__(kThreads) void k_extract_count(ExtractCounts a, TableClears clear)
 {
     __shared__ uint64_t s_red[kThreads / kWave];
-    const uint64_t total = (1ull << *table_log2) + kTableOverflow;
+    uint32_t b = blockIdx.x;
+    int t = 0;
+    while (b >= a.table[t].num_parts) b -= a.table[t++].num_parts;
+    const uint64_t* __restrict__ keys = a.table[t].keys;
+    const uint64_t total = (1ull << *a.table[t].log2) + kTableOverflow;
     const uint64_t ntiles = (total + kExtractTile - 1) / kExtractTile;
-    if (blockIdx.x == 0 && threadIdx.x == 0) *slots_out = total;
-    for (uint64_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
-        const uint64_t first = tile * kExtractTile;
-        uint32_t occ = 0;
-        // Unconditional loads (slots past the end read the last slot and are
-        // not counted), all in flight at once.
-        uint64_t v[kExtractIpt];
+    uint64_t t0, t1;
+    part_tiles(ntiles, b, a.table[t].num_parts, t0, t1);
+    const uint64_t end = min(t1 * kExtractTile, total);
+    uint32_t occ = 0;
+    constexpr int kAhead = 8;
+    for (uint64_t i = t0 * kExtractTile + threadIdx.x; i < end; i += kAhead * kThreads) {
+        // All in flight at once; slots past the part read its last and are not
+        // counted.
+        uint64_t v[kAhead];
 #pragma unroll
-        for (int k = 0; k < kExtractIpt; ++k) v[k] = table_keys[min(first + uint64_t(k) * kThreads + threadIdx.x, total - 1)];
+        for (int k = 0; k < kAhead; ++k) v[k] = keys[min(i + uint64_t(k) * kThreads, end - 1)];
 #pragma unroll
-        for (int k = 0; k < kExtractIpt; ++k)
-            occ += (first + uint64_t(k) * kThreads + threadIdx.x < total && v[k] != 0) ? 1u : 0u;
-        const uint64_t cnt = block_reduce_sum<kThreads>(occ, s_red);
-        if (threadIdx.x == 0) counts[tile] = uint32_t(cnt);
+        for (int k = 0; k < kAhead; ++k) occ += (i + uint64_t(k) * kThreads < end && v[k] != 0) ? 1u : 0u;
     }
+    const uint64_t cnt = block_reduce_sum<kThreads>(occ, s_red);
+    if (threadIdx.x == 0) a.table[t].parts[b] = uint32_t(cnt);
+    clear_tables(clear);
 }
 
 __global__ __launch_bounds__(kThreads) void k_level_extract(LevelExtractArgs g)
@@ -1644,7 +1676,10 @@ __global__ __launch_bounds__(kThreads) void k_level_extract(LevelExtractArgs g)
     const uint64_t total = (1ull << lg) + kTableOverflow;
     const uint64_t ntiles = (total + kExtractTile - 1) / kExtractTile;
     uint64_t wsum = 0;
-    for (uint64_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
+    uint64_t t0, t1;
+    part_tiles(ntiles, blockIdx.x, gridDim.x, t0, t1);
+    uint64_t tile_before = parts_before(g.parts, s_red);  // occupied slots before the tile
+    for (uint64_t tile = t0; tile < t1; ++tile) {
         const int64_t tile_base = int64_t(tile) * kExtractTile;
         const int64_t win_lo = tile_base - kHalo;
         const int64_t win_hi = tile_base + kExtractTile + kHalo;
@@ -1673,9 +1708,10 @@ __global__ __launch_bounds__(kThreads) void k_level_extract(LevelExtractArgs g)
         uint32_t occ = 0;
 #pragma unroll
         for (int j = 0; j < kExtractIpt; ++j) occ |= (s_win[first + j - win_lo] != 0 ? 1u : 0u) << j;
-        uint32_t unused;
-        const uint32_t local = block_exclusive_scan<kThreads>(__popc(occ), s_scan, unused);
-        uint64_t before = g.offsets[tile] + local;  // occupied slots before the current one
+        uint32_t tile_slots;
+        const uint32_t local = block_exclusive_scan<kThreads>(__popc(occ), s_scan, tile_slots);
+        uint64_t before = tile_before + local;  // occupied slots before the current one
+        tile_before += tile_slots;
         // Representatives' records, gathered up front (unoccupied slots read
         // parent 0, which is then ignored).
         uint32_t mask[kExtractIpt];
@@ -1738,6 +1774,7 @@ __global__ __launch_bounds__(kThreads) void k_level_extract(LevelExtractArgs g)
     }
     const uint64_t wtot = block_reduce_sum<kThreads>(wsum, s_red);
     if (threadIdx.x == 0 && wtot) atomicAdd((unsigned long long*)g.w_count, (unsigned long long)wtot);
+    if (threadIdx.x == 0 && blockIdx.x + 1 == gridDim.x) *g.q_count = tile_before;
 }
 
 // ---------------------------------------------------------------------------
@@ -1815,27 +1852,35 @@ __global__ __launch_bounds__(kThreads) void k_final_count(FinalArgs a)
     __shared__ FinalLds s_lv;
     stage_levels(a, s_lv);
     const uint64_t ntiles = (a.total_nodes + kFinalTile - 1) / kFinalTile;
-    for (uint64_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
+    uint64_t t0, t1;
+    part_tiles(ntiles, blockIdx.x, gridDim.x, t0, t1);
+    uint64_t sum = 0;
+    for (uint64_t tile = t0; tile < t1; ++tile) {
         uint32_t sizes[kFinalIpt];
-        const uint32_t sum = node_words(a, s_lv, tile * kFinalTile + uint64_t(threadIdx.x) * kFinalIpt, sizes);
-        const uint64_t tot = block_reduce_sum<kThreads>(sum, s_red);
-        if (threadIdx.x == 0) a.counts[tile] = uint32_t(tot);
+        sum += node_words(a, s_lv, tile * kFinalTile + uint64_t(threadIdx.x) * kFinalIpt, sizes);
     }
+    const uint64_t tot = block_reduce_sum<kThreads>(sum, s_red);
+    if (threadIdx.x == 0) a.parts[blockIdx.x] = uint32_t(tot);
 }
 
 __global__ __launch_bounds__(kThreads) void k_final_positions(FinalArgs a)
 {
     __shared__ uint32_t s_scan[kThreads / kWave];
+    __shared__ uint64_t s_red[kThreads / kWave];
     __shared__ FinalLds s_lv;
     stage_levels(a, s_lv);
     const uint64_t ntiles = (a.total_nodes + kFinalTile - 1) / kFinalTile;
-    for (uint64_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
+    uint64_t t0, t1;
+    part_tiles(ntiles, blockIdx.x, gridDim.x, t0, t1);
+    uint64_t before = parts_before(a.parts, s_red);
+    for (uint64_t tile = t0; tile < t1; ++tile) {
         const uint64_t first = tile * kFinalTile + uint64_t(threadIdx.x) * kFinalIpt;
         uint32_t sizes[kFinalIpt];
         const uint32_t sum = node_words(a, s_lv, first, sizes);
-        uint32_t unused;
-        const uint32_t local = block_exclusive_scan<kThreads>(sum, s_scan, unused);
-        uint64_t pos = a.offsets[tile] + local;
+        uint32_t tile_words;
+        const uint32_t local = block_exclusive_scan<kThreads>(sum, s_scan, tile_words);
+        uint64_t pos = before + local;
+        before += tile_words;
 #pragma unroll
         for (int j = 0; j < kFinalIpt; ++j) {
             if (first + j < a.total_nodes) a.positions[first + j] = uint32_t(pos);
@@ -2119,13 +2164,13 @@ void launch_scan_counts(hipStream_t s, const uint32_t* counts, uint64_t* offsets
                        items_host);
 }
 
-void launch_cell_reduce(hipStream_t s, const CellArgs& a, BuildCounters* c, int leaf_level)
+void launch_cell_reduce(hipStream_t s, const CellArgs& a, BuildCounters* c)
 {
     const uint64_t runs = cell_runs(a.cells, a.run_cells);
     {
         TimedLaunch t(kKLeafReduce, s);
         hipLaunchKernelGGL(k_cell_reduce, dim3(resident_grid(k_cell_reduce, kCellThreads, runs)), dim3(kCellThreads), 0,
-                           s, a, &c->n, &c->pre[leaf_level]);
+                           s, a, &c->n);
     }
     TimedLaunch t(kKLeafCompact, s);
     hipLaunchKernelGGL(k_cell_compact, dim3(resident_grid(k_cell_compact, kThreads, runs)), dim3(kThreads), 0, s, a,
@@ -2135,7 +2180,7 @@ void launch_cell_reduce(hipStream_t s, const CellArgs& a, BuildCounters* c, int 
 template <typename K>
 void launch_leaf_reduce(hipStream_t s, const K* sorted, BuildCounters* c, uint32_t group_bits, uint64_t* reg_code,
                         uint64_t* reg_mask, uint64_t* lp_code, uint64_t* lp_mask, uint64_t lp_capacity,
-                        uint32_t* tile_counts, uint64_t* tile_offsets, uint64_t n_bound, int leaf_level,
+                        uint32_t* tile_counts, uint64_t* tile_offsets, uint64_t n_bound,
                         uint64_t code_mask, const ChunkPrefix& buckets)
 {
     const uint64_t chunks = (n_bound + kReduceChunk - 1) / kReduceChunk;
@@ -2150,21 +2195,20 @@ void launch_leaf_reduce(hipStream_t s, const K* sorted, BuildCounters* c, uint32
                     hipLaunchKernelGGL((k_leaf_reduce<K, kBucketsLds>),
                                        dim3(resident_grid(k_leaf_reduce<K, kBucketsLds>, kThreads, units)),
                                        dim3(kThreads), 0, s, sorted, &c->n, code_mask, group_bits, reg_code, reg_mask,
-                                       tile_counts, &c->pre[leaf_level],
+                                       tile_counts,
                                        reinterpret_cast<unsigned long long*>(&c->error), buckets);
                 else
                     hipLaunchKernelGGL((k_leaf_reduce<K, kBucketsGlobal>),
                                        dim3(resident_grid(k_leaf_reduce<K, kBucketsGlobal>, kThreads, units)),
                                        dim3(kThreads), 0, s, sorted, &c->n, code_mask, group_bits, reg_code, reg_mask,
-                                       tile_counts, &c->pre[leaf_level],
+                                       tile_counts,
                                        reinterpret_cast<unsigned long long*>(&c->error), buckets);
             }
         }
         if (!bucketed)
             hipLaunchKernelGGL((k_leaf_reduce<K, kBucketsNone>),
                                dim3(resident_grid(k_leaf_reduce<K, kBucketsNone>, kThreads, units)), dim3(kThreads), 0,
-                               s, sorted, &c->n, code_mask, group_bits, reg_code, reg_mask, tile_counts,
-                               &c->pre[leaf_level], reinterpret_cast<unsigned long long*>(&c->error), ChunkPrefix{});
+                               s, sorted, &c->n, code_mask, group_bits, reg_code, reg_mask, tile_counts, reinterpret_cast<unsigned long long*>(&c->error), ChunkPrefix{});
     }
     launch_scan_counts(s, tile_counts, tile_offsets, &c->n, kReduceChunk, &c->leaf_positions);
     {
@@ -2175,18 +2219,16 @@ void launch_leaf_reduce(hipStream_t s, const K* sorted, BuildCounters* c, uint32
     }
 }
 template void launch_leaf_reduce<uint64_t>(hipStream_t, const uint64_t*, BuildCounters*, uint32_t, uint64_t*,
-                                           uint64_t*, uint64_t*, uint64_t*, uint64_t, uint32_t*, uint64_t*, uint64_t,
-                                           int, uint64_t, const ChunkPrefix&);
+                                           uint64_t*, uint64_t*, uint64_t*, uint64_t, uint32_t*, uint64_t*, uint64_t, uint64_t, const ChunkPrefix&);
 template void launch_leaf_reduce<uint32_t>(hipStream_t, const uint32_t*, BuildCounters*, uint32_t, uint64_t*,
-                                           uint64_t*, uint64_t*, uint64_t*, uint64_t, uint32_t*, uint64_t*, uint64_t,
-                                           int, uint64_t, const ChunkPrefix&);
+                                           uint64_t*, uint64_t*, uint64_t*, uint64_t, uint32_t*, uint64_t*, uint64_t, uint64_t, const ChunkPrefix&);
 
-void launch_table_clear(hipStream_t s, uint64_t* keys, const uint64_t* count_ptr, uint32_t* log2_out,
-                        uint32_t load_shift, uint32_t overflow, uint64_t slot_bound)
+void launch_table_clear(hipStream_t s, const TableClears& a)
 {
     TimedLaunch t(kKTableClear, s);
-    hipLaunchKernelGGL(k_table_clear, dim3(grid_for((slot_bound + kThreads - 1) / kThreads, 8)), dim3(kThreads), 0, s,
-                       keys, count_ptr, log2_out, load_shift, overflow);
+    uint64_t most = 1;
+    for (int i = 0; i < a.num; ++i) most = std::max(most, a.table[i].slot_bound);
+    hipLaunchKernelGGL(k_table_clear, dim3(grid_for((most + kThreads - 1) / kThreads, 8)), dim3(kThreads), 0, s, a);
 }
 
 void launch_leaf_insert(hipStream_t s, const uint64_t* lp_mask, const uint64_t* count_ptr, uint64_t* table_keys,
@@ -2226,21 +2268,28 @@ void launch_sketch_estimate(hipStream_t s, const uint32_t* regs, const uint64_t*
     hipLaunchKernelGGL(k_sketch_estimate, dim3(1), dim3(kEstimateThreads), 0, s, regs, bound_ptr, estimate);
 }
 
-void launch_level_build(hipStream_t s, const LevelBuildArgs& a, uint64_t child_bound, const TableClearArgs* clear)
+uint32_t level_build_parts(uint64_t child_bound)
 {
-    const uint64_t tiles = (child_bound + kBuildTile - 1) / kBuildTile;
-    {
-        TimedLaunch t(kKLevelCount, s);
-        const uint64_t work = clear ? std::max(tiles, (clear->slot_bound + kThreads - 1) / kThreads) : tiles;
-        const TableClearArgs ca = clear ? *clear : TableClearArgs{};  // by value: *clear may not outlive the call
-        hipLaunchKernelGGL(k_level_count, dim3(resident_grid(k_level_count, kThreads, work)), dim3(kThreads), 0, s,
-                           a.child_codes, a.child_count, a.tile_counts, a.next_count, ca);
-    }
-    launch_scan_counts(s, a.tile_counts, const_cast<uint64_t*>(a.offsets), a.child_count, kBuildTile, nullptr);
-    {
-        TimedLaunch t(kKLevelBuild, s);
-        hipLaunchKernelGGL(k_level_build, dim3(resident_grid(k_level_build, kThreads, tiles)), dim3(kThreads), 0, s, a);
-    }
+    return uint32_t(std::min<uint64_t>(kMaxParts, resident_grid(k_level_build, kThreads, tiles(child_bound, kBuildTile))));
+}
+
+uint32_t level_extract_parts(uint64_t slot_bound)
+{
+    return uint32_t(std::min<uint64_t>(kMaxParts, resident_grid(k_level_extract, kThreads, tiles(slot_bound, kExtractTile))));
+}
+
+void launch_level_count(hipStream_t s, const uint64_t* codes, const uint64_t* count, uint64_t bound, uint32_t* parts,
+                        uint64_t* pre, int level, int lowest)
+{
+    TimedLaunch t(kKLevelCount, s);
+    hipLaunchKernelGGL(k_level_count, dim3(level_build_parts(bound)), dim3(kThreads), 0, s, codes, count, parts, pre,
+                       level, lowest);
+}
+
+void launch_level_build(hipStream_t s, const LevelBuildArgs& a, uint64_t child_bound)
+{
+    TimedLaunch t(kKLevelBuild, s);
+    hipLaunchKernelGGL(k_level_build, dim3(level_build_parts(child_bound)), dim3(kThreads), 0, s, a);
 }
 
 void launch_level_tail(hipStream_t s, const TailArgs& a)
@@ -2249,20 +2298,20 @@ void launch_level_tail(hipStream_t s, const TailArgs& a)
     hipLaunchKernelGGL(k_level_tail, dim3(1), dim3(kTailThreads), 0, s, a);
 }
 
+void launch_extract_count(hipStream_t s, const ExtractCounts& a, const TableClears* clear)
+{
+    uint32_t grid = 0;
+    for (int i = 0; i < a.num; ++i) grid += a.table[i].num_parts;
+    if (grid == 0) return;
+    TimedLaunch t(kKExtractCount, s);
+    const TableClears tc = clear ? *clear : TableClears{};
+    hipLaunchKernelGGL(k_extract_count, dim3(grid), dim3(kThreads), 0, s, a, tc);
+}
+
 void launch_level_extract(hipStream_t s, const LevelExtractArgs& a, uint64_t slot_bound)
 {
-    const uint64_t tiles = (slot_bound + kExtractTile - 1) / kExtractTile;
-    {
-        TimedLaunch t(kKExtractCount, s);
-        hipLaunchKernelGGL(k_extract_count, dim3(resident_grid(k_extract_count, kThreads, tiles)), dim3(kThreads), 0,
-                           s, a.table_keys, a.table_log2, a.tile_counts, a.slots_scratch);
-    }
-    launch_scan_counts(s, a.tile_counts, const_cast<uint64_t*>(a.offsets), a.slots_scratch, kExtractTile, a.q_count);
-    {
-        TimedLaunch t(kKLevelExtract, s);
-        hipLaunchKernelGGL(k_level_extract, dim3(resident_grid(k_level_extract, kThreads, tiles)), dim3(kThreads), 0,
-                           s, a);
-    }
+    TimedLaunch t(kKLevelExtract, s);
+    hipLaunchKernelGGL(k_level_extract, dim3(level_extract_parts(slot_bound)), dim3(kThreads), 0, s, a);
 }
 
 void launch_level_check(hipStream_t s, const uint32_t* parent_slots, const uint32_t* table_rep,
@@ -2335,16 +2384,14 @@ void launch_final(hipStream_t s, const FinalArgs& a)
     if (a.total_nodes == 0 && a.num_leaves == 0) return;
     if (a.total_nodes) {
         const uint64_t tiles = (a.total_nodes + kFinalTile - 1) / kFinalTile;
+        const uint32_t parts = uint32_t(std::min<uint64_t>(kMaxParts, resident_grid(k_final_positions, kThreads, tiles)));
         {
             TimedLaunch t(kKFinalCount, s);
-            hipLaunchKernelGGL(k_final_count, dim3(resident_grid(k_final_count, kThreads, tiles)), dim3(kThreads), 0, s,
-                               a);
+            hipLaunchKernelGGL(k_final_count, dim3(parts), dim3(kThreads), 0, s, a);
         }
-        launch_scan_counts(s, a.counts, a.offsets, nullptr, kFinalTile, nullptr, a.total_nodes);
         {
             TimedLaunch t(kKFinalPositions, s);
-            hipLaunchKernelGGL(k_final_positions, dim3(resident_grid(k_final_positions, kThreads, tiles)),
-                               dim3(kThreads), 0, s, a);
+            hipLaunchKernelGGL(k_final_positions, dim3(parts), dim3(kThreads), 0, s, a);
         }
     }
     const uint64_t work = std::max(a.total_nodes, a.num_leaves);

@@ -214,7 +214,6 @@ struct BuildCounters {
     uint64_t collisions;
     uint64_t error;                           // kErr* bits
     uint32_t table_log2[SVDAG_MAX_LEVELS + 1];  // [l] level tables, [MAX] leaf table
-    uint64_t table_slots;                     // slots of the table being extracted
     uint64_t leaf_estimate;                   // table sizing count of the leaf dedup table
 };
 
@@ -273,14 +272,14 @@ void launch_scan_counts(hipStream_t s, const uint32_t* counts, uint64_t* offsets
 // leaves into the regions reg_code / reg_mask (kLeafRegionItems per chunk of
 // kPackTileItems keys), then compacted into lp_code / lp_mask (lp_capacity
 // entries); sets
-// c->leaf_positions and adds the leaf level's parent count to c->pre[leaf_level].
+// c->leaf_positions.
 // buckets.offsets non-null (32-bit keys only): the keys are local to the
 // buckets of a segmented sort, key i's code is (b << buckets.chunk_bits) | key
 // for the bucket b holding position i.
 template <typename K>
 void launch_leaf_reduce(hipStream_t s, const K* sorted, BuildCounters* c, uint32_t group_bits, uint64_t* reg_code,
                         uint64_t* reg_mask, uint64_t* lp_code, uint64_t* lp_mask, uint64_t lp_capacity,
-                        uint32_t* tile_counts, uint64_t* tile_offsets, uint64_t n_bound, int leaf_level,
+                        uint32_t* tile_counts, uint64_t* tile_offsets, uint64_t n_bound,
                         uint64_t code_mask, const ChunkPrefix& buckets = ChunkPrefix{});
 
 // Leaf ReduceByKey over keys grouped by cell (code >> kCellShift: 64^3 voxels,
@@ -314,12 +313,26 @@ struct CellArgs {
     uint64_t* lp_mask;
     uint64_t lp_capacity;
 };
-void launch_cell_reduce(hipStream_t s, const CellArgs& a, BuildCounters* c, int leaf_level);
+void launch_cell_reduce(hipStream_t s, const CellArgs& a, BuildCounters* c);
 
-// Clears an ordered (load_shift, overflow) or hashed table sized from *count_ptr
-// and records its log2 size.
-void launch_table_clear(hipStream_t s, uint64_t* keys, const uint64_t* count_ptr, uint32_t* log2_out,
-                        uint32_t load_shift, uint32_t overflow, uint64_t slot_bound);
+// Clears ordered (overflow > 0) and hashed tables, each sized from its count
+// (device memory), and records their log2 sizes.
+struct TableClears {
+    int num;
+    uint32_t load_shift;
+    struct {
+        uint64_t* keys;
+        const uint64_t* count;
+        uint32_t* log2_out;
+        uint32_t overflow;
+        uint64_t slot_bound;
+    } table[SVDAG_MAX_LEVELS + 1];
+    void add(uint64_t* keys, const uint64_t* count, uint32_t* log2_out, uint32_t overflow, uint64_t slot_bound)
+    {
+        table[num++] = {keys, count, log2_out, overflow, slot_bound};
+    }
+};
+void launch_table_clear(hipStream_t s, const TableClears& a);
 
 // Inserts every leaf mask into the hashed table and records its slot.
 void launch_leaf_insert(hipStream_t s, const uint64_t* lp_mask, const uint64_t* count_ptr, uint64_t* table_keys,
@@ -371,23 +384,25 @@ struct LevelBuildArgs {
     uint64_t* table_keys;
     uint32_t* table_rep;
     const uint32_t* table_log2;
-    uint32_t* tile_counts;    // tiles(child_bound, kBuildTileItems)
-    const uint64_t* offsets;  // same count, written by the scan
-    uint64_t* next_count;     // M of the level above (atomic adds), or null
+    const uint32_t* parts;    // parents started in each part of the children
+    // Non-null: the same counts for the level above (zero before; next_num
+    // parts of *parent_count, this level's node count).
+    uint32_t* next_parts;
+    uint32_t next_num;
+    const uint64_t* parent_count;
     BuildCounters* counters;
 };
-// The level's table clear (launch_table_clear's arguments), done by the
-// level's count kernel instead of a launch of its own.
-struct TableClearArgs {
-    uint64_t* keys;
-    const uint64_t* count;  // the level's node count (sizes the table)
-    uint32_t* log2_out;
-    uint32_t load_shift;
-    uint32_t overflow;
-    uint64_t slot_bound;
-};
-void launch_level_build(hipStream_t s, const LevelBuildArgs& a, uint64_t child_bound,
-                        const TableClearArgs* clear = nullptr);
+// Workgroups of a level's build and extract (their parts; at most kMaxParts and
+// at most one per tile).
+constexpr uint32_t kMaxParts = 2048;
+uint32_t level_build_parts(uint64_t child_bound);
+uint32_t level_extract_parts(uint64_t slot_bound);
+// Parents started in each part of the sorted child codes (level_build_parts of
+// them); with pre also the node counts of levels lowest .. level, added to
+// pre[...], which the codes below determine.
+void launch_level_count(hipStream_t s, const uint64_t* codes, const uint64_t* count, uint64_t bound, uint32_t* parts,
+                        uint64_t* pre, int level, int lowest);
+void launch_level_build(hipStream_t s, const LevelBuildArgs& a, uint64_t child_bound);
 
 // ---- small top levels -------------------------------------------------------
 // Levels 0..top with top <= kTailTopLevel hold at most 8^top <= 512 nodes; one
@@ -432,13 +447,27 @@ struct LevelExtractArgs {
     uint64_t* out_hashes;
     uint8_t* out_masks;
     uint32_t* out_children;
-    uint32_t* tile_counts;    // tiles(slot_bound, kExtractTileItems)
-    const uint64_t* offsets;
-    uint64_t* slots_scratch;  // receives the table's slot count
+    const uint32_t* parts;    // occupied slots of each part (launch_extract_count)
     uint64_t* q_count;        // receives the level's unique node count
     uint64_t* w_count;        // receives the level's word count (atomic adds)
 };
 void launch_level_extract(hipStream_t s, const LevelExtractArgs& a, uint64_t slot_bound);
+// Occupied slots per part (level_extract_parts of its slot bound) of each of
+// several ordered tables; also clears the tables of `clear`.
+struct ExtractCounts {
+    int num;
+    struct {
+        const uint64_t* keys;
+        const uint32_t* log2;
+        uint32_t* parts;
+        uint32_t num_parts;
+    } table[SVDAG_MAX_LEVELS];
+    void add(const uint64_t* keys, const uint32_t* log2, uint32_t* parts, uint32_t num_parts)
+    {
+        table[num++] = {keys, log2, parts, num_parts};
+    }
+};
+void launch_extract_count(hipStream_t s, const ExtractCounts& a, const TableClears* clear = nullptr);
 
 void launch_level_check(hipStream_t s, const uint32_t* parent_slots, const uint32_t* table_rep,
                         const uint8_t* parent_masks, const uint32_t* parent_children, const uint64_t* count_ptr,
@@ -460,8 +489,7 @@ struct FinalArgs {
     uint64_t leaves_start;   // word index of the first leaf
     uint32_t* positions;     // [total_nodes] absolute word offset of each node
     uint32_t* words;
-    uint32_t* counts;        // tiles(total_nodes, kFinalTileItems)
-    uint64_t* offsets;
+    uint32_t* parts;         // words of each part of the nodes (one per tile at most)
 };
 void launch_final(hipStream_t s, const FinalArgs& a);
 

@@ -61,11 +61,6 @@ __device__ __forceinline__ uint64_t split_by_3(uint32_t a)
     return x;
 }
 
-// Morton layout of src/DAG_Compression_Fast.cpp:223-236.
-__device__ __forceinline__ uint64_t morton3(uint32_t x, uint32_t y, uint32_t z)
-{
-    return split_by_3(x) << 2 | split_by_3(y) << 1 | split_by_3(z);
-}
 
 // A triangle with a non-finite coordinate gets no rows and sets kErrKeyRange
 // in *err.

@@ -309,7 +309,6 @@ struct BuildLayout {
     uint64_t level_nodes[SVDAG_MAX_LEVELS] = {}, level_slots_of[SVDAG_MAX_LEVELS] = {};
     // Per hashed level: counts per part of its children and of its table's slots.
     uint64_t build_parts[SVDAG_MAX_LEVELS] = {}, extract_parts[SVDAG_MAX_LEVELS] = {};
-    uint64_t tail_codes[2] = {}, tail_ranks[2] = {}, tail_masks = 0, tail_children = 0, tail_hash = 0;
     uint64_t n = 0, leaf_bound = 0, level_bound = 0, leaf_slots = 0, level_slots = 0;
     uint32_t group_bits = 0;
     SortPlan key_plan{};
@@ -396,13 +395,6 @@ BuildLayout plan_build(uint64_t n, int depth, int key_bytes, uint32_t load_shift
         L.trep[l] = c.take(4 * L.level_slots_of[l]);
     }
     for (int i = 0; i < 2; ++i) L.trank[i] = c.take(4 * widest_slots);
-    for (int i = 0; i < 2; ++i) {
-        L.tail_codes[i] = c.take(8 * kTailMaxParents);
-        L.tail_ranks[i] = c.take(4 * kTailMaxParents);
-    }
-    L.tail_masks = c.take(kTailMaxParents);
-    L.tail_children = c.take(32 * kTailMaxParents);
-    L.tail_hash = c.take(8 * 8 * kTailMaxParents);
     L.total = c.off;
     // The leaf-reduce regions are read only by the compaction, before any of
     // the buffers from the leaf table on is written.
@@ -1091,13 +1083,6 @@ int build(svdag_context* ctx, const K* d_keys, uint64_t n, int depth, svdag_dag*
             t.child_count = &c->pre[tail_top + 1];
         }
         t.child_rank_of_slot = below;
-        for (int i = 0; i < 2; ++i) {
-            t.codes[i] = reinterpret_cast<uint64_t*>(A + L.tail_codes[i]);
-            t.ranks[i] = reinterpret_cast<uint32_t*>(A + L.tail_ranks[i]);
-        }
-        t.masks = reinterpret_cast<uint8_t*>(A + L.tail_masks);
-        t.children = reinterpret_cast<uint32_t*>(A + L.tail_children);
-        t.child_hash = reinterpret_cast<uint64_t*>(A + L.tail_hash);
         for (int l = 0; l <= tail_top; ++l) {
             t.out_hashes[l] = reinterpret_cast<uint64_t*>(O + S.hashes[l]);
             t.out_masks[l] = reinterpret_cast<uint8_t*>(O + S.masks[l]);
@@ -1215,13 +1200,6 @@ int merge_device(svdag_context* ctx, const svdag_dag* dags, uint64_t count, int 
     // Few enough chunk levels take the one-workgroup tail (at most
     // kTailMaxChildren roots below it).
     const bool tail = k >= 1 && k - 1 <= kTailTopLevel;
-    uint64_t o_tcodes[2], o_tranks[2];
-    for (int i = 0; i < 2; ++i) {
-        o_tcodes[i] = cv.take(8 * kTailMaxParents);
-        o_tranks[i] = cv.take(4 * kTailMaxParents);
-    }
-    const uint64_t o_tmasks = cv.take(kTailMaxParents), o_tchildren = cv.take(32 * kTailMaxParents);
-    const uint64_t o_thash = cv.take(64 * kTailMaxParents);
     TRY(ensure_arena(ctx, cv.off));
     char* A = ctx->arena;
     BuildCounters* c = reinterpret_cast<BuildCounters*>(A + o_counters);
@@ -1350,13 +1328,6 @@ int merge_device(svdag_context* ctx, const svdag_dag* dags, uint64_t count, int 
         t.child_hashes = reinterpret_cast<const uint64_t*>(O + S.hashes[k]);
         t.child_count = &c->pre[k];
         t.child_rank_of_slot = child_rank;
-        for (int i = 0; i < 2; ++i) {
-            t.codes[i] = reinterpret_cast<uint64_t*>(A + o_tcodes[i]);
-            t.ranks[i] = reinterpret_cast<uint32_t*>(A + o_tranks[i]);
-        }
-        t.masks = reinterpret_cast<uint8_t*>(A + o_tmasks);
-        t.children = reinterpret_cast<uint32_t*>(A + o_tchildren);
-        t.child_hash = reinterpret_cast<uint64_t*>(A + o_thash);
         for (int l = 0; l < k; ++l) {
             t.out_hashes[l] = reinterpret_cast<uint64_t*>(O + S.hashes[l]);
             t.out_masks[l] = reinterpret_cast<uint8_t*>(O + S.masks[l]);
@@ -2618,13 +2589,6 @@ int svdag_resident_dag(svdag_resident* r, svdag_dag* out)
     const uint64_t o_leaf_rank = cv.take(4 * r->leaf_slots);
     const uint64_t o_rank[2] = {cv.take(4 * max_slots), cv.take(4 * max_slots)};
     const uint64_t o_codes = cv.take(8 * nslots), o_rslots = cv.take(4 * nslots), o_rcount = cv.take(8);
-    uint64_t o_tcodes[2], o_tranks[2];
-    for (int i = 0; i < 2; ++i) {
-        o_tcodes[i] = cv.take(8 * kTailMaxParents);
-        o_tranks[i] = cv.take(4 * kTailMaxParents);
-    }
-    const uint64_t o_tmasks = cv.take(kTailMaxParents), o_tchildren = cv.take(32 * kTailMaxParents);
-    const uint64_t o_thash = cv.take(64 * kTailMaxParents);
     TRY(ensure_arena(ctx, cv.off));
     char* A = ctx->arena;
     BuildCounters* c = reinterpret_cast<BuildCounters*>(A + o_counters);
@@ -2692,13 +2656,6 @@ int svdag_resident_dag(svdag_resident* r, svdag_dag* out)
     t.child_rank_of_slot = below;
     t.child_hashes = reinterpret_cast<const uint64_t*>(O + S.hashes[r->top]);
     t.child_count = rcount;
-    for (int i = 0; i < 2; ++i) {
-        t.codes[i] = reinterpret_cast<uint64_t*>(A + o_tcodes[i]);
-        t.ranks[i] = reinterpret_cast<uint32_t*>(A + o_tranks[i]);
-    }
-    t.masks = reinterpret_cast<uint8_t*>(A + o_tmasks);
-    t.children = reinterpret_cast<uint32_t*>(A + o_tchildren);
-    t.child_hash = reinterpret_cast<uint64_t*>(A + o_thash);
     for (int l = 0; l < r->top; ++l) {
         t.out_hashes[l] = reinterpret_cast<uint64_t*>(O + S.hashes[l]);
         t.out_masks[l] = reinterpret_cast<uint8_t*>(O + S.masks[l]);

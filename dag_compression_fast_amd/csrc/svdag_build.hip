@@ -1202,32 +1202,11 @@ __device__ __forceinline__ uint32_t ordered_insert(uint64_t* __restrict__ tk, ui
 
 // ---------------------------------------------------------------------------
 // Level build: children (Morton-sorted codes of the level below, their table
-// slots) -> parents.  A parent belongs to the thread holding its first child and
-// has at most 8 children, so a run extends at most 7 keys past the thread.
+// slots) -> parents.  A parent belongs to the tile holding its first child and
+// has at most 8 children, so a run extends at most 7 children past the tile.
 // ---------------------------------------------------------------------------
-constexpr int kBuildIpt = 4;
+constexpr int kBuildIpt = 2;
 constexpr int kBuildTile = kThreads * kBuildIpt;
-
-__device__ __forceinline__ void parent_runs(const uint64_t* __restrict__ codes, uint64_t n, uint64_t first,
-                                            uint64_t (&code)[kBuildIpt], uint32_t& starts, uint32_t& gstarts)
-{
-    // Unconditional loads (positions past the end read the last code and are
-    // never starts), so that all of them are in flight at once.  n >= 1 here.
-#pragma unroll
-    for (int j = 0; j < kBuildIpt; ++j) code[j] = codes[min(first + j, n - 1)];
-    const uint64_t before = first > 0 ? codes[min(first - 1, n - 1)] : ~0ull;
-    starts = 0;   // bit j: child j starts a parent
-    gstarts = 0;  // bit j: it starts a grandparent too
-#pragma unroll
-    for (int j = 0; j < kBuildIpt; ++j) {
-        const uint64_t prev = j ? code[j - 1] : before;
-        const bool head = first + j == 0;
-        if (first + j < n && (head || (code[j] >> 3) != (prev >> 3))) {
-            starts |= 1u << j;
-            gstarts |= (head || (code[j] >> 6) != (prev >> 6)) ? 1u << j : 0u;
-        }
-    }
-}
 
 // The parents that each part of the children starts (the workgroups of
 // k_level_build take the same parts).  With pre set, also the node counts of
@@ -1282,329 +1261,366 @@ __global__ __launch_bounds__(kThreads) void k_level_count(const uint64_t* __rest
     }
 }
 
-struct ParentAcc {
-    uint64_t code;
-    uint32_t mask;
-    uint32_t child[8];
-    uint64_t hash[8];
-};
+// A tile's children are read coalesced and staged in LDS with the starts of
+// their parents; then one thread per parent takes its children from LDS (they
+// are sorted, so slot s's child is the popcount of the mask below s), writes the
+// record and inserts the hash into the level's table.  The next tile's children
+// are loaded before the inserts.  Bound by the chain of each tile's dependent
+// steps (loads, two barriers, probe, CAS) and the waves in flight to hide it.
+// All builds of 2048^3 triangles 359 -> 285 us, of 64 chunks (12.8M keys) 137 ->
+// 96, against a thread per run of children whose last parent walked on through
+// global memory child by child.  Two children per thread: with four the
+// registers (130) leave 12 waves per CU (331 us), with one a tile has too little
+// between its barriers (356); not loading ahead takes 305.
+constexpr int kBuildHalo = 8;
+constexpr int kBuildWaves = kThreads / kWave;
 
-__device__ __forceinline__ void acc_reset(ParentAcc& a, uint64_t code)
-{
-    a.code = code;
-    a.mask = 0;
-#pragma unroll
-    for (int s = 0; s < 8; ++s) {
-        a.child[s] = kEmptyChild;
-        a.hash[s] = 0;
-    }
-}
-
-__device__ __forceinline__ void acc_add(ParentAcc& a, uint32_t slot, uint32_t rank, uint64_t hash)
-{
-    a.mask |= 1u << slot;
-#pragma unroll
-    for (int s = 0; s < 8; ++s) {
-        a.child[s] = slot == uint32_t(s) ? rank : a.child[s];
-        a.hash[s] = slot == uint32_t(s) ? hash : a.hash[s];
-    }
-}
-
-// Writes a parent's record and returns its hash.
-__device__ __forceinline__ uint64_t acc_emit(const ParentAcc& a, uint64_t p, const LevelBuildArgs& g)
-{
-    g.parent_codes[p] = a.code;
-    g.parent_masks[p] = uint8_t(a.mask);
-    uint4* dst = reinterpret_cast<uint4*>(g.parent_children + 8 * p);
-    dst[0] = make_uint4(a.child[0], a.child[1], a.child[2], a.child[3]);
-    dst[1] = make_uint4(a.child[4], a.child[5], a.child[6], a.child[7]);
-    const uint64_t h = hash_children(a.hash);
-    if (g.parent_hashes) g.parent_hashes[p] = h;
-    return h;
-}
-
-// A thread owns kBuildIpt consecutive children; their loads (or rank and hash
-// gathers) are issued together.  The tile's parent hashes are staged in LDS and
-// inserted into the level's table one thread per parent.
 __global__ __launch_bounds__(kThreads) void k_level_build(LevelBuildArgs g)
 {
-    __shared__ uint32_t s_scan[kThreads / kWave];
-    __shared__ uint64_t s_red[kThreads / kWave];
-    __shared__ uint32_t s_heads[kThreads / kWave];
-    __shared__ uint64_t s_hash[kBuildTile];
-    __shared__ uint32_t s_elect[kThreads / kWave][kElectBuckets];
+    __shared__ uint64_t s_hash[kBuildTile + kBuildHalo];
+    __shared__ uint32_t s_slot[kBuildTile + kBuildHalo];
+    __shared__ uint8_t s_sub[kBuildTile + kBuildHalo];
+    __shared__ uint16_t s_start[kBuildTile + 1];
+    __shared__ uint32_t s_cnt[kBuildIpt * kBuildWaves];
+    __shared__ uint32_t s_heads[kBuildWaves];
+    __shared__ uint32_t s_end;
+    __shared__ uint64_t s_red[kBuildWaves];
+    __shared__ uint32_t s_elect[kBuildWaves][kElectBuckets];
     const uint64_t n = *g.child_count;
     const uint64_t ntiles = (n + kBuildTile - 1) / kBuildTile;
     const uint64_t next_tiles = g.next_parts ? (*g.parent_count + kBuildTile - 1) / kBuildTile : 0;
     uint64_t t0, t1;
     part_tiles(ntiles, blockIdx.x, gridDim.x, t0, t1);
     if (t0 >= t1) return;  // the whole workgroup
-    uint64_t p0 = parts_before(g.parts, s_red);
+    const uint32_t tid = threadIdx.x, lane = lane_id();
+    const uint32_t w = uint32_t(__builtin_amdgcn_readfirstlane(int(tid / kWave)));
     const uint32_t lg = *g.table_log2;
     const uint64_t limit = (1ull << lg) + kTableOverflow;
-    const uint32_t* __restrict__ slots = g.child_slots;
-    const uint32_t* __restrict__ rank_of_slot = g.child_rank_of_slot;
-    const uint64_t* __restrict__ hashes = g.child_hashes;
-    const uint64_t* __restrict__ seq = g.child_hash_seq;
-    for (uint64_t tile = t0; tile < t1; ++tile) {
-        const uint64_t first = tile * kBuildTile + uint64_t(threadIdx.x) * kBuildIpt;
-        uint64_t code[kBuildIpt];
-        uint32_t starts, gstarts;
-        parent_runs(g.child_codes, n, first, code, starts, gstarts);
-        uint32_t tile_parents;
-        const uint32_t local = block_exclusive_scan<kThreads>(__popc(starts), s_scan, tile_parents);
-        if (g.next_parts) {
-            // Parents of this level's nodes, for the parts of the next build:
-            // the tile's nodes [p0, p0 + tile_parents) lie in at most two of
-            // its tiles (low half: the first, high half: the second).
-            const uint32_t cut = uint32_t(kBuildTile - p0 % kBuildTile);
-            uint32_t heads = 0;
-#pragma unroll
-            for (int j = 0; j < kBuildIpt; ++j) {
-                const uint32_t q = local + uint32_t(__popc(starts & ((1u << j) - 1u)));
-                heads += ((gstarts >> j) & 1u) ? (q < cut ? 1u : 1u << 16) : 0u;
-            }
-            heads = wave_reduce_sum32(heads);
-            if (lane_id() == 0) s_heads[threadIdx.x / kWave] = heads;
-        }
 
-        // Indices are clamped into [0, n): loads past the end read a valid child
-        // that is then ignored.
-        // rank[] holds the child pointers: slots with sequential hashes, else ranks.
-        uint32_t rank[kBuildIpt];
-        uint64_t hsh[kBuildIpt];
-        if (seq) {
-#pragma unroll
-            for (int j = 0; j < kBuildIpt; ++j) {
-                rank[j] = slots[min(first + j, n - 1)];
-                hsh[j] = seq[min(first + j, n - 1)];
-            }
+    // A tile's children in registers: row j holds child j * kThreads + tid, the
+    // halo (threads 0 .. 7) those past the tile; before[j]: the code before the
+    // wave's row.  Indices are clamped into [0, n): what lies past the end is
+    // not used.
+    uint64_t code[kBuildIpt], hash[kBuildIpt], before[kBuildIpt], halo_code = 0, halo_hash = 0;
+    uint32_t slot[kBuildIpt], halo_slot = 0;
+    auto child = [&](uint64_t i, uint64_t& h, uint32_t& sl) {
+        if (g.child_hash_seq) {
+            sl = g.child_slots[i];
+            h = g.child_hash_seq[i];
         } else {
-#pragma unroll
-            for (int j = 0; j < kBuildIpt; ++j) rank[j] = rank_of_slot[slots[min(first + j, n - 1)]];
-#pragma unroll
-            for (int j = 0; j < kBuildIpt; ++j) hsh[j] = hashes[rank[j]];
+            sl = g.child_rank_of_slot[g.child_slots[i]];
+            h = g.child_hashes[sl];
         }
-
-        uint32_t q = local;
-        bool open = false;
-        ParentAcc acc;
-        acc_reset(acc, 0);
+    };
+    auto load = [&](uint64_t tile) {
+        const uint64_t base = tile * kBuildTile;
 #pragma unroll
         for (int j = 0; j < kBuildIpt; ++j) {
-            if ((starts >> j) & 1u) {
-                if (open) {
-                    s_hash[q] = acc_emit(acc, p0 + q, g);
-                    ++q;
-                }
-                open = true;
-                acc_reset(acc, code[j] >> 3);
-            }
-            if (open && first + j < n) acc_add(acc, uint32_t(code[j] & 7), rank[j], hsh[j]);
+            const uint64_t row = base + uint64_t(j) * kThreads + w * kWave;
+            code[j] = g.child_codes[min(row + lane, n - 1)];
+            before[j] = g.child_codes[row > 0 ? min(row - 1, n - 1) : 0];
         }
-        if (open) {
-            // The last parent may take children past this thread's (at most 7).
-            for (uint64_t i = first + kBuildIpt; i < n; ++i) {
-                const uint64_t cc = g.child_codes[i];
-                if ((cc >> 3) != acc.code) break;
-                if (seq) {
-                    acc_add(acc, uint32_t(cc & 7), slots[i], seq[i]);
-                } else {
-                    const uint32_t r = rank_of_slot[slots[i]];
-                    acc_add(acc, uint32_t(cc & 7), r, hashes[r]);
-                }
-            }
-            s_hash[q] = acc_emit(acc, p0 + q, g);
+#pragma unroll
+        for (int j = 0; j < kBuildIpt; ++j) child(min(base + uint64_t(j) * kThreads + tid, n - 1), hash[j], slot[j]);
+        if (tid < uint32_t(kBuildHalo)) {
+            const uint64_t i = min(base + kBuildTile + tid, n - 1);
+            halo_code = g.child_codes[i];
+            child(i, halo_hash, halo_slot);
         }
+    };
+    load(t0);
+    uint64_t p0 = parts_before(g.parts, s_red);
+    for (uint64_t tile = t0; tile < t1; ++tile) {
+        const uint64_t base = tile * kBuildTile;
+        const uint32_t here = uint32_t(min(uint64_t(kBuildTile), n - base));
+        // Row by row: which children start a parent (a grandparent), as ballots.
+        uint64_t starts[kBuildIpt], gstarts[kBuildIpt];
+#pragma unroll
+        for (int j = 0; j < kBuildIpt; ++j) {
+            const uint32_t i = uint32_t(j) * kThreads + tid;
+            uint64_t prev = __shfl_up(code[j], 1, kWave);
+            if (lane == 0) prev = before[j];
+            const uint64_t x = base + i == 0 ? ~0ull : code[j] ^ prev;
+            starts[j] = __ballot(i < here && (x >> 3) != 0);
+            gstarts[j] = __ballot(i < here && (x >> 6) != 0);
+            if (lane == 0) s_cnt[j * kBuildWaves + w] = uint32_t(__popcll(starts[j]));
+            s_hash[i] = hash[j];
+            s_slot[i] = slot[j];
+            s_sub[i] = uint8_t(code[j] & 7u);
+        }
+        if (tid < uint32_t(kBuildHalo)) {
+            s_hash[kBuildTile + tid] = halo_hash;
+            s_slot[kBuildTile + tid] = halo_slot;
+            s_sub[kBuildTile + tid] = uint8_t(halo_code & 7u);
+        }
+        // End of the tile's last run: the halo's children of the last child's
+        // parent (a prefix of it, the codes being sorted).  The last wave holds
+        // that child, the first the halo: through LDS.
+        if (tid == uint32_t(kThreads - 1)) s_red[0] = code[kBuildIpt - 1] >> 3;
         __syncthreads();
-        if (g.next_parts && threadIdx.x < 2) {
+        if (w == 0) {
+            const uint64_t B = __ballot(lane < uint32_t(kBuildHalo) && base + kBuildTile + lane < n &&
+                                        (halo_code >> 3) == s_red[0]);
+            if (lane == 0) s_end = here + uint32_t(__popcll(B));
+        }
+        uint32_t local[kBuildIpt], tile_parents = 0;
+#pragma unroll
+        for (int i = 0; i < kBuildIpt * kBuildWaves; ++i) {
+            if (uint32_t(i % kBuildWaves) == w) local[i / kBuildWaves] = tile_parents;
+            tile_parents += s_cnt[i];
+        }
+        // The tile's nodes [p0, p0 + tile_parents) lie in at most two tiles of
+        // the next build: its parents in the first (low half) and the second.
+        const uint32_t cut = uint32_t(kBuildTile - p0 % kBuildTile);
+        uint32_t heads = 0;
+#pragma unroll
+        for (int j = 0; j < kBuildIpt; ++j) {
+            const uint32_t q = local[j] + uint32_t(__popcll(starts[j] & lanemask_lt()));
+            if ((starts[j] >> lane) & 1ull) {
+                s_start[q] = uint16_t(uint32_t(j) * kThreads + tid);
+                g.parent_codes[p0 + q] = code[j] >> 3;
+            }
+            heads += ((gstarts[j] >> lane) & 1ull) ? (q < cut ? 1u : 1u << 16) : 0u;
+        }
+        if (g.next_parts) {
+            heads = wave_reduce_sum32(heads);
+            if (lane == 0) s_heads[w] = heads;
+        }
+        if (tile + 1 < t1) load(tile + 1);
+        __syncthreads();
+        if (g.next_parts && tid < 2) {
             uint32_t sum = 0;
 #pragma unroll
-            for (int i = 0; i < kThreads / kWave; ++i) sum += (s_heads[i] >> (16 * threadIdx.x)) & 0xFFFFu;
-            const uint64_t t = p0 / kBuildTile + threadIdx.x;
+            for (int i = 0; i < kBuildWaves; ++i) sum += (s_heads[i] >> (16 * tid)) & 0xFFFFu;
+            const uint64_t t = p0 / kBuildTile + tid;
             if (sum) atomicAdd(&g.next_parts[part_of_tile(next_tiles, t, g.next_num)], sum);
         }
-        // Equal parents (identical subtrees) often sit side by side: one lane
-        // per distinct hash in a wave probes the table, the others take its slot.
         for (uint32_t k0 = 0; k0 < tile_parents; k0 += kThreads) {
-            const uint32_t k = k0 + threadIdx.x;
+            const uint32_t k = k0 + tid;
             const bool valid = k < tile_parents;
-            const uint64_t h = valid ? s_hash[k] : 0ull;
+            uint64_t h = 0;
+            if (valid) {
+                const uint32_t st = s_start[k], en = k + 1 < tile_parents ? s_start[k + 1] : s_end;
+                uint32_t mask = 0;
+#pragma unroll
+                for (uint32_t c = 0; c < 8; ++c) mask |= st + c < en ? 1u << s_sub[min(st + c, en - 1)] : 0u;
+                uint32_t ch[8];
+                uint64_t hs[8];
+#pragma unroll
+                for (uint32_t c = 0; c < 8; ++c) {
+                    const bool there = (mask >> c) & 1u;
+                    const uint32_t i = st + uint32_t(__popc(mask & ((1u << c) - 1u)));
+                    const uint32_t at = min(i, en - 1);
+                    ch[c] = there ? s_slot[at] : kEmptyChild;
+                    hs[c] = there ? s_hash[at] : 0ull;
+                }
+                const uint64_t p = p0 + k;
+                g.parent_masks[p] = uint8_t(mask);
+                uint4* dst = reinterpret_cast<uint4*>(g.parent_children + 8 * p);
+                dst[0] = make_uint4(ch[0], ch[1], ch[2], ch[3]);
+                dst[1] = make_uint4(ch[4], ch[5], ch[6], ch[7]);
+                h = hash_children(hs);
+                if (g.parent_hashes) g.parent_hashes[p] = h;
+            }
+            // Equal parents (identical subtrees) often sit side by side: one lane
+            // per distinct hash in a wave probes the table, the others take its
+            // slot.
             bool follower;
-            const uint32_t leader = elect_leader(h, valid, s_elect[threadIdx.x / kWave], follower);
-            uint32_t slot = 0;
+            const uint32_t leader = elect_leader(h, valid, s_elect[w], follower);
+            uint32_t at = 0;
             if (valid && !follower)
-                slot = ordered_insert(g.table_keys, g.table_rep, lg, limit, h, uint32_t(p0 + k), g.counters);
-            slot = uint32_t(__shfl(int(slot), int(leader), kWave));
-            if (valid) g.parent_slots[p0 + k] = slot;
+                at = ordered_insert(g.table_keys, g.table_rep, lg, limit, h, uint32_t(p0 + k), g.counters);
+            at = uint32_t(__shfl(int(at), int(leader), kWave));
+            if (valid) g.parent_slots[p0 + k] = at;
         }
         p0 += tile_parents;
-        __syncthreads();  // s_hash is rewritten by the next tile
+        __syncthreads();  // the staged children are rewritten by the next tile
     }
 }
 
 // ---------------------------------------------------------------------------
-// Small top levels in one workgroup.  Per level (top down to 0): parents are
-// the runs of equal code >> 3 among the children; one thread per parent reads
-// its (at most 8) children and forms its mask, child ranks and hash; the
-// (hash, parent) pairs are sorted in LDS (bitonic), equal hashes get one rank,
-// and the level is written in ascending hash order.  The parents' ranks are
-// the next level's child ranks.
+// Small top levels in one workgroup, all in LDS.  Level l <= 3 has at most 8^l
+// <= 512 nodes, so its children lie in a dense array indexed by code (empty:
+// rank kEmptyChild, hash 0): parent p's are entries 8p .. 8p + 7, and a parent's
+// rank and hash are an entry of the next level's array.  Per level: one thread
+// per parent forms its mask and hash; the (hash, parent) pairs are sorted (each
+// wave 64 of them in registers, then merges by binary search); equal hashes get
+// one rank, and the level is written in ascending hash order.  Bound by latency
+// (one workgroup): four levels take 20 to 24 us; with the children scattered
+// through global memory and a bitonic sort of 45 barriers they took 45 to 58.
 // ---------------------------------------------------------------------------
 constexpr int kTailThreads = 1024;
+constexpr int kTailChildren = int(kTailMaxChildren) / kTailThreads;
+
+// True when (ka, ia) sorts before (kb, ib).
+__device__ __forceinline__ bool pair_less(uint64_t ka, uint32_t ia, uint64_t kb, uint32_t ib)
+{
+    return ka < kb || (ka == kb && ia < ib);
+}
 
 __global__ __launch_bounds__(kTailThreads) void k_level_tail(TailArgs a)
 {
+    // Children of level l (dense), then of level l - 1 behind them: 8^(l + 1)
+    // entries each, in two arrays used in turn.
+    __shared__ uint64_t s_hash[kTailMaxChildren + kTailMaxParents];
+    __shared__ uint32_t s_rank[kTailMaxChildren + kTailMaxParents];
     __shared__ uint64_t s_key[kTailMaxParents];
     __shared__ uint16_t s_idx[kTailMaxParents];
-    __shared__ uint32_t s_start[kTailMaxParents + 1];
     __shared__ uint32_t s_scan[kTailThreads / kWave];
     __shared__ uint64_t s_red[kTailThreads / kWave];
-    const uint32_t tid = threadIdx.x;
+    const uint32_t tid = threadIdx.x, lane = lane_id();
     BuildCounters* c = a.counters;
-    uint32_t C = uint32_t(*a.child_count);
-    int cur = 0;
-    for (int l = a.top; l >= 0; --l, cur ^= 1) {
-        const bool first = l == a.top;
-        const uint64_t* ccodes = first ? a.child_codes : a.codes[cur ^ 1];
-        const uint32_t* cranks = first ? nullptr : a.ranks[cur ^ 1];
-        const uint64_t* chashes = first ? a.child_hashes : a.out_hashes[l + 1];
-        // Child rank and hash of child i.
-        auto child_rank = [&](uint32_t i) -> uint32_t {
-            return first ? a.child_rank_of_slot[a.child_slots[i]] : cranks[i];
-        };
-
-        // 1. Run heads (parents) in child order.
-        uint32_t M = 0;
-        for (uint32_t base = 0; base < C; base += kTailThreads) {
-            const uint32_t i = base + tid;
-            bool head = false;
-            if (i < C) head = i == 0 || (ccodes[i] >> 3) != (ccodes[i - 1] >> 3);
-            uint32_t total;
-            const uint32_t ex = block_exclusive_scan<kTailThreads>(head ? 1u : 0u, s_scan, total);
-            if (head) s_start[M + ex] = i;
-            M += total;
+    {
+        // The children of level `top`; all loads of a step are issued together.
+        const uint32_t C = uint32_t(min(*a.child_count, uint64_t(kTailMaxChildren)));
+        uint32_t code[kTailChildren], r[kTailChildren];
+        uint64_t h[kTailChildren];
+#pragma unroll
+        for (int k = 0; k < kTailChildren; ++k) {
+            const uint32_t i = min(uint32_t(k) * kTailThreads + tid, C ? C - 1 : 0u);
+            code[k] = C ? uint32_t(a.child_codes[i]) & (kTailMaxChildren - 1) : 0u;
+            r[k] = C ? a.child_slots[i] : 0u;
         }
-        if (tid == 0) s_start[M] = C;
-        __syncthreads();
-
-        // 2. Children scatter their rank and hash into their parent's slot (the
-        //    gathers of all children are independent), then one thread per
-        //    parent reads its 8 slots and forms mask, record and hash.
-        uint64_t* pcodes = a.codes[cur];
-        for (uint32_t k = tid; k < 8 * M; k += kTailThreads) {
-            a.children[k] = kEmptyChild;
-            a.child_hash[k] = 0;
+#pragma unroll
+        for (int k = 0; k < kTailChildren; ++k) r[k] = C ? a.child_rank_of_slot[r[k]] : 0u;
+#pragma unroll
+        for (int k = 0; k < kTailChildren; ++k) h[k] = C ? a.child_hashes[r[k]] : 0ull;
+        for (uint32_t i = tid; i < kTailMaxChildren; i += kTailThreads) {
+            s_rank[i] = kEmptyChild;
+            s_hash[i] = 0;
         }
         __syncthreads();
-#pragma unroll 4
-        for (uint32_t i = tid; i < C; i += kTailThreads) {
-            // Parent of child i: the last run start <= i.
-            uint32_t lo = 0, hi = M;
-            while (hi - lo > 1) {
-                const uint32_t mid = (lo + hi) / 2;
-                if (s_start[mid] <= i) lo = mid;
-                else hi = mid;
+#pragma unroll
+        for (int k = 0; k < kTailChildren; ++k) {
+            if (uint32_t(k) * kTailThreads + tid < C) {
+                s_rank[code[k]] = r[k];
+                s_hash[code[k]] = h[k];
             }
-            const uint32_t slot = uint32_t(ccodes[i] & 7);
-            const uint32_t r = child_rank(i);
-            a.children[8 * lo + slot] = r;
-            a.child_hash[8 * lo + slot] = chashes[r];
         }
         __syncthreads();
-        for (uint32_t p = tid; p < M; p += kTailThreads) {
-            const uint4* cs = reinterpret_cast<const uint4*>(a.children + 8 * uint64_t(p));
-            const uint4 c0 = cs[0], c1 = cs[1];
-            const uint32_t ch[8] = {c0.x, c0.y, c0.z, c0.w, c1.x, c1.y, c1.z, c1.w};
-            uint32_t mask = 0;
+    }
+    uint32_t in = 0, out = kTailMaxChildren;  // where the children and the parents' entries are
+    for (int l = a.top; l >= 0; --l) {
+        const uint32_t P = 1u << (3 * l);  // parents there may be
+        // 1. Parents: mask and hash (absent ones sort last).
+        const uint32_t p = tid;
+        uint32_t mask = 0;
+        uint64_t key = ~0ull;
+        uint32_t idx = 0xFFFFu;
+        if (p < P) {
             uint64_t hs[8];
 #pragma unroll
-            for (int k = 0; k < 8; ++k) {
-                mask |= ch[k] != kEmptyChild ? 1u << k : 0u;
-                hs[k] = a.child_hash[8 * uint64_t(p) + k];
+            for (uint32_t k = 0; k < 8; ++k) {
+                mask |= s_rank[in + 8 * p + k] != kEmptyChild ? 1u << k : 0u;
+                hs[k] = s_hash[in + 8 * p + k];
             }
-            pcodes[p] = ccodes[s_start[p]] >> 3;
-            a.masks[p] = uint8_t(mask);
-            s_key[p] = hash_children(hs);
-            s_idx[p] = uint16_t(p);
+            if (mask) {
+                key = hash_children(hs);
+                idx = p;
+            } else {
+                idx = 0x8000u | p;
+            }
+            s_rank[out + p] = kEmptyChild;
+            s_hash[out + p] = mask ? key : 0ull;
         }
-        // Pad to a power of two; (max key, index 0xFFFF) sorts after every parent.
-        uint32_t n2 = 1;
-        while (n2 < M) n2 <<= 1;
-        for (uint32_t p = M + tid; p < n2; p += kTailThreads) {
-            s_key[p] = ~0ull;
-            s_idx[p] = 0xFFFF;
-        }
-        __syncthreads();
-
-        // 3. Bitonic sort of (key, index), ascending.
-        for (uint32_t size = 2; size <= n2; size <<= 1) {
-            for (uint32_t stride = size >> 1; stride > 0; stride >>= 1) {
-                for (uint32_t t = tid; t < n2 / 2; t += kTailThreads) {
-                    const uint32_t lo = 2 * t - (t & (stride - 1));
-                    const uint32_t hi = lo + stride;
-                    const bool up = (lo & size) == 0;
-                    const uint64_t ka = s_key[lo], kb = s_key[hi];
-                    const uint16_t ia = s_idx[lo], ib = s_idx[hi];
-                    const bool greater = ka > kb || (ka == kb && ia > ib);
-                    if (greater == up) {
-                        s_key[lo] = kb;
-                        s_key[hi] = ka;
-                        s_idx[lo] = ib;
-                        s_idx[hi] = ia;
+        // 2. Ascending sort of (key, idx): each wave's 64 by a bitonic network
+        //    in registers, then runs of 64, 128, ... merged in pairs: an
+        //    element's place is its own plus the elements of the other run
+        //    before it.  Waves without parents only keep the barriers.
+        const bool mine = (tid & ~uint32_t(kWave - 1)) < P;
+        const uint32_t net = min(P, uint32_t(kWave));  // lanes of one network
+        if (mine) {
+            for (uint32_t size = 2; size <= net; size <<= 1) {
+                for (uint32_t stride = size >> 1; stride > 0; stride >>= 1) {
+                    const uint64_t ok = __shfl_xor(key, int(stride), kWave);
+                    const uint32_t oi = uint32_t(__shfl_xor(int(idx), int(stride), kWave));
+                    const bool up = (lane & size) == 0 || size == net;
+                    const bool keep_low = ((lane & stride) == 0) == up;
+                    const bool less = pair_less(key, idx, ok, oi);
+                    // Equal pairs (padding) may stay.
+                    if (less != keep_low && pair_less(ok, oi, key, idx) == keep_low) {
+                        key = ok;
+                        idx = oi;
                     }
                 }
-                __syncthreads();
             }
         }
-
-        // 4. Unique ranks; the first of each equal-hash run represents it.
-        uint32_t* pranks = a.ranks[cur];
-        uint32_t Q = 0;
-        uint64_t words = 0, bad = 0;
-        for (uint32_t base = 0; base < M; base += kTailThreads) {
-            const uint32_t q = base + tid;
-            bool lead = false;
-            if (q < M) lead = q == 0 || s_key[q] != s_key[q - 1];
-            uint32_t total;
-            const uint32_t ex = block_exclusive_scan<kTailThreads>(lead ? 1u : 0u, s_scan, total);
-            if (q < M) {
-                const uint32_t r = Q + ex + (lead ? 1u : 0u) - 1u;
-                const uint32_t p = s_idx[q];
-                pranks[p] = r;
-                if (lead) {
-                    const uint32_t m = a.masks[p];
-                    a.out_hashes[l][r] = s_key[q];
-                    a.out_masks[l][r] = uint8_t(m);
-                    const uint4* src = reinterpret_cast<const uint4*>(a.children + 8 * uint64_t(p));
-                    uint4* dst = reinterpret_cast<uint4*>(a.out_children[l] + 8 * uint64_t(r));
-                    dst[0] = src[0];
-                    dst[1] = src[1];
-                    words += 1 + __popc(m);
-                } else if (a.check_collisions) {
-                    // Compare with the run's representative (content must be equal).
-                    uint32_t f = q;
-                    while (f > 0 && s_key[f - 1] == s_key[q]) --f;
-                    const uint32_t rp = s_idx[f];
-                    bool diff = a.masks[p] != a.masks[rp];
-                    for (int k = 0; k < 8; ++k) diff |= a.children[8 * p + k] != a.children[8 * rp + k];
-                    bad += diff ? 1 : 0;
+        uint32_t pos = tid;
+        if (mine) {
+            s_key[pos] = key;
+            s_idx[pos] = uint16_t(idx);
+        }
+        __syncthreads();
+        for (uint32_t run = kWave; run < P; run *= 2) {
+            if (mine) {
+                const uint32_t other = (pos & ~(run - 1)) ^ run;
+                uint32_t lo = 0, hi = run;
+                while (lo < hi) {
+                    const uint32_t mid = (lo + hi) / 2;
+                    if (pair_less(s_key[other + mid], s_idx[other + mid], key, idx)) lo = mid + 1;
+                    else hi = mid;
                 }
+                pos = (pos & ~(2 * run - 1)) + (pos & (run - 1)) + lo;
             }
-            Q += total;
+            __syncthreads();
+            if (mine) {
+                s_key[pos] = key;
+                s_idx[pos] = uint16_t(idx);
+            }
+            __syncthreads();
         }
-        words = block_reduce_sum<kTailThreads>(words, s_red);
-        bad = block_reduce_sum<kTailThreads>(bad, s_red);
+        // 3. Unique ranks; the first of each equal-hash run represents it.  One
+        //    scan carries the ranks and, above them, the totals: duplicates
+        //    (at most 511: 9 bits from bit 10) and the representatives'
+        //    children (at most 4096: 13 bits from bit 19).
+        const uint32_t q = tid;
+        uint64_t bad = 0;
+        const uint32_t qp = q < P ? s_idx[q] : 0xFFFFu;
+        const bool there = qp < kTailMaxParents;
+        const uint64_t qk = there ? s_key[q] : 0ull;
+        const bool lead = there && (q == 0 || qk != s_key[q - 1]);
+        uint32_t ch[8], m = 0;
+        if (there) {
+#pragma unroll
+            for (uint32_t k = 0; k < 8; ++k) {
+                ch[k] = s_rank[in + 8 * qp + k];
+                m |= ch[k] != kEmptyChild ? 1u << k : 0u;
+            }
+        }
+        uint32_t total;
+        const uint32_t ex = block_exclusive_scan<kTailThreads>(
+            lead ? 1u | uint32_t(__popc(m)) << 19 : there ? 1u << 10 : 0u, s_scan, total) & 1023u;
+        const uint32_t Q = total & 1023u;
+        if (there) {
+            const uint32_t r = ex + (lead ? 1u : 0u) - 1u;
+            s_rank[out + qp] = r;
+            if (lead) {
+                a.out_hashes[l][r] = qk;
+                a.out_masks[l][r] = uint8_t(m);
+                uint4* dst = reinterpret_cast<uint4*>(a.out_children[l] + 8 * uint64_t(r));
+                dst[0] = make_uint4(ch[0], ch[1], ch[2], ch[3]);
+                dst[1] = make_uint4(ch[4], ch[5], ch[6], ch[7]);
+            } else if (a.check_collisions) {
+                // Compare with the run's representative (content must be equal).
+                uint32_t f = q;
+                while (f > 0 && s_key[f - 1] == qk) --f;
+                const uint32_t rp = s_idx[f];
+                bool diff = false;
+                for (uint32_t k = 0; k < 8; ++k) diff |= ch[k] != s_rank[in + 8 * rp + k];
+                bad = diff ? 1 : 0;
+            }
+        }
+        if (a.check_collisions) bad = block_reduce_sum<kTailThreads>(bad, s_red);
         if (tid == 0) {
-            c->pre[l] = M;
+            c->pre[l] = Q + (total >> 10 & 511u);
             c->uniq[l] = Q;
-            c->words[l] = words;
+            c->words[l] = Q + (total >> 19);
             if (bad) c->collisions += bad;
         }
-        // The next level reads this level's codes, ranks and hashes (the
-        // barrier orders the global writes within the workgroup).
-        __syncthreads();
-        C = M;
+        __syncthreads();  // ranks written, keys read
+        const uint32_t t = in;
+        in = out;
+        out = t;
     }
 }
 

@@ -228,7 +228,7 @@ constexpr uint64_t kErrOffsets = 16;    // device chunk offsets invalid or past 
 constexpr uint64_t kPackTileItems = 4096;     // grouped keys per leaf-reduce chunk
 constexpr uint32_t kLeafGroupBits = 9;        // low leaf-code bits the key sort leaves unsorted
 constexpr uint64_t kLeafRegionItems = kPackTileItems + (1u << kLeafGroupBits);  // leaves one chunk may emit
-constexpr uint64_t kBuildTileItems = 1024;    // child codes per level-build tile
+constexpr uint64_t kBuildTileItems = 512;     // child codes per level-build tile
 constexpr uint64_t kExtractTileItems = 256;   // table slots per extract tile
 constexpr uint64_t kFinalTileItems = 4096;    // nodes per final-layout tile
 inline uint64_t tiles(uint64_t n, uint64_t per) { return (n + per - 1) / per; }
@@ -420,13 +420,6 @@ struct TailArgs {
     const uint32_t* child_rank_of_slot;
     const uint64_t* child_hashes;
     const uint64_t* child_count;
-    // Scratch, each at least kTailMaxParents entries (two ping-pong halves for
-    // codes and ranks).
-    uint64_t* codes[2];
-    uint32_t* ranks[2];
-    uint8_t* masks;
-    uint32_t* children;                   // 8 per parent
-    uint64_t* child_hash;                 // 8 per parent
     // Output levels 0..top.
     uint64_t* out_hashes[kTailTopLevel + 1];
     uint8_t* out_masks[kTailTopLevel + 1];

@@ -12,21 +12,30 @@
 // result is a function of IEEE operations alone and a host build of the same
 // steps gives the same pixels.
 //
-// Layout per wave: 8x8 pixels (neighbouring rays walk the same nodes), four
-// waves per workgroup (16x16 pixels).  The walk's stack (one entry per level:
-// node word index, child mask, children still to visit) lives in LDS as a
-// 32-bit index array and a 16-bit mask array (31.5 KB: five workgroups per
-// CU), level-major so a wave's 64 entries of one level are consecutive.
+// Layout per wave: 8x8 pixels (neighbouring rays walk the same nodes), one wave
+// per workgroup: waves differ several times over in the nodes they visit, and a
+// workgroup of four holds its LDS until the slowest is done.  The walk's stack
+// (one entry per level: node word index, child mask, children still to visit)
+// lives in LDS as a 32-bit index array and a 16-bit mask array, sized by the
+// depth and level-major so a wave's 64 entries of one level are consecutive.
+// Bound by the chain of each visit (two dependent loads and about 160 vector
+// instructions; the vector units are half busy) of the longest rays: on average
+// a third of the wave slots are held.  1920x1080 through 20M keys of triangles
+// at depth 11: 571 us with 21-level stacks, workgroups of four waves and the
+// next child searched bit by bit; 493 with a 12-level stack and masks permuted
+// once a node; 470 with one wave a workgroup.
 #include "svdag_device.hpp"
 #include "svdag_internal.hpp"
+
+#include <type_traits>
 
 #pragma clang fp contract(off)
 
 namespace svdag {
 namespace {
 
-constexpr int kTraceThreads = 256;
-constexpr int kTraceTile = 16;  // pixels per workgroup side
+constexpr int kTraceThreads = 64;
+constexpr int kTraceTile = 8;   // pixels per workgroup side
 constexpr int kTraceMaxDepth = 21;
 
 // max and min with the reference's operand order and NaN behaviour
@@ -84,15 +93,15 @@ __device__ __forceinline__ uint32_t crossed_children(bool root, int level, int d
     return m;
 }
 
-// First set child of `mask` in the ray's front-to-back order.
-__device__ __forceinline__ uint32_t next_child(uint32_t order, uint32_t mask)
+// Children in visiting order are c ^ order for c = 0..7: bit c of the result is
+// the mask's bit c ^ order, so the first child to visit is the lowest set bit.
+// XOR-ing a bit of the index swaps neighbours, pairs or halves.
+__device__ __forceinline__ uint32_t visiting_order(uint32_t order, uint32_t mask)
 {
-    // Children in visiting order are child ^ order for child = 0..7; the first
-    // one set is the lowest set bit of the mask permuted by XOR with order.
-    uint32_t permuted = 0;
-#pragma unroll
-    for (uint32_t c = 0; c < 8; ++c) permuted |= ((mask >> (c ^ order)) & 1u) << c;
-    return uint32_t(__builtin_ctz(permuted)) ^ order;
+    const uint32_t a = order & 1u, b = order & 2u, c = order & 4u;
+    mask = (mask & 0xAAu) >> a | (mask & 0x55u) << a;
+    mask = (mask & 0xCCu) >> b | (mask & 0x33u) << b;
+    return (mask & 0xF0u) >> c | (mask & 0x0Fu) << c;
 }
 
 __device__ __forceinline__ uint32_t murmur32(uint32_t h)
@@ -111,16 +120,17 @@ __device__ __forceinline__ uint32_t rgb888(float r, float g, float b)
     return uint32_t(R * 255.0f) | uint32_t(G * 255.0f) << 8 | uint32_t(B * 255.0f) << 16;
 }
 
+// LEVELS: stack entries, at least the depth.
+template <int LEVELS>
 __global__ __launch_bounds__(kTraceThreads) void k_trace_paths(const uint32_t* __restrict__ words, uint64_t n_words,
                                                                int depth, svdag_trace_params p,
                                                                uint32_t* __restrict__ paths,
                                                                uint32_t* __restrict__ colors)
 {
-    __shared__ uint32_t s_index[kTraceMaxDepth][kTraceThreads];
-    __shared__ uint16_t s_masks[kTraceMaxDepth][kTraceThreads];  // child mask | children to visit << 8
-    const uint32_t w = threadIdx.x / kWave, lane = threadIdx.x % kWave;
-    const uint32_t px = blockIdx.x * kTraceTile + (w & 1u) * 8u + (lane & 7u);
-    const uint32_t py = blockIdx.y * kTraceTile + (w >> 1) * 8u + (lane >> 3);
+    __shared__ uint32_t s_index[LEVELS][kTraceThreads];
+    __shared__ uint16_t s_masks[LEVELS][kTraceThreads];  // child mask | children to visit (in their order) << 8
+    const uint32_t px = blockIdx.x * kTraceTile + (threadIdx.x & 7u);
+    const uint32_t py = blockIdx.y * kTraceTile + (threadIdx.x >> 3);
     if (px >= p.width || py >= p.height) return;
     // Entry l of this thread's stack: stack_index[l * kTraceThreads], stack_masks[...].
     uint32_t* const stack_index = &s_index[0][threadIdx.x];
@@ -149,7 +159,7 @@ __global__ __launch_bounds__(kTraceThreads) void k_trace_paths(const uint32_t* _
     uint32_t leaf_lo = 0, leaf_hi = 0;
     if (n_words > 0) {
         child_mask = words[0] & 0xFFu;
-        visit = child_mask & crossed_children(true, 0, depth, path, r);
+        visit = visiting_order(r.order, child_mask & crossed_children(true, 0, depth, path, r));
     }
     int level = 0;
     // Each pass either clears one child of the current node or returns to an
@@ -171,8 +181,8 @@ __global__ __launch_bounds__(kTraceThreads) void k_trace_paths(const uint32_t* _
         for (int a = 0; a < 3; ++a) path[a] >>= uint32_t(level - up);
         level = up;
 
-        const uint32_t child = next_child(r.order, visit);
-        visit &= ~(1u << child);
+        const uint32_t child = uint32_t(__builtin_ctz(visit)) ^ r.order;
+        visit &= visit - 1u;
         path[0] = path[0] << 1 | (child >> 2 & 1u);
         path[1] = path[1] << 1 | (child >> 1 & 1u);
         path[2] = path[2] << 1 | (child & 1u);
@@ -217,7 +227,7 @@ __global__ __launch_bounds__(kTraceThreads) void k_trace_paths(const uint32_t* _
             // Inside a leaf: the child's byte of the occupancy.
             child_mask = ((child & 4u) ? leaf_hi : leaf_lo) >> ((child & 3u) * 8u) & 0xFFu;
         }
-        visit = child_mask & crossed_children(false, level, depth, path, r);
+        visit = visiting_order(r.order, child_mask & crossed_children(false, level, depth, path, r));
     }
 
     const uint64_t pix = uint64_t(py) * p.width + px;
@@ -248,7 +258,15 @@ void launch_trace_paths(hipStream_t s, const uint32_t* words, uint64_t n_words, 
     if (p.width == 0 || p.height == 0) return;
     TimedLaunch t(kKTracePaths, s);
     const dim3 grid((p.width + kTraceTile - 1) / kTraceTile, (p.height + kTraceTile - 1) / kTraceTile);
-    hipLaunchKernelGGL(k_trace_paths, grid, dim3(kTraceThreads), 0, s, words, n_words, depth, p, paths, colors);
+    auto run = [&](auto levels) {
+        hipLaunchKernelGGL((k_trace_paths<decltype(levels)::value>), grid, dim3(kTraceThreads), 0, s, words, n_words,
+                           depth, p, paths, colors);
+    };
+    // A stack of the depth's own size leaves room for more workgroups.
+    if (depth <= 9) run(std::integral_constant<int, 9>{});
+    else if (depth <= 12) run(std::integral_constant<int, 12>{});
+    else if (depth <= 16) run(std::integral_constant<int, 16>{});
+    else run(std::integral_constant<int, kTraceMaxDepth>{});
 }
 
 }  // namespace svdag

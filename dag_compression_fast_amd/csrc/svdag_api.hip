@@ -42,7 +42,8 @@ const char* const kKernelNames[kNumKernelIds] = {
     "leaf_order",     "level_count", "level_build",   "level_check",        "extract_count",      "level_extract",
     "final_count",    "final_positions", "final_write", "merge_insert",     "sketch",             "level_tail",
     "query_voxels",   "vox_setup",   "vox_count",     "vox_write",
-    "trace_paths",    "resident_insert", "sort_scatter_top", "seg_count",   "seg_scatter"};
+    "trace_paths",    "resident_insert", "sort_scatter_top", "seg_count",   "seg_scatter",
+    "copy_out"};
 
 // Event pairs around the launches of the kernels selected by `mask`; resolved
 // into per-kernel totals once the stream has drained.
@@ -1765,19 +1766,28 @@ int svdag_dag_to_host(svdag_context* ctx, const svdag_dag* dag, svdag_dag* out)
 {
     TRY(check_ctx(ctx));
     if (!dag || !out) return set_error(SVDAG_ERR_ARGUMENT, "null argument");
-    uint64_t total = 8 * dag->num_leaves + 8;
-    for (int l = 0; l < dag->num_levels; ++l) total += 41 * dag->levels[l].num_nodes + 32;
+    uint64_t total = 8 * dag->num_leaves + 16;
+    for (int l = 0; l < dag->num_levels; ++l) total += 41 * dag->levels[l].num_nodes + 48;
     char* mem = static_cast<char*>(host_alloc(total));
     if (!mem) return set_error(SVDAG_ERR_MEMORY, "host allocation failed");
     *out = *dag;
     out->location = SVDAG_HOST;
     out->storage = mem;
     const hipMemcpyKind kind = dag->location == SVDAG_DEVICE ? hipMemcpyDeviceToHost : hipMemcpyHostToHost;
+    // A device DAG leaves in one kernel; arrays off a 16-byte boundary (not this
+    // library's own) are copies of their own.
+    CopyOut co{};
+    const bool packed = kind == hipMemcpyDeviceToHost;
     char* p = mem;
     auto copy = [&](void* src, uint64_t bytes) -> void* {
         void* dst = p;
-        if (bytes) (void)hipMemcpyAsync(dst, src, bytes, kind, ctx->stream);
-        p += (bytes + 7) / 8 * 8;
+        if (bytes && packed && reinterpret_cast<uintptr_t>(src) % 16 == 0) {
+            co.seg[co.num++] = {src, dst, bytes};
+            co.pieces += uint32_t((bytes + kCopyPiece - 1) / kCopyPiece);
+        } else if (bytes) {
+            (void)hipMemcpyAsync(dst, src, bytes, kind, ctx->stream);
+        }
+        p += (bytes + 15) / 16 * 16;
         return dst;
     };
     for (int l = 0; l < dag->num_levels; ++l) {
@@ -1787,6 +1797,7 @@ int svdag_dag_to_host(svdag_context* ctx, const svdag_dag* dag, svdag_dag* out)
         out->levels[l].masks = static_cast<uint8_t*>(copy(dag->levels[l].masks, q));
     }
     out->leaves = static_cast<uint64_t*>(copy(dag->leaves, 8 * dag->num_leaves));
+    launch_copy_out(ctx->stream, co);
     const hipError_t e = hipStreamSynchronize(ctx->stream);
     if (e != hipSuccess) {
         host_release(mem);

@@ -1945,6 +1945,43 @@ __global__ __launch_bounds__(kThreads) void k_final_write(FinalArgs a)
 }
 
 // ---------------------------------------------------------------------------
+// A DAG's arrays to pinned host memory in one launch.  A workgroup takes pieces
+// of 16 KB: 4 loads of 16 bytes per thread in flight, then 4 stores over the
+// link.  A DAG has three arrays a level: as copies of their own, most of them a
+// few KB, they took 7 to 10 us each (0.56 MB in 19 arrays: 125 us, now 26; 10.5
+// MB in 28: 389 and 207; 73 MB: 1479 and 1358, the link's 54 GB/s).
+// ---------------------------------------------------------------------------
+__global__ __launch_bounds__(kThreads) void k_copy_out(CopyOut a)
+{
+    constexpr uint32_t kWords = uint32_t(kCopyPiece / 16), kAhead = kWords / kThreads;
+    for (uint32_t piece = blockIdx.x; piece < a.pieces; piece += gridDim.x) {
+        uint32_t at = piece;
+        int g = 0;
+        for (;; ++g) {
+            const uint32_t here = uint32_t((a.seg[g].bytes + kCopyPiece - 1) / kCopyPiece);
+            if (at < here) break;
+            at -= here;
+        }
+        const uint64_t bytes = a.seg[g].bytes;
+        const uint64_t words = bytes / 16, first = uint64_t(at) * kWords + threadIdx.x;
+        const uint4* __restrict__ src = static_cast<const uint4*>(a.seg[g].src);
+        uint4* __restrict__ dst = static_cast<uint4*>(a.seg[g].dst);
+        if (words) {
+            uint4 v[kAhead];
+#pragma unroll
+            for (uint32_t k = 0; k < kAhead; ++k) v[k] = src[min(first + uint64_t(k) * kThreads, words - 1)];
+#pragma unroll
+            for (uint32_t k = 0; k < kAhead; ++k)
+                if (first + uint64_t(k) * kThreads < words) dst[first + uint64_t(k) * kThreads] = v[k];
+        }
+        // The last bytes of a segment, with its first piece.
+        const uint64_t tail = 16 * words + threadIdx.x;
+        if (at == 0 && tail < bytes)
+            static_cast<uint8_t*>(a.seg[g].dst)[tail] = static_cast<const uint8_t*>(a.seg[g].src)[tail];
+    }
+}
+
+// ---------------------------------------------------------------------------
 // Merge insert (MergeDAGs, src/DAGCompression.cu:1109-1320): the nodes of one
 // level of many sub-DAGs, concatenated, enter one shared dedup table.  A node's
 // hash depends only on its content, so it is reused; its children are remapped
@@ -2415,6 +2452,13 @@ void launch_final(hipStream_t s, const FinalArgs& a)
         TimedLaunch t(kKFinalWrite, s);
         hipLaunchKernelGGL(k_final_write, dim3(grid_for((work + kThreads - 1) / kThreads, 8)), dim3(kThreads), 0, s, a);
     }
+}
+
+void launch_copy_out(hipStream_t s, const CopyOut& a)
+{
+    if (a.pieces == 0) return;
+    TimedLaunch t(kKCopyOut, s);
+    hipLaunchKernelGGL(k_copy_out, dim3(grid_for(a.pieces, 2)), dim3(kThreads), 0, s, a);
 }
 
 void launch_resident_leaves(hipStream_t s, const uint64_t* leaves, uint64_t count, uint64_t* table_keys, uint32_t lg,

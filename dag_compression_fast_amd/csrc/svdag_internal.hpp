@@ -50,6 +50,7 @@ enum KernelId : int {
     kKSortScatterTop,  // top-digit pass of a top-digit-first key sort (64-bit in, 32-bit out)
     kKSegCount,        // segmented sort: per-tile counts
     kKSegScatter,      // segmented sort: scatter passes
+    kKCopyOut,         // results to the host
     kNumKernelIds
 };
 
@@ -544,6 +545,22 @@ void launch_trace_paths(hipStream_t s, const uint32_t* words, uint64_t n_words, 
 // 2 the walk left the words).
 void launch_query_voxels(hipStream_t s, const uint32_t* words, uint64_t n_words, int depth, const uint64_t* codes,
                          uint64_t n, uint8_t* out);
+
+// ---- copies to the host ----------------------------------------------------
+// Arrays in device memory to pinned host memory; both ends 16-byte aligned, any
+// length.
+constexpr int kMaxCopySegments = 3 * SVDAG_MAX_LEVELS + 1;
+constexpr uint64_t kCopyPiece = 16384;  // bytes per workgroup step
+struct CopyOut {
+    int num;
+    uint32_t pieces;  // of all segments
+    struct {
+        const void* src;
+        void* dst;
+        uint64_t bytes;
+    } seg[kMaxCopySegments];
+};
+void launch_copy_out(hipStream_t s, const CopyOut& a);
 
 // ---- merge ----------------------------------------------------------------
 // Remaps and inserts the nodes of many sub-DAG levels into one shared table.

@@ -1408,9 +1408,55 @@ int sort_keys_entry(svdag_context* ctx, const K* d_keys, uint64_t n, int32_t bit
     const uint64_t o_a = cv.take(sizeof(K) * n), o_b = cv.take(sizeof(K) * n);
     TRY(ensure_arena(ctx, cv.off));
     char* A = ctx->arena;
-    launch_fill_u64(st, reinterpret_cast<uint64_t*>(A + o_zero), (o_n - o_zero) / 8, 0);
-    launch_fill_u64(st, reinterpret_cast<uint64_t*>(A + o_n), 1, n);
-    launch_fill_u64(st, reinterpret_cast<uint64_t*>(A + o_or), 1, 0);
+    // The digit totals, then the count and the OR of the keys.
+    auto reset = [&] {
+        launch_fill_u64(st, reinterpret_cast<uint64_t*>(A + o_zero), (o_or + 8 - o_zero) / 8, 0, (o_n - o_zero) / 8, n);
+    };
+    reset();
+    if constexpr (sizeof(K) == 8) {
+        // Top digit first, from three digits on, where the rest fits 32 bits:
+        // 32-bit keys in the two halves of the first buffer, the tables in the
+        // second.  A key with bits above the sorted ones (read back after the
+        // histogram) has to keep them, which only the LSD sort does.
+        const uint32_t top_bits = uint32_t(std::min(ctx->radix_bits, kMaxRadixBits));
+        const uint32_t top_shift = uint32_t(bits) > top_bits ? uint32_t(bits) - top_bits : 0;
+        if (ctx->top_first != kTopFirstNever && plan.passes >= 3 && top_shift <= 32 &&
+            (n >= kTopSortMinKeys || ctx->top_first == kTopFirstAlways) && n < (1ull << 30)) {
+            const SortPlan below = make_sort_plan(0, int(top_shift), int(top_bits), kSortIptSmall);
+            uint32_t widest = 0;
+            for (int p = 0; p < below.passes; ++p) widest = std::max(widest, below.bits[p]);
+            const uint64_t buckets = 1ull << top_bits, tb = seg_tile_bound(n, buckets);
+            Carver t;
+            t.off = o_b;
+            SegScratch sc;
+            uint64_t* const bucket_start = reinterpret_cast<uint64_t*>(A + t.take(8 * (buckets + 1)));
+            sc.tiles = reinterpret_cast<SegTile*>(A + t.take(sizeof(SegTile) * tb));
+            sc.chunk_tiles = reinterpret_cast<uint32_t*>(A + t.take(4 * (buckets + 1)));
+            sc.counts = reinterpret_cast<uint32_t*>(A + t.take(4 * (tb << widest)));
+            sc.totals = reinterpret_cast<uint32_t*>(A + t.take(4 * (buckets << widest)));
+            sc.starts = reinterpret_cast<uint32_t*>(A + t.take(4 * (buckets << widest)));
+            sc.ntiles = reinterpret_cast<uint64_t*>(A + t.take(8));
+            sc.slices = reinterpret_cast<uint32_t*>(A + o_counts);  // free after the top pass
+            sc.slice_words = sort_count_words(n);
+            if (t.off <= cv.off) {
+                uint32_t* const zero = reinterpret_cast<uint32_t*>(A + o_zero);
+                uint32_t* const counts = reinterpret_cast<uint32_t*>(A + o_counts);
+                const uint64_t* const n_ptr = reinterpret_cast<const uint64_t*>(A + o_n);
+                launch_top_histogram(st, d_keys, top_shift, top_bits, n_ptr, n, zero, counts,
+                                     reinterpret_cast<unsigned long long*>(A + o_or));
+                HIP_TRY(hipMemcpyAsync(&ctx->h_counters->key_or, A + o_or, 8, hipMemcpyDeviceToHost, st));
+                TRY(finish(ctx, "sort_keys"));
+                if ((ctx->h_counters->key_or >> bits) == 0) {
+                    uint32_t* const a = reinterpret_cast<uint32_t*>(A + o_a);
+                    launch_top_sort(st, d_keys, a, a + n, d_out, top_shift, top_bits, below, n_ptr, n, zero, counts,
+                                    bucket_start, sc);
+                    HIP_TRY(hipGetLastError());
+                    return finish(ctx, "sort_keys");
+                }
+                reset();
+            }
+        }
+    }
     const int where = launch_sort<K>(st, plan, d_keys, reinterpret_cast<K*>(A + o_a),
                                      reinterpret_cast<K*>(A + o_b), d_out,
                                      reinterpret_cast<const uint64_t*>(A + o_n), n,

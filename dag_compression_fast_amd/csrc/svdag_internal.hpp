@@ -195,6 +195,20 @@ int launch_cell_sort(hipStream_t stream, const K* keys_in, uint32_t* keys_out, i
                      const uint64_t* n_ptr, uint64_t n_bound, uint32_t* zero, uint32_t* counts,
                      unsigned long long* key_or, uint32_t* starts);
 
+// Full key sort, top digit first (keys below 2^(top_shift + top_bits), top_shift
+// <= 32): the histogram (also the OR of the keys), then the passes.  below:
+// digits covering [0, top_shift); keys_a and keys_b: n 32-bit keys; the
+// segmented sort's scratch has 2^top_bits chunks and digits of below's widths.
+void launch_top_histogram(hipStream_t stream, const uint64_t* keys_in, uint32_t top_shift, uint32_t top_bits,
+                          const uint64_t* n_ptr, uint64_t n, uint32_t* zero, uint32_t* counts,
+                          unsigned long long* key_or);
+void launch_top_sort(hipStream_t stream, const uint64_t* keys_in, uint32_t* keys_a, uint32_t* keys_b,
+                     uint64_t* keys_out, uint32_t top_shift, uint32_t top_bits, const SortPlan& below,
+                     const uint64_t* n_ptr, uint64_t n, uint32_t* zero, uint32_t* counts, uint64_t* bucket_start,
+                     const SegScratch& sc);
+// From how many keys svdag_sort_keys takes it.
+constexpr uint64_t kTopSortMinKeys = 1ull << 22;
+
 template <typename K>
 int launch_sort(hipStream_t stream, const SortPlan& plan, const K* keys_in, K* keys_a, K* keys_b, K* final_keys,
                 const uint64_t* n_ptr, uint64_t n_bound, uint32_t* zero, uint32_t* counts,

@@ -329,6 +329,36 @@ __global__ __launch_bounds__(kScanThreads) void k_sort_scan(uint32_t* __restrict
     }
 }
 
+// Where the counts of the tiles are.  A workgroup of the count kernel takes
+// `per` consecutive tiles and keeps counting over them, so that only slices
+// (its tiles of one chunk) are left to scan: slice (t / per + chunk) of tile t
+// (both terms only grow, so no two slices share a row) holds the keys of each
+// digit before the slice, tile t's row those before the tile in the slice.
+// per == 1: the tile rows alone, as slice rows.  (8 chunks of 67M keys have so
+// many tiles and so few workgroups in the scan that scanning tile rows took 415
+// us a pass; slices take 11.)  All rows are R words, written
+// and read whole.
+struct SegRows {
+    uint32_t* tile;   // per > 1: ntiles rows
+    uint32_t* slice;  // per == 1: ntiles rows; else ntiles / per + num_chunks rows
+    uint32_t per;
+};
+__device__ __forceinline__ uint64_t seg_slice(const SegRows& rows, uint64_t t, uint64_t chunk)
+{
+    return rows.per == 1 ? t : uint32_t(t) / rows.per + chunk;
+}
+
+// The tiles of a segmented pass (none crosses a chunk), with the offset rows of
+// its digits; keys written wider than they are read get their chunk above
+// high_shift.
+struct SegPass {
+    const SegTile* tiles = nullptr;
+    const uint64_t* ntiles = nullptr;
+    const uint32_t* starts = nullptr;
+    SegRows rows{nullptr, nullptr, 1};
+    uint32_t high_shift = 0;
+};
+
 // Ranking of a scatter pass: unstable (the first pass of a key-only sort),
 // stable, or adaptive: unstable for a tile whose keys all agree on the bits
 // the earlier passes sorted (their order within a digit is then free; the
@@ -341,7 +371,8 @@ enum RankMode { kRankUnstable = 0, kRankStable = 1, kRankAdaptive = 2 };
 
 // KO narrower than K (the top-digit pass of a 64-bit key sort): each key is
 // written without its digit and the bits above it, as a key local to its digit.
-template <typename K, int MODE, int IPT, int THREADS, typename KO = K>
+// SEG: tiles and offsets from seg (n_ptr, offsets, stride and prefix unused).
+template <typename K, int MODE, int IPT, int THREADS, typename KO = K, bool SEG = false>
 __global__ __launch_bounds__(THREADS) void k_sort_scatter(const K* __restrict__ keys_in, KO* __restrict__ keys_out,
                                                                const uint64_t* __restrict__ n_ptr, uint32_t shift,
                                                                uint32_t digit_mask,
@@ -349,7 +380,7 @@ __global__ __launch_bounds__(THREADS) void k_sort_scatter(const K* __restrict__ 
                                                                ChunkPrefix prefix, uint32_t sorted_shift,
                                                                uint32_t sorted_mask,
                                                                const unsigned long long* __restrict__ key_or,
-                                                               uint32_t end_bit)
+                                                               uint32_t end_bit, SegPass seg)
 {
     constexpr bool MATCH = MODE != kRankUnstable;  // needs the stable ranking's tables
     constexpr bool DCNT = MODE != kRankStable;     // needs the unstable ranking's counters
@@ -375,8 +406,8 @@ __global__ __launch_bounds__(THREADS) void k_sort_scatter(const K* __restrict__ 
     const uint32_t tid = threadIdx.x;
     const uint32_t w = tid / kWave;
     const uint32_t lane = lane_id();
-    const uint64_t n = *n_ptr;
-    const uint64_t ntiles = (n + kTile - 1) / kTile;
+    const uint64_t n = SEG ? 0 : *n_ptr;
+    const uint64_t ntiles = SEG ? *seg.ntiles : (n + kTile - 1) / kTile;
     const uint32_t radix = digit_mask + 1;
 
     // Keys above the sorted bits: every tile ranks stably.
@@ -386,9 +417,14 @@ __global__ __launch_bounds__(THREADS) void k_sort_scatter(const K* __restrict__ 
     K key[IPT];
     // Keys of tile t (loaded one tile ahead).  Full tiles, the common case, load
     // without per-key guards.
+    auto tile_of = [&](uint64_t t) -> SegTile {
+        if constexpr (SEG) return seg.tiles[t];
+        else return SegTile{t * kTile, uint32_t(min(uint64_t(kTile), n - t * kTile)), 0u};
+    };
     auto load_tile = [&](uint64_t t) {
-        const uint64_t base = t * kTile;
-        const uint32_t cnt = t < walk.end ? uint32_t(min(uint64_t(kTile), n - base)) : 0u;
+        const SegTile next = t < walk.end ? tile_of(t) : SegTile{0, 0, 0};
+        const uint64_t base = next.start;
+        const uint32_t cnt = next.count;
         const K* src = keys_in + base + wave_base + lane;
         if (cnt == kTile) {
             // Each key is read once: non-temporal loads (measured 4% faster
@@ -419,8 +455,8 @@ __global__ __launch_bounds__(THREADS) void k_sort_scatter(const K* __restrict__ 
     // barrier after the clear also orders the previous tile's stores (reads of
     // s_keys and s_base) before this tile's writes of them.
     for (uint64_t tile = walk.tile; tile < walk.end; tile += walk.step) {
-        const uint64_t tile_base = tile * kTile;
-        const uint32_t tile_n = uint32_t(min(uint64_t(kTile), n - tile_base));
+        const SegTile here = tile_of(tile);
+        const uint32_t tile_n = here.count;
         if constexpr (MODE == kRankAdaptive) {
             // The span of the earlier passes' bits over the tile's keys.
             uint32_t lo = 0xFFFFFFFFu, hi = 0;
@@ -530,7 +566,12 @@ __global__ __launch_bounds__(THREADS) void k_sort_scatter(const K* __restrict__ 
             const uint32_t d = tid * DPT + k;
             if (d < radix) {
                 s_lstart[d] = uint16_t(lstart);
-                s_base[d] = offsets[uint64_t(d) * stride + tile] - lstart;
+                if constexpr (SEG)
+                    s_base[d] = seg.starts[uint64_t(here.chunk) * radix + d] +
+                                seg.rows.slice[seg_slice(seg.rows, tile, here.chunk) * radix + d] +
+                                (seg.rows.per != 1 ? seg.rows.tile[tile * radix + d] : 0u) - lstart;
+                else
+                    s_base[d] = offsets[uint64_t(d) * stride + tile] - lstart;
             }
             lstart += dtot[k];
         }
@@ -554,7 +595,9 @@ __global__ __launch_bounds__(THREADS) void k_sort_scatter(const K* __restrict__ 
             const K k = s_keys[j];
             const uint32_t d = uint32_t(k >> shift) & digit_mask;
             const uint32_t o = s_base[d] + j;
-            if constexpr (sizeof(KO) < sizeof(K))
+            if constexpr (SEG && sizeof(KO) > sizeof(K))
+                keys_out[o] = KO(here.chunk) << seg.high_shift | k;
+            else if constexpr (sizeof(KO) < sizeof(K))
                 keys_out[o] = KO(k & ((K(1) << shift) - 1));
             else
                 keys_out[o] = k;
@@ -639,7 +682,7 @@ static void launch_pass(hipStream_t stream, const K* src, K* dst, const uint64_t
         TimedLaunch t(kKSortScatterKeys, stream);
         hipLaunchKernelGGL((k_sort_scatter<K, kRankUnstable, IPT, kSortThreads>), dim3(scatter_grid),
                            dim3(kSortThreads), kUnstableExtraLds, stream, src, dst, n_ptr, shift,
-                           dmask, counts, stride, prefix, sorted_lo, sorted_mask, nullptr, 64u);
+                           dmask, counts, stride, prefix, sorted_lo, sorted_mask, nullptr, 64u, SegPass{});
     } else if (span_fits || (first && wide_or)) {
         // Later key-only passes: tiles uniform in the earlier passes' bits (the
         // common case: the input is sorted on them, in runs longer than a tile)
@@ -647,12 +690,12 @@ static void launch_pass(hipStream_t stream, const K* src, K* dst, const uint64_t
         TimedLaunch t(kKSortScatterKeys, stream);
         hipLaunchKernelGGL((k_sort_scatter<K, kRankAdaptive, IPT, kSortThreads>), dim3(scatter_grid),
                            dim3(kSortThreads), 0, stream, src, dst, n_ptr, shift, dmask, counts,
-                           stride, prefix, sorted_lo, sorted_mask, wide_or, end_bit);
+                           stride, prefix, sorted_lo, sorted_mask, wide_or, end_bit, SegPass{});
     } else {
         TimedLaunch t(kKSortScatterKeys, stream);
         hipLaunchKernelGGL((k_sort_scatter<K, kRankStable, IPT, kSortThreads>), dim3(scatter_grid),
                            dim3(kSortThreads), 0, stream, src, dst, n_ptr, shift, dmask, counts,
-                           stride, prefix, sorted_lo, sorted_mask, nullptr, 64u);
+                           stride, prefix, sorted_lo, sorted_mask, nullptr, 64u, SegPass{});
     }
 }
 
@@ -748,25 +791,6 @@ constexpr int kSegDigitsPerThread = int(kSegMaxDigits / kSegThreads);
 static_assert(kSegDigitsPerThread * kSegThreads == int(kSegMaxDigits), "digits spread evenly over the threads");
 static_assert(kSegTile == kSegTileItems, "tile size shared with the planner");
 static_assert(kSegWideThreads * kSegIpt <= 65536 && kSegMaxBins <= 65536, "bin and rank packed in 16 bits each");
-
-// Where the counts of the tiles are.  A workgroup of the count kernel takes
-// `per` consecutive tiles and keeps counting over them, so that only slices
-// (its tiles of one chunk) are left to scan: slice (t / per + chunk) of tile t
-// (both terms only grow, so no two slices share a row) holds the keys of each
-// digit before the slice, tile t's row those before the tile in the slice.
-// per == 1: the tile rows alone, as slice rows.  (8 chunks of 67M keys have so
-// many tiles and so few workgroups in the scan that scanning tile rows took 415
-// us a pass; slices take 11.)  All rows are R words, written
-// and read whole.
-struct SegRows {
-    uint32_t* tile;   // per > 1: ntiles rows
-    uint32_t* slice;  // per == 1: ntiles rows; else ntiles / per + num_chunks rows
-    uint32_t per;
-};
-__device__ __forceinline__ uint64_t seg_slice(const SegRows& rows, uint64_t t, uint64_t chunk)
-{
-    return rows.per == 1 ? t : uint32_t(t) / rows.per + chunk;
-}
 
 // Tile table of the segmented sort, planned on the device from the chunk
 // offsets (no host planning, so a captured build replays for any offsets
@@ -1264,7 +1288,7 @@ int launch_top_digit_sort(hipStream_t stream, const uint64_t* keys_in, uint32_t*
         // (207 against 243 us on 70M keys).
         TimedLaunch t(kKSortScatterTop, stream);
         hipLaunchKernelGGL((k_sort_scatter<uint64_t, kRankUnstable, I, kSortThreads, uint32_t>),
-                           dim3(scatter_grid), dim3(kSortThreads), 0, stream, keys_in, local, n_ptr, top_shift, dmask, counts, stride, ChunkPrefix{}, 0u, 0u, nullptr, 64u);
+                           dim3(scatter_grid), dim3(kSortThreads), 0, stream, keys_in, local, n_ptr, top_shift, dmask, counts, stride, ChunkPrefix{}, 0u, 0u, nullptr, 64u, SegPass{});
     };
     if (ipt == kSortIptLarge) run(std::integral_constant<int, kSortIptLarge>{});
     else run(std::integral_constant<int, kSortIptSmall>{});
@@ -1306,7 +1330,7 @@ int launch_cell_sort(hipStream_t stream, const K* keys_in, uint32_t* keys_out, i
         TimedLaunch t(kKSortScatterKeys, stream);
         hipLaunchKernelGGL((k_sort_scatter<K, kRankUnstable, I, kSortThreads, uint32_t>), dim3(scatter_grid),
                            dim3(kSortThreads), 0, stream, keys_in, keys_out, n_ptr, shift, dmask, counts, stride,
-                           ChunkPrefix{}, 0u, 0u, nullptr, 64u);
+                           ChunkPrefix{}, 0u, 0u, nullptr, 64u, SegPass{});
     };
     if (ipt == kSortIptLarge) run(std::integral_constant<int, kSortIptLarge>{});
     else run(std::integral_constant<int, kSortIptSmall>{});
@@ -1319,5 +1343,110 @@ template int launch_cell_sort<uint64_t>(hipStream_t, const uint64_t*, uint32_t*,
 template int launch_cell_sort<uint32_t>(hipStream_t, const uint32_t*, uint32_t*, int, uint32_t, uint32_t,
                                         const uint64_t*, uint64_t, uint32_t*, uint32_t*, unsigned long long*,
                                         uint32_t*);
+
+// ---------------------------------------------------------------------------
+// Full sort of 64-bit keys below 2^(top_shift + top_bits), top digit first: the
+// top pass leaves 32-bit keys grouped by their top digit, stable segmented LSD
+// passes sort the rest inside each group, and the last one writes the 64-bit
+// keys.  Against an LSD sort of all digits a pass after the first moves 12 bytes
+// a key instead of 24.  The caller has launched launch_top_histogram and knows
+// that no key has a bit above the digit (those would be lost).
+// ---------------------------------------------------------------------------
+void launch_top_histogram(hipStream_t stream, const uint64_t* keys_in, uint32_t top_shift, uint32_t top_bits,
+                          const uint64_t* n_ptr, uint64_t n, uint32_t* zero, uint32_t* counts,
+                          unsigned long long* key_or)
+{
+    constexpr int I = kSortIptSmall;
+    HistPlan hp{};
+    hp.passes = 1;
+    hp.shift[0] = top_shift;
+    hp.mask[0] = (1u << top_bits) - 1u;
+    const uint64_t stride = sort_tiles(n, I);
+    TimedLaunch t(kKHistogram, stream);
+    hipLaunchKernelGGL((k_histogram<uint64_t, I>), dim3(histogram_grid<uint64_t, I>(stride)), dim3(kSortThreads), 0,
+                       stream, keys_in, n_ptr, hp, zero, key_or, counts, stride, ChunkPrefix{});
+}
+
+void launch_top_sort(hipStream_t stream, const uint64_t* keys_in, uint32_t* keys_a, uint32_t* keys_b,
+                     uint64_t* keys_out, uint32_t top_shift, uint32_t top_bits, const SortPlan& below,
+                     const uint64_t* n_ptr, uint64_t n, uint32_t* zero, uint32_t* counts, uint64_t* bucket_start,
+                     const SegScratch& sc)
+{
+    constexpr int I = kSortIptSmall;
+    static_assert(kSortThreads == kSegThreads && I == kSegIpt, "one tile size");
+    const uint32_t top_mask = (1u << top_bits) - 1u, buckets = top_mask + 1;
+    const uint64_t stride = sort_tiles(n, I);
+    const int cus = device_cu_count();
+    auto tile_grid = [&](uint64_t tiles) {
+        return dim3(uint32_t(std::max<uint64_t>(
+            kXcds, std::min<uint64_t>((tiles + kXcds - 1) / kXcds * kXcds, uint64_t(cus) * 64) / kXcds * kXcds)));
+    };
+    const uint64_t tile_count = seg_tile_bound(n, buckets);
+    const dim3 grid = tile_grid(tile_count);
+    {
+        TimedLaunch t(kKSortScan, stream);
+        if (stride <= kSmallScanTiles)
+            hipLaunchKernelGGL(k_sort_scan<kWave>, dim3(buckets), dim3(kWave), 0, stream, counts, zero, n_ptr, stride,
+                               uint64_t(kSortThreads) * I, nullptr);
+        else
+            hipLaunchKernelGGL(k_sort_scan<kScanThreads>, dim3(buckets), dim3(kScanThreads), 0, stream, counts, zero,
+                               n_ptr, stride, uint64_t(kSortThreads) * I, nullptr);
+        hipLaunchKernelGGL(k_digit_starts, dim3(1), dim3(kRadix), 0, stream, zero, buckets, n_ptr, bucket_start);
+    }
+    {
+        TimedLaunch t(kKSortScatterTop, stream);
+        hipLaunchKernelGGL((k_sort_scatter<uint64_t, kRankUnstable, I, kSortThreads, uint32_t>), tile_grid(stride),
+                           dim3(kSortThreads), 0, stream, keys_in, keys_a, n_ptr, top_shift, top_mask, counts, stride,
+                           ChunkPrefix{}, 0u, 0u, nullptr, 64u, SegPass{});
+    }
+    {
+        TimedLaunch t(kKSortScan, stream);
+        hipLaunchKernelGGL(k_seg_plan_chunks, dim3(1), dim3(kPlanThreads), 0, stream, bucket_start, uint64_t(buckets),
+                           n_ptr, sc.chunk_tiles, sc.ntiles, kSegTile);
+        hipLaunchKernelGGL(k_seg_plan_tiles,
+                           dim3(int(std::max<uint64_t>(1, std::min<uint64_t>((tile_count + 255) / 256, uint64_t(cus) * 8)))),
+                           dim3(256), 0, stream, bucket_start, sc.chunk_tiles, uint64_t(buckets), sc.ntiles, sc.tiles,
+                           kSegTile);
+    }
+    uint32_t *src = keys_a, *dst = keys_b;
+    for (int p = 0; p < below.passes; ++p) {
+        const uint32_t shift = below.shift[p], mask = (1u << below.bits[p]) - 1u, R = mask + 1;
+        const uint64_t col_jobs = uint64_t(buckets) * ((R + kWave - 1) / kWave);
+        const int col_grid = int(std::max<uint64_t>(1, std::min<uint64_t>(col_jobs, uint64_t(cus) * 16)));
+        SegPass seg{sc.tiles, sc.ntiles, sc.starts, SegRows{sc.counts, sc.counts, 1}, top_shift};
+        const uint32_t per = uint32_t(std::min<uint64_t>(kSegMaxSlice, tile_count / kSegUnits));
+        if (per > 1 && (tile_count / per + buckets + 1) * R <= sc.slice_words)
+            seg.rows = SegRows{sc.counts, sc.slices, per};
+        {
+            TimedLaunch t(kKSegCount, stream);
+            hipLaunchKernelGGL((k_seg_count<false, uint32_t, kSegThreads>), grid, dim3(kSegThreads), 0, stream,
+                               static_cast<const uint32_t*>(src), sc.tiles, sc.ntiles, shift, mask, top_shift, seg.rows,
+                               nullptr);
+        }
+        {
+            TimedLaunch t(kKSortScan, stream);
+            hipLaunchKernelGGL(k_seg_scan_cols, dim3(col_grid), dim3(kColThreads), 0, stream, sc.chunk_tiles,
+                               uint64_t(buckets), R, seg.rows, sc.totals);
+            hipLaunchKernelGGL(k_seg_scan_digits, dim3(buckets), dim3(kSegThreads), 0, stream, bucket_start,
+                               uint64_t(buckets), R, sc.totals, sc.starts);
+        }
+        TimedLaunch t(kKSegScatter, stream);
+        const bool last = p + 1 == below.passes;
+        const uint32_t sorted = shift == 0 ? 0u : (1u << shift) - 1u;  // bits the earlier passes sorted
+        auto pass = [&](auto mode, auto out) {
+            using KO = std::remove_pointer_t<decltype(out)>;
+            hipLaunchKernelGGL((k_sort_scatter<uint32_t, decltype(mode)::value, I, kSortThreads, KO, true>), grid,
+                               dim3(kSortThreads), 0, stream, src, out, nullptr, shift, mask, nullptr, 0ull,
+                               ChunkPrefix{}, 0u, sorted, nullptr, 64u, seg);
+        };
+        using Unstable = std::integral_constant<int, kRankUnstable>;
+        using Adaptive = std::integral_constant<int, kRankAdaptive>;
+        if (p == 0 && last) pass(Unstable{}, keys_out);
+        else if (p == 0) pass(Unstable{}, dst);
+        else if (last) pass(Adaptive{}, keys_out);
+        else pass(Adaptive{}, dst);
+        std::swap(src, dst);
+    }
+}
 
 }  // namespace svdag

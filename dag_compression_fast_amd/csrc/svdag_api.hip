@@ -701,6 +701,8 @@ struct BatchLayout {
     bool segmented = false;
     uint32_t seg_lo = 0, seg_chunk_bits = 0;
     uint64_t cells = 0;  // the sort's one pass groups the keys by 64^3 cell
+    uint64_t chunks = 0;  // chunks sorted: all, or (compact) those that hold keys
+    bool compact = false;
 };
 
 BatchLayout plan_batch(const BuildLayout& L, uint64_t n, const BatchInfo* batch, uint32_t first_bits)
@@ -710,6 +712,7 @@ BatchLayout plan_batch(const BuildLayout& L, uint64_t n, const BatchInfo* batch,
     Carver c;
     c.off = L.total;
     B.offsets = c.take(8 * (batch->num_chunks + 1));
+    B.chunks = batch->num_chunks;
     // Batched builds whose chunk-local sort spans at most kSegMaxBits bits sort
     // inside each chunk (the chunk order is the input order); the tiles are
     // planned on the device from the offsets.
@@ -721,10 +724,23 @@ BatchLayout plan_batch(const BuildLayout& L, uint64_t n, const BatchInfo* batch,
     // its two passes.
     if (B.segmented && first_bits == 0 && batch->chunk_depth > 6 &&
         B.seg_chunk_bits - kCellShift <= kMaxSegDigitBits) {
-        const uint64_t cells = batch->num_chunks << (B.seg_chunk_bits - kCellShift);
-        if (cells_pay(cells, n)) {
+        // Where most chunks are empty (a round of a served grid), only the
+        // others are sorted; their offsets and indices fit the offsets' room.
+        // Five chunks of a 4096-chunk grid, 2M keys: the tables of all of them
+        // (2M cells) left the sort at two passes with scans of 15 us each.
+        uint64_t live = batch->num_chunks;
+        if (batch->h_offsets) {
+            live = 0;
+            for (uint64_t i = 0; i < batch->num_chunks; ++i) live += batch->h_offsets[i + 1] > batch->h_offsets[i];
+        }
+        const bool compact = 2 * live <= batch->num_chunks;
+        const uint64_t chunks = compact ? live : batch->num_chunks;
+        const uint64_t cells = chunks << (B.seg_chunk_bits - kCellShift);
+        if (chunks != 0 && cells_pay(cells, n)) {
             B.cells = cells;
             B.seg_lo = kCellShift;
+            B.chunks = chunks;
+            B.compact = compact;
         }
     }
     if (B.segmented) {
@@ -790,8 +806,10 @@ int build(svdag_context* ctx, const K* d_keys, uint64_t n, int depth, svdag_dag*
     char* O = static_cast<char*>(storage);
     const bool capture = fixed && fixed->captured;
     bool forked = false;  // work is in flight on the side stream
+    std::vector<uint64_t> live_chunks;  // offsets, then (32-bit) indices; read by a copy until the stream drains
     auto fail = [&](int code) {
         if (forked) (void)hipStreamSynchronize(ctx->side);
+        if (!live_chunks.empty()) (void)hipStreamSynchronize(st);
         if (!fixed) device_release(ctx, storage);
         out->storage = nullptr;
         return code;
@@ -817,7 +835,22 @@ int build(svdag_context* ctx, const K* d_keys, uint64_t n, int depth, svdag_dag*
     if (batch) {
         if (!d_off) {
             uint64_t* up = reinterpret_cast<uint64_t*>(A + B.offsets);
-            if (hipMemcpyAsync(up, batch->h_offsets, 8 * (batch->num_chunks + 1), hipMemcpyHostToDevice, st) != hipSuccess)
+            const uint64_t* from = batch->h_offsets;
+            uint64_t words = batch->num_chunks + 1;
+            if (B.compact) {
+                words = B.chunks + 1 + (B.chunks + 1) / 2;
+                live_chunks.resize(words);
+                uint32_t* const ids = reinterpret_cast<uint32_t*>(live_chunks.data() + B.chunks + 1);
+                uint64_t j = 0;
+                for (uint64_t i = 0; i < batch->num_chunks; ++i)
+                    if (from[i + 1] > from[i]) {
+                        live_chunks[j] = from[i];
+                        ids[j++] = uint32_t(i);
+                    }
+                live_chunks[j] = from[batch->num_chunks];
+                from = live_chunks.data();
+            }
+            if (hipMemcpyAsync(up, from, 8 * words, hipMemcpyHostToDevice, st) != hipSuccess)
                 return fail(set_error(SVDAG_ERR_HIP, "offset upload failed"));
             d_off = up;
         }
@@ -844,7 +877,7 @@ int build(svdag_context* ctx, const K* d_keys, uint64_t n, int depth, svdag_dag*
             sc.slice_words = sort_count_words(n);
             where = launch_segmented_sort(st, reinterpret_cast<const uint64_t*>(d_keys),
                                           reinterpret_cast<uint32_t*>(ka), reinterpret_cast<uint32_t*>(kb), d_off,
-                                          batch->num_chunks, &c->n, n, sc, B.seg_lo, B.seg_chunk_bits, err,
+                                          B.chunks, &c->n, n, sc, B.seg_lo, B.seg_chunk_bits, err,
                                           ctx->seg_first_bits);
         } else {
             where = launch_sort<uint64_t>(st, L.key_plan, reinterpret_cast<const uint64_t*>(d_keys), ka, kb,
@@ -903,7 +936,11 @@ int build(svdag_context* ctx, const K* d_keys, uint64_t n, int depth, svdag_dag*
         ca.keys = static_cast<const uint32_t*>(sorted);
         ca.starts = reinterpret_cast<const uint32_t*>(A + (batch ? B.seg_starts : L.cell_starts));
         ca.cells = batch ? B.cells : L.cells;
-        ca.run_cells = cell_run_length(ca.cells, sort_count_words(n));
+        if (B.compact) {
+            ca.chunk_ids = reinterpret_cast<const uint32_t*>(d_off + B.chunks + 1);
+            ca.chunk_cells = 1u << (B.seg_chunk_bits - kCellShift);
+        }
+        ca.run_cells = cell_run_length(ca.cells, sort_count_words(n), B.compact ? ca.chunk_cells : kMaxRunCells);
         ca.reg_mask = reg_code;
         ca.reg_code = reinterpret_cast<uint32_t*>(reg_mask);
         ca.run_counts = sort_counts;  // free once the sort is done

@@ -581,7 +581,10 @@ __global__ __launch_bounds__(kThreads) void k_cell_compact(CellArgs a, const uin
             const uint32_t cnt = uint32_t(__shfl(int(count), int(r), kWave));
             const uint64_t src = uint32_t(__shfl(int(start), int(r), kWave));
             const uint64_t dst = before + uint32_t(__shfl(int(upto), int(r), kWave)) - cnt;
-            const uint64_t high = (batch + r) * a.run_cells * kCellLeaves;
+            uint64_t cell = (batch + r) * a.run_cells;
+            if (a.chunk_ids)
+                cell = uint64_t(a.chunk_ids[cell / a.chunk_cells]) * a.chunk_cells + cell % a.chunk_cells;
+            const uint64_t high = cell * kCellLeaves;
             if (dst + cnt > a.lp_capacity) {
                 if (lane == 0) atomicOr(err, (unsigned long long)kErrInternal);
                 continue;

@@ -306,10 +306,13 @@ void launch_leaf_reduce(hipStream_t s, const K* sorted, BuildCounters* c, uint32
 constexpr uint32_t kCellShift = 18;
 constexpr uint32_t kCellLeaves = 1u << (kCellShift - 6);
 constexpr uint32_t kMaxRunCells = 32;
-inline uint32_t cell_run_length(uint64_t cells, uint64_t max_runs)
+// A power of two, at most `most`.
+inline uint32_t cell_run_length(uint64_t cells, uint64_t max_runs, uint64_t most)
 {
-    const uint64_t runs = std::min<uint64_t>(16384, max_runs);
-    return uint32_t(std::max<uint64_t>(1, std::min<uint64_t>(kMaxRunCells, (cells + runs - 1) / runs)));
+    const uint64_t runs = std::min<uint64_t>(16384, max_runs), top = std::min<uint64_t>(kMaxRunCells, most);
+    uint32_t len = 1;
+    while (len < top && cells > len * runs) len *= 2;
+    return len;
 }
 __host__ __device__ inline uint64_t cell_runs(uint64_t cells, uint32_t run_cells) { return (cells + run_cells - 1) / run_cells; }
 // A cell costs its workgroup a pass over 4096 table words however few keys it
@@ -327,6 +330,11 @@ struct CellArgs {
     uint64_t* lp_code;
     uint64_t* lp_mask;
     uint64_t lp_capacity;
+    // Non-null: the cells are those of some chunks only, chunk_cells each (a
+    // power of two that run_cells divides), chunk j's at chunk_ids[j] in the
+    // order of all chunks.
+    const uint32_t* chunk_ids;
+    uint32_t chunk_cells;
 };
 void launch_cell_reduce(hipStream_t s, const CellArgs& a, BuildCounters* c);
 

@@ -111,3 +111,25 @@ def test_cells_on_gpu(gpu, oracle):
     run_plain(gpu, oracle)
     run_below_top(gpu, oracle, [(10, 1_100_000, 1), (11, 1_100_000, 1), (12, 4_300_000, 1), (12, 1_100_000, 1)])
     run_batched(gpu, oracle)
+
+
+def run_sparse(m, oracle):
+    """Batched builds most of whose chunks are empty sort only the others: half
+    of the chunks (the most that takes it), one, the first and the last."""
+    rng = np.random.default_rng(0xCE14)
+    for depth, num, live in ((7, 8, (0, 3, 5, 7)), (9, 64, (63,)), (8, 64, (0, 17, 18, 63)), (9, 8, (2,)),
+                             (7, 8, (0, 1, 2, 3, 4))):
+        chunks = [np.empty(0, dtype=np.uint64) for _ in range(num)]
+        last = (1 << (3 * depth - 18)) - 1
+        for i in live:
+            chunks[i] = cell_keys(rng, depth, [0, last, last // 2], [700, 1, 4100])
+        batched(m, oracle, chunks, depth)
+
+
+def test_sparse_chunks_on_the_cpu_emulator(emu, oracle):
+    run_sparse(emu, oracle)
+
+
+@pytest.mark.gpu
+def test_sparse_chunks_on_gpu(gpu, oracle):
+    run_sparse(gpu, oracle)

@@ -631,6 +631,8 @@ struct BatchInfo {
     const uint64_t* d_offsets = nullptr;
 };
 
+constexpr uint64_t kSketchMinLeaves = 1ull << 15;  // 64K slots of 8 bytes at load 1/2
+
 // Returned by build() when a table sized from an estimate overflowed; the
 // caller repeats the build with bound-sized tables.
 constexpr int kRetryWithBounds = -100;
@@ -967,8 +969,9 @@ int build(svdag_context* ctx, const K* d_keys, uint64_t n, int depth, svdag_dag*
     uint32_t* ls1 = reinterpret_cast<uint32_t*>(A + L.list_slots[1]);
     // The leaf table is sized from a distinct-count estimate of the masks (or,
     // on a retry, from the leaf positions, an upper bound).
+    // Small tables stay in the caches anyway: two launches less.
     const uint64_t* leaf_size = &c->leaf_positions;
-    if (estimate) {
+    if (estimate && L.leaf_bound > kSketchMinLeaves) {
         uint32_t* regs = reinterpret_cast<uint32_t*>(A + L.sketch);
         launch_sketch(st, lp_mask, &c->leaf_positions, regs, L.leaf_bound);
         launch_sketch_estimate(st, regs, &c->leaf_positions, &c->leaf_estimate);

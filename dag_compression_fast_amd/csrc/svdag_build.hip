@@ -1169,6 +1169,49 @@ __global__ __launch_bounds__(kOrderSortThreads) void k_order_sort(const uint64_t
     }
 }
 
+// The whole order of at most kOrderCap masks in one workgroup: occupied slots
+// gathered into LDS in any order, sorted, and each slot's rank found by a search.
+// Four launches less three: 1000 keys, whose build is bound by launches (6 us
+// each), 199 -> 163 us with the sketch's two and the layout's count left out too.
+constexpr uint32_t kOrderSmallSlots = 8 * kOrderCap;
+
+__global__ __launch_bounds__(kSampleThreads) void k_order_small(const uint64_t* __restrict__ table_keys,
+                                                                const uint32_t* __restrict__ table_log2,
+                                                                uint64_t* __restrict__ out,
+                                                                uint32_t* __restrict__ rank_of_slot,
+                                                                uint64_t* __restrict__ count)
+{
+    __shared__ uint64_t s_key[kOrderCap];
+    __shared__ uint32_t s_n;
+    const uint32_t slots = 1u << *table_log2;
+    if (threadIdx.x == 0) s_n = 0;
+    __syncthreads();
+    for (uint32_t i = threadIdx.x; i < slots; i += kSampleThreads) {
+        const uint64_t k = table_keys[i];
+        if (k) {
+            const uint32_t at = atomicAdd(&s_n, 1u);
+            if (at < kOrderCap) s_key[at] = k;  // always: the caller's bound
+        }
+    }
+    __syncthreads();
+    const uint32_t n = min(s_n, kOrderCap);
+    block_merge_sort<kSampleThreads, int(kOrderCap) / kSampleThreads>(s_key, n);
+    for (uint32_t i = threadIdx.x; i < n; i += kSampleThreads) out[i] = s_key[i];
+    for (uint32_t i = threadIdx.x; i < slots; i += kSampleThreads) {
+        const uint64_t k = table_keys[i];
+        if (k) {
+            uint32_t lo = 0, hi = n;
+            while (lo < hi) {
+                const uint32_t mid = (lo + hi) / 2;
+                if (s_key[mid] < k) lo = mid + 1;
+                else hi = mid;
+            }
+            rank_of_slot[i] = lo;
+        }
+    }
+    if (threadIdx.x == 0) *count = n;
+}
+
 // Ordered-table probe: home = top lg bits of the hash, linear probing forward
 // into an overflow tail (no wrap), so every key sits at or after its home slot.
 // `won` tells whether this call placed the key.
@@ -2298,6 +2341,11 @@ void launch_leaf_insert(hipStream_t s, const uint64_t* lp_mask, const uint64_t* 
 void launch_leaf_order(hipStream_t s, const LeafOrderArgs& a, uint64_t slot_bound, uint64_t leaf_bound)
 {
     TimedLaunch t(kKLeafOrder, s);
+    if (leaf_bound <= kOrderCap && slot_bound <= kOrderSmallSlots) {
+        hipLaunchKernelGGL(k_order_small, dim3(1), dim3(kSampleThreads), 0, s, a.table_keys, a.table_log2, a.out,
+                           a.rank_of_slot, a.count);
+        return;
+    }
     const int grid = grid_for((slot_bound + kOrderTile - 1) / kOrderTile, 4);
     hipLaunchKernelGGL(k_leaf_sample, dim3(1), dim3(kSampleThreads), 0, s, a.table_keys, a.table_log2, a.split);
     hipLaunchKernelGGL(k_order_count, dim3(grid), dim3(kThreads), 0, s, a.table_keys, a.table_log2, a.split, a.totals);
@@ -2441,7 +2489,7 @@ void launch_final(hipStream_t s, const FinalArgs& a)
     if (a.total_nodes) {
         const uint64_t tiles = (a.total_nodes + kFinalTile - 1) / kFinalTile;
         const uint32_t parts = uint32_t(std::min<uint64_t>(kMaxParts, resident_grid(k_final_positions, kThreads, tiles)));
-        {
+        if (parts > 1) {  // one part starts at 0
             TimedLaunch t(kKFinalCount, s);
             hipLaunchKernelGGL(k_final_count, dim3(parts), dim3(kThreads), 0, s, a);
         }

@@ -1,7 +1,8 @@
 """Level builds and extracts over parts of tiles (a count per part, summed by
 the workgroups), and the merge whose top levels take one workgroup (up to 8^4
 chunks) or the hashed levels (8^5).  Leaf counts sit at the edges of a tile
-(1024 children), with one and with eight leaves a parent; inputs that leave all
+(512 children), of the leaf order in one workgroup (4096 keys) and of the
+estimated table (32768), with one and with eight leaves a parent; inputs that leave all
 but one part empty and levels of one node are among them."""
 import numpy as np
 import pytest
@@ -21,7 +22,7 @@ def check(m, oracle, keys, depth):
 
 def run_builds(m, oracle):
     rng = np.random.default_rng(0x9A77)
-    for leaves in (1, 8, 1023, 1024, 1025, 2047, 2049, 4097, 16385):
+    for leaves in (1, 8, 511, 512, 513, 1023, 1024, 1025, 2047, 2049, 4095, 4096, 4097, 16385, 32769):
         # Consecutive leaves (8 a parent), and one leaf a parent.
         for step, depth in ((1, 8), (8, 9), (64, 9)):
             codes = np.arange(leaves, dtype=np.uint64) * np.uint64(step) + np.uint64(step - 1)

@@ -37,9 +37,10 @@ SPACE = {
 }
 
 # Batched builds sorted inside each chunk: the first pass's digit width of that
-# sort, and the table load factor.
+# sort (0: the library's choice, one pass over 64^3 cells where they pay), and
+# the table load factor.
 SEG_SPACE = {
-    "seg_first_bits": (4, 5, 6, 7, 8),
+    "seg_first_bits": (0, 4, 5, 6, 7),
     "table_load_shift": (1, 2, 3),
 }
 
@@ -74,7 +75,7 @@ def space_for(chunk_depth=None):
 
 def default_setting(space, chunk_depth=None):
     """The library's default setting expressed in `space`'s options (the
-    segmented sort's default split is half its bits)."""
+    segmented sort's default split of two passes is half its bits)."""
     out = {}
     for name in space:
         v = DEFAULTS[name]

@@ -422,15 +422,18 @@ __global__ __launch_bounds__(kThreads) void k_leaf_compact(const uint64_t* __res
 // ---------------------------------------------------------------------------
 // Leaf reduce of keys grouped by 64^3 cell (code >> kCellShift) with known cell
 // starts: one workgroup ORs a cell's keys into a table of its 4096 leaves in
-// LDS (32 KB: four workgroups of 8 waves per CU) and writes the leaves present
+// LDS (32 KB; three workgroups of 8 waves per CU) and writes the leaves present
 // in order.  Against the 32^3 groups of k_leaf_reduce the sort orders 3 bits
 // less (one pass instead of two up to depth 9 in a chunk), no wave looks for
 // group starts, and the table words are 32 bits wide (64-bit LDS atomics take
 // twice the bank cycles).  Bound by the keys' read and the LDS atomics where
-// cells are full (512^3 noise, 67M keys: 304 -> 62 us, with 268 us of sort
-// saved), by the two barriers and the table pass a cell where they are not
-// (512 chunks, 645 keys a cell: 364 -> 415 us, with 640 us of sort saved; 690
-// before the next cell's keys were loaded ahead).
+// cells are full (512^3 noise, 67M keys: 304 -> 56 us, with 268 us of sort
+// saved; 2048^3 triangles 153 -> 125), by the two barriers and the table pass a
+// cell where they are not (512 chunks, 645 keys a cell: 364 -> 395 us, with 640
+// us of sort saved; 690 before the next cell's keys were loaded ahead).  Full
+// rounds of keys go without their guards (138 -> 125 us of the triangles);
+// registers for a fourth workgroup gain 26 us of the chunks and lose 18 of
+// 1024^3 noise (540).
 // A cell of k keys emits at most min(k, 4096) leaves, so a run of cells writes
 // into its own keys' positions of the regions; codes there are 32-bit, local to
 // the run.
@@ -489,6 +492,12 @@ __global__ __launch_bounds__(kCellThreads) void k_cell_reduce(CellArgs a, const 
     // The keys of one round, from p on; rows past the cell's end stay unread.
     uint32_t k[kCellKeys];
     auto load = [&](uint32_t p, uint32_t left) {
+        if (left >= uint32_t(kCellThreads * kCellKeys)) {
+#pragma unroll
+            for (int i = 0; i < kCellKeys; ++i)
+                k[i] = __builtin_nontemporal_load(a.keys + p + uint32_t(i) * kCellThreads + threadIdx.x);
+            return;
+        }
 #pragma unroll
         for (int i = 0; i < kCellKeys; ++i)
             if (uint32_t(i) * kCellThreads < left)
@@ -504,10 +513,15 @@ __global__ __launch_bounds__(kCellThreads) void k_cell_reduce(CellArgs a, const 
         const uint32_t base = uint32_t(__builtin_amdgcn_readlane(int(bound), 0));
         for (uint32_t p = s;;) {
             const uint32_t left = e - p;
+            auto add = [&](uint32_t key) { atomicOr(&tab[(key >> 5) & (2 * kCellLeaves - 1)], 1u << (key & 31u)); };
+            if (left >= uint32_t(kCellThreads * kCellKeys)) {
 #pragma unroll
-            for (int i = 0; i < kCellKeys; ++i)
-                if (uint32_t(i) * kCellThreads + threadIdx.x < left)
-                    atomicOr(&tab[(k[i] >> 5) & (2 * kCellLeaves - 1)], 1u << (k[i] & 31u));
+                for (int i = 0; i < kCellKeys; ++i) add(k[i]);
+            } else {
+#pragma unroll
+                for (int i = 0; i < kCellKeys; ++i)
+                    if (uint32_t(i) * kCellThreads < left && uint32_t(i) * kCellThreads + threadIdx.x < left) add(k[i]);
+            }
             if (left <= uint32_t(kCellThreads * kCellKeys)) break;
             p += kCellThreads * kCellKeys;
             load(p, e - p);

@@ -92,13 +92,19 @@ typedef enum svdag_option {
                                          longer stages its keys */
     SVDAG_OPT_SEG_FIRST_BITS = 10,    /* batched builds that sort inside each chunk (chunk
                                          depth <= 9): digit width of that sort's first pass,
-                                         0 = half the chunk-local bits (default); clamped so
-                                         that neither pass is wider than 9 bits */
+                                         clamped so that neither pass is wider than 9 bits;
+                                         0 (default): one pass that groups the keys by 64^3
+                                         voxels where that pays (chunk depths 7 to 9), else
+                                         half the bits */
     SVDAG_OPT_TOP_DIGIT_FIRST = 11    /* plain builds of 64-bit keys: sort the top digit first
                                          and the rest inside each top-digit bucket as 32-bit
-                                         keys; 0 = never, 1 = from 2^20 keys on (default),
+                                         keys.  0 = never, 1 = from 2^20 keys on (default),
                                          2 = always.  Used where the bits below the top digit
-                                         fit 32 and at most 12 of them need sorting. */
+                                         fit 32 and at most 12 of them need sorting.  With 1
+                                         the keys are grouped by 64^3 voxels where that pays
+                                         (one pass at depths 7 to 9, 32-bit keys too).
+                                         svdag_sort_keys: the same order of digits for 64-bit
+                                         keys from 2^22 keys on (1). */
 } svdag_option;
 
 /* --- context ------------------------------------------------------------ */

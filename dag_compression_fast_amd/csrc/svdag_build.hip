@@ -422,18 +422,18 @@ __global__ __launch_bounds__(kThreads) void k_leaf_compact(const uint64_t* __res
 // ---------------------------------------------------------------------------
 // Leaf reduce of keys grouped by 64^3 cell (code >> kCellShift) with known cell
 // starts: one workgroup ORs a cell's keys into a table of its 4096 leaves in
-// LDS (32 KB; three workgroups of 8 waves per CU) and writes the leaves present
+// LDS (32 KB; four workgroups of 8 waves per CU) and writes the leaves present
 // in order.  Against the 32^3 groups of k_leaf_reduce the sort orders 3 bits
 // less (one pass instead of two up to depth 9 in a chunk), no wave looks for
 // group starts, and the table words are 32 bits wide (64-bit LDS atomics take
 // twice the bank cycles).  Bound by the keys' read and the LDS atomics where
 // cells are full (512^3 noise, 67M keys: 304 -> 56 us, with 268 us of sort
 // saved; 2048^3 triangles 153 -> 125), by the two barriers and the table pass a
-// cell where they are not (512 chunks, 645 keys a cell: 364 -> 395 us, with 640
+// cell where they are not (512 chunks, 645 keys a cell: 364 -> 374 us, with 640
 // us of sort saved; 690 before the next cell's keys were loaded ahead).  Full
 // rounds of keys go without their guards (138 -> 125 us of the triangles);
-// registers for a fourth workgroup gain 26 us of the chunks and lose 18 of
-// 1024^3 noise (540).
+// registers are held to 64 for the fourth workgroup per CU, which gains 26 us of
+// the chunks and loses 18 of 1024^3 noise (540).
 // A cell of k keys emits at most min(k, 4096) leaves, so a run of cells writes
 // into its own keys' positions of the regions; codes there are 32-bit, local to
 // the run.
@@ -444,7 +444,7 @@ constexpr int kCellKeys = 8;  // keys per thread in flight
 constexpr int kCellRows = int(kCellLeaves) / kCellThreads;
 static_assert(kCellRows * kCellThreads == int(kCellLeaves) && kMaxRunCells < kWave, "rows and starts per lane");
 
-__global__ __launch_bounds__(kCellThreads) void k_cell_reduce(CellArgs a, const uint64_t* __restrict__ n_ptr)
+__global__ __launch_bounds__(kCellThreads, 8) void k_cell_reduce(CellArgs a, const uint64_t* __restrict__ n_ptr)
 {
     __shared__ uint64_t s_tab[kCellLeaves];
     __shared__ uint32_t s_cnt[kCellWaves];

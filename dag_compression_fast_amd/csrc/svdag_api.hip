@@ -705,6 +705,7 @@ struct BatchLayout {
     uint64_t cells = 0;  // the sort's one pass groups the keys by 64^3 cell
     uint64_t chunks = 0;  // chunks sorted: all, or (compact) those that hold keys
     bool compact = false;
+    uint64_t count_words = 0;  // u32 words at seg_counts
 };
 
 BatchLayout plan_batch(const BuildLayout& L, uint64_t n, const BatchInfo* batch, uint32_t first_bits)
@@ -749,7 +750,8 @@ BatchLayout plan_batch(const BuildLayout& L, uint64_t n, const BatchInfo* batch,
         const uint64_t tb = seg_tile_bound(n, batch->num_chunks);
         B.seg_tiles = c.take(sizeof(SegTile) * tb);
         B.seg_ct = c.take(4 * (batch->num_chunks + 1));
-        B.seg_counts = c.take(4 * (tb << kMaxSegDigitBits));
+        B.count_words = tb << kMaxSegDigitBits;
+        B.seg_counts = c.take(4 * B.count_words);
         B.seg_totals = c.take(4 * (batch->num_chunks << kMaxSegDigitBits));
         B.seg_starts = c.take(4 * (batch->num_chunks << kMaxSegDigitBits));
         B.seg_ntiles = c.take(8);
@@ -945,7 +947,12 @@ int build(svdag_context* ctx, const K* d_keys, uint64_t n, int depth, svdag_dag*
         ca.run_cells = cell_run_length(ca.cells, sort_count_words(n), B.compact ? ca.chunk_cells : kMaxRunCells);
         ca.reg_mask = reg_code;
         ca.reg_code = reinterpret_cast<uint32_t*>(reg_mask);
-        ca.run_counts = sort_counts;  // free once the sort is done
+        // The sort's counts are free once it is done.  A batched build's hold at
+        // least a word per cell (2^kMaxSegDigitBits per chunk, which has no more
+        // cells); a plain build's runs number at most 256 or n / 512.
+        ca.run_counts = batch ? reinterpret_cast<uint32_t*>(A + B.seg_counts) : sort_counts;
+        if (cell_runs(ca.cells, ca.run_cells) > (batch ? B.count_words : sort_count_words(n)))
+            return fail(set_error(SVDAG_ERR_INTERNAL, "cell runs exceed their counts"));
         ca.lp_code = lp_code;
         ca.lp_mask = lp_mask;
         ca.lp_capacity = L.leaf_bound;

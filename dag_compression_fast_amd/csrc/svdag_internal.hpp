@@ -306,7 +306,8 @@ void launch_leaf_reduce(hipStream_t s, const K* sorted, BuildCounters* c, uint32
 constexpr uint32_t kCellShift = 18;
 constexpr uint32_t kCellLeaves = 1u << (kCellShift - 6);
 constexpr uint32_t kMaxRunCells = 32;
-// A power of two, at most `most`.
+// Cells per run: a power of two, at most `most`; the shortest with at most
+// max_runs (and 16384) runs, if `most` allows it.
 inline uint32_t cell_run_length(uint64_t cells, uint64_t max_runs, uint64_t most)
 {
     const uint64_t runs = std::min<uint64_t>(16384, max_runs), top = std::min<uint64_t>(kMaxRunCells, most);

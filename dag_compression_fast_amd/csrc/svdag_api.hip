@@ -21,6 +21,7 @@
 #include <cstring>
 #include <map>
 #include <mutex>
+#include <new>
 #include <string>
 #include <thread>
 #include <unordered_map>
@@ -137,6 +138,9 @@ struct svdag_context {
     uint64_t arena_cap = 0;
     // Source table of the last gathered build (kept until its copy is done).
     std::vector<GatherSource> gather_src;
+    // Likewise: offsets, then (32-bit) indices of the chunks with keys of the
+    // last batched build that sorted only those.
+    std::vector<uint64_t> live_chunks;
     // Result blocks (DAG storage, final words): reused across calls, returned
     // by svdag_free_dag / svdag_free_words, released by svdag_free_all.
     std::multimap<uint64_t, void*> free_blocks;
@@ -810,10 +814,8 @@ int build(svdag_context* ctx, const K* d_keys, uint64_t n, int depth, svdag_dag*
     char* O = static_cast<char*>(storage);
     const bool capture = fixed && fixed->captured;
     bool forked = false;  // work is in flight on the side stream
-    std::vector<uint64_t> live_chunks;  // offsets, then (32-bit) indices; read by a copy until the stream drains
     auto fail = [&](int code) {
         if (forked) (void)hipStreamSynchronize(ctx->side);
-        if (!live_chunks.empty()) (void)hipStreamSynchronize(st);
         if (!fixed) device_release(ctx, storage);
         out->storage = nullptr;
         return code;
@@ -843,7 +845,13 @@ int build(svdag_context* ctx, const K* d_keys, uint64_t n, int depth, svdag_dag*
             uint64_t words = batch->num_chunks + 1;
             if (B.compact) {
                 words = B.chunks + 1 + (B.chunks + 1) / 2;
-                live_chunks.resize(words);
+                std::vector<uint64_t>& live_chunks = ctx->live_chunks;
+                try {
+                    live_chunks.resize(words);
+                } catch (const std::bad_alloc&) {
+                    return fail(set_error(SVDAG_ERR_MEMORY, "cannot allocate %llu bytes of host memory",
+                                          (unsigned long long)(8 * words)));
+                }
                 uint32_t* const ids = reinterpret_cast<uint32_t*>(live_chunks.data() + B.chunks + 1);
                 uint64_t j = 0;
                 for (uint64_t i = 0; i < batch->num_chunks; ++i)

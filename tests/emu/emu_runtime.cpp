@@ -283,6 +283,13 @@ int g_schedule = 0;
 // runtime reports an invalid configuration) instead of running the kernel.
 int g_sticky_error = 0;
 uint64_t g_launches = 0, g_bad_launches = 0;
+// Failures on request (tests of error paths): streams that never report their
+// work done, the n-th next launch or copy refused (0: none), and how often a
+// caller waited for a stream without a bound.
+int g_stalled = 0;
+int g_fail_launch = 0, g_fail_copy = 0;
+uint64_t g_stream_waits = 0;
+bool due(int& countdown) { return countdown > 0 && --countdown == 0; }
 
 bool valid_config(dim3 grid, dim3 block)
 {
@@ -327,6 +334,10 @@ void run_launch(dim3 grid, dim3 block, std::function<void()>& body)
         std::abort();
     }
     ++g_launches;
+    if (due(g_fail_launch)) {
+        g_sticky_error = 9;  // hipErrorInvalidConfiguration
+        return;
+    }
     if (!valid_config(grid, block)) {
         std::fprintf(stderr, "emu: invalid launch configuration grid (%u, %u, %u) block (%u, %u, %u)\n", grid.x,
                      grid.y, grid.z, block.x, block.y, block.z);
@@ -386,6 +397,7 @@ hipError_t hipHostFree(void* p) { return hipFree(p); }
 hipError_t hipMemcpy(void* d, const void* s, size_t n, int) { if (n) std::memmove(d, s, n); return hipSuccess; }
 hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, int k, hipStream_t)
 {
+    if (emu::due(emu::g_fail_copy)) return hipErrorInvalidValue;
     if (emu::g_capture) {
         emu::GraphOp op;
         op.dst = d;
@@ -433,7 +445,11 @@ hipError_t hipGraphDestroy(hipGraph_t g)
     return hipSuccess;
 }
 hipError_t hipMemsetAsync(void* d, int v, size_t n, hipStream_t) { std::memset(d, v, n); return hipSuccess; }
-hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
+hipError_t hipStreamSynchronize(hipStream_t)
+{
+    ++emu::g_stream_waits;
+    return hipSuccess;
+}
 hipError_t hipDeviceSynchronize() { return hipSuccess; }
 hipError_t hipGetLastError()
 {
@@ -443,6 +459,10 @@ hipError_t hipGetLastError()
 }
 hipError_t hipPeekAtLastError() { return emu::g_sticky_error; }
 void emu_set_schedule(int mode) { emu::g_schedule = mode; }
+void emu_set_stalled(int on) { emu::g_stalled = on; }
+void emu_fail_launch(int nth) { emu::g_fail_launch = nth; }
+void emu_fail_copy(int nth) { emu::g_fail_copy = nth; }
+uint64_t emu_stream_waits() { return emu::g_stream_waits; }
 uint64_t emu_launch_count() { return emu::g_launches; }
 uint64_t emu_bad_launch_count() { return emu::g_bad_launches; }
 const char* hipGetErrorString(hipError_t) { return "emulator error"; }
@@ -461,8 +481,8 @@ hipError_t hipMemPoolTrimTo(hipMemPool_t, size_t) { return hipSuccess; }
 hipError_t hipEventCreate(void** e) { *e = std::malloc(8); return hipSuccess; }
 hipError_t hipEventCreateWithFlags(void** e, unsigned) { *e = std::malloc(8); return hipSuccess; }
 hipError_t hipEventRecord(void*, void*) { return hipSuccess; }
-hipError_t hipEventQuery(void*) { return hipSuccess; }
-hipError_t hipStreamQuery(void*) { return hipSuccess; }
+hipError_t hipEventQuery(void*) { return emu::g_stalled ? hipError_t(hipErrorNotReady) : hipError_t(hipSuccess); }
+hipError_t hipStreamQuery(void*) { return emu::g_stalled ? hipError_t(hipErrorNotReady) : hipError_t(hipSuccess); }
 hipError_t hipEventSynchronize(void*) { return hipSuccess; }
 hipError_t hipEventElapsedTime(float* ms, void*, void*) { *ms = 0; return hipSuccess; }
 hipError_t hipEventDestroy(void* e) { std::free(e); return hipSuccess; }

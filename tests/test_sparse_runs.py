@@ -60,9 +60,9 @@ def emu():
     svd = emu_ctypes.use_emulator()
     yield svd, ctypes.CDLL(emu_ctypes.EMU_LIB)
     from dag_compression_fast_amd import _lib
+    svd._default = None  # the emulator's context goes before its library
     _lib._lib = None
     _lib._hip = None
-    svd._default = None
 
 
 def test_sparse_runs_on_the_cpu_emulator(emu, oracle):

@@ -1878,6 +1878,7 @@ int svdag_dag_to_host(svdag_context* ctx, const svdag_dag* dag, svdag_dag* out)
     // A device DAG leaves in one kernel; arrays off a 16-byte boundary (not this
     // library's own) are copies of their own.
     CopyOut co{};
+    hipError_t e = hipSuccess;
     const bool packed = kind == hipMemcpyDeviceToHost;
     char* p = mem;
     auto copy = [&](void* src, uint64_t bytes) -> void* {
@@ -1885,8 +1886,8 @@ int svdag_dag_to_host(svdag_context* ctx, const svdag_dag* dag, svdag_dag* out)
         if (bytes && packed && reinterpret_cast<uintptr_t>(src) % 16 == 0) {
             co.seg[co.num++] = {src, dst, bytes};
             co.pieces += uint32_t((bytes + kCopyPiece - 1) / kCopyPiece);
-        } else if (bytes) {
-            (void)hipMemcpyAsync(dst, src, bytes, kind, ctx->stream);
+        } else if (bytes && e == hipSuccess) {
+            e = hipMemcpyAsync(dst, src, bytes, kind, ctx->stream);
         }
         p += (bytes + 15) / 16 * 16;
         return dst;
@@ -1898,11 +1899,16 @@ int svdag_dag_to_host(svdag_context* ctx, const svdag_dag* dag, svdag_dag* out)
         out->levels[l].masks = static_cast<uint8_t*>(copy(dag->levels[l].masks, q));
     }
     out->leaves = static_cast<uint64_t*>(copy(dag->leaves, 8 * dag->num_leaves));
-    launch_copy_out(ctx->stream, co);
-    const hipError_t e = hipStreamSynchronize(ctx->stream);
+    if (e == hipSuccess) {
+        launch_copy_out(ctx->stream, co);
+        e = hipGetLastError();
+    }
+    // Also after a refused copy or launch: the others may be writing the block.
+    const hipError_t drained = hipStreamSynchronize(ctx->stream);
+    if (e == hipSuccess) e = drained;
     if (e != hipSuccess) {
         host_release(mem);
-        out->storage = nullptr;
+        empty_dag(out, out->num_levels, SVDAG_HOST);
         return set_error(SVDAG_ERR_HIP, "copy to host failed: %s", hipGetErrorString(e));
     }
     return 0;

@@ -1875,15 +1875,41 @@ int svdag_dag_to_host(svdag_context* ctx, const svdag_dag* dag, svdag_dag* out)
     out->location = SVDAG_HOST;
     out->storage = mem;
     const hipMemcpyKind kind = dag->location == SVDAG_DEVICE ? hipMemcpyDeviceToHost : hipMemcpyHostToHost;
-    // A device DAG leaves in one kernel; arrays off a 16-byte boundary (not this
-    // library's own) are copies of their own.
+    // A device DAG leaves in one kernel.  Arrays that it cannot read (another
+    // device's: the caller's DAG may be from any context) or that lie off a
+    // 16-byte boundary are copies of their own; an array that the DAG does not
+    // have stays null.  [known, known_end): memory of this device, the DAG's own
+    // block or the allocation last asked about.
+    uintptr_t known = 0, known_end = 0;
+    if (const auto own = ctx->block_size.find(dag->storage); own != ctx->block_size.end()) {
+        known = reinterpret_cast<uintptr_t>(own->first);
+        known_end = known + own->second;
+    }
+    auto readable = [&](void* src, uint64_t bytes) {
+        const uintptr_t at = reinterpret_cast<uintptr_t>(src);
+        if (at % 16 != 0) return false;
+        if (at < known || at + bytes > known_end) {
+            hipPointerAttribute_t info{};
+            hipDeviceptr_t base = nullptr;
+            size_t size = 0;
+            if (hipPointerGetAttributes(&info, src) != hipSuccess || info.type != hipMemoryTypeDevice ||
+                info.device != ctx->device || hipMemGetAddressRange(&base, &size, src) != hipSuccess) {
+                (void)hipGetLastError();
+                return false;
+            }
+            known = reinterpret_cast<uintptr_t>(base);
+            known_end = known + size;
+        }
+        return at >= known && at + bytes <= known_end;
+    };
     CopyOut co{};
     hipError_t e = hipSuccess;
     const bool packed = kind == hipMemcpyDeviceToHost;
     char* p = mem;
     auto copy = [&](void* src, uint64_t bytes) -> void* {
         void* dst = p;
-        if (bytes && packed && reinterpret_cast<uintptr_t>(src) % 16 == 0) {
+        if (!src) return nullptr;
+        if (bytes && packed && readable(src, bytes)) {
             co.seg[co.num++] = {src, dst, bytes};
             co.pieces += uint32_t((bytes + kCopyPiece - 1) / kCopyPiece);
         } else if (bytes && e == hipSuccess) {

@@ -13,6 +13,7 @@
 #include <chrono>
 #include <cstdio>
 #include <cstdlib>
+#include <map>
 #include <mutex>
 #include <thread>
 #include <unistd.h>
@@ -382,8 +383,56 @@ static void* emu_alloc(size_t n)
     return p;
 }
 
-hipError_t hipMalloc(void** p, size_t n) { *p = emu_alloc(n); return *p ? hipSuccess : hipErrorOutOfMemory; }
-hipError_t hipFree(void* p) { std::free(p); return hipSuccess; }
+// Allocations (address -> size) and the device all of them claim to be on.
+static std::mutex g_alloc_mutex;
+static std::map<uintptr_t, size_t> g_allocs;
+static int g_pointer_device = 0;
+
+static bool find_alloc(const void* p, uintptr_t& base, size_t& size)
+{
+    std::lock_guard<std::mutex> lock(g_alloc_mutex);
+    const uintptr_t at = reinterpret_cast<uintptr_t>(p);
+    auto it = g_allocs.upper_bound(at);
+    if (it == g_allocs.begin()) return false;
+    --it;
+    base = it->first;
+    size = it->second;
+    return at < base + size;
+}
+
+hipError_t hipMalloc(void** p, size_t n)
+{
+    *p = emu_alloc(n);
+    if (!*p) return hipErrorOutOfMemory;
+    std::lock_guard<std::mutex> lock(g_alloc_mutex);
+    g_allocs[reinterpret_cast<uintptr_t>(*p)] = n;
+    return hipSuccess;
+}
+hipError_t hipFree(void* p)
+{
+    {
+        std::lock_guard<std::mutex> lock(g_alloc_mutex);
+        g_allocs.erase(reinterpret_cast<uintptr_t>(p));
+    }
+    std::free(p);
+    return hipSuccess;
+}
+hipError_t hipPointerGetAttributes(hipPointerAttribute_t* a, const void* p)
+{
+    uintptr_t base;
+    size_t size;
+    if (!find_alloc(p, base, size)) return hipErrorInvalidValue;
+    *a = hipPointerAttribute_t{hipMemoryTypeDevice, g_pointer_device};
+    return hipSuccess;
+}
+hipError_t hipMemGetAddressRange(hipDeviceptr_t* base, size_t* size, hipDeviceptr_t p)
+{
+    uintptr_t at;
+    if (!find_alloc(p, at, *size)) return hipErrorInvalidValue;
+    *base = reinterpret_cast<void*>(at);
+    return hipSuccess;
+}
+void emu_set_pointer_device(int device) { g_pointer_device = device; }
 // Device globals are host globals here: the symbol is its own address.
 hipError_t hipGetSymbolAddress(void** p, const void* symbol)
 {

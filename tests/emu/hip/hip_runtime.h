@@ -160,11 +160,16 @@ enum hipMemcpyKind { hipMemcpyHostToHost = 0, hipMemcpyHostToDevice = 1, hipMemc
                      hipMemcpyDeviceToDevice = 3, hipMemcpyDefault = 4 };
 enum { hipMemPoolAttrReleaseThreshold = 4 };
 enum { hipHostMallocDefault = 0 };
+enum hipMemoryType { hipMemoryTypeUnregistered = 0, hipMemoryTypeHost = 1, hipMemoryTypeDevice = 2 };
+struct hipPointerAttribute_t { hipMemoryType type; int device; };
+typedef void* hipDeviceptr_t;
 struct hipDeviceProp_t { int multiProcessorCount; char name[256]; };
 
 extern "C" {
 hipError_t hipMalloc(void** p, size_t n);
 hipError_t hipFree(void* p);
+hipError_t hipPointerGetAttributes(hipPointerAttribute_t* a, const void* p);
+hipError_t hipMemGetAddressRange(hipDeviceptr_t* base, size_t* size, hipDeviceptr_t p);
 hipError_t hipGetSymbolAddress(void** p, const void* symbol);
 hipError_t hipMallocAsync(void** p, size_t n, hipStream_t s);
 hipError_t hipFreeAsync(void* p, hipStream_t s);

@@ -1,6 +1,8 @@
 """svdag_dag_to_host reports what it could not copy: a refused kernel launch or
-copy is an error, and the result holds nothing then.  On the CPU emulator,
-which refuses a chosen launch or copy."""
+copy is an error, and the result holds nothing then.  Its kernel reads memory of
+the context's own device only, and an array that the DAG does not have stays
+null.  On the CPU emulator, which refuses a chosen launch or copy and counts
+launches."""
 import ctypes
 
 import numpy as np
@@ -78,4 +80,43 @@ def test_a_refused_copy_is_an_error(emu):
     assert rc == 0
     got = svd.Dag(out, dag.ctx)
     assert np.array_equal(got.to_numpy()["leaves"], dag.to_numpy()["leaves"])
+    got.free()
+
+
+def test_memory_of_another_device_is_not_read_by_the_kernel(emu):
+    svd, lib = emu
+    other = svd.Context()
+    try:
+        dag = svd.create_dag(np.arange(0, 200000, 37, dtype=np.uint64), 6, ctx=other)  # not in the default context's pool
+        for device, kernels in ((0, 1), (1, 0)):
+            lib.emu_set_pointer_device(device)
+            before = lib.emu_launch_count()
+            rc, out = to_host(svd, dag.raw)
+            assert rc == 0 and lib.emu_launch_count() - before == kernels
+            got, want = svd.Dag(out, svd.default_context()), dag.to_numpy()
+            for a, b in zip(got.to_numpy()["levels"], want["levels"]):
+                assert all(np.array_equal(a[k], b[k]) for k in b)
+            got.free()
+        dag.free()
+    finally:
+        lib.emu_set_pointer_device(0)
+        other.close()
+
+
+def test_an_array_that_is_not_there_stays_null(emu):
+    svd, _ = emu
+    from dag_compression_fast_amd import _lib
+    dag = a_dag(svd)
+    raw = _lib.SvdagDag.from_buffer_copy(dag.raw)
+    for l in range(raw.num_levels):
+        raw.levels[l].hashes = None
+    rc, out = to_host(svd, raw)
+    assert rc == 0
+    assert all(not out.levels[l].hashes for l in range(out.num_levels))
+    for l in range(out.num_levels):
+        out.levels[l].hashes = out.levels[l].children  # to_numpy reads every array
+    got, want = svd.Dag(out, dag.ctx), dag.to_numpy()
+    assert np.array_equal(got.to_numpy()["leaves"], want["leaves"])
+    for a, b in zip(got.to_numpy()["levels"], want["levels"]):
+        assert np.array_equal(a["masks"], b["masks"]) and np.array_equal(a["children"], b["children"])
     got.free()

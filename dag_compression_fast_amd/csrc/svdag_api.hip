@@ -1904,7 +1904,7 @@ int svdag_dag_to_host(svdag_context* ctx, const svdag_dag* dag, svdag_dag* out)
     };
     CopyOut co{};
     hipError_t e = hipSuccess;
-    const bool packed = kind == hipMemcpyDeviceToHost;
+    const bool packed = kind == hipMemcpyDeviceToHost && total < kCopyOutMaxBytes;
     char* p = mem;
     auto copy = [&](void* src, uint64_t bytes) -> void* {
         void* dst = p;

@@ -574,6 +574,13 @@ void launch_query_voxels(hipStream_t s, const uint32_t* words, uint64_t n_words,
 // length.
 constexpr int kMaxCopySegments = 3 * SVDAG_MAX_LEVELS + 1;
 constexpr uint64_t kCopyPiece = 16384;  // bytes per workgroup step
+// DAGs from this size on leave by the copy engine, array by array: it reaches 57
+// GB/s against the kernel's 53.5 but takes about 7 us more an array (28 arrays,
+// kernel and copies: 126 MB 2337 and 2398 us, 228 MB 4223 and 4190, 314 MB 5860
+// and 5710, 1.76 GB 32.9 and 31.0 ms).  Copies of the large arrays beside a
+// kernel for the others took 2 to 3% less than either, but a few processes in
+// thirty then kept to 31 GB/s.
+constexpr uint64_t kCopyOutMaxBytes = 160ull << 20;
 struct CopyOut {
     int num;
     uint32_t pieces;  // of all segments

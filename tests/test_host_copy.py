@@ -1,8 +1,8 @@
 """svdag_dag_to_host reports what it could not copy: a refused kernel launch or
 copy is an error, and the result holds nothing then.  Its kernel reads memory of
 the context's own device only, and an array that the DAG does not have stays
-null.  On the CPU emulator, which refuses a chosen launch or copy and counts
-launches."""
+null.  DAGs of 160 MiB or more are copied array by array.  On the CPU emulator,
+which refuses a chosen launch or copy and counts launches."""
 import ctypes
 
 import numpy as np
@@ -120,3 +120,20 @@ def test_an_array_that_is_not_there_stays_null(emu):
     for a, b in zip(got.to_numpy()["levels"], want["levels"]):
         assert np.array_equal(a["masks"], b["masks"]) and np.array_equal(a["children"], b["children"])
     got.free()
+
+
+@pytest.mark.parametrize("words, kernels", [((160 << 17) - 9, 1), ((160 << 17) - 8, 0)])
+def test_large_dags_leave_by_the_copy_engine(emu, words, kernels):
+    # Leaves alone, and the 16 + 48 bytes of padding a one-level DAG is given.
+    svd, lib = emu
+    from dag_compression_fast_amd import _lib
+    leaves = svd.DeviceBuffer.from_numpy(np.arange(words, dtype=np.uint64) * np.uint64(0x9E3779B97F4A7C15))
+    raw = _lib.SvdagDag()
+    raw.num_levels, raw.location, raw.num_leaves, raw.leaves = 1, svd.SVDAG_DEVICE, words, leaves.address
+    before = lib.emu_launch_count()
+    rc, out = to_host(svd, raw)
+    assert rc == 0 and lib.emu_launch_count() - before == kernels
+    got = svd.Dag(out, svd.default_context())
+    assert np.array_equal(got.to_numpy()["leaves"], leaves.to_numpy(np.uint64, words))
+    got.free()
+    leaves.free()

@@ -228,13 +228,15 @@ void mark(svdag_context* ctx, const char* name)
     if (hipEventRecord(ctx->marks[ctx->num_marks], ctx->stream) == hipSuccess) ctx->mark_names[ctx->num_marks++] = name;
 }
 
-// Waits for the stream with a deadline instead of blocking without bound; on
-// expiry the error names the first stage whose marker has not completed.
-int finish(svdag_context* ctx, const char* what)
+// Waits until `query` reports success, with a deadline instead of blocking
+// without bound; on expiry the error names the first stage whose marker has not
+// completed.
+template <typename Query>
+int wait_for(svdag_context* ctx, const char* what, Query query)
 {
     const auto start = std::chrono::steady_clock::now();
     for (;;) {
-        const hipError_t e = hipStreamQuery(ctx->stream);
+        const hipError_t e = query();
         if (e == hipSuccess) break;
         if (e != hipErrorNotReady) {
             ctx->num_marks = 0;
@@ -259,6 +261,13 @@ int finish(svdag_context* ctx, const char* what)
         if (waited < 0.05) std::this_thread::yield();
         else std::this_thread::sleep_for(std::chrono::microseconds(200));
     }
+    return 0;
+}
+
+// All of the stream's work.
+int finish(svdag_context* ctx, const char* what)
+{
+    TRY(wait_for(ctx, what, [&] { return hipStreamQuery(ctx->stream); }));
     ctx->num_marks = 0;
     ctx->recorder.resolve(true);
     return 0;
@@ -1471,8 +1480,8 @@ int sort_keys_entry(svdag_context* ctx, const K* d_keys, uint64_t n, int32_t bit
     if constexpr (sizeof(K) == 8) {
         // Top digit first, from three digits on, where the rest fits 32 bits:
         // 32-bit keys in the two halves of the first buffer, the tables in the
-        // second.  A key with bits above the sorted ones (read back after the
-        // histogram) has to keep them, which only the LSD sort does.
+        // second.  Keys with bits above the sorted ones keep them as 64-bit keys
+        // in the first buffer and the output, in turn.
         const uint32_t top_bits = uint32_t(std::min(ctx->radix_bits, kMaxRadixBits));
         const uint32_t top_shift = uint32_t(bits) > top_bits ? uint32_t(bits) - top_bits : 0;
         if (ctx->top_first != kTopFirstNever && plan.passes >= 3 && top_shift <= 32 &&
@@ -1498,13 +1507,31 @@ int sort_keys_entry(svdag_context* ctx, const K* d_keys, uint64_t n, int32_t bit
                 uint32_t* const counts = reinterpret_cast<uint32_t*>(A + o_counts);
                 const uint64_t* const n_ptr = reinterpret_cast<const uint64_t*>(A + o_n);
                 launch_top_histogram(st, d_keys, top_shift, top_bits, n_ptr, n, zero, counts,
-                                     reinterpret_cast<unsigned long long*>(A + o_or));
-                HIP_TRY(hipMemcpyAsync(&ctx->h_counters->key_or, A + o_or, 8, hipMemcpyDeviceToHost, st));
-                TRY(finish(ctx, "sort_keys"));
+                                     reinterpret_cast<unsigned long long*>(A + o_or), bucket_start,
+                                     &ctx->h_counters->key_or);
+                // The plan runs while the host reads the OR.
+                const int marks = ctx->num_marks;
+                mark(ctx, "sort histogram");
+                launch_top_plan(st, top_bits, n_ptr, n, zero, counts, bucket_start, sc);
+                HIP_TRY(hipGetLastError());
+                if (ctx->num_marks > marks)
+                    TRY(wait_for(ctx, "sort_keys", [&] { return hipEventQuery(ctx->marks[marks]); }));
+                else
+                    TRY(finish(ctx, "sort_keys"));
+                uint64_t* const a = reinterpret_cast<uint64_t*>(A + o_a);
+                const bool even = below.passes % 2 == 0;
                 if ((ctx->h_counters->key_or >> bits) == 0) {
-                    uint32_t* const a = reinterpret_cast<uint32_t*>(A + o_a);
-                    launch_top_sort(st, d_keys, a, a + n, d_out, top_shift, top_bits, below, n_ptr, n, zero, counts,
-                                    bucket_start, sc);
+                    uint32_t* const low = reinterpret_cast<uint32_t*>(a);
+                    launch_top_passes<uint32_t>(st, d_keys, low, low + n, d_out, top_shift, top_bits, below, n_ptr, n,
+                                                counts, bucket_start, sc);
+                    HIP_TRY(hipGetLastError());
+                    return finish(ctx, "sort_keys");
+                }
+                // The top pass writes the output where an even number of passes
+                // follows; an input that reaches into it takes the LSD sort.
+                if (!even || d_out + n <= d_keys || d_keys + n <= d_out) {
+                    launch_top_passes<uint64_t>(st, d_keys, even ? d_out : a, even ? a : d_out, d_out, top_shift,
+                                                top_bits, below, n_ptr, n, counts, bucket_start, sc);
                     HIP_TRY(hipGetLastError());
                     return finish(ctx, "sort_keys");
                 }

@@ -195,17 +195,24 @@ int launch_cell_sort(hipStream_t stream, const K* keys_in, uint32_t* keys_out, i
                      const uint64_t* n_ptr, uint64_t n_bound, uint32_t* zero, uint32_t* counts,
                      unsigned long long* key_or, uint32_t* starts);
 
-// Full key sort, top digit first (keys below 2^(top_shift + top_bits), top_shift
-// <= 32): the histogram (also the OR of the keys), then the passes.  below:
-// digits covering [0, top_shift); keys_a and keys_b: n 32-bit keys; the
+// Stable sort of 64-bit keys on bits [0, top_shift + top_bits) (top_shift <=
+// 32), top digit first.  launch_top_histogram: the digit totals (zero), the
+// top digit's tile counts and group starts, and the OR of the keys, also into
+// *or_out (pinned).  launch_top_plan: the tables that the passes need.
+// launch_top_passes: below = digits covering [0, top_shift); KL = uint32_t when
+// no key has a bit above the sorted ones, else uint64_t; first and second: n
+// keys each, used in turn (for uint64_t, second may be keys_out if below.passes
+// is odd, and first if it is even; neither may overlap keys_in then).  The
 // segmented sort's scratch has 2^top_bits chunks and digits of below's widths.
 void launch_top_histogram(hipStream_t stream, const uint64_t* keys_in, uint32_t top_shift, uint32_t top_bits,
                           const uint64_t* n_ptr, uint64_t n, uint32_t* zero, uint32_t* counts,
-                          unsigned long long* key_or);
-void launch_top_sort(hipStream_t stream, const uint64_t* keys_in, uint32_t* keys_a, uint32_t* keys_b,
-                     uint64_t* keys_out, uint32_t top_shift, uint32_t top_bits, const SortPlan& below,
-                     const uint64_t* n_ptr, uint64_t n, uint32_t* zero, uint32_t* counts, uint64_t* bucket_start,
-                     const SegScratch& sc);
+                          unsigned long long* key_or, uint64_t* bucket_start, unsigned long long* or_out);
+void launch_top_plan(hipStream_t stream, uint32_t top_bits, const uint64_t* n_ptr, uint64_t n, const uint32_t* zero,
+                     uint32_t* counts, const uint64_t* bucket_start, const SegScratch& sc);
+template <typename KL>
+void launch_top_passes(hipStream_t stream, const uint64_t* keys_in, KL* first, KL* second, uint64_t* keys_out,
+                       uint32_t top_shift, uint32_t top_bits, const SortPlan& below, const uint64_t* n_ptr, uint64_t n,
+                       uint32_t* counts, const uint64_t* bucket_start, const SegScratch& sc);
 // From how many keys svdag_sort_keys takes it.
 constexpr uint64_t kTopSortMinKeys = 1ull << 22;
 

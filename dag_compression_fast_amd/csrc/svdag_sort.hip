@@ -1232,10 +1232,13 @@ template int launch_segmented_sort<uint32_t>(hipStream_t, const uint32_t*, uint3
 // ---------------------------------------------------------------------------
 namespace {
 
-// starts[d] = keys with a smaller top digit (d < R); starts[R] = n.
+// starts[d] = keys with a smaller top digit (d < R); starts[R] = n.  With
+// key_or, its value also goes to *or_out (pinned host memory).
 __global__ __launch_bounds__(kRadix) void k_digit_starts(const uint32_t* __restrict__ hist, uint32_t R,
                                                          const uint64_t* __restrict__ n_ptr,
-                                                         uint64_t* __restrict__ starts)
+                                                         uint64_t* __restrict__ starts,
+                                                         const unsigned long long* __restrict__ key_or,
+                                                         unsigned long long* __restrict__ or_out)
 {
     __shared__ uint32_t s_scan[kRadix / kWave];
     const uint32_t d = threadIdx.x;
@@ -1243,6 +1246,7 @@ __global__ __launch_bounds__(kRadix) void k_digit_starts(const uint32_t* __restr
     const uint32_t ex = block_exclusive_scan<kRadix>(d < R ? hist[d] : 0u, s_scan, total);
     if (d < R) starts[d] = ex;
     if (d == 0) starts[R] = *n_ptr;
+    if (d == 0 && key_or) *or_out = *key_or;
 }
 
 }  // namespace
@@ -1281,7 +1285,8 @@ int launch_top_digit_sort(hipStream_t stream, const uint64_t* keys_in, uint32_t*
             else
                 hipLaunchKernelGGL(k_sort_scan<kScanThreads>, dim3(R), dim3(kScanThreads), 0, stream, counts, zero,
                                    n_ptr, stride, uint64_t(kSortThreads) * I, nullptr);
-            hipLaunchKernelGGL(k_digit_starts, dim3(1), dim3(kRadix), 0, stream, zero, R, n_ptr, bucket_start);
+            hipLaunchKernelGGL(k_digit_starts, dim3(1), dim3(kRadix), 0, stream, zero, R, n_ptr, bucket_start,
+                               nullptr, nullptr);
         }
         // Without the LDS that holds the 64-bit LSD pass to two workgroups per
         // CU: this pass writes half the bytes and measured faster at four
@@ -1345,16 +1350,27 @@ template int launch_cell_sort<uint32_t>(hipStream_t, const uint32_t*, uint32_t*,
                                         uint32_t*);
 
 // ---------------------------------------------------------------------------
-// Full sort of 64-bit keys below 2^(top_shift + top_bits), top digit first: the
-// top pass leaves 32-bit keys grouped by their top digit, stable segmented LSD
-// passes sort the rest inside each group, and the last one writes the 64-bit
-// keys.  Against an LSD sort of all digits a pass after the first moves 12 bytes
-// a key instead of 24.  The caller has launched launch_top_histogram and knows
-// that no key has a bit above the digit (those would be lost).
+// Full sort of 64-bit keys on bits [0, top_shift + top_bits), top digit first:
+// the top pass groups the keys by their top digit, stable segmented LSD passes
+// sort the rest inside each group, and the last one writes the result.
+//   launch_top_histogram  digit totals and group starts; the OR of the keys,
+//                         also into pinned host memory
+//   launch_top_plan       the tile tables, which either kind of key needs (the
+//                         host reads the OR meanwhile)
+//   launch_top_passes     uint32_t: keys without bits above the sorted ones are
+//                         32-bit keys inside their group, and the last pass puts
+//                         the group back above them; against an LSD sort of all
+//                         digits a pass after the first moves 12 bytes a key
+//                         instead of 24 (100M keys at 33 bits: 1807 us, LSD
+//                         2454).  uint64_t: keys with higher bits keep them, at
+//                         about the LSD sort's cost (100M keys at 33 bits 2466
+//                         and 2609 us, at 19 bits 1829 and 1780; 4.2M at 27 bits
+//                         223 and 216); that sort after this histogram would
+//                         read all keys once more (2803, 1985 and 284 us).
 // ---------------------------------------------------------------------------
 void launch_top_histogram(hipStream_t stream, const uint64_t* keys_in, uint32_t top_shift, uint32_t top_bits,
                           const uint64_t* n_ptr, uint64_t n, uint32_t* zero, uint32_t* counts,
-                          unsigned long long* key_or)
+                          unsigned long long* key_or, uint64_t* bucket_start, unsigned long long* or_out)
 {
     constexpr int I = kSortIptSmall;
     HistPlan hp{};
@@ -1362,17 +1378,43 @@ void launch_top_histogram(hipStream_t stream, const uint64_t* keys_in, uint32_t 
     hp.shift[0] = top_shift;
     hp.mask[0] = (1u << top_bits) - 1u;
     const uint64_t stride = sort_tiles(n, I);
-    TimedLaunch t(kKHistogram, stream);
-    hipLaunchKernelGGL((k_histogram<uint64_t, I>), dim3(histogram_grid<uint64_t, I>(stride)), dim3(kSortThreads), 0,
-                       stream, keys_in, n_ptr, hp, zero, key_or, counts, stride, ChunkPrefix{});
+    {
+        TimedLaunch t(kKHistogram, stream);
+        hipLaunchKernelGGL((k_histogram<uint64_t, I>), dim3(histogram_grid<uint64_t, I>(stride)), dim3(kSortThreads), 0,
+                           stream, keys_in, n_ptr, hp, zero, key_or, counts, stride, ChunkPrefix{});
+    }
+    TimedLaunch t(kKSortScan, stream);
+    hipLaunchKernelGGL(k_digit_starts, dim3(1), dim3(kRadix), 0, stream, zero, 1u << top_bits, n_ptr, bucket_start,
+                       key_or, or_out);
 }
 
-void launch_top_sort(hipStream_t stream, const uint64_t* keys_in, uint32_t* keys_a, uint32_t* keys_b,
-                     uint64_t* keys_out, uint32_t top_shift, uint32_t top_bits, const SortPlan& below,
-                     const uint64_t* n_ptr, uint64_t n, uint32_t* zero, uint32_t* counts, uint64_t* bucket_start,
-                     const SegScratch& sc)
+void launch_top_plan(hipStream_t stream, uint32_t top_bits, const uint64_t* n_ptr, uint64_t n, const uint32_t* zero,
+                     uint32_t* counts, const uint64_t* bucket_start, const SegScratch& sc)
 {
     constexpr int I = kSortIptSmall;
+    const uint32_t buckets = 1u << top_bits;
+    const uint64_t stride = sort_tiles(n, I), tile_count = seg_tile_bound(n, buckets);
+    TimedLaunch t(kKSortScan, stream);
+    if (stride <= kSmallScanTiles)
+        hipLaunchKernelGGL(k_sort_scan<kWave>, dim3(buckets), dim3(kWave), 0, stream, counts, zero, n_ptr, stride,
+                           uint64_t(kSortThreads) * I, nullptr);
+    else
+        hipLaunchKernelGGL(k_sort_scan<kScanThreads>, dim3(buckets), dim3(kScanThreads), 0, stream, counts, zero,
+                           n_ptr, stride, uint64_t(kSortThreads) * I, nullptr);
+    hipLaunchKernelGGL(k_seg_plan_chunks, dim3(1), dim3(kPlanThreads), 0, stream, bucket_start, uint64_t(buckets),
+                       n_ptr, sc.chunk_tiles, sc.ntiles, kSegTile);
+    const uint64_t plan_grid = std::min<uint64_t>((tile_count + 255) / 256, uint64_t(device_cu_count()) * 8);
+    hipLaunchKernelGGL(k_seg_plan_tiles, dim3(int(std::max<uint64_t>(1, plan_grid))), dim3(256), 0, stream,
+                       bucket_start, sc.chunk_tiles, uint64_t(buckets), sc.ntiles, sc.tiles, kSegTile);
+}
+
+template <typename KL>
+void launch_top_passes(hipStream_t stream, const uint64_t* keys_in, KL* first, KL* second, uint64_t* keys_out,
+                       uint32_t top_shift, uint32_t top_bits, const SortPlan& below, const uint64_t* n_ptr, uint64_t n,
+                       uint32_t* counts, const uint64_t* bucket_start, const SegScratch& sc)
+{
+    constexpr int I = kSortIptSmall;
+    constexpr bool kLocal = sizeof(KL) < sizeof(uint64_t);  // keys without their group
     static_assert(kSortThreads == kSegThreads && I == kSegIpt, "one tile size");
     const uint32_t top_mask = (1u << top_bits) - 1u, buckets = top_mask + 1;
     const uint64_t stride = sort_tiles(n, I);
@@ -1384,31 +1426,12 @@ void launch_top_sort(hipStream_t stream, const uint64_t* keys_in, uint32_t* keys
     const uint64_t tile_count = seg_tile_bound(n, buckets);
     const dim3 grid = tile_grid(tile_count);
     {
-        TimedLaunch t(kKSortScan, stream);
-        if (stride <= kSmallScanTiles)
-            hipLaunchKernelGGL(k_sort_scan<kWave>, dim3(buckets), dim3(kWave), 0, stream, counts, zero, n_ptr, stride,
-                               uint64_t(kSortThreads) * I, nullptr);
-        else
-            hipLaunchKernelGGL(k_sort_scan<kScanThreads>, dim3(buckets), dim3(kScanThreads), 0, stream, counts, zero,
-                               n_ptr, stride, uint64_t(kSortThreads) * I, nullptr);
-        hipLaunchKernelGGL(k_digit_starts, dim3(1), dim3(kRadix), 0, stream, zero, buckets, n_ptr, bucket_start);
-    }
-    {
         TimedLaunch t(kKSortScatterTop, stream);
-        hipLaunchKernelGGL((k_sort_scatter<uint64_t, kRankUnstable, I, kSortThreads, uint32_t>), tile_grid(stride),
-                           dim3(kSortThreads), 0, stream, keys_in, keys_a, n_ptr, top_shift, top_mask, counts, stride,
-                           ChunkPrefix{}, 0u, 0u, nullptr, 64u, SegPass{});
+        hipLaunchKernelGGL((k_sort_scatter<uint64_t, kLocal ? kRankUnstable : kRankStable, I, kSortThreads, KL>),
+                           tile_grid(stride), dim3(kSortThreads), 0, stream, keys_in, first, n_ptr, top_shift, top_mask,
+                           counts, stride, ChunkPrefix{}, 0u, 0u, nullptr, 64u, SegPass{});
     }
-    {
-        TimedLaunch t(kKSortScan, stream);
-        hipLaunchKernelGGL(k_seg_plan_chunks, dim3(1), dim3(kPlanThreads), 0, stream, bucket_start, uint64_t(buckets),
-                           n_ptr, sc.chunk_tiles, sc.ntiles, kSegTile);
-        hipLaunchKernelGGL(k_seg_plan_tiles,
-                           dim3(int(std::max<uint64_t>(1, std::min<uint64_t>((tile_count + 255) / 256, uint64_t(cus) * 8)))),
-                           dim3(256), 0, stream, bucket_start, sc.chunk_tiles, uint64_t(buckets), sc.ntiles, sc.tiles,
-                           kSegTile);
-    }
-    uint32_t *src = keys_a, *dst = keys_b;
+    KL *src = first, *dst = second;
     for (int p = 0; p < below.passes; ++p) {
         const uint32_t shift = below.shift[p], mask = (1u << below.bits[p]) - 1u, R = mask + 1;
         const uint64_t col_jobs = uint64_t(buckets) * ((R + kWave - 1) / kWave);
@@ -1419,8 +1442,8 @@ void launch_top_sort(hipStream_t stream, const uint64_t* keys_in, uint32_t* keys
             seg.rows = SegRows{sc.counts, sc.slices, per};
         {
             TimedLaunch t(kKSegCount, stream);
-            hipLaunchKernelGGL((k_seg_count<false, uint32_t, kSegThreads>), grid, dim3(kSegThreads), 0, stream,
-                               static_cast<const uint32_t*>(src), sc.tiles, sc.ntiles, shift, mask, top_shift, seg.rows,
+            hipLaunchKernelGGL((k_seg_count<false, KL, kSegThreads>), grid, dim3(kSegThreads), 0, stream,
+                               static_cast<const KL*>(src), sc.tiles, sc.ntiles, shift, mask, top_shift, seg.rows,
                                nullptr);
         }
         {
@@ -1435,18 +1458,26 @@ void launch_top_sort(hipStream_t stream, const uint64_t* keys_in, uint32_t* keys
         const uint32_t sorted = shift == 0 ? 0u : (1u << shift) - 1u;  // bits the earlier passes sorted
         auto pass = [&](auto mode, auto out) {
             using KO = std::remove_pointer_t<decltype(out)>;
-            hipLaunchKernelGGL((k_sort_scatter<uint32_t, decltype(mode)::value, I, kSortThreads, KO, true>), grid,
+            hipLaunchKernelGGL((k_sort_scatter<KL, decltype(mode)::value, I, kSortThreads, KO, true>), grid,
                                dim3(kSortThreads), 0, stream, src, out, nullptr, shift, mask, nullptr, 0ull,
                                ChunkPrefix{}, 0u, sorted, nullptr, 64u, seg);
         };
-        using Unstable = std::integral_constant<int, kRankUnstable>;
-        using Adaptive = std::integral_constant<int, kRankAdaptive>;
-        if (p == 0 && last) pass(Unstable{}, keys_out);
-        else if (p == 0) pass(Unstable{}, dst);
-        else if (last) pass(Adaptive{}, keys_out);
-        else pass(Adaptive{}, dst);
+        // Keys that are equal on the sorted bits and below are one value unless
+        // they have higher bits: only then must every tile rank stably.
+        using First = std::integral_constant<int, kLocal ? kRankUnstable : kRankStable>;
+        using Later = std::integral_constant<int, kLocal ? kRankAdaptive : kRankStable>;
+        if (p == 0 && last) pass(First{}, keys_out);
+        else if (p == 0) pass(First{}, dst);
+        else if (last) pass(Later{}, keys_out);
+        else pass(Later{}, dst);
         std::swap(src, dst);
     }
 }
+template void launch_top_passes<uint32_t>(hipStream_t, const uint64_t*, uint32_t*, uint32_t*, uint64_t*, uint32_t,
+                                          uint32_t, const SortPlan&, const uint64_t*, uint64_t, uint32_t*,
+                                          const uint64_t*, const SegScratch&);
+template void launch_top_passes<uint64_t>(hipStream_t, const uint64_t*, uint64_t*, uint64_t*, uint64_t*, uint32_t,
+                                          uint32_t, const SortPlan&, const uint64_t*, uint64_t, uint32_t*,
+                                          const uint64_t*, const SegScratch&);
 
 }  // namespace svdag

@@ -27,6 +27,7 @@
 #include "svdag_device.hpp"
 #include "svdag_internal.hpp"
 
+#include <algorithm>
 #include <type_traits>
 
 #pragma clang fp contract(off)
@@ -130,7 +131,7 @@ __global__ __launch_bounds__(kTraceThreads) void k_trace_paths(const uint32_t* _
     __shared__ uint32_t s_index[LEVELS][kTraceThreads];
     __shared__ uint16_t s_masks[LEVELS][kTraceThreads];  // child mask | children to visit (in their order) << 8
     const uint32_t px = blockIdx.x * kTraceTile + (threadIdx.x & 7u);
-    const uint32_t py = blockIdx.y * kTraceTile + (threadIdx.x >> 3);
+    const uint32_t py = (blockIdx.z * gridDim.y + blockIdx.y) * kTraceTile + (threadIdx.x >> 3);
     if (px >= p.width || py >= p.height) return;
     // Entry l of this thread's stack: stack_index[l * kTraceThreads], stack_masks[...].
     uint32_t* const stack_index = &s_index[0][threadIdx.x];
@@ -257,7 +258,11 @@ void launch_trace_paths(hipStream_t s, const uint32_t* words, uint64_t n_words, 
 {
     if (p.width == 0 || p.height == 0) return;
     TimedLaunch t(kKTracePaths, s);
-    const dim3 grid((p.width + kTraceTile - 1) / kTraceTile, (p.height + kTraceTile - 1) / kTraceTile);
+    // Rows of tiles past a grid's 65535 (images of more than 524280 rows) take
+    // its third dimension.
+    constexpr uint32_t kMaxRows = 1u << 15;
+    const uint32_t rows = (p.height + kTraceTile - 1) / kTraceTile;
+    const dim3 grid((p.width + kTraceTile - 1) / kTraceTile, std::min(rows, kMaxRows), (rows + kMaxRows - 1) / kMaxRows);
     auto run = [&](auto levels) {
         hipLaunchKernelGGL((k_trace_paths<decltype(levels)::value>), grid, dim3(kTraceThreads), 0, s, words, n_words,
                            depth, p, paths, colors);

@@ -73,9 +73,16 @@ def space_for(chunk_depth=None):
     return SEG_SPACE if chunk_depth is not None and segmented(chunk_depth) else SPACE
 
 
+def library_setting(space):
+    """The options of a fresh context, by `space`'s names."""
+    return {name: DEFAULTS[name] for name in space}
+
+
 def default_setting(space, chunk_depth=None):
-    """The library's default setting expressed in `space`'s options (the
-    segmented sort's default split of two passes is half its bits)."""
+    """The library's options with the segmented sort's digit spelled out as two
+    passes take it (half the bits).  A fresh context leaves that digit to the
+    library, which groups the keys by cell in one pass where that pays:
+    library_setting."""
     out = {}
     for name in space:
         v = DEFAULTS[name]
@@ -107,8 +114,9 @@ def autotune(ctx, build, fetch, reps=3, space=None, clock=time.perf_counter, chu
     result kept by the callee) under every candidate setting; `fetch()` returns
     the last build's flat layout as a numpy array for the equality check.
     Returns {"best": setting, "best_ms": ms, "table": [(setting, ms), ...],
-    "default_ms": ms of the library's default setting when it is a candidate}
-    and leaves the best setting applied to ctx."""
+    "default_ms": ms of a fresh context's options when they are a candidate}
+    and leaves the best setting applied to ctx.  chunk_depth changes nothing
+    (the defaults no longer depend on it)."""
     table = []
     reference = None
     for setting in candidates(space):
@@ -128,7 +136,7 @@ def autotune(ctx, build, fetch, reps=3, space=None, clock=time.perf_counter, chu
         table.append((setting, best * 1e3))
     best_setting, best_ms = min(table, key=lambda row: row[1])
     apply(ctx, best_setting)
-    want = default_setting(space or SPACE, chunk_depth)
+    want = library_setting(space or SPACE)
     default_ms = next((ms for st, ms in table if st == want), None)
     return {"best": best_setting, "best_ms": best_ms, "table": table, "default_ms": default_ms}
 

@@ -370,7 +370,8 @@ BuildLayout plan_build(uint64_t n, int depth, int key_bytes, uint32_t load_shift
     L.zero_begin = c.off;
     L.counters = c.take(sizeof(BuildCounters));
     L.key_sort_zero = c.take(4 * sort_zero_words(L.key_plan));
-    L.order_zero = c.take(4 * kOrderZeroWords);
+    const bool small_order = order_is_small(L.leaf_slots, L.leaf_bound);
+    if (!small_order) L.order_zero = c.take(4 * kOrderZeroWords);
     L.sketch = c.take(4 * kSketchRegs);
     for (int l = tail_top + 1; l <= depth - 3; ++l) {
         const uint64_t children = l == depth - 3 ? L.leaf_bound : L.level_nodes[l + 1];
@@ -379,7 +380,6 @@ BuildLayout plan_build(uint64_t n, int depth, int key_bytes, uint32_t load_shift
     L.zero_end = c.off;
     for (int l = tail_top + 1; l <= depth - 3; ++l)
         L.extract_parts[l] = c.take(4 * std::min<uint64_t>(kMaxParts, tiles(L.level_slots_of[l], kExtractTileItems)));
-    L.order_split = c.take(8 * kOrderMaxBuckets);
     L.sort_counts = c.take(4 * sort_count_words(n));
     L.tile_counts = c.take(4 * stage_tiles);
     L.tile_offsets = c.take(8 * stage_tiles);
@@ -395,6 +395,7 @@ BuildLayout plan_build(uint64_t n, int depth, int key_bytes, uint32_t load_shift
         L.list_keys[i] = c.take(8 * L.leaf_bound);
         L.list_slots[i] = c.take(4 * L.leaf_bound);
     }
+    if (!small_order) L.order_split = c.take(8 * kOrderMaxBuckets);
     for (int i = 0; i < 2; ++i) {
         L.codes[i] = c.take(8 * L.level_bound);
         L.slots[i] = c.take(4 * L.level_bound);
@@ -1240,9 +1241,11 @@ int merge_device(svdag_context* ctx, const svdag_dag* dags, uint64_t count, int 
     uint64_t o_codes[2];
     o_codes[0] = cv.take(8 * nlive);
     const uint64_t upload_bytes = cv.off;
-    const uint64_t o_order_zero = cv.take(4 * kOrderZeroWords);
-    const uint64_t o_order_split = cv.take(8 * kOrderMaxBuckets);
-    const uint64_t o_parts = cv.take(4 * kMaxParts);
+    const bool small_order = order_is_small(leaf_slots, total_leaves);
+    const uint64_t o_order_zero = small_order ? 0 : cv.take(4 * kOrderZeroWords);
+    const uint64_t o_order_split = small_order ? 0 : cv.take(8 * kOrderMaxBuckets);
+    const uint64_t o_parts = cv.take(4 * std::min<uint64_t>(kMaxParts, std::max(tiles(level_slots, kExtractTileItems),
+                                                                               tiles(nlive, kBuildTileItems))));
     const uint64_t o_leaf_slot_of = cv.take(4 * total_leaves);
     const uint64_t o_leaf_table = cv.take(8 * leaf_slots);
     const uint64_t o_leaf_rank = cv.take(4 * leaf_slots);
@@ -1316,7 +1319,7 @@ int merge_device(svdag_context* ctx, const svdag_dag* dags, uint64_t count, int 
     // The upload buffer must outlive the copy: finish it before returning.
     if (hipStreamSynchronize(st) != hipSuccess) return fail(set_error(SVDAG_ERR_HIP, "merge upload failed"));
 
-    launch_fill_u64(st, reinterpret_cast<uint64_t*>(A + o_order_zero), kOrderZeroWords / 2, 0);
+    if (!small_order) launch_fill_u64(st, reinterpret_cast<uint64_t*>(A + o_order_zero), kOrderZeroWords / 2, 0);
 
     // Leaves: shared hashed table, its order, ranks.
     uint64_t* leaf_table = reinterpret_cast<uint64_t*>(A + o_leaf_table);
@@ -2748,15 +2751,22 @@ int svdag_resident_dag(svdag_resident* r, svdag_dag* out)
     Carver cv;
     const uint64_t o_zero = cv.off;
     const uint64_t o_counters = cv.take(sizeof(BuildCounters));
-    const uint64_t o_order_zero = cv.take(4 * kOrderZeroWords);
+    const bool small_order = order_is_small(r->leaf_slots, L);
+    // The extracts' parts lie over the leaf order's tables and lists: they are
+    // counted after it.
+    Carver parts_cv = cv;
+    uint64_t o_parts[SVDAG_MAX_LEVELS];
+    for (int i = 0; i < r->rlevels; ++i)
+        o_parts[i] = parts_cv.take(4 * std::min<uint64_t>(kMaxParts, tiles(r->slots[i], kExtractTileItems)));
+    const uint64_t o_order_zero = small_order ? cv.off : cv.take(4 * kOrderZeroWords);
     const uint64_t zero_end = cv.off;
-    const uint64_t o_order_split = cv.take(8 * kOrderMaxBuckets);
-    const uint64_t o_parts = cv.take(4 * kMaxParts * r->rlevels);
+    const uint64_t o_order_split = small_order ? 0 : cv.take(8 * kOrderMaxBuckets);
     uint64_t o_lk[2], o_ls[2];
     for (int i = 0; i < 2; ++i) {
         o_lk[i] = cv.take(8 * L);
         o_ls[i] = cv.take(4 * L);
     }
+    cv.off = std::max(cv.off, parts_cv.off);
     const uint64_t o_leaf_rank = cv.take(4 * r->leaf_slots);
     const uint64_t o_rank[2] = {cv.take(4 * max_slots), cv.take(4 * max_slots)};
     const uint64_t o_codes = cv.take(8 * nslots), o_rslots = cv.take(4 * nslots), o_rcount = cv.take(8);
@@ -2789,10 +2799,10 @@ int svdag_resident_dag(svdag_resident* r, svdag_dag* out)
                       r->leaf_slots, L);
     // Resident levels bottom-up, each in ascending hash order with its
     // children's slots turned into ranks of the level below.
-    uint32_t* const level_parts = reinterpret_cast<uint32_t*>(A + o_parts);
+    auto level_parts = [&](int i) { return reinterpret_cast<uint32_t*>(A + o_parts[i]); };
     ExtractCounts occupied{};
     for (int i = 0; i < r->rlevels; ++i)
-        occupied.add(r->tkeys[i], r->d_lg + i, level_parts + uint64_t(kMaxParts) * i, level_extract_parts(r->slots[i]));
+        occupied.add(r->tkeys[i], r->d_lg + i, level_parts(i), level_extract_parts(r->slots[i]));
     launch_extract_count(st, occupied);
     const uint32_t* below = leaf_rank;
     int cur = 0;
@@ -2809,7 +2819,7 @@ int svdag_resident_dag(svdag_resident* r, svdag_dag* out)
         e.out_hashes = reinterpret_cast<uint64_t*>(O + S.hashes[l]);
         e.out_masks = reinterpret_cast<uint8_t*>(O + S.masks[l]);
         e.out_children = reinterpret_cast<uint32_t*>(O + S.children[l]);
-        e.parts = level_parts + uint64_t(kMaxParts) * i;
+        e.parts = level_parts(i);
         e.q_count = &c->uniq[l];
         e.w_count = &c->words[l];
         launch_level_extract(st, e, r->slots[i]);

@@ -848,7 +848,6 @@ constexpr uint32_t kSampleMax = 4096;        // masks sampled at most
 constexpr uint32_t kSamplePerBucket = 8;     // aimed at; fewer past 2^9 buckets
 constexpr uint32_t kSampleScanMax = 1u << 18;  // slots looked at for a small sample
 constexpr uint32_t kOrderMean = 1024;        // masks per bucket aimed at
-constexpr uint32_t kOrderCap = 4096;         // masks one LDS sort takes
 constexpr int kOrderSortThreads = 512;
 constexpr int kOrderIpt = 16;
 constexpr uint32_t kOrderTile = kThreads * kOrderIpt;
@@ -1187,8 +1186,6 @@ __global__ __launch_bounds__(kOrderSortThreads) void k_order_sort(const uint64_t
 // gathered into LDS in any order, sorted, and each slot's rank found by a search.
 // Four launches less three: 1000 keys, whose build is bound by launches (6 us
 // each), 199 -> 163 us with the sketch's two and the layout's count left out too.
-constexpr uint32_t kOrderSmallSlots = 8 * kOrderCap;
-
 __global__ __launch_bounds__(kSampleThreads) void k_order_small(const uint64_t* __restrict__ table_keys,
                                                                 const uint32_t* __restrict__ table_log2,
                                                                 uint64_t* __restrict__ out,
@@ -2355,7 +2352,7 @@ void launch_leaf_insert(hipStream_t s, const uint64_t* lp_mask, const uint64_t* 
 void launch_leaf_order(hipStream_t s, const LeafOrderArgs& a, uint64_t slot_bound, uint64_t leaf_bound)
 {
     TimedLaunch t(kKLeafOrder, s);
-    if (leaf_bound <= kOrderCap && slot_bound <= kOrderSmallSlots) {
+    if (order_is_small(slot_bound, leaf_bound)) {
         hipLaunchKernelGGL(k_order_small, dim3(1), dim3(kSampleThreads), 0, s, a.table_keys, a.table_log2, a.out,
                            a.rank_of_slot, a.count);
         return;

@@ -375,6 +375,13 @@ void launch_leaf_insert(hipStream_t s, const uint64_t* lp_mask, const uint64_t* 
 constexpr uint32_t kOrderMaxLog2 = 11;
 constexpr uint32_t kOrderMaxBuckets = 1u << kOrderMaxLog2;
 constexpr uint64_t kOrderZeroWords = 2 * kOrderMaxBuckets;  // u32 words that must be zero at launch
+// Orders that one workgroup takes whole: they need no split, totals or lists.
+constexpr uint32_t kOrderCap = 4096;  // masks one LDS sort takes
+constexpr uint32_t kOrderSmallSlots = 8 * kOrderCap;
+inline bool order_is_small(uint64_t slot_bound, uint64_t leaf_bound)
+{
+    return leaf_bound <= kOrderCap && slot_bound <= kOrderSmallSlots;
+}
 struct LeafOrderArgs {
     const uint64_t* table_keys;
     const uint32_t* table_log2;

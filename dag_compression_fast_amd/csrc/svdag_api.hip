@@ -2204,33 +2204,42 @@ int svdag_voxelize_triangles(svdag_context* ctx, const double* d_tris, uint64_t 
         return rc;
     }
     const uint64_t ntiles = tiles(units, kVoxUnitTile);
-    Carver unit_cv;
-    const uint64_t o_bits = unit_cv.take(2 * units);
-    const uint64_t o_tcnt = unit_cv.take(4 * ntiles), o_toff = unit_cv.take(8 * ntiles), o_trow = unit_cv.take(8 * (ntiles + 1));
-    void* unit_mem = nullptr;
-    if ((rc = device_alloc(ctx, &unit_mem, unit_cv.off)) != 0) {
-        device_release(ctx, mem);
-        return rc;
-    }
-    char* W = static_cast<char*>(unit_mem);
-    uint16_t* bits = reinterpret_cast<uint16_t*>(W + o_bits);
-    uint32_t* tcounts = reinterpret_cast<uint32_t*>(W + o_tcnt);
-    uint64_t* toffs = reinterpret_cast<uint64_t*>(W + o_toff);
-    uint64_t* trow = reinterpret_cast<uint64_t*>(W + o_trow);
-    launch_vox_count(st, setup, R, cnt + 1, cnt + 2, units, depth, trow, bits, tcounts);
-    launch_scan_counts(st, tcounts, toffs, cnt + 2, kVoxUnitTile, cnt + 3);
-    if (hipMemcpyAsync(h, cnt, sizeof(h), hipMemcpyDeviceToHost, st) != hipSuccess)
-        rc = set_error(SVDAG_ERR_HIP, "count read-back failed");
-    if (rc == 0) rc = finish(ctx, "voxelize (count)");
-    const uint64_t keys = h[3];
     void* out = nullptr;
-    if (rc == 0 && keys) rc = device_alloc(ctx, &out, 8 * keys);
-    if (rc == 0 && keys) {
-        launch_vox_write(st, setup, R, trow, cnt + 2, units, depth, bits, toffs, static_cast<uint64_t*>(out));
-        rc = hipGetLastError() == hipSuccess ? finish(ctx, "voxelize (write)")
-                                             : set_error(SVDAG_ERR_HIP, "voxelizer launch failed");
+    uint64_t keys = 0;
+    // The count pass stores the units' bits for the write pass; where there is
+    // no room for them beside the keys, the write pass makes the tests again.
+    auto unit_stage = [&](bool store) -> int {
+        Carver unit_cv;
+        const uint64_t o_tcnt = unit_cv.take(4 * ntiles), o_toff = unit_cv.take(8 * ntiles), o_trow = unit_cv.take(8 * (ntiles + 1));
+        const uint64_t o_bits = store ? unit_cv.take(2 * units) : 0;
+        void* unit_mem = nullptr;
+        TRY(device_alloc(ctx, &unit_mem, unit_cv.off));
+        char* W = static_cast<char*>(unit_mem);
+        uint16_t* bits = store ? reinterpret_cast<uint16_t*>(W + o_bits) : nullptr;
+        uint32_t* tcounts = reinterpret_cast<uint32_t*>(W + o_tcnt);
+        uint64_t* toffs = reinterpret_cast<uint64_t*>(W + o_toff);
+        uint64_t* trow = reinterpret_cast<uint64_t*>(W + o_trow);
+        launch_vox_count(st, setup, R, cnt + 1, cnt + 2, units, depth, trow, bits, tcounts);
+        launch_scan_counts(st, tcounts, toffs, cnt + 2, kVoxUnitTile, cnt + 3);
+        int result = 0;
+        if (hipMemcpyAsync(h, cnt, sizeof(h), hipMemcpyDeviceToHost, st) != hipSuccess)
+            result = set_error(SVDAG_ERR_HIP, "count read-back failed");
+        if (result == 0) result = finish(ctx, "voxelize (count)");
+        keys = h[3];
+        if (result == 0 && keys) result = device_alloc(ctx, &out, 8 * keys);
+        if (result == 0 && keys) {
+            launch_vox_write(st, setup, R, trow, cnt + 2, units, depth, bits, toffs, static_cast<uint64_t*>(out));
+            result = hipGetLastError() == hipSuccess ? finish(ctx, "voxelize (write)")
+                                                     : set_error(SVDAG_ERR_HIP, "voxelizer launch failed");
+        }
+        device_release(ctx, unit_mem);
+        return result;
+    };
+    rc = unit_stage(true);
+    if (rc == SVDAG_ERR_MEMORY) {
+        pool_trim(ctx);
+        rc = unit_stage(false);
     }
-    device_release(ctx, unit_mem);
     device_release(ctx, mem);
     if (rc != 0) {
         device_release(ctx, out);

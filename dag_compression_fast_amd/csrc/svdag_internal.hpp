@@ -564,8 +564,8 @@ void launch_row_setup(hipStream_t s, const TriSetup* setup, const uint64_t* row_
                       uint64_t* tile_off, uint64_t* total_units_dev, unsigned long long* err);
 // Voxels per tile of kVoxUnitTile units (total_units in all, also in
 // *total_units_dev) into tile_counts, and per unit the voxels that are in
-// (bits).  tile_row (tiles + 1 entries) receives each tile's first row; the
-// write pass reads both.
+// (bits, may be null).  tile_row (tiles + 1 entries) receives each tile's first
+// row; the write pass reads both (with null bits it makes the tests again).
 void launch_vox_count(hipStream_t s, const TriSetup* setup, const VoxRows& rows, const uint64_t* n_rows_dev,
                       const uint64_t* total_units_dev, uint64_t total_units, int depth, uint64_t* tile_row,
                       uint16_t* bits, uint32_t* tile_counts);

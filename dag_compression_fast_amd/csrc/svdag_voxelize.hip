@@ -24,7 +24,8 @@
 //                   per column, keys per tile of 256 units
 //   (scan)          key offsets per tile
 //   k_vox_write     the columns with a bit set again, now only for their keys,
-//                   staged in LDS and written in runs
+//                   staged in LDS and written in runs (no room for the bits: all
+//                   tests again)
 // A unit never leaves its row, so a thread keeps its triangle's edge functions
 // in registers and the wave has no row changes to diverge on.  Threads that
 // walked 8 columns across rows reloaded them at nearly every column (some lane
@@ -293,8 +294,59 @@ __device__ __forceinline__ Unit unit_of(const RowTable& R, const uint64_t* __res
     return Unit{R.tri[r], R.u[r], R.w0[r] + first, int(min(uint32_t(kUnitCols), R.cols[r] - first))};
 }
 
-// bits[unit]: bit 2i + j says that voxel lo + j of the unit's column i is in
-// (lo: column_range); counts[tile] = the tile's bits set.
+// Unit U's voxels: bit 2i + j says that voxel lo + j of its column i is in (lo:
+// column_range).
+__device__ __forceinline__ uint32_t unit_bits(const TriSetup& S, const Unit& U, int64_t side)
+{
+    uint32_t found = 0;
+    const int a = S.a, u = S.u, w = S.w, planes = S.planes;
+    const double cu = double(int64_t(U.u)) + 0.5;
+    // Edge functions of the planes (u, w), (a, u) and (w, a), with the
+    // terms that the row fixes multiplied out.
+    double uu[3], uw[3], ud[3], aa[3], au[3], ad[3], ww[3], wa[3], wd[3];
+#pragma unroll
+    for (int e = 0; e < 3; ++e) {
+        uu[e] = S.ex[u][e] * cu;
+        uw[e] = S.ey[u][e];
+        ud[e] = S.ed[u][e];
+        aa[e] = S.ex[a][e];
+        au[e] = S.ey[a][e] * cu;
+        ad[e] = S.ed[a][e];
+        ww[e] = S.ex[w][e];
+        wa[e] = S.ey[w][e];
+        wd[e] = S.ed[w][e];
+    }
+    const double q = S.nd - pick3(S.n, u) * cu, nw = pick3(S.n, w), na = pick3(S.n, a);
+    const bool plane_a = (planes >> a) & 1, plane_w = (planes >> w) & 1;  // else edge-on there
+#pragma unroll 1
+    for (int i = 0; i < U.cols; ++i) {
+        const double cw = double(int64_t(U.w0) + i) + 0.5;
+        // The dominant projection sees only the column.
+        bool in = true;
+#pragma unroll
+        for (int e = 0; e < 3; ++e) in &= !(uu[e] + uw[e] * cw + ud[e] < 0);
+        if (!in) continue;
+        const double ac = (q - nw * cw) / na;
+        int32_t lo, hi;
+        column_range(ac, side, lo, hi);
+        double wx[3];
+#pragma unroll
+        for (int e = 0; e < 3; ++e) wx[e] = ww[e] * cw;
+        for (int32_t kk = lo; kk <= hi; ++kk) {
+            const double ck = double(kk) + 0.5;
+            bool ok = !(fabs(ck - ac) > 0.5);
+#pragma unroll
+            for (int e = 0; e < 3; ++e) {
+                ok &= !(plane_a && aa[e] * ck + au[e] + ad[e] < 0);
+                ok &= !(plane_w && wx[e] + wa[e] * ck + wd[e] < 0);
+            }
+            found |= uint32_t(ok) << (2 * i + (kk - lo));
+        }
+    }
+    return found;
+}
+
+// counts[tile] = the tile's voxels; with bits, also the units' bits.
 __global__ __launch_bounds__(kVoxThreads) void k_vox_count(const TriSetup* __restrict__ setup, RowTable R,
                                                            const uint64_t* __restrict__ tile_row,
                                                            const uint64_t* __restrict__ total_ptr, int64_t side,
@@ -307,52 +359,8 @@ __global__ __launch_bounds__(kVoxThreads) void k_vox_count(const TriSetup* __res
         const Unit U = unit_of(R, tile_row, total, tile);
         uint32_t found = 0;
         if (U.cols) {
-            const TriSetup& S = setup[U.tri];
-            const int a = S.a, u = S.u, w = S.w, planes = S.planes;
-            const double cu = double(int64_t(U.u)) + 0.5;
-            // Edge functions of the planes (u, w), (a, u) and (w, a), with the
-            // terms that the row fixes multiplied out.
-            double uu[3], uw[3], ud[3], aa[3], au[3], ad[3], ww[3], wa[3], wd[3];
-#pragma unroll
-            for (int e = 0; e < 3; ++e) {
-                uu[e] = S.ex[u][e] * cu;
-                uw[e] = S.ey[u][e];
-                ud[e] = S.ed[u][e];
-                aa[e] = S.ex[a][e];
-                au[e] = S.ey[a][e] * cu;
-                ad[e] = S.ed[a][e];
-                ww[e] = S.ex[w][e];
-                wa[e] = S.ey[w][e];
-                wd[e] = S.ed[w][e];
-            }
-            const double q = S.nd - pick3(S.n, u) * cu, nw = pick3(S.n, w), na = pick3(S.n, a);
-            const bool plane_a = (planes >> a) & 1, plane_w = (planes >> w) & 1;  // else edge-on there
-#pragma unroll 1
-            for (int i = 0; i < U.cols; ++i) {
-                const double cw = double(int64_t(U.w0) + i) + 0.5;
-                // The dominant projection sees only the column.
-                bool in = true;
-#pragma unroll
-                for (int e = 0; e < 3; ++e) in &= !(uu[e] + uw[e] * cw + ud[e] < 0);
-                if (!in) continue;
-                const double ac = (q - nw * cw) / na;
-                int32_t lo, hi;
-                column_range(ac, side, lo, hi);
-                double wx[3];
-#pragma unroll
-                for (int e = 0; e < 3; ++e) wx[e] = ww[e] * cw;
-                for (int32_t kk = lo; kk <= hi; ++kk) {
-                    const double ck = double(kk) + 0.5;
-                    bool ok = !(fabs(ck - ac) > 0.5);
-#pragma unroll
-                    for (int e = 0; e < 3; ++e) {
-                        ok &= !(plane_a && aa[e] * ck + au[e] + ad[e] < 0);
-                        ok &= !(plane_w && wx[e] + wa[e] * ck + wd[e] < 0);
-                    }
-                    found |= uint32_t(ok) << (2 * i + (kk - lo));
-                }
-            }
-            bits[tile * kVoxThreads + threadIdx.x] = uint16_t(found);
+            found = unit_bits(setup[U.tri], U, side);
+            if (bits) bits[tile * kVoxThreads + threadIdx.x] = uint16_t(found);
         }
         const uint64_t sum = block_reduce_sum<kVoxThreads>(uint64_t(__popc(found)), s_red);
         if (threadIdx.x == 0) counts[tile] = uint32_t(sum);
@@ -360,6 +368,8 @@ __global__ __launch_bounds__(kVoxThreads) void k_vox_count(const TriSetup* __res
 }
 
 // The keys of the voxels whose bit is set, in unit, column and voxel order.
+// Without STORED bits (no memory was left for them) the tests are made again.
+template <bool STORED>
 __global__ __launch_bounds__(kVoxThreads) void k_vox_write(const TriSetup* __restrict__ setup, RowTable R,
                                                            const uint64_t* __restrict__ tile_row,
                                                            const uint64_t* __restrict__ total_ptr, int64_t side,
@@ -374,7 +384,13 @@ __global__ __launch_bounds__(kVoxThreads) void k_vox_write(const TriSetup* __res
     const uint64_t ntiles = (total + kVoxThreads - 1) / kVoxThreads;
     for (uint64_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
         const uint64_t g = tile * kVoxThreads + threadIdx.x;
-        uint32_t left = g < total ? bits[g] : 0u;
+        uint32_t left = 0;
+        if constexpr (STORED) {
+            if (g < total) left = bits[g];
+        } else {
+            const Unit U = unit_of(R, tile_row, total, tile);
+            if (U.cols) left = unit_bits(setup[U.tri], U, side);
+        }
         uint32_t tile_keys;
         uint32_t o = block_exclusive_scan<kVoxThreads>(uint32_t(__popc(left)), s_scan, tile_keys);
         if (left) {
@@ -452,8 +468,12 @@ void launch_vox_write(hipStream_t s, const TriSetup* setup, const VoxRows& rows,
     TimedLaunch t(kKVoxWrite, s);
     const uint64_t tiles = (total_units + kVoxThreads - 1) / kVoxThreads;
     const RowTable R{rows.tri, rows.u, rows.w0, rows.cols, rows.unit_off};
-    hipLaunchKernelGGL(k_vox_write, dim3(resident_grid(k_vox_write, kVoxThreads, tiles)), dim3(kVoxThreads), 0, s, setup,
-                       R, tile_row, total_units_dev, int64_t(1) << depth, bits, tile_offsets, keys);
+    auto run = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(resident_grid(kernel, kVoxThreads, tiles)), dim3(kVoxThreads), 0, s, setup, R,
+                           tile_row, total_units_dev, int64_t(1) << depth, bits, tile_offsets, keys);
+    };
+    if (bits) run(k_vox_write<true>);
+    else run(k_vox_write<false>);
 }
 
 }  // namespace svdag

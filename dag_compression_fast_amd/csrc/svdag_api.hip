@@ -1028,10 +1028,10 @@ int build(svdag_context* ctx, const K* d_keys, uint64_t n, int depth, svdag_dag*
         ls = ctx->side;
         forked = true;
     }
-    // The sort's launches are issued after the first level builds' (below):
-    // the side stream already waits for the leaf dedup (fork_ev), and issuing
-    // builds first keeps the main stream busy while the host issues the sort's
-    // two dozen small launches.
+    // Its four launches (one for small builds) are issued after the first level
+    // builds' (below); the side stream already waits for the leaf dedup
+    // (fork_ev).  Issuing them here measured the same (17M to 70M keys within
+    // 0.5%, 150M 1% less).
     bool ordered = false;
     auto order_leaves = [&]() -> int {
         if (ordered) return 0;
@@ -1096,10 +1096,8 @@ int build(svdag_context* ctx, const K* d_keys, uint64_t n, int depth, svdag_dag*
         if (ctx->check_collisions)
             launch_level_check(st, a.parent_slots, a.table_rep, a.parent_masks, a.parent_children, &c->pre[l],
                                &c->collisions, L.level_nodes[l]);
-        // The unique-leaf sort's two dozen small launches go out once the two
-        // largest level builds are queued: the main stream then has enough
-        // work not to wait while the host issues them, and the sort starts
-        // early enough on the side stream to end beside the builds.
+        // The leaf order goes out once the two largest level builds are queued:
+        // early enough to end beside the builds.
         if (l == std::max(depth - 4, tail_top + 1)) TRY(order_leaves());
     }
     // Stage markers (the completion deadline names the first stage not done)

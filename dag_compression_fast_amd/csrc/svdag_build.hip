@@ -1,9 +1,11 @@
 // svdag_build.hip -- gfx950 kernels of the bottom-up DAG build.
 //
 // Reference path (src/DAGCompression.cu):
-//   SelectUnique + leaf ReduceByKey  :1035-1068  -> k_leaf_reduce / k_leaf_compact
-//       (one pass over the keys grouped by code >> 15: duplicates OR into the
-//       same 4^3 mask, so no separate unique step is needed)
+//   SelectUnique + leaf ReduceByKey  :1035-1068  -> k_cell_reduce /
+//       k_cell_compact (keys grouped by 64^3 cell, code >> 18, with known cell
+//       starts) or k_leaf_reduce / k_leaf_compact (keys grouped by code >> 15):
+//       one pass over the keys; duplicates OR into the same 4^3 mask, so no
+//       separate unique step is needed
 //   SortLevel(Leaves)               :1070-1071  -> k_table_clear / k_leaf_insert
 //       (hash table keyed by the mask) + a sample sort of its occupied slots
 //       (k_leaf_sample, k_order_*)

@@ -1,8 +1,11 @@
-// svdag_sort.hip -- LSD radix sort for gfx950 (wave64), reduce-then-scan.
+// svdag_sort.hip -- radix sorts for gfx950 (wave64), reduce-then-scan.
 //
 // Replaces the CUB DeviceRadixSort calls of the reference (SortKeys,
-// src/DAGCompression.cu:336-357).  Digits are up to 9
-// bits wide.  No workgroup ever waits on another one: every pass is
+// src/DAGCompression.cu:336-357): an LSD sort (launch_sort), sorts inside
+// segments (launch_segmented_sort), top digit first with the rest sorted inside
+// each digit's keys (launch_top_digit_sort, launch_top_passes), and one pass
+// that groups by a digit (launch_cell_sort).  Digits are up to 9 bits wide.  No
+// workgroup ever waits on another one: every LSD pass is
 //   k_sort_count    tile t (a fixed range of 4096 keys) -> per-digit counts
 //   k_sort_scan     one workgroup per digit scans that digit's row of tile
 //                   counts and adds the digit's global start (from the pass's
@@ -776,7 +779,9 @@ namespace {
 // spreads a 4096-key tile over 512 digits in runs of 8 keys, 32 bytes: 67M keys
 // a chunk took 2170 us of scatter with 256 threads, 1515 with 1024 (1630 with
 // 512); buckets of 140k keys and 64 digits 105 and 162 us, chunks of 330k keys
-// and 512 digits 436 and 460.
+// and 512 digits 436 and 460.  Between, whole builds of 8 chunks take the same
+// (0.6M to 8M keys a chunk within 0.5%; 16M 4765 us wide, 4790 not; 32M 6160 and
+// 6380), so the line may lie anywhere there.
 constexpr int kSegThreads = 256;
 constexpr int kSegWideThreads = 1024;
 constexpr uint64_t kSegWideKeys = 1ull << 22;

@@ -139,9 +139,9 @@ int svdag_create_dag(svdag_context* ctx, const uint64_t* d_keys, uint64_t n,
  * process ends) and its result in the caller's device buffer d_storage, of
  * storage_bytes >= svdag_result_bytes(n, depth).  Calls no hipMalloc, hipFree
  * or allocating routine.  A build needing more scratch than the array holds
- * (svdag_scratch_bytes(n, depth, 8) at load shift 1; about 5M keys at depth 9,
- * 1M at depth 10, 900k at depth 11, 650k at depth 12) or more storage than given fails with SVDAG_ERR_MEMORY
- * before any device work.  `out` points into d_storage and owns nothing
+ * (svdag_scratch_bytes(n, depth, 8) at load shift 1; about 5.6M keys at depth 9,
+ * 1.0M at depth 10, 950k at depth 11, 660k at depth 12) or more storage than
+ * given fails with SVDAG_ERR_MEMORY before any device work.  `out` points into d_storage and owns nothing
  * (out->storage is NULL; svdag_free_dag releases nothing).  Every call on a
  * GPU shares that GPU's array, which keeps the last call's contents (each call
  * clears what must start at zero): calls that overlap on one GPU, from any
@@ -209,7 +209,8 @@ int svdag_create_final_dag(svdag_context* ctx, const svdag_dag* dag,
                            uint32_t** d_words, uint64_t* n_words);
 
 /* Copies between host (FCpuDag-like) and device residency.  `out` is a new
- * DAG owned by the caller. */
+ * DAG owned by the caller.  svdag_dag_to_host leaves an array that the DAG does
+ * not have (a null pointer) null; on an error `out` holds nothing. */
 int svdag_dag_to_host(svdag_context* ctx, const svdag_dag* dag, svdag_dag* out);
 int svdag_dag_to_device(svdag_context* ctx, const svdag_dag* dag, svdag_dag* out);
 

@@ -431,7 +431,7 @@ __global__ __launch_bounds__(kThreads) void k_leaf_compact(const uint64_t* __res
 // twice the bank cycles).  Bound by the keys' read and the LDS atomics where
 // cells are full (512^3 noise, 67M keys: 304 -> 56 us, with 268 us of sort
 // saved; 2048^3 triangles 153 -> 125), by the two barriers and the table pass a
-// cell where they are not (512 chunks, 645 keys a cell: 364 -> 374 us, with 640
+// cell where they are not (512 chunks, 645 keys a cell: 364 -> 390 us, with 640
 // us of sort saved; 690 before the next cell's keys were loaded ahead).  Full
 // rounds of keys go without their guards (138 -> 125 us of the triangles);
 // registers are held to 64 for the fourth workgroup per CU, which gains 26 us of
